@@ -8,6 +8,7 @@ import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "lib", "libmixed_gemv_amd.so")
+PY_CALLS_PATH = os.path.join(_PKG_DIR, "lib", "py_calls.so")
 
 _c = ctypes
 _u16p = _c.c_void_p  # fp16 bit patterns; passed as raw addresses (host numpy or device pointers)
@@ -97,6 +98,20 @@ def lib():
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def py_calls():
+    """The extension module that unpacks torch tensors and calls the library (csrc/py_calls.cpp); raises if it is
+    missing.  The library is loaded in front of it, so that the two share one copy."""
+    import importlib.machinery
+    import importlib.util
+    lib()
+    if not os.path.exists(PY_CALLS_PATH):
+        raise ImportError(f"{PY_CALLS_PATH} not found: not built (run `python -m mixed_gemv_amd.build`)")
+    loader = importlib.machinery.ExtensionFileLoader("py_calls", PY_CALLS_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("py_calls", loader))
+    loader.exec_module(module)
+    return module
 
 
 def check(status, where):

@@ -37,18 +37,22 @@ def _host_ptr(a):
     return ctypes.c_void_p(a.ctypes.data)
 
 
-def _dev_ptr(t):
+def _dev_address(t):
     if t is None:
-        return ctypes.c_void_p(0)
+        return 0
     if isinstance(t, int):
-        return ctypes.c_void_p(t)
+        return t
     if hasattr(t, "data_ptr"):
         if not t.is_cuda:
             raise ValueError("device entry points need GPU tensors; there is no CPU path")
         if not t.is_contiguous():
             raise ValueError("tensors must be contiguous")
-        return ctypes.c_void_p(t.data_ptr())
+        return t.data_ptr()
     raise TypeError(f"cannot take a device address from {type(t)!r}")
+
+
+def _dev_ptr(t):
+    return ctypes.c_void_p(_dev_address(t))
 
 
 def _is_bf16(element, probe):
@@ -62,13 +66,27 @@ def _is_bf16(element, probe):
     return element == "bf16"
 
 
-def _stream_ptr(stream):
+def _stream_address(stream):
     if stream is None:
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
-        return ctypes.c_void_p(stream)
-    return ctypes.c_void_p(stream.cuda_stream)
+        return stream
+    return stream.cuda_stream
+
+
+def _stream_ptr(stream):
+    return ctypes.c_void_p(_stream_address(stream))
+
+
+_calls = None  # the device entry points as CPython calls (csrc/py_calls.cpp), loaded with the first of them
+
+
+def _native_calls():
+    global _calls
+    if _calls is None:
+        _calls = _lib.py_calls()
+    return _calls
 
 
 def _shape_arg(shape):
@@ -229,20 +247,10 @@ def device_gemv(ptr_A, ptr_B, ptr_scale, ptr_zero_point, ptr_C, ptr_D, B, M, N, 
     ptr_zero_point the folded fp16 term -z*s, ptr_C an optional fp16 bias.  The quant mode is
     a run-time argument (a compile-time constant in the reference).  element: "f16" / "bf16" for
     every 16-bit operand; None takes it from ptr_B when that is a torch tensor, else fp16."""
-    bf16 = _is_bf16(element, ptr_B)
-    gemv = _lib.lib().mgemv_gemv_bf16 if bf16 else _lib.lib().mgemv_gemv
-    gemv_batched = _lib.lib().mgemv_gemv_batched_bf16 if bf16 else _lib.lib().mgemv_gemv_batched
-    if B == 1 and not batch_strides:
-        st = gemv(_dev_ptr(ptr_A), _dev_ptr(ptr_B), _dev_ptr(ptr_scale), _dev_ptr(ptr_zero_point),
-                                   _dev_ptr(ptr_C), _dev_ptr(ptr_D), int(M), int(N), int(K), int(group_size),
-                                   int(quant_op), int(weight_bits), _stream_ptr(stream))
-    else:
-        sa, sb, ss, sc, sd = batch_strides or (0, 0, 0, 0, 0)
-        st = gemv_batched(_dev_ptr(ptr_A), _dev_ptr(ptr_B), _dev_ptr(ptr_scale),
-                          _dev_ptr(ptr_zero_point), _dev_ptr(ptr_C), _dev_ptr(ptr_D), int(B), int(M),
-                          int(N), int(K), int(group_size), int(quant_op), int(weight_bits),
-                          int(sa), int(sb), int(ss), int(sc), int(sd), _stream_ptr(stream))
-    _lib.check(st, "device_gemv")
+    st = (_calls or _native_calls()).gemv(ptr_A, ptr_B, ptr_scale, ptr_zero_point, ptr_C, ptr_D, B, M, N, K, group_size,
+                                          quant_op, weight_bits, stream, batch_strides, element)
+    if st:
+        raise _lib.MixedGemvError(st, "device_gemv")
 
 
 def device_gemv_routed(ptr_A, ptr_B, ptr_scale, ptr_zero_point, ptr_C, ptr_D, route, stack_entries, B, M, N, K,
@@ -253,12 +261,11 @@ def device_gemv_routed(ptr_A, ptr_B, ptr_scale, ptr_zero_point, ptr_C, ptr_D, ro
     stack of stack_entries matrices; x and y are stepped by b.  batch_strides = (weights in bytes, x,
     scale, bias, y) as in device_gemv; a stride of 0 for x gives every problem the same activations.
     The reference steps through a stack at a fixed stride only (gemv/kernel/mixed_gemv.h:140-149)."""
-    fn = _lib.lib().mgemv_gemv_routed_bf16 if _is_bf16(element, ptr_B) else _lib.lib().mgemv_gemv_routed
-    sa, sb, ss, sc, sd = batch_strides
-    st = fn(_dev_ptr(ptr_A), _dev_ptr(ptr_B), _dev_ptr(ptr_scale), _dev_ptr(ptr_zero_point), _dev_ptr(ptr_C),
-            _dev_ptr(ptr_D), _dev_ptr(route), int(stack_entries), int(B), int(M), int(N), int(K), int(group_size),
-            int(quant_op), int(weight_bits), int(sa), int(sb), int(ss), int(sc), int(sd), _stream_ptr(stream))
-    _lib.check(st, "device_gemv_routed")
+    st = (_calls or _native_calls()).gemv_routed(ptr_A, ptr_B, ptr_scale, ptr_zero_point, ptr_C, ptr_D, route,
+                                                 stack_entries, B, M, N, K, group_size, batch_strides, quant_op,
+                                                 weight_bits, stream, element)
+    if st:
+        raise _lib.MixedGemvError(st, "device_gemv_routed")
 
 
 class GemvAdaptor:
@@ -305,11 +312,10 @@ def dequantize(ptr_A, ptr_scale, ptr_zero_point, ptr_out, M, K, group_size,
                quant_op=WeightOnlyQuantOp.FINEGRAINED_SCALE_AND_ZEROS, weight_bits=4, stream=None, element=None):
     """Writes dequantised weights [M][K] (fp16, or bf16 with element="bf16" / a torch.bfloat16 scale
     tensor) with the kernels' own converter + dequantiser."""
-    fn = _lib.lib().mgemv_dequantize_bf16 if _is_bf16(element, ptr_scale) else _lib.lib().mgemv_dequantize
-    st = fn(_dev_ptr(ptr_A), _dev_ptr(ptr_scale), _dev_ptr(ptr_zero_point), _dev_ptr(ptr_out),
-                                     int(M), int(K), int(group_size), int(quant_op), int(weight_bits),
-                                     _stream_ptr(stream))
-    _lib.check(st, "dequantize")
+    st = (_calls or _native_calls()).dequantize(ptr_A, ptr_scale, ptr_zero_point, ptr_out, M, K, group_size, quant_op,
+                                                weight_bits, stream, element)
+    if st:
+        raise _lib.MixedGemvError(st, "dequantize")
 
 
 def set_launch_override(split_k_waves=0, tiles_per_workgroup=0, tiles_per_wave=0, max_workgroups=0):

@@ -11,6 +11,8 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")   # objects and the compiler's intermediate files (the device assembly among them)
 LIB_PATH = os.path.join(LIB_DIR, "libmixed_gemv_amd.so")
+PY_CALLS_SOURCE = "py_calls.cpp"         # CPython extension module over the library (torch tensors in, C-ABI calls out)
+PY_CALLS_PATH = os.path.join(LIB_DIR, "py_calls.so")
 LINT_REPORT = os.path.join(LIB_DIR, "isa_lint.json")
 MIN_DOT_INSTRUCTIONS = 10000
 
@@ -93,6 +95,27 @@ def write_default_plans(path):
     return len(lines)
 
 
+def build_py_calls(verbose=True):
+    """csrc/py_calls.cpp -> lib/py_calls.so.  PyTorch's libraries are named without a path: the process that loads the
+    module has them already."""
+    import sysconfig
+    import torch
+    torch_dir = os.path.dirname(torch.__file__)
+    torch_include = os.path.join(torch_dir, "include")
+    rocm_include = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc()))), "include")
+    cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(REPO_DIR, "include"), "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", torch_include, "-isystem", os.path.join(torch_include, "torch", "csrc", "api", "include"),
+           "-isystem", rocm_include, os.path.join(CSRC, PY_CALLS_SOURCE), "-o", PY_CALLS_PATH,
+           "-L", LIB_DIR, "-lmixed_gemv_amd", "-L", os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return PY_CALLS_PATH
+
+
 def build_library(verbose=True, extra_flags=(), jobs=None, lint=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     write_default_plans(os.path.join(OBJ_DIR, "default_plans.inc"))
@@ -115,6 +138,7 @@ def build_library(verbose=True, extra_flags=(), jobs=None, lint=True):
     subprocess.run(cmd, check=True)
     if lint:
         lint_device_code(verbose)
+    build_py_calls(verbose)
     return LIB_PATH
 
 
