@@ -8,6 +8,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "kernel_common.h"
@@ -18,95 +19,147 @@ struct DequantParams {
   const uint8_t* weights;
   const half_t* scale;
   const half_t* zero_add;
-  int n_out, k, group_size, tiles, ksteps, flags;
+  int n_out, k, group_size, num_groups, tiles, ksteps, flags;
 };
 
-// One wave per unit; writes the dequantised weights of its 16 rows x kStepK columns with the
-// same converters, and the same wave-uniform choice between them, as the GEMV kernels.
-template <int BITS, int QOP, int ACT>
-__global__ void __launch_bounds__(256) dequantize_kernel(const DequantParams p, half_t* __restrict__ out) {
-  using G = Geometry<BITS>;
+// The scales (or zeros) of the 16 rows of a tile in one group: 32 neighbouring bytes of the table, row 2i in the low and
+// row 2i + 1 in the high half of word i.  Rows past the table read as zero.
+struct TileScales {
+  uint32_t v[kTileRows / 2];
+};
+__device__ __forceinline__ TileScales load_tile_scales(__amdgpu_buffer_rsrc_t table, int byte_offset) {
+  TileScales t;
+#pragma unroll
+  for (int i = 0; i < kTileRows / 2; i += 4) {
+    const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(table, byte_offset + i * 4, 0, kCacheDefault);
+    t.v[i] = q[0]; t.v[i + 1] = q[1]; t.v[i + 2] = q[2]; t.v[i + 3] = q[3];
+  }
+  return t;
+}
+
+// True when all 16 scales permit the short (fp16, int4) resp. fused (bf16) dequantiser, in every lane.
+template <int ACT>
+__device__ __forceinline__ bool tile_scales_permit_short_form(const TileScales& s) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  constexpr uint16_t kFirst = ACT == kActBf16 ? 0x0d80 : 0x0001, kPast = ACT == kActBf16 ? 0x7b00 : 0x2800;
+  u16x2 most = u16x2{0, 0};
+#pragma unroll
+  for (int i = 0; i < kTileRows / 2; ++i)
+    most = __builtin_elementwise_max(most, (u16x2)(__builtin_bit_cast(u16x2, s.v[i]) - u16x2{kFirst, kFirst}));
+  return __builtin_amdgcn_ballot_w64((most[0] > most[1] ? most[0] : most[1]) >= kPast - kFirst) == 0;
+}
+
+// Eight consecutive weights of one row (one word of int4, two of int8) to 16 bytes, with the converters of the GEMV kernels.
+template <int BITS, int QOP, int ACT, bool SHORT>
+__device__ __forceinline__ u32x4 dequantize_eight(const uint32_t (&w)[8 * BITS / 32], const ConvertRegs& c, uint32_t s_bits,
+                                                  uint32_t z_bits) {
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
+  u32x4 out;
+  if constexpr (ACT == kActBf16) {
+    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? z_bits : 0u);
+    if constexpr (BITS == 4) {
+      uint32_t d[4];
+      dequant_int4_word_bf16<kHasZero, SHORT>(w[0], c, bs, d);
+      out = u32x4{d[0], d[1], d[2], d[3]};
+    } else {
+      uint32_t d0[2], d1[2];
+      dequant_int8_word_bf16<kHasZero, SHORT>(w[0], bs, d0);
+      dequant_int8_word_bf16<kHasZero, SHORT>(w[1], bs, d1);
+      out = u32x4{d0[0], d0[1], d1[0], d1[1]};
+    }
+  } else {
+    const half2_t s2 = splat_low(s_bits), z2 = kHasZero ? splat_low(z_bits) : half2_t{};
+    half2_t d[4];
+    if constexpr (BITS == 4 && SHORT) {
+      dequant_int4_word_short<kHasZero>(w[0], c, make_short_form_scale(s2), z2, d);
+    } else {
+      half2_t q[4];
+      if constexpr (BITS == 4) {
+        convert_int4_word(w[0], c, q);
+      } else {
+        half2_t q0[2], q1[2];
+        convert_int8_word(w[0], c, q0);
+        convert_int8_word(w[1], c, q1);
+        q[0] = q0[0]; q[1] = q0[1]; q[2] = q1[0]; q[3] = q1[1];
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h) d[h] = dequant_pair<kHasZero>(q[h], s2, z2);
+    }
+    out = u32x4{as_u32(d[0]), as_u32(d[1]), as_u32(d[2]), as_u32(d[3])};
+  }
+  return out;
+}
+
+// One wave per unit; writes the dequantised weights of its 16 rows x kStepK columns with the same converters, and the
+// same wave-uniform choice between them, as the GEMV kernels.
+// Bound by its stores (four bytes out for one byte of int4 in), so the lanes are dealt out along the OUTPUT: a store
+// instruction of the wave writes one whole row of the unit (int4: 64 lanes x 16 bytes = 512 k) or two (int8), contiguous,
+// and each lane picks the one or two weight words it needs for that out of the 16-byte chunks of the tile layout (the four
+// or eight lanes of a chunk share its cache line, and the 16 rows of a unit read each of its lines 8 times out of the L1).
+// With a lane per row, as the GEMV kernels have it, every store instruction scatters 64 pieces of 4 bytes.
+constexpr int kDequantWaves = 4;
+template <int BITS, int QOP, int ACT>
+__global__ void __launch_bounds__(kWave * kDequantWaves) dequantize_kernel(const DequantParams p, half_t* __restrict__ out) {
+  using G = Geometry<BITS>;
+  constexpr int kWords = 8 * BITS / 32;                // weight words of eight weights: 1 | 2
+  constexpr int kLanesPerRow = G::kStepK / 8;          // 64 | 32
+  constexpr int kRowsPerStore = kWave / kLanesPerRow;  // 1 | 2
+  typedef u32x4 __attribute__((aligned(4))) u32x4_any;  // the caller's rows are 4-byte aligned
   const int lane = threadIdx.x % kWave;
-  const long long unit = (long long)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  const long long unit = (long long)blockIdx.x * kDequantWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (unit >= (long long)p.tiles * p.ksteps) return;  // whole waves only
   const int tile = (int)(unit / p.ksteps), kstep = (int)(unit % p.ksteps);
-  const int row = tile * kTileRows + lane % kTileRows;
-  const int k_run = kstep * G::kStepK + (lane / kTileRows) * G::kRunK;
-  const ConvertRegs c = make_convert_regs();
-  const uint8_t* base = p.weights + (size_t)unit * kUnitBytes + (size_t)lane * kChunkBytes;
-  const int row_c = row < p.n_out ? row : p.n_out - 1;
-  uint32_t s_bits[kBlocksPerUnit];
-  half_t s[kBlocksPerUnit], z[kBlocksPerUnit];
+  const int piece = lane % kLanesPerRow, sub_row = lane / kLanesPerRow;  // eight weights of a row; which row of the store
+  const int k0 = kstep * G::kStepK + piece * 8;
+  const int row0 = tile * kTileRows;
+
+  const int slice = piece * 8 / G::kRunK, block = piece * 8 % G::kRunK / G::kChunkK, word = piece % (G::kChunkK / 8) * kWords;
+  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(p.weights + (size_t)unit * kUnitBytes, kUnitBytes);
+  const int w_offset = block * kBlockBytes + (slice * kTileRows + sub_row) * kChunkBytes + word * 4;
+  uint32_t w[kTileRows / kRowsPerStore][kWords];
 #pragma unroll
-  for (int i = 0; i < kBlocksPerUnit; ++i) {
-    z[i] = (half_t)0.0f;
-    if constexpr (QOP == MGEMV_PER_COLUMN_SCALE_ONLY) {
-      s[i] = p.scale[row_c];
+  for (int i = 0; i < kTileRows / kRowsPerStore; ++i) {
+    const int off = w_offset + i * kRowsPerStore * kChunkBytes;
+    if constexpr (BITS == 4) {
+      w[i][0] = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, off, 0, kCacheDefault);
     } else {
-      Problem geo{};
-      geo.k = p.k;
-      geo.group_size = p.group_size;
-      const int idx = group_of(geo, k_run + i * G::kChunkK) * p.n_out + row_c;
-      s[i] = p.scale[idx];
-      if constexpr (kHasZero) z[i] = p.zero_add[idx];
-    }
-    s_bits[i] = (uint32_t)__builtin_bit_cast(uint16_t, s[i]);
-  }
-  const bool take_short = (BITS == 4 || ACT == kActBf16) && (p.flags & kExactIntegerFormOnly) == 0 &&
-                          wave_scales_permit_short_form<ACT>(s_bits);
-#pragma unroll
-  for (int i = 0; i < kBlocksPerUnit; ++i) {
-    const int k0 = k_run + i * G::kChunkK;
-    const u32x4 w = *reinterpret_cast<const u32x4*>(base + i * kBlockBytes);
-    const half2_t s2 = splat(s[i]), z2 = splat(z[i]);
-    if (row >= p.n_out || k0 >= p.k) continue;
-    half_t* dst = out + (size_t)row * (size_t)p.k + k0;
-    if constexpr (ACT == kActBf16) {
-      constexpr int kPairs = BITS == 4 ? 4 : 2;
-      const uint32_t z_bits = (uint32_t)__builtin_bit_cast(uint16_t, z[i]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (k0 + j * G::kWordK >= p.k) continue;  // k is a multiple of 8: whole words
-        uint32_t d[kPairs];
-        if (take_short) {
-          const Bf16Scale bs = make_bf16_scale<BITS, true>(s_bits[i], z_bits);
-          if constexpr (BITS == 4) dequant_int4_word_bf16<kHasZero, true>(w[j], c, bs, d);
-          else dequant_int8_word_bf16<kHasZero, true>(w[j], bs, d);
-        } else {
-          const Bf16Scale bs = make_bf16_scale<BITS, false>(s_bits[i], z_bits);
-          if constexpr (BITS == 4) dequant_int4_word_bf16<kHasZero, false>(w[j], c, bs, d);
-          else dequant_int8_word_bf16<kHasZero, false>(w[j], bs, d);
-        }
-#pragma unroll
-        for (int h = 0; h < kPairs; ++h) *reinterpret_cast<uint32_t*>(dst + j * 2 * kPairs + h * 2) = d[h];
-      }
-      continue;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (k0 + j * G::kWordK >= p.k) continue;  // k is a multiple of 8: whole words
-      if constexpr (BITS == 4) {
-        half2_t d[4];
-        if (take_short) {
-          dequant_int4_word_short<kHasZero>(w[j], c, make_short_form_scale(s2), z2, d);
-        } else {
-          half2_t q[4];
-          convert_int4_word(w[j], c, q);
-#pragma unroll
-          for (int h = 0; h < 4; ++h) d[h] = dequant_pair<kHasZero>(q[h], s2, z2);
-        }
-#pragma unroll
-        for (int h = 0; h < 4; ++h) *reinterpret_cast<half2_t*>(dst + j * 8 + h * 2) = d[h];
-      } else {
-        half2_t q[2];
-        convert_int8_word(w[j], c, q);
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          *reinterpret_cast<half2_t*>(dst + j * 4 + h * 2) = dequant_pair<kHasZero>(q[h], s2, z2);
-      }
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(w_rsrc, off, 0, kCacheDefault);
+      w[i][0] = v[0]; w[i][1] = v[1];
     }
   }
+  int group = 0;
+  if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) {
+    Problem geo{};
+    geo.k = p.k;
+    geo.group_size = p.group_size;
+    group = group_of(geo, k0);
+  }
+  const int table_offset = (group * p.n_out + row0) * 2;
+  const uint32_t table_bytes = (uint32_t)p.num_groups * (uint32_t)p.n_out * 2u;
+  const TileScales s = load_tile_scales(make_rsrc(p.scale, table_bytes), table_offset);
+  TileScales z{};
+  if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) z = load_tile_scales(make_rsrc(p.zero_add, table_bytes), table_offset);
+
+  const ConvertRegs c = make_convert_regs();
+  half_t* const dst = out + (size_t)(row0 + sub_row) * (size_t)p.k + k0;
+  const bool inside = k0 < p.k;  // k is a multiple of 8
+  auto write_rows = [&](auto short_form) {
+    constexpr bool kShort = decltype(short_form)::value;
+#pragma unroll
+    for (int i = 0; i < kTileRows / kRowsPerStore; ++i) {
+      const int row = i * kRowsPerStore + sub_row;
+      const int shift = kRowsPerStore == 1 ? 16 * (i & 1) : 16 * sub_row;
+      const int entry = kRowsPerStore == 1 ? i / 2 : i;
+      const u32x4 d = dequantize_eight<BITS, QOP, ACT, kShort>(w[i], c, (s.v[entry] >> shift) & 0xffffu, (z.v[entry] >> shift) & 0xffffu);
+      if (inside && row0 + row < p.n_out)
+        __builtin_nontemporal_store(d, reinterpret_cast<u32x4_any*>(dst + (size_t)(i * kRowsPerStore) * (size_t)p.k));
+    }
+  };
+  // rows past n_out read the next group's scales or zeros: they may only cost the short form
+  if ((BITS == 4 || ACT == kActBf16) && (p.flags & kExactIntegerFormOnly) == 0 && tile_scales_permit_short_form<ACT>(s))
+    write_rows(std::true_type{});
+  else
+    write_rows(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -688,7 +741,7 @@ hipError_t launch_gemv(const GemvLaunch& g, int bits, int qop, int mb, int gpr, 
 template <int BITS, int ACT>
 hipError_t launch_dequant(const DequantParams& p, int qop, half_t* out, hipStream_t stream) {
   const long long units = (long long)p.tiles * p.ksteps;
-  const dim3 block(256), grid((unsigned)((units + 3) / 4));
+  const dim3 block(kWave * kDequantWaves), grid((unsigned)((units + kDequantWaves - 1) / kDequantWaves));
   switch (qop) {
     case 1: return launch(dequantize_kernel<BITS, 1, ACT>, grid, block, 0, stream, p, out);
     case 2: return launch(dequantize_kernel<BITS, 2, ACT>, grid, block, 0, stream, p, out);
@@ -867,6 +920,7 @@ int dequantize_any(const void* weights, const uint16_t* scale, const uint16_t* z
   p.n_out = n_out;
   p.k = k;
   p.group_size = group_size;
+  p.num_groups = k / group_size;
   p.tiles = num_tiles(n_out);
   p.ksteps = num_ksteps(k, weight_bits);
   p.flags = g_dequant_flags.load();
