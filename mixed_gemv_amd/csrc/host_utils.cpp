@@ -10,48 +10,54 @@
 
 namespace {
 
-// ---- binary16 helpers (host) ---------------------------------------------------------------
+// ---- binary16 helpers (host): eight values at a time, selects instead of branches -----------
 
-inline uint32_t bits_of(float f) {
-  uint32_t u;
-  std::memcpy(&u, &f, 4);
-  return u;
-}
-inline float float_of(uint32_t u) {
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
-}
+typedef uint16_t u16x8 __attribute__((vector_size(16)));
+typedef int8_t i8x8 __attribute__((vector_size(8)));
+typedef uint32_t u32x8 __attribute__((vector_size(32)));
+typedef float f32x8 __attribute__((vector_size(32)));
 
-// Exact widening binary16 -> binary32 through a power-of-two rescale.
-inline float half_bits_to_float(uint16_t h) {
-  const uint32_t sign = (uint32_t)(h & 0x8000u) << 16;
-  const uint32_t body = (uint32_t)(h & 0x7fffu);
-  if (body >= 0x7c00u) return float_of(sign | 0x7f800000u | ((body & 0x3ffu) << 13));
+// (by reference: a 32-byte vector argument has no agreed place without AVX)
+inline void half_bits_to_float(const u16x8& h16, f32x8& f) {
   // Place exponent+mantissa in the binary32 fields, then multiply by 2^(127-15) = 2^112:
   // exact for normals, and it normalises subnormals for free.
-  const float scaled = float_of(body << 13) * float_of(0x77800000u);
-  return float_of(sign | bits_of(scaled));
+  const u32x8 h = __builtin_convertvector(h16, u32x8);
+  const u32x8 sign = (h & 0x8000u) << 16, body = h & 0x7fffu;
+  const u32x8 scaled = (u32x8)((f32x8)(body << 13) * 0x1p112f);
+  const u32x8 special = 0x7f800000u | ((body & 0x3ffu) << 13);
+  f = (f32x8)(sign | (body >= 0x7c00u ? special : scaled));
 }
 
 // binary32 -> binary16, round-to-nearest-even.
-inline uint16_t float_to_half_bits(float f) {
-  uint32_t x = bits_of(f);
-  const uint16_t sign = (uint16_t)((x >> 16) & 0x8000u);
-  x &= 0x7fffffffu;
-  if (x >= 0x47800000u) {  // |f| >= 65536, inf or nan
-    return (uint16_t)(sign | (x > 0x7f800000u ? 0x7e00u : 0x7c00u));
+inline void float_to_half_bits(const f32x8& f, u16x8& h) {
+  const u32x8 sign = ((u32x8)f >> 16) & 0x8000u, x = (u32x8)f & 0x7fffffffu;
+  const u32x8 nan = (u32x8){} + 0x7e00u, inf = (u32x8){} + 0x7c00u;
+  const u32x8 big = x > 0x7f800000u ? nan : inf;  // |f| >= 65536, inf or nan
+  // |f| < 2^-14: the result is subnormal (or zero).  Adding 0.5 shifts the value so that the binary32 unit in the last
+  // place is 2^-24, the subnormal half spacing; the hardware's RNE does the rounding.
+  const u32x8 small = (u32x8)((f32x8)x + 0.5f) - 0x3f000000u;
+  // rebias the exponent by (15 - 127) and add the rounding bias 0xfff, and one more where ties have to go up to even
+  const u32x8 normal = (x + 0xc8000fffu + ((x >> 13) & 1u)) >> 13;
+  const u32x8 body = x < 0x38800000u ? small : normal;
+  h = __builtin_convertvector(sign | (x >= 0x47800000u ? big : body), u16x8);
+}
+
+// Elements a thread should have at least (a few microseconds' work: what starting the others costs).
+constexpr size_t kGrain = (size_t)1 << 15;
+
+// fn(first, last) over pieces of `grain` elements of [0, n), side by side where there is enough to do.
+template <typename Fn>
+void in_pieces(size_t n, size_t grain, Fn fn) {
+  const size_t pieces = (n + grain - 1) / grain;
+  if (pieces <= 1) {
+    fn((size_t)0, n);
+    return;
   }
-  if (x < 0x38800000u) {  // |f| < 2^-14: the result is subnormal (or zero)
-    // Adding 0.5 shifts the value so that the binary32 unit in the last place is 2^-24,
-    // the subnormal half spacing; the hardware's RNE does the rounding.
-    const float shifted = float_of(x) + 0.5f;
-    return (uint16_t)(sign | (bits_of(shifted) - 0x3f000000u));
+#pragma omp parallel for schedule(static)
+  for (long long i = 0; i < (long long)pieces; ++i) {
+    const size_t first = (size_t)i * grain;
+    fn(first, first + grain < n ? first + grain : n);
   }
-  const uint32_t odd = (x >> 13) & 1u;
-  x += 0xc8000fffu;  // rebias exponent by (15 - 127) and add the rounding bias 0xfff
-  x += odd;          // ties go to even
-  return (uint16_t)(sign | (x >> 13));
 }
 
 bool shape_ok(const size_t* shape, int rank, size_t& experts, size_t& k, size_t& n_out) {
@@ -97,70 +103,90 @@ void transpose_quantised(uint8_t* dst, const uint8_t* src, size_t k, size_t n_ou
   }
 }
 
-// Walks the chunks of row n in ascending k and hands each (source byte offset inside the row,
-// byte offset inside the tiled buffer, bytes of the chunk that lie inside the row -- fewer than 16
-// only for the last chunk of a row whose k is not a multiple of the chunk) to `visit`; nested
-// loops instead of chunk_offset() keep integer divisions out of the inner loop.
-template <typename Visit>
-inline void for_each_chunk_of_row(size_t n, size_t k, size_t ksteps, int bits, Visit visit) {
-  const size_t ck = (size_t)mgemv::chunk_k(bits);
-  const size_t tile = n / mgemv::kTileRows, r = n % mgemv::kTileRows;
-  size_t k0 = 0;
-  for (size_t s = 0; s < ksteps && k0 < k; ++s) {
-    const size_t unit = (tile * ksteps + s) * (size_t)mgemv::kUnitBytes;
-    for (size_t slice = 0; slice < (size_t)mgemv::kKSlices && k0 < k; ++slice) {
-      const size_t lane_off = (slice * mgemv::kTileRows + r) * (size_t)mgemv::kChunkBytes;
-      for (size_t blk = 0; blk < (size_t)mgemv::kBlocksPerUnit && k0 < k; ++blk, k0 += ck)
-        visit(k0 * (size_t)bits / 8, unit + blk * (size_t)mgemv::kBlockBytes + lane_off,
-              (k - k0 < ck ? k - k0 : ck) * (size_t)bits / 8);
+// Four words at a time; the compiler makes SSE2 of it (or whatever the target has).
+typedef uint32_t word4 __attribute__((vector_size(16), aligned(4), may_alias));
+template <typename W>
+inline W encode_int4(W natural) {
+  const W b = natural ^ 0x88888888u;
+  const W f5 = b & 0x00f00000u;
+  return ((b & 0x0000000fu) << 7) | ((b & 0x000000f0u) << 19) | ((b & 0x00000f00u) >> 5) | ((b & 0x0000f000u) << 7) |
+         ((b & 0x000f0000u) >> 1) | (f5 << 11) | (f5 >> 21) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
+}
+template <typename W>
+inline W decode_int4(W w) {
+  const W f5 = ((w >> 11) | (w << 21)) & 0x00f00000u;
+  return (((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) | ((w >> 7) & 0x0000f000u) |
+          ((w << 1) & 0x000f0000u) | f5 | ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u)) ^ 0x88888888u;
+}
+template <int BITS, bool DECODE>
+inline word4 recode_chunk(word4 w) {
+  if (BITS == 8) return w ^ 0x80808080u;
+  return DECODE ? decode_int4(w) : encode_int4(w);
+}
+
+// One 16-row tile between rows (row_bytes apart, `rows` of them) and its units.  A lane's run -- 64 bytes of one row, whose
+// four chunks go to the four blocks of a unit -- is a cache line of the row, and the unit's 4 KiB stay in the first-level
+// cache while the runs of 16 rows x 4 slices fill them, so that both sides are walked line by line.  (A row at a time,
+// as the first version of this loop had it, comes back to each line of the tiled side four times.)
+template <int BITS, bool DECODE>
+void recode_tile(uint8_t* units, uint8_t* rows_base, size_t rows, size_t row_bytes, size_t ksteps) {
+  constexpr size_t kRunBytes = (size_t)mgemv::kBlocksPerUnit * mgemv::kChunkBytes;
+  for (size_t s = 0; s < ksteps; ++s) {
+    uint8_t* const unit = units + s * (size_t)mgemv::kUnitBytes;
+    for (size_t slice = 0; slice < (size_t)mgemv::kKSlices; ++slice) {
+      const size_t off = (s * mgemv::kKSlices + slice) * kRunBytes;
+      if (off >= row_bytes) break;  // a run past k: left as it is (zero)
+      const size_t here = row_bytes - off < kRunBytes ? row_bytes - off : kRunBytes;
+      for (size_t r = 0; r < rows; ++r) {
+        uint8_t* const row = rows_base + r * row_bytes + off;
+        uint8_t* const lane = unit + (slice * mgemv::kTileRows + r) * mgemv::kChunkBytes;
+        if (here == kRunBytes) {
+          for (int blk = 0; blk < mgemv::kBlocksPerUnit; ++blk) {
+            word4* const in_row = reinterpret_cast<word4*>(row + blk * mgemv::kChunkBytes);
+            word4* const in_unit = reinterpret_cast<word4*>(lane + blk * mgemv::kBlockBytes);
+            if (DECODE) *in_row = recode_chunk<BITS, true>(*in_unit); else *in_unit = recode_chunk<BITS, false>(*in_row);
+          }
+          continue;
+        }
+        for (size_t blk = 0; blk * mgemv::kChunkBytes < here; ++blk) {
+          const size_t valid = here - blk * mgemv::kChunkBytes < (size_t)mgemv::kChunkBytes ? here - blk * mgemv::kChunkBytes
+                                                                                           : (size_t)mgemv::kChunkBytes;
+          word4 w = {0, 0, 0, 0};  // positions past k inside a chunk: any value, they only ever meet zero activations
+          uint8_t* const in_unit = lane + blk * mgemv::kBlockBytes;
+          std::memcpy(&w, DECODE ? in_unit : row + blk * mgemv::kChunkBytes, DECODE ? (size_t)mgemv::kChunkBytes : valid);
+          w = recode_chunk<BITS, DECODE>(w);
+          std::memcpy(DECODE ? row + blk * mgemv::kChunkBytes : in_unit, &w, DECODE ? valid : (size_t)mgemv::kChunkBytes);
+        }
+      }
     }
   }
 }
 
-// One matrix: rows of k elements (n_out rows) -> tile layout.
-void tile_one_matrix(uint8_t* dst, const uint8_t* src, size_t n_out, size_t k, int bits) {
-  const size_t ksteps = (size_t)mgemv::num_ksteps((int)k, bits);
-  const size_t row_bytes = k * (size_t)bits / 8;
-  // zero bytes only where the layout pads: whole rows past n_out, reduction positions past k
-  if (n_out % mgemv::kTileRows != 0 || k % (size_t)mgemv::step_k(bits) != 0) {
-    const size_t total = mgemv::preprocessed_bytes(n_out, k, bits), piece = (size_t)1 << 20;
-#pragma omp parallel for schedule(static)
-    for (long long off = 0; off < (long long)total; off += (long long)piece)
-      std::memset(dst + off, 0, total - (size_t)off < piece ? total - (size_t)off : piece);
-  }
-#pragma omp parallel for schedule(static)
-  for (long long n = 0; n < (long long)n_out; ++n) {
-    const uint8_t* row = src + (size_t)n * row_bytes;
-    for_each_chunk_of_row((size_t)n, k, ksteps, bits, [&](size_t src_off, size_t dst_off, size_t valid) {
-      uint32_t words[4] = {0, 0, 0, 0};  // positions past k: any value, they only ever meet zero activations
-      std::memcpy(words, row + src_off, valid);
-      if (bits == 4) {
-        for (int j = 0; j < 4; ++j) words[j] = mgemv::encode_int4_word(words[j]);
-      } else {
-        for (int j = 0; j < 4; ++j) words[j] = mgemv::encode_int8_word(words[j]);
-      }
-      std::memcpy(dst + dst_off, words, mgemv::kChunkBytes);
-    });
+// One matrix between rows of k elements (n_out rows) and the tile layout.
+template <int BITS, bool DECODE>
+void recode_matrix(uint8_t* tiled, uint8_t* rows, size_t n_out, size_t k) {
+  const size_t ksteps = (size_t)mgemv::num_ksteps((int)k, BITS), tiles = (size_t)mgemv::num_tiles((int)n_out);
+  const size_t row_bytes = k * (size_t)BITS / 8, tile_bytes = ksteps * (size_t)mgemv::kUnitBytes;
+  const bool padded = k % (size_t)mgemv::step_k(BITS) != 0;
+#pragma omp parallel for schedule(static) if (tiles * tile_bytes >= 4 * kGrain)
+  for (long long t = 0; t < (long long)tiles; ++t) {
+    const size_t row0 = (size_t)t * mgemv::kTileRows;
+    const size_t here = n_out - row0 < (size_t)mgemv::kTileRows ? n_out - row0 : (size_t)mgemv::kTileRows;
+    uint8_t* const tile = tiled + (size_t)t * tile_bytes;
+    // zero bytes only where the layout pads: rows past n_out, reduction positions past k
+    if (!DECODE && (padded || here < (size_t)mgemv::kTileRows)) std::memset(tile, 0, tile_bytes);
+    recode_tile<BITS, DECODE>(tile, rows + row0 * row_bytes, here, row_bytes, ksteps);
   }
 }
 
+void tile_one_matrix(uint8_t* dst, const uint8_t* src, size_t n_out, size_t k, int bits) {
+  uint8_t* const rows = const_cast<uint8_t*>(src);  // only read
+  if (bits == 4) recode_matrix<4, false>(dst, rows, n_out, k); else recode_matrix<8, false>(dst, rows, n_out, k);
+}
+
 void untile_one_matrix(uint8_t* dst, const uint8_t* src, size_t n_out, size_t k, int bits) {
-  const size_t ksteps = (size_t)mgemv::num_ksteps((int)k, bits);
-  const size_t row_bytes = k * (size_t)bits / 8;
-#pragma omp parallel for schedule(static)
-  for (long long n = 0; n < (long long)n_out; ++n) {
-    uint8_t* row = dst + (size_t)n * row_bytes;
-    for_each_chunk_of_row((size_t)n, k, ksteps, bits, [&](size_t row_off, size_t tiled_off, size_t valid) {
-      uint32_t words[4];
-      std::memcpy(words, src + tiled_off, mgemv::kChunkBytes);
-      if (bits == 4) {
-        for (int j = 0; j < 4; ++j) words[j] = mgemv::decode_int4_word(words[j]);
-      } else {
-        for (int j = 0; j < 4; ++j) words[j] = mgemv::decode_int8_word(words[j]);
-      }
-      std::memcpy(row + row_off, words, valid);
-    });
-  }
+  uint8_t* const tiled = const_cast<uint8_t*>(src);  // only read
+  if (bits == 4) recode_matrix<4, true>(tiled, dst, n_out, k); else recode_matrix<8, true>(tiled, dst, n_out, k);
 }
 
 int check_dims(size_t n_out, size_t k, int bits) {
@@ -179,56 +205,84 @@ int mgemv_pack_int4(uint8_t* packed, const int8_t* unpacked, size_t n_unpacked) 
   if (n_unpacked == 0) return MGEMV_OK;
   if (packed == nullptr || unpacked == nullptr) return MGEMV_ERR_NULL_POINTER;
   if (n_unpacked % 2) return MGEMV_ERR_SIZE;  // two elements per byte
-  const size_t n_bytes = n_unpacked / 2;
-  for (size_t i = 0; i < n_bytes; ++i) {
-    const unsigned lo = (unsigned)unpacked[2 * i] & 0xfu;
-    const unsigned hi = (unsigned)unpacked[2 * i + 1] & 0xfu;
-    packed[i] = (uint8_t)(lo | (hi << 4));
-  }
+  // 32 elements at a time: a 16-bit pair holds element 2i in its low byte and 2i + 1 in its high one
+  typedef uint16_t pairs16 __attribute__((vector_size(32), aligned(1), may_alias));
+  typedef uint8_t bytes16 __attribute__((vector_size(16), aligned(1), may_alias));
+  in_pieces(n_unpacked / 2, kGrain, [=](size_t first, size_t last) {
+    size_t i = first;
+    for (; i + 16 <= last; i += 16) {
+      const pairs16 v = *reinterpret_cast<const pairs16*>(unpacked + 2 * i);
+      *reinterpret_cast<bytes16*>(packed + i) = __builtin_convertvector((v & 0x000f) | ((v >> 4) & 0x00f0), bytes16);
+    }
+    for (; i < last; ++i)
+      packed[i] = (uint8_t)(((unsigned)unpacked[2 * i] & 0xfu) | (((unsigned)unpacked[2 * i + 1] & 0xfu) << 4));
+  });
   return MGEMV_OK;
 }
 
 int mgemv_unpack_int4(int8_t* unpacked, const uint8_t* packed, size_t n_packed) {
   if (n_packed == 0) return MGEMV_OK;
   if (packed == nullptr || unpacked == nullptr) return MGEMV_ERR_NULL_POINTER;
-  for (size_t i = 0; i < n_packed; ++i) {
-    const int lo = packed[i] & 0xf, hi = packed[i] >> 4;
-    unpacked[2 * i] = (int8_t)(lo >= 8 ? lo - 16 : lo);
-    unpacked[2 * i + 1] = (int8_t)(hi >= 8 ? hi - 16 : hi);
-  }
+  typedef int8_t bytes16 __attribute__((vector_size(16), aligned(1), may_alias));
+  in_pieces(n_packed, kGrain, [=](size_t first, size_t last) {
+    size_t i = first;
+    for (; i + 16 <= last; i += 16) {
+      const bytes16 v = *reinterpret_cast<const bytes16*>(packed + i);
+      const bytes16 lo = ((v & 0xf) ^ 8) - 8, hi = (((v >> 4) & 0xf) ^ 8) - 8;
+      bytes16* const to = reinterpret_cast<bytes16*>(unpacked + 2 * i);
+      to[0] = __builtin_shufflevector(lo, hi, 0, 16, 1, 17, 2, 18, 3, 19, 4, 20, 5, 21, 6, 22, 7, 23);
+      to[1] = __builtin_shufflevector(lo, hi, 8, 24, 9, 25, 10, 26, 11, 27, 12, 28, 13, 29, 14, 30, 15, 31);
+    }
+    for (; i < last; ++i) {
+      unpacked[2 * i] = (int8_t)(((packed[i] & 0xf) ^ 8) - 8);
+      unpacked[2 * i + 1] = (int8_t)(((packed[i] >> 4) ^ 8) - 8);
+    }
+  });
   return MGEMV_OK;
 }
 
 int mgemv_fold_zero_points(uint16_t* out, const uint16_t* scales, const int8_t* zeros, size_t n) {
   if (n == 0) return MGEMV_OK;
   if (out == nullptr || scales == nullptr || zeros == nullptr) return MGEMV_ERR_NULL_POINTER;
-  for (size_t i = 0; i < n; ++i) {
-    // -z is an integer of magnitude <= 128: exact in binary16.  The binary32 product of two
-    // halves is exact, so one rounding to binary16 is the correctly rounded fp16 multiply.
-    const float neg_z = (float)(-(int)zeros[i]);
-    out[i] = float_to_half_bits(neg_z * half_bits_to_float(scales[i]));
-  }
+  // -z is an integer of magnitude <= 128: exact in binary16.  The binary32 product of two
+  // halves is exact, so one rounding to binary16 is the correctly rounded fp16 multiply.
+  in_pieces(n, kGrain / 4, [=](size_t first, size_t last) {
+    for (size_t i = first; i < last; i += 8) {
+      const size_t here = last - i < 8 ? last - i : 8;
+      u16x8 s = {}, r;
+      i8x8 z = {};
+      std::memcpy(&s, scales + i, here == 8 ? 16 : here * 2);
+      std::memcpy(&z, zeros + i, here == 8 ? 8 : here);
+      f32x8 f;
+      half_bits_to_float(s, f);
+      typedef int32_t i32x8 __attribute__((vector_size(32)));
+      float_to_half_bits(__builtin_convertvector(-__builtin_convertvector(z, i32x8), f32x8) * f, r);
+      std::memcpy(out + i, &r, here == 8 ? 16 : here * 2);
+    }
+  });
   return MGEMV_OK;
 }
 
 int mgemv_fold_zero_points_bf16(uint16_t* out, const uint16_t* scales, const int8_t* zeros, size_t n) {
   if (n == 0) return MGEMV_OK;
   if (out == nullptr || scales == nullptr || zeros == nullptr) return MGEMV_ERR_NULL_POINTER;
-  for (size_t i = 0; i < n; ++i) {
-    // -z has at most 8 significant bits: exact in bfloat16.  The binary32 product of two
-    // bfloat16 values is exact, so one rounding (nearest even) is the correctly rounded multiply.
-    const uint32_t s_bits = (uint32_t)scales[i] << 16;
-    float s;
-    std::memcpy(&s, &s_bits, 4);
-    const float prod = (float)(-(int)zeros[i]) * s;
-    uint32_t bits;
-    std::memcpy(&bits, &prod, 4);
-    if ((bits & 0x7fffffffu) > 0x7f800000u) {
-      out[i] = (uint16_t)((bits >> 16) | 0x0040u);  // NaN stays NaN
-    } else {
-      out[i] = (uint16_t)((bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16);
+  in_pieces(n, kGrain / 4, [=](size_t first, size_t last) {
+    for (size_t i = first; i < last; ++i) {
+      // -z has at most 8 significant bits: exact in bfloat16.  The binary32 product of two
+      // bfloat16 values is exact, so one rounding (nearest even) is the correctly rounded multiply.
+      const uint32_t s_bits = (uint32_t)scales[i] << 16;
+      float s;
+      std::memcpy(&s, &s_bits, 4);
+      const float prod = (float)(-(int)zeros[i]) * s;
+      uint32_t bits;
+      std::memcpy(&bits, &prod, 4);
+      if ((bits & 0x7fffffffu) > 0x7f800000u) {
+        out[i] = (uint16_t)((bits >> 16) | 0x0040u);  // NaN stays NaN
+      } else {
+        out[i] = (uint16_t)((bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16);
+      }
     }
-  }
+  });
   return MGEMV_OK;
 }
 
