@@ -102,8 +102,8 @@ struct ShortFormScale {
   half2_t m8s;   // (-8 s, -8 s)
 };
 
-// fp16 bit pattern of a scale for which the short form is exact: 0x0001 .. 0x27ff.
-__device__ __forceinline__ bool short_form_ok(uint32_t scale_bits) { return ((scale_bits & 0xffffu) - 1u) < 0x27ffu; }
+// fp16 bit patterns of the scales for which the short form is exact: 0x0001 .. 0x27ff.
+constexpr uint32_t kShortF16First = 0x0001, kShortF16Past = 0x2800;
 
 __device__ __forceinline__ ShortFormScale make_short_form_scale(half2_t s2) {
   ShortFormScale f;
@@ -187,11 +187,9 @@ __device__ __forceinline__ void settle_dot_chain(float& acc) { asm volatile("s_n
 // for the sum, rounding the fp32 sum to bf16 equals rounding the exact sum once (24 >= 2*8+2).
 // Values are kept as packed pairs of bf16 bit patterns, (low, high) = ascending k.
 //
-// Two forms, as for fp16.  With 8u (int4) or u (int8) from v_cvt_f32_ubyteN:
-//   fused    fma(8u, s/8, -8s) resp. fma(u, s, -128s): exact, hence = q*s, for 2^-100 <= s < 2^119
-//            (-8s / -128s stays finite; for s > 0 a zero product is +0 on both routes).  For int4
-//            the fma and the conversions around it are v_dot2_f32_bf16 instructions on packed
-//            pairs (dequant_int4_word_bf16), which needs s/8 to be a normal bf16;
+// Two forms each, as for fp16:
+//   short    int4: the products of the fp16 short form, exact in fp16, widened to fp32 by the matrix unit and rounded
+//            (dequant_int4_word_bf16_short); int8: fma(u, s, -128 s), exact for 2^-100 <= s < 2^119;
 //   general  (8u - 64) * (s/8) resp. (u - 128) * s: exact for every finite s, with the sign of
 //            a zero product as the reference's multiply gives it.
 // ---------------------------------------------------------------------------------------------
@@ -199,10 +197,6 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-#ifndef MGEMV_BF16_DOT_DEQUANT
-#define MGEMV_BF16_DOT_DEQUANT 1
-#endif
-constexpr bool kBf16DotDequant = MGEMV_BF16_DOT_DEQUANT != 0;  // 0: the v_cvt / v_fma route for int4 as well
 constexpr int kActF16 = 0;
 constexpr int kActBf16 = 1;
 
@@ -216,120 +210,152 @@ __device__ __forceinline__ float byte_to_f32(uint32_t v) {
   return (float)((v >> (8 * BYTE)) & 0xffu);  // v_cvt_f32_ubyteN
 }
 
-// bf16 bit pattern of a scale for which the fused form is exact (both weight widths):
-// 0x0d80 .. 0x7aff, i.e. 2^-100 <= s < 2^119 -- positive, s/8 a normal bf16, -128 s finite.
-__device__ __forceinline__ bool fused_form_ok_bf16(uint32_t scale_bits) { return ((scale_bits & 0xffffu) - 0x0d80u) < (0x7b00u - 0x0d80u); }
+// Which scales the short form takes, by bf16 bit pattern.
+// int8: 2^-100 .. 2^119 -- positive, every product with an integer a normal number, -128 s finite.
+// int4: the products q s have 11 significant bits and must not fall off either end of fp16: 2^-17 <= s < 2^-5, scaled by
+// any 2^shift that is the same for the whole wave (the widening step takes it back).
+constexpr uint32_t kShortBf16Int8First = 0x0d80, kShortBf16Int8Past = 0x7b00;
+constexpr uint32_t kShortBf16Int4First = (127 - 17) << 7, kShortBf16Int4Past = (127 - 5) << 7;
+constexpr int kShortBf16MinShift = -14, kShortBf16MaxShift = 15;  // 2^shift is a normal fp16 value
+constexpr int kNoShortForm = 0x7fffffff;
+
+// One lane's row of the 4x4 identity, as a mask on four packed 16-bit values: the operand of the widening steps below.
+struct Identity4 {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ Identity4 make_identity4() {
+  const uint32_t row = threadIdx.x & 3u;  // lane i of each four holds row i
+  const uint32_t half = (row & 1u) != 0 ? 0xffff0000u : 0x0000ffffu;
+  return Identity4{row < 2 ? half : 0u, row < 2 ? 0u : half};
+}
+
+// v_mfma_f32_4x4x4_16b with the 4x4 identity as one operand gives every lane its own four 16-bit values back as fp32 --
+// times the identity's value, plus the lane's accumulator operand: one instruction of 8 cycles on the otherwise idle
+// matrix unit in place of four conversions (and four additions) of the vector unit.  Every instruction these kernels issue costs
+// a wave about 4.3 cycles (measured with 4 waves per SIMD), so what counts is their number.
+// The other three values of a lane's block meet zero factors: all of them must be finite.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 widen_f16(const u32x2& identity, half2_t a, half2_t b) {
+  return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, identity), __builtin_bit_cast(half4_t, u32x2{as_u32(a), as_u32(b)}),
+                                            f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+}
+// Bf16 values plus the additive zero, rounded to bf16, PAIRS packed pairs at a time.  r + z carries at most 17 significant
+// bits wherever it comes near the middle between two bf16 values, so its rounding to bf16 is that of the exact sum (checked
+// on the device against the vector unit over 8e8 pairs, subnormal zeros included).
+// A matrix instruction's result is there five issue slots later.  The barriers keep the compiler from lining up each
+// instruction with its own conversions, where it would have to fill those slots with waits (100 of them a unit): first all
+// instructions, then all conversions.
+template <int PAIRS>
+__device__ __forceinline__ void add_zero_bf16(uint32_t (&d)[PAIRS], const u32x2& identity, const f32x4& z) {
+  f32x4 sum[PAIRS / 2];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < PAIRS / 2; ++i)
+    sum[i] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, identity),
+                                                    __builtin_bit_cast(s16x4, u32x2{d[2 * i], d[2 * i + 1]}), z, 0, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < PAIRS / 2; ++i) {
+    d[2 * i] = pack_bf16(sum[i][0], sum[i][1]);
+    d[2 * i + 1] = pack_bf16(sum[i][2], sum[i][3]);
+  }
+}
 
 struct Bf16Scale {
-  float mul;        // int4: s/8; int8: s
-  float add;        // fused form: -8s resp. -128s (int4 through the dot instructions: -24s); general form: unused
-  float z;          // additive zero
-  uint32_t sel_lo;  // int4 fused form through the dot instructions: the bf16 pairs (s/8, 0) ...
-  uint32_t sel_hi;  // ... and (0, s/8)
+  float mul;              // int4, general: s/8; int8: s
+  float add;              // int8, short: -128 s
+  f32x4 z;                // additive zero, four times: the accumulator operand of add_zero_bf16
+  ShortFormScale f16;     // int4, short: of s * 2^-shift
+  u32x2 widen, identity;  // 2^shift (fp16) and 1 (bf16) times the lane's row of the identity
 };
 
-template <int BITS, bool FUSED>
-__device__ __forceinline__ Bf16Scale make_bf16_scale(uint32_t s_bits, uint32_t z_bits) {
-  const float s = bf16_low_to_f32(s_bits);
-  Bf16Scale f;
-  f.mul = BITS == 4 ? s * 0.125f : s;
-  f.add = FUSED ? s * (BITS == 4 ? (kBf16DotDequant ? -24.0f : -8.0f) : -128.0f) : 0.0f;
-  f.z = bf16_low_to_f32(z_bits);
-  f.sel_lo = f.sel_hi = 0;
-  if constexpr (BITS == 4 && FUSED && kBf16DotDequant) {
-    f.sel_lo = (s_bits & 0xffffu) - 0x0180u;  // s/8: three off the exponent of a normal s (the fused range has no other)
-    f.sel_hi = f.sel_lo << 16;
+// shift: int4 short form only.
+template <int BITS, bool SHORT>
+__device__ __forceinline__ Bf16Scale make_bf16_scale(uint32_t s_bits, uint32_t z_bits, const Identity4& id, int shift) {
+  const float s = bf16_low_to_f32(s_bits), z = bf16_low_to_f32(z_bits);
+  Bf16Scale f{};
+  if constexpr (BITS == 4 && SHORT) {
+    auto scaled = [&](uint32_t power_bits) { return splat((half_t)(s * __builtin_bit_cast(float, power_bits - ((uint32_t)shift << 23)))); };  // exact
+    f.f16.s17 = scaled(0x48000000u);  // 2^17
+    f.f16.s21 = scaled(0x4a000000u);
+    f.f16.m8s = scaled(0xc1000000u);  // -8
+    const uint32_t unit = (uint32_t)(15 + shift) << 10;
+    f.widen = u32x2{id.lo & (unit | unit << 16), id.hi & (unit | unit << 16)};
+  } else {
+    f.mul = BITS == 4 ? s * 0.125f : s;
+    f.add = s * -128.0f;
   }
+  f.identity = u32x2{id.lo & 0x3f803f80u, id.hi & 0x3f803f80u};
+  f.z = f32x4{z, z, z, z};
   return f;
 }
 
-// (a, b): the integers 8u (int4) or u (int8) of a k-adjacent pair -> packed bf16 pair of
-// rn(rn(q s) + z) resp. rn(q s).
-template <int BITS, bool HAS_ZERO, bool FUSED>
+// General form.  (a, b): the integers 8u (int4) or u (int8) of a k-adjacent pair -> packed bf16 pair of
+// rn(rn(q s) + z) resp. rn(q s).  (The products may overflow, so the sum stays on the vector unit.)
+template <int BITS, bool HAS_ZERO>
 __device__ __forceinline__ uint32_t dequant_pair_bf16(float a, float b, const Bf16Scale& f) {
-  float p0, p1;
-  if constexpr (FUSED) {
-    p0 = __builtin_fmaf(a, f.mul, f.add);
-    p1 = __builtin_fmaf(b, f.mul, f.add);
-  } else {
-    constexpr float kBias = BITS == 4 ? 64.0f : 128.0f;
-    p0 = (a - kBias) * f.mul;
-    p1 = (b - kBias) * f.mul;
-  }
-  uint32_t d = pack_bf16(p0, p1);
-  if constexpr (HAS_ZERO) d = pack_bf16(bf16_low_to_f32(d) + f.z, bf16_high_to_f32(d) + f.z);
+  constexpr float kBias = BITS == 4 ? 64.0f : 128.0f;
+  uint32_t d = pack_bf16((a - kBias) * f.mul, (b - kBias) * f.mul);
+  if constexpr (HAS_ZERO) d = pack_bf16(bf16_low_to_f32(d) + f.z[0], bf16_high_to_f32(d) + f.z[0]);
   return d;
 }
 
-// Eight bf16 values (four packed pairs a[0..3]) through out = rn_bf16(a * m + c), fp32 inside:
-// v_dot2_f32_bf16 with the factor pair sel_lo = (m, 0) resp. sel_hi = (0, m) computes
-// a.lo * m + c resp. a.hi * m + c straight from the packed pair -- fused, one rounding (checked
-// exhaustively by the tests) -- and v_cvt_pk_bf16_f32 rounds to bf16.  The product with the zero
-// factor vanishes as long as every a is finite, which the fused form's scale range guarantees.
-// One asm block, because the compiler does not know these are dot instructions: their results
-// must not be read by another kind of instruction within three issue slots, and the order
-// below keeps at least three instructions between each dot and the conversion that consumes it.
-__device__ __forceinline__ void dot_round_bf16x8(const uint32_t (&a)[4], uint32_t sel_lo, uint32_t sel_hi, float c,
-                                                 uint32_t (&out)[4]) {
-  float t0, t1, t2, t3, t4, t5, t6, t7;
-  asm("v_dot2_f32_bf16 %4, %12, %16, %18\n\t"
-      "v_dot2_f32_bf16 %5, %12, %17, %18\n\t"
-      "v_dot2_f32_bf16 %6, %13, %16, %18\n\t"
-      "v_dot2_f32_bf16 %7, %13, %17, %18\n\t"
-      "v_dot2_f32_bf16 %8, %14, %16, %18\n\t"
-      "v_dot2_f32_bf16 %9, %14, %17, %18\n\t"
-      "v_dot2_f32_bf16 %10, %15, %16, %18\n\t"
-      "v_dot2_f32_bf16 %11, %15, %17, %18\n\t"
-      "v_cvt_pk_bf16_f32 %0, %4, %5\n\t"
-      "v_cvt_pk_bf16_f32 %1, %6, %7\n\t"
-      "v_cvt_pk_bf16_f32 %2, %8, %9\n\t"
-      "v_cvt_pk_bf16_f32 %3, %10, %11"
-      : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3]), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3),
-        "=&v"(t4), "=&v"(t5), "=&v"(t6), "=&v"(t7)
-      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(sel_lo), "v"(sel_hi), "v"(c));
-}
-
-// int4: the fields of elements (2,3) sit at bits 3-6 of bytes 0 and 2, those of (6,7) at bits 3-6
-// of bytes 1 and 3; (0,1) and (4,5) come to bytes 0 and 2 after a shift by 4 resp. a rotation
-// by 12 (tile_layout.h).  A masked byte converts to 8u.
-template <bool HAS_ZERO, bool FUSED>
-__device__ __forceinline__ void dequant_int4_word_bf16(uint32_t w, const ConvertRegs& c, const Bf16Scale& f,
-                                                       uint32_t (&d)[4]) {
-  if constexpr (FUSED && kBf16DotDequant) {
-    // A field at bits 3-6 of a half-word under the bf16 pattern 0x4300 (128.0, mantissa step 1) IS
-    // the bf16 value 128 + 8u -- the route of gemv/interleaved_numeric_conversion.h:340-401 on
-    // these field positions -- and (128 + 8u) * (s/8) - 24 s = (u - 8) s exactly.
-    uint32_t magic;  // in a VGPR, so that mask (an SGPR) and magic fit one v_and_or_b32
-    asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
-    uint32_t m[4];
-    m[0] = ((w >> 4) & c.mask3) | magic;
-    m[1] = (w & c.mask3) | magic;
-    m[2] = (__builtin_amdgcn_alignbit(w, w, 12) & c.mask3) | magic;
-    m[3] = ((w >> 8) & c.mask3) | magic;
-    if constexpr (HAS_ZERO) {
-      uint32_t pb[4];
-      dot_round_bf16x8(m, f.sel_lo, f.sel_hi, f.add, pb);
-      dot_round_bf16x8(pb, 0x00003f80u, 0x3f800000u, f.z, d);   // factors (1, 0) and (0, 1)
-    } else {
-      dot_round_bf16x8(m, f.sel_lo, f.sel_hi, f.add, d);
+// WORDS words of int4 (field positions: tile_layout.h), 8 WORDS weights, to packed bf16 pairs in ascending k.
+// Short: 17 vector and 4 matrix instructions a word with a zero, 13 and 2
+// without; 98 cycles a word and SIMD with the product's matrix instruction (4 waves; the scale applied in fp32, one field at
+// a time, 122; v_dot2_f32_bf16 on packed pairs, with the zero, 35 instructions).
+// General: a field masked at bits 3-6 of a byte converts to 8u.
+template <bool HAS_ZERO, bool SHORT, int WORDS>
+__device__ __forceinline__ void dequant_int4_words_bf16(const uint32_t (&words)[WORDS], const ConvertRegs& c, const Bf16Scale& f,
+                                                        uint32_t (&d)[4 * WORDS]) {
+  if constexpr (SHORT) {
+    half2_t q[WORDS][4];
+#pragma unroll
+    for (int i = 0; i < WORDS; ++i) dequant_int4_word_short<false>(words[i], c, f.f16, half2_t{}, q[i]);  // q s 2^-shift, exact
+    f32x4 p[2 * WORDS];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * WORDS; ++i) p[i] = widen_f16(f.widen, q[i / 2][2 * (i % 2)], q[i / 2][2 * (i % 2) + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * WORDS; ++i) {
+      d[2 * i] = pack_bf16(p[i][0], p[i][1]);
+      d[2 * i + 1] = pack_bf16(p[i][2], p[i][3]);
     }
-    return;
+    if constexpr (HAS_ZERO) add_zero_bf16(d, f.identity, f.z);
+  } else {
+    uint32_t mask = c.mask3;  // a value of its own: shared masked words would be computed, and kept, in front of the branch between the forms
+    asm("" : "+s"(mask));
+#pragma unroll
+    for (int i = 0; i < WORDS; ++i) {
+      const uint32_t w = words[i];
+      const uint32_t e01 = (w >> 4) & mask;
+      const uint32_t e23 = w & mask;
+      const uint32_t e45 = __builtin_amdgcn_alignbit(w, w, 12) & mask;
+      const uint32_t e67 = w & 0x78007800u;
+      d[4 * i + 0] = dequant_pair_bf16<4, HAS_ZERO>(byte_to_f32<0>(e01), byte_to_f32<2>(e01), f);
+      d[4 * i + 1] = dequant_pair_bf16<4, HAS_ZERO>(byte_to_f32<0>(e23), byte_to_f32<2>(e23), f);
+      d[4 * i + 2] = dequant_pair_bf16<4, HAS_ZERO>(byte_to_f32<0>(e45), byte_to_f32<2>(e45), f);
+      d[4 * i + 3] = dequant_pair_bf16<4, HAS_ZERO>(byte_to_f32<1>(e67), byte_to_f32<3>(e67), f);
+    }
   }
-  const uint32_t e01 = (w >> 4) & c.mask3;
-  const uint32_t e23 = w & c.mask3;
-  const uint32_t e45 = __builtin_amdgcn_alignbit(w, w, 12) & c.mask3;
-  const uint32_t e67 = w & 0x78007800u;
-  d[0] = dequant_pair_bf16<4, HAS_ZERO, FUSED>(byte_to_f32<0>(e01), byte_to_f32<2>(e01), f);
-  d[1] = dequant_pair_bf16<4, HAS_ZERO, FUSED>(byte_to_f32<0>(e23), byte_to_f32<2>(e23), f);
-  d[2] = dequant_pair_bf16<4, HAS_ZERO, FUSED>(byte_to_f32<0>(e45), byte_to_f32<2>(e45), f);
-  d[3] = dequant_pair_bf16<4, HAS_ZERO, FUSED>(byte_to_f32<1>(e67), byte_to_f32<3>(e67), f);
 }
 
-// int8: 4 biased bytes in natural order.
-template <bool HAS_ZERO, bool FUSED>
-__device__ __forceinline__ void dequant_int8_word_bf16(uint32_t w, const Bf16Scale& f, uint32_t (&d)[2]) {
-  d[0] = dequant_pair_bf16<8, HAS_ZERO, FUSED>(byte_to_f32<0>(w), byte_to_f32<1>(w), f);
-  d[1] = dequant_pair_bf16<8, HAS_ZERO, FUSED>(byte_to_f32<2>(w), byte_to_f32<3>(w), f);
+// WORDS words of int8: 4 biased bytes each in natural order.
+template <bool HAS_ZERO, bool SHORT, int WORDS>
+__device__ __forceinline__ void dequant_int8_words_bf16(const uint32_t (&words)[WORDS], const Bf16Scale& f, uint32_t (&d)[2 * WORDS]) {
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i) {
+    const uint32_t w = words[i];
+    if constexpr (SHORT) {
+      d[2 * i] = pack_bf16(__builtin_fmaf(byte_to_f32<0>(w), f.mul, f.add), __builtin_fmaf(byte_to_f32<1>(w), f.mul, f.add));
+      d[2 * i + 1] = pack_bf16(__builtin_fmaf(byte_to_f32<2>(w), f.mul, f.add), __builtin_fmaf(byte_to_f32<3>(w), f.mul, f.add));
+    } else {
+      d[2 * i] = dequant_pair_bf16<8, HAS_ZERO>(byte_to_f32<0>(w), byte_to_f32<1>(w), f);
+      d[2 * i + 1] = dequant_pair_bf16<8, HAS_ZERO>(byte_to_f32<2>(w), byte_to_f32<3>(w), f);
+    }
+  }
+  if constexpr (SHORT && HAS_ZERO) add_zero_bf16(d, f.identity, f.z);
 }
 
 // bf16 counterpart of dot2_row_bcast (same hazards, same settle_dot_chain afterwards).

@@ -206,33 +206,34 @@ __device__ __forceinline__ void compute_word(float (&acc)[MB], uint32_t w, const
   }
 }
 
-// The same for bf16 operands; SHORT selects the fused form.
+// The same for bf16 operands, two words at a time: J and J + 1.
 template <int BITS, bool HAS_ZERO, bool SHORT, int MB, int I, int J>
-__device__ __forceinline__ void compute_word_bf16(float (&acc)[MB], uint32_t w,
-                                                  const uint32_t (&x)[MB][BITS == 4 ? 4 : 2], const ConvertRegs& c,
-                                                  const Bf16Scale& f) {
+__device__ __forceinline__ void compute_words_bf16(float (&acc)[MB], uint32_t w0, uint32_t w1,
+                                                   const uint32_t (&x)[MB][BITS == 4 ? 4 : 2], const ConvertRegs& c,
+                                                   const Bf16Scale& f) {
   constexpr int kPairs = BITS == 4 ? 4 : 2;
-  uint32_t d[kPairs];
-  if constexpr (BITS == 4) dequant_int4_word_bf16<HAS_ZERO, SHORT>(w, c, f, d);
-  else dequant_int8_word_bf16<HAS_ZERO, SHORT>(w, f, d);
+  uint32_t d[2 * kPairs];
+  if constexpr (BITS == 4) dequant_int4_words_bf16<HAS_ZERO, SHORT, 2>({w0, w1}, c, f, d);
+  else dequant_int8_words_bf16<HAS_ZERO, SHORT, 2>({w0, w1}, f, d);
 #pragma unroll
-  for (int h = 0; h < kPairs; ++h) {
+  for (int h = 0; h < kPairs; ++h)
 #pragma unroll
     for (int m = 0; m < MB; ++m) dot2_row_bcast_bf16<4 * I + J>(acc[m], x[m][h], d[h]);
-  }
+#pragma unroll
+  for (int h = 0; h < kPairs; ++h)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) dot2_row_bcast_bf16<4 * I + J + 1>(acc[m], x[m][h], d[kPairs + h]);
 }
 
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool SHORT, int I, int ACT>
 __device__ __forceinline__ void compute_block(float (&acc)[MB], const UnitFragment<BITS, MB, GROUPS_PER_RUN>& f,
-                                              const ConvertRegs& c) {
+                                              const ConvertRegs& c, int shift) {
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   constexpr int gi = I * GROUPS_PER_RUN / kBlocksPerUnit;
   if constexpr (ACT == kActBf16) {
-    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(f.s[gi], kHasZero ? f.z[gi] : 0u);
-    compute_word_bf16<BITS, kHasZero, SHORT, MB, I, 0>(acc, f.w[I][0], f.x, c, bs);
-    compute_word_bf16<BITS, kHasZero, SHORT, MB, I, 1>(acc, f.w[I][1], f.x, c, bs);
-    compute_word_bf16<BITS, kHasZero, SHORT, MB, I, 2>(acc, f.w[I][2], f.x, c, bs);
-    compute_word_bf16<BITS, kHasZero, SHORT, MB, I, 3>(acc, f.w[I][3], f.x, c, bs);
+    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(f.s[gi], kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
+    compute_words_bf16<BITS, kHasZero, SHORT, MB, I, 0>(acc, f.w[I][0], f.w[I][1], f.x, c, bs);
+    compute_words_bf16<BITS, kHasZero, SHORT, MB, I, 2>(acc, f.w[I][2], f.w[I][3], f.x, c, bs);
   } else {
     const half2_t s2 = splat_low(f.s[gi]);
     half2_t z2 = half2_t{};
@@ -248,12 +249,12 @@ __device__ __forceinline__ void compute_block(float (&acc)[MB], const UnitFragme
 
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool SHORT, int ACT>
 __device__ __forceinline__ void compute_unit_form(float (&acc)[MB], const UnitFragment<BITS, MB, GROUPS_PER_RUN>& f,
-                                                  const ConvertRegs& regs) {
+                                                  const ConvertRegs& regs, int shift) {
   const ConvertRegs c = (ACT == kActF16 && BITS == 4 && !SHORT) ? general_form_regs(regs) : regs;
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 0, ACT>(acc, f, c);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 1, ACT>(acc, f, c);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 2, ACT>(acc, f, c);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 3, ACT>(acc, f, c);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 0, ACT>(acc, f, c, shift);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 1, ACT>(acc, f, c, shift);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 2, ACT>(acc, f, c, shift);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 3, ACT>(acc, f, c, shift);
   // The two forms meet again after this call, and the compiler may place a register copy of
   // the accumulators at that join: make them safe to read by any instruction first.
 #pragma unroll
@@ -281,12 +282,13 @@ __device__ __forceinline__ void compute_unit(float (&acc)[MB], const UnitFragmen
     return;
   }
   if constexpr (BITS == 4 || ACT == kActBf16) {
-    if (short_allowed && wave_scales_permit_short_form<ACT>(f.s)) {
-      compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, true, ACT>(acc, f, c);
+    const int shift = short_allowed ? wave_short_form<BITS, ACT>(f.s) : kNoShortForm;
+    if (shift != kNoShortForm) {
+      compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, true, ACT>(acc, f, c, shift);
       return;
     }
   }
-  compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, false, ACT>(acc, f, c);
+  compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, false, ACT>(acc, f, c, 0);
 }
 
 // Epilogue: fp32 add of the bias, one rounding to fp16

@@ -37,11 +37,12 @@ __device__ __forceinline__ TileScales load_tile_scales(__amdgpu_buffer_rsrc_t ta
   return t;
 }
 
-// True when all 16 scales permit the short (fp16, int4) resp. fused (bf16) dequantiser, in every lane.
-template <int ACT>
+// True when all 16 scales permit the short dequantiser (with shift 0), in every lane.
+template <int BITS, int ACT>
 __device__ __forceinline__ bool tile_scales_permit_short_form(const TileScales& s) {
   typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-  constexpr uint16_t kFirst = ACT == kActBf16 ? 0x0d80 : 0x0001, kPast = ACT == kActBf16 ? 0x7b00 : 0x2800;
+  constexpr uint16_t kFirst = ACT != kActBf16 ? kShortF16First : BITS == 4 ? kShortBf16Int4First : kShortBf16Int8First;
+  constexpr uint16_t kPast = ACT != kActBf16 ? kShortF16Past : BITS == 4 ? kShortBf16Int4Past : kShortBf16Int8Past;
   u16x2 most = u16x2{0, 0};
 #pragma unroll
   for (int i = 0; i < kTileRows / 2; ++i)
@@ -56,17 +57,11 @@ __device__ __forceinline__ u32x4 dequantize_eight(const uint32_t (&w)[8 * BITS /
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   u32x4 out;
   if constexpr (ACT == kActBf16) {
-    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? z_bits : 0u);
-    if constexpr (BITS == 4) {
-      uint32_t d[4];
-      dequant_int4_word_bf16<kHasZero, SHORT>(w[0], c, bs, d);
-      out = u32x4{d[0], d[1], d[2], d[3]};
-    } else {
-      uint32_t d0[2], d1[2];
-      dequant_int8_word_bf16<kHasZero, SHORT>(w[0], bs, d0);
-      dequant_int8_word_bf16<kHasZero, SHORT>(w[1], bs, d1);
-      out = u32x4{d0[0], d0[1], d1[0], d1[1]};
-    }
+    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? z_bits : 0u, make_identity4(), 0);
+    uint32_t d[4];
+    if constexpr (BITS == 4) dequant_int4_words_bf16<kHasZero, SHORT, 1>(w, c, bs, d);
+    else dequant_int8_words_bf16<kHasZero, SHORT, 2>(w, bs, d);
+    out = u32x4{d[0], d[1], d[2], d[3]};
   } else {
     const half2_t s2 = splat_low(s_bits), z2 = kHasZero ? splat_low(z_bits) : half2_t{};
     half2_t d[4];
@@ -156,7 +151,7 @@ __global__ void __launch_bounds__(kWave * kDequantWaves) dequantize_kernel(const
     }
   };
   // rows past n_out read the next group's scales or zeros: they may only cost the short form
-  if ((BITS == 4 || ACT == kActBf16) && (p.flags & kExactIntegerFormOnly) == 0 && tile_scales_permit_short_form<ACT>(s))
+  if ((BITS == 4 || ACT == kActBf16) && (p.flags & kExactIntegerFormOnly) == 0 && tile_scales_permit_short_form<BITS, ACT>(s))
     write_rows(std::true_type{});
   else
     write_rows(std::false_type{});

@@ -169,16 +169,25 @@ struct ScaleTables {
   __amdgpu_buffer_rsrc_t scale, zero;
 };
 
-// True when the scale of every lane of the wave (all groups of the unit) permits the short
-// (fp16, int4) resp. fused (bf16) dequantiser; wave-uniform, so the choice costs one scalar
-// branch per unit.
-template <int ACT, typename Bits, int GROUPS_PER_RUN>
-__device__ __forceinline__ bool wave_scales_permit_short_form(const Bits (&scale_bits)[GROUPS_PER_RUN]) {
-  bool ok = true;
+// Which form a unit takes, wave-uniform, so the choice costs one scalar branch per unit: kNoShortForm when the scale of
+// some lane (any group of the unit) does not permit the short one, else the short form's shift (int4 weights with bf16
+// scales; 0 otherwise).
+template <int BITS, int ACT, int GROUPS_PER_RUN>
+__device__ __forceinline__ int wave_short_form(const uint32_t (&scale_bits)[GROUPS_PER_RUN]) {
+  auto all_within = [&](uint32_t first, uint32_t past) {
+    bool ok = true;
 #pragma unroll
-  for (int gi = 0; gi < GROUPS_PER_RUN; ++gi)
-    ok = ok && (ACT == kActBf16 ? fused_form_ok_bf16(scale_bits[gi]) : short_form_ok(scale_bits[gi]));
-  return __builtin_amdgcn_ballot_w64(!ok) == 0;
+    for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) ok = ok && (scale_bits[gi] & 0xffffu) - first < past - first;
+    return __builtin_amdgcn_ballot_w64(!ok) == 0;
+  };
+  if constexpr (ACT != kActBf16) return all_within(kShortF16First, kShortF16Past) ? 0 : kNoShortForm;
+  if constexpr (BITS == 8) return all_within(kShortBf16Int8First, kShortBf16Int8Past) ? 0 : kNoShortForm;
+  if (all_within(kShortBf16Int4First, kShortBf16Int4Past)) return 0;
+  // other magnitudes: the same range of 12 binades, moved around the first lane's scale
+  const int exponent = (int)(__builtin_amdgcn_readfirstlane(scale_bits[0]) >> 7 & 0xffu);
+  const int shift = exponent - (127 - 11);
+  if (shift < kShortBf16MinShift || shift > kShortBf16MaxShift) return kNoShortForm;
+  return all_within(kShortBf16Int4First + (uint32_t)(shift * 128), kShortBf16Int4Past + (uint32_t)(shift * 128)) ? shift : kNoShortForm;
 }
 
 // Epilogue value before the final rounding: alpha * acc + beta * bias in fp32, the outer

@@ -102,8 +102,6 @@ gemv_mfma_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, c
       short_ok[t] = (tail.flags & kExactIntegerFormOnly) == 0;
       if constexpr (QOP == MGEMV_PER_COLUMN_SCALE_ONLY) {
         col_scale[t] = splat(p.scale[row[t]]);
-        const uint32_t bits[1] = {as_u32(col_scale[t])};
-        short_ok[t] = short_ok[t] && wave_scales_permit_short_form<kActF16>(bits);
       }
     }
     const ConvertRegs c = make_convert_regs();
@@ -292,8 +290,6 @@ gemv_mfma_lds_kernel(const uint8_t* weights, const half_t* x, const half_t* scal
   bool short_ok = (tail.flags & kExactIntegerFormOnly) == 0;
   if constexpr (QOP == MGEMV_PER_COLUMN_SCALE_ONLY) {
     col_scale = splat(p.scale[row]);
-    const uint32_t bits[1] = {as_u32(col_scale)};
-    short_ok = short_ok && wave_scales_permit_short_form<ACT>(bits);
   }
   const ConvertRegs c = make_convert_regs();
 

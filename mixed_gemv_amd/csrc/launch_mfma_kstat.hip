@@ -187,8 +187,6 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     bool short_ok = short_allowed;
     if constexpr (QOP == MGEMV_PER_COLUMN_SCALE_ONLY) {
       col_scale = splat_low(f.s[0]);
-      const uint32_t bits[1] = {f.s[0]};
-      short_ok = short_ok && wave_scales_permit_short_form<ACT>(bits);
     }
     if constexpr (PROBE == kProbeLoadsOnly) {
       uint32_t t = xa.x[0][0][0];

@@ -86,7 +86,7 @@ __device__ __forceinline__ void load_block_operands(const Activations& xa, int i
 template <int BITS, int QOP, int GROUPS_PER_RUN, bool SHORT, int ACT, typename Activations>
 __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWeights<BITS, GROUPS_PER_RUN>& f,
                                                        const Activations& xa, const ConvertRegs& c,
-                                                       half2_t col_scale2) {
+                                                       half2_t col_scale2, int shift) {
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   constexpr int kFrags = BITS == 4 ? 4 : 2;
   // The operands of block i+1 are requested before block i is dequantised, and the request is
@@ -101,24 +101,25 @@ __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWei
     const u32x4 (&op)[kFrags] = ops[i & 1];
     const int gi = i * GROUPS_PER_RUN / kBlocksPerUnit;
     if constexpr (ACT == kActBf16) {
-      // bf16: the same dequantiser as the VALU kernel (SHORT = fused form), v_mfma_f32_16x16x32_bf16
+      // bf16: the same dequantiser as the VALU kernel, v_mfma_f32_16x16x32_bf16
       const uint32_t s_bits = QOP != MGEMV_PER_COLUMN_SCALE_ONLY ? f.s[gi] : as_u32(col_scale2);
-      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u);
+      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
+      // two matrix instructions' worth of weights at a time
 #pragma unroll
-      for (int j = 0; j < kFrags; ++j) {
-        u32x4 a;
+      for (int j = 0; j < kFrags; j += 2) {
+        uint32_t d[8];
         if constexpr (BITS == 4) {
-          uint32_t d[4];
-          dequant_int4_word_bf16<kHasZero, SHORT>(f.w[i][j], c, bs, d);
-          a = u32x4{d[0], d[1], d[2], d[3]};
+          dequant_int4_words_bf16<kHasZero, SHORT, 2>({f.w[i][j], f.w[i][j + 1]}, c, bs, d);
         } else {
-          uint32_t d0[2], d1[2];
-          dequant_int8_word_bf16<kHasZero, SHORT>(f.w[i][2 * j], bs, d0);
-          dequant_int8_word_bf16<kHasZero, SHORT>(f.w[i][2 * j + 1], bs, d1);
-          a = u32x4{d0[0], d0[1], d1[0], d1[1]};
+          dequant_int8_words_bf16<kHasZero, SHORT, 4>({f.w[i][0], f.w[i][1], f.w[i][2], f.w[i][3]}, bs, d);
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                      __builtin_bit_cast(bf16x8_t, op[j]), acc, 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f32x4& sum = acc;
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, u32x4{d[4 * h], d[4 * h + 1], d[4 * h + 2], d[4 * h + 3]}),
+              __builtin_bit_cast(bf16x8_t, op[j + h]), sum, 0, 0, 0);
+        }
       }
       continue;
     }
@@ -168,14 +169,21 @@ __device__ __forceinline__ void compute_unit_mfma(f32x4& acc, const MfmaWeights<
                                                   const Activations& xa, const ConvertRegs& c,
                                                   half2_t col_scale2, bool short_allowed) {
   if constexpr (BITS == 4 || ACT == kActBf16) {
-    bool take_short = short_allowed;
-    if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) take_short = take_short && wave_scales_permit_short_form<ACT>(f.s);
-    if (take_short) {
-      compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, true, ACT>(acc, f, xa, c, col_scale2);
+    int shift = short_allowed ? 0 : kNoShortForm;
+    if (short_allowed) {
+      if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) {
+        shift = wave_short_form<BITS, ACT>(f.s);
+      } else {
+        const uint32_t bits[1] = {as_u32(col_scale2)};
+        shift = wave_short_form<BITS, ACT>(bits);
+      }
+    }
+    if (shift != kNoShortForm) {
+      compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, true, ACT>(acc, f, xa, c, col_scale2, shift);
       return;
     }
   }
-  compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2);
+  compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2, 0);
 }
 
 // Weights, scales and zeros of unit `unit` of the wave's k range through descriptors: everything
