@@ -139,7 +139,7 @@ __device__ __forceinline__ void load_operands(UnitFragment<BITS, MB, GROUPS_PER_
   for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
     int voffset;
     if constexpr (GROUPS_PER_RUN == 4) {
-      voffset = (group_of(p, c.k_run + gi * G::kChunkK) * p.n_out + c.row) * 2;
+      voffset = (group_of<4>(p, c.k_run + gi * G::kChunkK) * p.n_out + c.row) * 2;
     } else {
       voffset = c.sz_voffset[gi];
     }

@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(kWave * kDequantWaves) dequantize_kernel(const
     Problem geo{};
     geo.k = p.k;
     geo.group_size = p.group_size;
-    group = group_of(geo, k0);
+    group = group_of<4>(geo, k0);
   }
   const int table_offset = (group * p.n_out + row0) * 2;
   const uint32_t table_bytes = (uint32_t)p.num_groups * (uint32_t)p.n_out * 2u;

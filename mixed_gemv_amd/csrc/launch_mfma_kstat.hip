@@ -114,7 +114,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     const int k_run = kw * G::kStepK + slice * G::kRunK;
 #pragma unroll
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-      const int grp = QOP == MGEMV_PER_COLUMN_SCALE_ONLY ? 0 : group_of(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
+      const int grp = QOP == MGEMV_PER_COLUMN_SCALE_ONLY ? 0 : group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
       group_offset[gi] = grp * p.n_out * 2;
     }
   }

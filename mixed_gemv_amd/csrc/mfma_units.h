@@ -53,7 +53,7 @@ __device__ __forceinline__ void load_weights_mfma(MfmaWeights<BITS, GROUPS_PER_R
     const int k_run = kstep * G::kStepK + (lane / kTileRows) * G::kRunK;
 #pragma unroll
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-      const int grp = group_of(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
+      const int grp = group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
       const int idx = grp * p.n_out + row;
       f.s[gi] = load_half_bits(p.scale + idx);
       if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) f.z[gi] = load_half_bits(p.zero_add + idx);
@@ -201,7 +201,7 @@ __device__ __forceinline__ void load_weights_lds_mfma(MfmaWeights<BITS, GROUPS_P
     const int k_run = kstep * G::kStepK + (lane / kTileRows) * G::kRunK;
 #pragma unroll
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-      const int grp = group_of(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
+      const int grp = group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
       const int off = (grp * p.n_out + row) * 2;
       f.s[gi] = load_b16_low(tables.scale, off);
       if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) f.z[gi] = load_b16_low(tables.zero, off);
