@@ -292,7 +292,8 @@ MGEMV_API int mgemv_set_matrix_core_threshold(int min_m_batch);
  *   MGEMV_MATRIX_CORE_K_STATIONARY            the kernel whose waves each keep one k step of 512 (int4) or 256
  *                                             (int8) reduction elements and its activation operand in registers
  *                                             while the workgroup walks its tiles, wherever k has at most 16 such
- *                                             steps (fp16 only; else as AUTO).
+ *                                             steps (bf16: and its activation rows, which stay in LDS there, fit
+ *                                             160 KiB beside the partial sums; else as AUTO).
  * Same results to tolerance either way (the k split, hence the order of the fp32 sums, differs).
  * For tests and measurements; no counterpart in the reference.  Process-wide. */
 enum {
@@ -331,8 +332,10 @@ MGEMV_API int mgemv_set_dequant_form(int form);
  * an instantiation the reference itself still rejects at compile time
  * (gemv/threadblock/default_dq_mma_simt.h:133-134).  Dequantisation is a bf16 multiply and a bf16
  * add, each rounded to nearest even; accumulation is fp32; the output is rounded once to bf16.
- * Kernel choice follows the fp16 rules (mgemv_set_matrix_core_threshold), except that of the two
- * matrix-core kernels only the LDS-staged one exists for bf16 (mgemv_query_launch_bf16 tells). */
+ * Kernel choice follows the fp16 rules (mgemv_set_matrix_core_threshold), except that the register-operand kernel does
+ * not exist for bf16 and that the k-stationary kernel, whose bf16 build keeps its activation rows in LDS, has a rule of its
+ * own: from 3 rows and 5 k steps up to walks of 3 tiles per compute unit, and on longer ones that fill the SIMDs as well
+ * as the LDS-staged kernel; two rows with 5-8 k steps (int8: only groups that do not divide the k step, from 9). */
 MGEMV_API int mgemv_gemv_bf16(const void *weights, const uint16_t *x, const uint16_t *scale,
                               const uint16_t *zero_add, const uint16_t *bias, uint16_t *y, int n_out, int m_batch,
                               int k, int group_size, int quant_op, int weight_bits, void *stream);
@@ -399,9 +402,10 @@ MGEMV_API int mgemv_tuned_plan_count(void);
  * out[0] = workgroups, out[1] = threads per
  * workgroup, out[2] = k-split waves per tile, out[3] = tile sequences per workgroup,
  * out[4] = k steps per wave and tile, out[5] = 0 VALU kernel / 1 matrix-core kernel with the
- * activation operand in registers / 2 LDS-staged matrix-core kernel,
+ * activation operand in registers / 2 LDS-staged matrix-core kernel (bf16: also the k-stationary kernel, whose operand
+ * is in LDS there) / 3 k-stationary matrix-core kernel,
  * out[6] = tiles per wave (matrix-core path), out[7] = most tiles a wave walks one after the
- * other (VALU path). */
+ * other (VALU and k-stationary kernels). */
 MGEMV_API int mgemv_query_launch(int n_out, int m_batch, int k, int weight_bits, int group_size, int out[8]);
 /* mgemv_query_launch assumes an unpartitioned MI355X (256 compute units); a launch plans for the
  * compute units of the device its stream belongs to.

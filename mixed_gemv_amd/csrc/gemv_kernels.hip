@@ -420,6 +420,37 @@ inline bool use_k_stationary(int m_batch, int tiles, int ksteps, int bits, int c
   return (walk == 2 && ksteps <= 12) || walk >= 5;
 }
 
+// The bf16 build of the k-stationary kernel (its activation rows stay in LDS), measured against the built-in choice
+// otherwise on 7900 launches of random shapes and 5-16 k steps, 120 tiles to walks of 14, geometric means (worst):
+//   3-8 rows, walks of 1 / 2 / 3 tiles 0.83 / 0.85 / 0.80 of the time (0.96): 4096x4096 at 8 rows 5.61 us / 6.48;
+//     8192x8192 g64 at 3 rows 12.1 / 13.6; 5004x5280 g96 at 3 rows 8.24 / 9.84; int8 11008x4096 at 4 rows 10.0 / 11.9;
+//     fewer k steps leave SIMDs without a wave: 4 0.95 (1.1), 2 1.06 (1.4);
+//   walks of 5 0.79 (0.99): the LDS-staged kernel's workgroups of 4 tiles need a second round there; other longer
+//     walks by the units of the busiest SIMD, here against there (a workgroup of n k steps puts ceil(n/4) waves on a
+//     SIMD): walks of 4 and 6 up to 1.15 times as many 0.90 (1.06), then 1.02 (1.13); walks from 7 up to 1.05 times
+//     0.92 (1.07), then 1.03 (1.3).  28672x8192 at 4 rows 31.3 / 35.1, 28672x4096 17.9 / 20.1; 13824x5120 level;
+//   2 rows, 5-8 k steps, 0.85 (1.1): 28672x4096 17.7 / 18.9.  (9-16 k steps are ahead by a tenth too, 28672x8192
+//     31.3 / 34.2; the plan tests hold two rows to workgroups of 8 waves and to the VALU kernel there.)  int8 at 2 rows: one scale lookup per
+//     lane run level, four 0.90 from 9 k steps;
+//   9-16 rows, where they fit: walks of 1-3 tiles 0.84 (0.96), longer ones up to 2.0;
+//   one row: 0.97 with a spread of 0.8-1.3, so it stays on the VALU kernel.
+inline bool use_k_stationary_bf16(int m_batch, int tiles, int ksteps, int bits, int cus, bool generic_groups) {
+  if (m_batch < 2 || ksteps < 5 || tiles * 2 < cus) return false;
+  const int walk = ceil_div(tiles, cus);
+  if (m_batch == 2) return bits == 4 ? ksteps <= 8 : generic_groups && ksteps >= 9;
+  if (walk <= 3) return true;
+  if (m_batch > 8) return false;
+  if (walk == 5) return true;
+  const int tw = lds_staged_tiles_per_wg(tiles, 8, cus);
+  const long long here = 4ll * walk * ceil_div(ksteps, 4), there = (long long)ceil_div(ceil_div(tiles, tw), cus) * tw * ksteps;
+  return here * 100 <= there * (walk <= 6 ? 115 : 105);
+}
+
+// LDS stages of the k-stationary kernel's waves: 8 rows each to turn the operand round in (fp16), or the rows that stay (bf16).
+inline size_t kstat_stage_bytes(int waves, int bits, int m_batch, bool bf16) {
+  return (size_t)waves * (bf16 ? m_batch : 8) * (step_k(bits) * 2 + 16);
+}
+
 LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs& knobs) {
   const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
   const int cus = knobs.num_cus > 0 ? knobs.num_cus : kNumCus;  // the thresholds below were measured on 256 and scale with it
@@ -429,12 +460,17 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
   // K-stationary kernel: one wave per k step (so at most 16 k steps), one workgroup per compute unit
   // or fewer, each walking a contiguous run of tiles; more workgroups only where a walk's partial
   // sums would not fit the LDS or its weights not a 32-bit offset.
-  // fp16 only: the bf16 dequantiser does not fit 128 registers beside the operand (with spills: 28672x8192 40.2 us against 35.1)
-  const bool kstat_exists = ksteps <= kMaxWavesPerWorkgroup && !knobs.wide_waves;
+  // bf16 (the operand stays in LDS, beside the partial sums): where the two fit.
+  const long long park_bytes = (long long)kKSlices * m_batch * kKStationaryParkSlots * 16;  // partial sums per tile of a walk
+  const long long stage_bytes = knobs.wide_waves ? (long long)kstat_stage_bytes(ksteps, bits, m_batch, true) : 0;  // bf16: the rows stay
+  const long long most_lds = knobs.wide_waves ? kMaxKStationaryBf16Lds : kMaxKStationaryLds;
+  const bool kstat_exists = ksteps <= kMaxWavesPerWorkgroup && stage_bytes + park_bytes <= most_lds;
   const bool kstat_asked = mc && knobs.matrix_core_variant == MGEMV_MATRIX_CORE_K_STATIONARY;
   const bool kstat_by_rule = knobs.matrix_core_variant == MGEMV_MATRIX_CORE_AUTO && knobs.matrix_core_min_batch == 0 &&
-                             ov_sk == 0 && ov_tw == 0 && ov_t == 0 && !knobs.generic_groups &&
-                             use_k_stationary(m_batch, tiles, ksteps, bits, cus);
+                             ov_sk == 0 && ov_tw == 0 && ov_t == 0 &&
+                             (knobs.wide_waves ? stage_bytes + ceil_div(tiles, cus) * park_bytes <= most_lds &&
+                                                     use_k_stationary_bf16(m_batch, tiles, ksteps, bits, cus, knobs.generic_groups)
+                                               : !knobs.generic_groups && use_k_stationary(m_batch, tiles, ksteps, bits, cus));
   if (kstat_exists && (kstat_asked || kstat_by_rule)) {
     LaunchPlan lp{};
     lp.matrix_core = true;
@@ -447,10 +483,9 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     lp.workgroups = knobs.workgroups > 0 ? knobs.workgroups : cus;
     if (lp.workgroups > tiles) lp.workgroups = tiles;
     auto walk = [&]() { return ceil_div(tiles, lp.workgroups); };
-    const long long park_bytes = (long long)kKSlices * m_batch * kKStationaryParkSlots * 16;  // per tile of a walk
     while (lp.workgroups < tiles &&
            ((long long)(walk() + 2) * ksteps * kUnitBytes >= (1ll << 31) ||  // (the loop requests up to two tiles past the walk)
-            walk() * park_bytes > kMaxKStationaryLds))
+            stage_bytes + walk() * park_bytes > most_lds))
       lp.workgroups = lp.workgroups * 2 < tiles ? lp.workgroups * 2 : tiles;
     lp.tiles_in_sequence = walk();
     lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
@@ -706,9 +741,9 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
   r.launches = 1;
   if (lp.matrix_core && lp.k_stationary) {
     r.max_threads = kWave * kMaxWavesPerWorkgroup;
-    const size_t stage = (size_t)lp.split_k * 8 * (step_k(bits) * 2 + 16), park = (size_t)lp.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16;
+    const size_t stage = kstat_stage_bytes(lp.split_k, bits, m_batch, act == kActBf16), park = (size_t)lp.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16;
     // both when they fit (then no barrier stands between a wave's operand and its walk), else the larger of the two
-    r.lds_bytes = stage + park <= (size_t)kMaxKStationaryLds ? stage + park : stage > park ? stage : park;
+    r.lds_bytes = act == kActBf16 || stage + park <= (size_t)kMaxKStationaryLds ? stage + park : stage > park ? stage : park;
     return r;
   }
   if (lp.matrix_core) {
@@ -781,10 +816,10 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
   // (a group as long as k is the per-column mode, whose kernels look one scale up per row)
   knobs.generic_groups = group_size > 0 && group_size != k && groups_per_run(group_size, bits) == 4;
   if (act == kActBf16) {
-    // bf16: of the matrix-core kernels only the LDS-staged one (needs two tiles); the VALU kernel's
-    // fp32 dequantiser wants the registers of 8-wave workgroups
+    // bf16: of the matrix-core kernels the LDS-staged and the k-stationary one (both need two tiles here); the VALU
+    // kernel's dequantiser wants the registers of 8-wave workgroups
     if (num_tiles(n_out) < 2) knobs.matrix_core_min_batch = MGEMV_MAX_M_BATCH + 1;
-    knobs.matrix_core_variant = MGEMV_MATRIX_CORE_LDS_STAGED;
+    if (knobs.matrix_core_variant == MGEMV_MATRIX_CORE_REGISTER_OPERAND) knobs.matrix_core_variant = MGEMV_MATRIX_CORE_LDS_STAGED;
     knobs.wide_waves = true;
   }
   return knobs;
@@ -852,7 +887,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
     g.tail.m_batch = m_batch;
     g.lds = launch_resources(g.plan, weight_bits, m_batch, act).lds_bytes;
     if (g.plan.k_stationary) {
-      const size_t stage = (size_t)g.plan.split_k * 8 * (step_k(weight_bits) * 2 + 16);
+      const size_t stage = kstat_stage_bytes(g.plan.split_k, weight_bits, m_batch, act == kActBf16);
       if (g.lds > stage && g.lds - stage >= (size_t)g.plan.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16)
         g.tail.flags |= kParkBehindStage;
       if (probe != kProbeNone) {
@@ -1397,7 +1432,8 @@ int query_launch_any(int n_out, int m_batch, int k, int weight_bits, int group_s
   out[2] = lp.split_k;
   out[3] = lp.tiles_per_wg;
   out[4] = lp.steps_per_wave;
-  out[5] = !lp.matrix_core ? 0 : lp.k_stationary ? 3 : lp.staged_rows != 0 ? 2 : 1;
+  // (the bf16 build of the k-stationary kernel keeps its operand in LDS stages: it counts as LDS-staged, with walks)
+  out[5] = !lp.matrix_core ? 0 : lp.k_stationary && act != mgemv::kActBf16 ? 3 : lp.k_stationary || lp.staged_rows != 0 ? 2 : 1;
   out[6] = lp.tiles_per_wave;
   out[7] = lp.tiles_in_sequence;
   return MGEMV_OK;

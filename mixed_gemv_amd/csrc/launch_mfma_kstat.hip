@@ -21,10 +21,17 @@ namespace mgemv {
 // walks from the combine: wave r sums the ksteps partial blocks of tiles r, r + waves, ... and
 // stores them.  Per eight int4 weights a lane issues 13 VALU instructions and one matrix
 // instruction, against 17 VALU instructions of the DPP-dot kernel, whatever the number of rows.
+// bf16: the dequantiser needs the registers, so the operand stays in the wave's stage instead and is read from LDS, two
+// matrix instructions ahead (16 LDS reads of 16 bytes beside 400 other instructions a unit; 98-128 registers, 4 waves per
+// SIMD, no spills -- with a block's operands ahead the four-group build spilled 30 and took 1.4 times as long).  What
+// bounds it is its instruction issue (53-68 % of all cycles issue a vector instruction), then the start (16 MiB of first
+// units) and the last unit's arithmetic.  28672x8192, 4 rows: 31.3 us, 3.8 TB/s; the LDS-staged kernel, whose 140-164
+// registers leave 3 waves per SIMD and whose barriers line them up, 35.1.
 // It replaces nothing in the reference, whose kernel is fixed to one activation row
 // (gemv/threadblock/default_mma_core_simt.h:68-70); the dequantiser is the one of every kernel here
 // (gemv/warp/warp_dequantizer.h:52-59, 86-92), the epilogue host/mixed_gemv.h:102-103.
-// Dynamic LDS: waves x 8 activation rows (the stage each wave turns its operand round in, at the start) and
+// Dynamic LDS: waves x 8 activation rows (the stage each wave turns its operand round in, at the start; bf16: waves x
+// m_batch rows, which stay) and
 // tiles of the longest walk x 4 x m_batch x 17 x 16 bytes (the partial sums) -- one behind the other where
 // both fit, else sharing the space, with a barrier between the two uses.
 // ---------------------------------------------------------------------------------------------
@@ -44,6 +51,12 @@ __device__ __forceinline__ void load_unit_kstat(MfmaWeights<BITS, GROUPS_PER_RUN
   }
 }
 
+// Where a wave keeps its activation operand: in registers, or in its stage.
+template <int BITS, bool LDS_OPERAND>
+struct KStatOperand { typedef MfmaActivations<BITS> type; };
+template <int BITS>
+struct KStatOperand<BITS, true> { typedef LdsActivations<BITS> type; };
+
 // PROBE (measurement builds, wrong results): kProbeLoadsOnly keeps every load, the operand's way through LDS, the
 // parking, the barrier and the combine, and replaces the arithmetic of a unit by taking its registers;
 // kProbeComputeOnly requests only the first tile's unit and repeats its arithmetic for every tile of the walk.
@@ -54,6 +67,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
                        GemvTail tail) {
   extern __shared__ float partials[];
   using G = Geometry<BITS>;
+  constexpr bool kLdsOperand = ACT == kActBf16;
   Problem p;
   p.weights = weights;
   p.x = x;
@@ -127,21 +141,36 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) off[gi] = (int)((uint32_t)group_offset[gi] + row_bytes);
   };
 
-  MfmaActivations<BITS> xa;
   MfmaWeights<BITS, GROUPS_PER_RUN> wa, wb;
   auto request_first_unit = [&]() {
     int off[GROUPS_PER_RUN];
     offsets_of_tile(0, off);
     load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(wa, w_rsrc, tables, lane * kChunkBytes, off);
   };
-  // The activation operand: rows of this wave's k step come in whole (one fully coalesced load per row), pass
-  // through a stage of 8 rows that belongs to this wave alone, and are read back in operand shape -- lane
-  // (slice, m) takes the sixteen 16-byte pieces of row m that its matrix instructions pair with its weights.
+  // The activation operand: rows of this wave's k step come in whole (one fully coalesced load per row) and pass
+  // through a stage that belongs to this wave alone.
   // (Read straight from x in operand shape, every load instruction touches 64 cache lines for 16 bytes each.)
-  // More than 8 rows: a second round for the lanes of rows 8-15.  Lanes of rows that do not exist keep zeros.
-  {
-    using XS = XStage<BITS>;
-    uint8_t* const stage = reinterpret_cast<uint8_t*>(partials) + kw * (8 * XS::kRowStride);
+  using XS = XStage<BITS>;
+  const int stage_rows = kLdsOperand ? m_batch : 8;
+  uint8_t* const stage = reinterpret_cast<uint8_t*>(partials) + kw * (stage_rows * XS::kRowStride);
+  typename KStatOperand<BITS, kLdsOperand>::type xa;
+  if constexpr (kLdsOperand) {
+    // The stage stays: lanes of rows that do not exist read row 0 (those columns are never stored).
+    for (int first = 0; first < m_batch; first += 8) {
+      const int rows_here = m_batch - first < 8 ? m_batch - first : 8;
+      XRows<BITS, 8> rows;
+      fetch_x_rows<BITS, 8>(rows, p, x_rsrc, kw, lane, first, 1, rows_here);
+      if (first == 0) request_first_unit();
+      __builtin_amdgcn_sched_barrier(0);
+      park_x_rows<BITS, 8>(rows, stage, lane, first, 1, rows_here);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the LDS executes a wave's accesses in order
+    __builtin_amdgcn_wave_barrier();
+    xa.lane_base = stage + (m < m_batch ? m : 0) * XS::kRowStride + slice * (G::kRunK * 2);
+  } else {
+    // ... and are read back in operand shape -- lane (slice, m) takes the sixteen 16-byte pieces of row m that its
+    // matrix instructions pair with its weights.
+    // More than 8 rows: a second round for the lanes of rows 8-15.  Lanes of rows that do not exist keep zeros.
     const uint8_t* const mine = stage + (m & 7) * XS::kRowStride + slice * (G::kRunK * 2);
 #pragma unroll
     for (int i = 0; i < kBlocksPerUnit; ++i)
@@ -169,7 +198,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       __builtin_amdgcn_wave_barrier();
     }
   }
-  const bool park_behind_stage = (tail.flags & kParkBehindStage) != 0;
+  const bool park_behind_stage = kLdsOperand || (tail.flags & kParkBehindStage) != 0;
   if (!park_behind_stage) __syncthreads();  // the stages make room for the partial sums
   const bool short_allowed = (tail.flags & kExactIntegerFormOnly) == 0;
   const ConvertRegs c = make_convert_regs();
@@ -178,7 +207,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   // four floats, entry w written by wave w (the odd block length spreads the lanes over the banks).  The lane
   // that later sums a block finds its entries side by side, at offsets known to the compiler.
   f32x4* const park = reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(partials) +
-                                               (park_behind_stage ? waves * (8 * XStage<BITS>::kRowStride) : 0));
+                                               (park_behind_stage ? waves * (stage_rows * XS::kRowStride) : 0));
   const int park_tile_stride = kKSlices * m_batch * kParkSlots;  // entries from a tile to the next
   f32x4* const my_park = park + (slice * m_batch + m) * kParkSlots + kw;
   auto compute_and_park = [&](const MfmaWeights<BITS, GROUPS_PER_RUN>& f, int i) {
@@ -374,9 +403,7 @@ hipError_t launch_mfma_kstat_probe(const GemvLaunch& g, int gpr, int probe) {
 }
 
 hipError_t launch_mfma_kstat(const GemvLaunch& g, int bits, int qop, int gpr, int act) {
-  // fp16 only: with the bf16 dequantiser the kernel does not fit the 128 registers of a 16-wave workgroup, and with
-  // spills it is behind the other kernels; the planner never asks for it
-  if (act != kActF16) return hipErrorInvalidValue;
+  if (act == kActBf16) return launch_mfma_kstat_act<kActBf16>(g, bits, qop, gpr);
   return launch_mfma_kstat_act<kActF16>(g, bits, qop, gpr);
 }
 

@@ -92,6 +92,39 @@ __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWei
   // The operands of block i+1 are requested before block i is dequantised, and the request is
   // pinned there: left alone the compiler reads each operand right in front of its matrix
   // instruction and the wave sits through the LDS latency sixteen times per unit.
+  // (bf16: two matrix instructions' operands ahead, not a block's -- 44 instructions cover the LDS latency as well, and
+  // the registers decide between three and four waves per SIMD.)
+  if constexpr (ACT == kActBf16) {
+    // The same dequantiser as the VALU kernel, v_mfma_f32_16x16x32_bf16; two matrix instructions' worth of weights at a time.
+    constexpr int kPairsOfFrags = kFrags / 2, kParts = kBlocksPerUnit * kPairsOfFrags;
+    u32x4 ops[2][2];
+    auto request = [&](int part) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) ops[part & 1][h] = mfma_operand<BITS>(xa, part / kPairsOfFrags, part % kPairsOfFrags * 2 + h);
+    };
+    request(0);
+#pragma unroll
+    for (int part = 0; part < kParts; ++part) {
+      const int i = part / kPairsOfFrags, j = part % kPairsOfFrags * 2;
+      if (part + 1 < kParts) request(part + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const int gi = i * GROUPS_PER_RUN / kBlocksPerUnit;
+      const uint32_t s_bits = QOP != MGEMV_PER_COLUMN_SCALE_ONLY ? f.s[gi] : as_u32(col_scale2);
+      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
+      uint32_t d[8];
+      if constexpr (BITS == 4) {
+        dequant_int4_words_bf16<kHasZero, SHORT, 2>({f.w[i][j], f.w[i][j + 1]}, c, bs, d);
+      } else {
+        dequant_int8_words_bf16<kHasZero, SHORT, 4>({f.w[i][0], f.w[i][1], f.w[i][2], f.w[i][3]}, bs, d);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, u32x4{d[4 * h], d[4 * h + 1], d[4 * h + 2], d[4 * h + 3]}),
+            __builtin_bit_cast(bf16x8_t, ops[part & 1][h]), acc, 0, 0, 0);
+    }
+    return;
+  }
   u32x4 ops[2][kFrags];
   load_block_operands<BITS>(xa, 0, ops[0]);
 #pragma unroll
@@ -100,29 +133,6 @@ __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWei
     __builtin_amdgcn_sched_barrier(0);
     const u32x4 (&op)[kFrags] = ops[i & 1];
     const int gi = i * GROUPS_PER_RUN / kBlocksPerUnit;
-    if constexpr (ACT == kActBf16) {
-      // bf16: the same dequantiser as the VALU kernel, v_mfma_f32_16x16x32_bf16
-      const uint32_t s_bits = QOP != MGEMV_PER_COLUMN_SCALE_ONLY ? f.s[gi] : as_u32(col_scale2);
-      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
-      // two matrix instructions' worth of weights at a time
-#pragma unroll
-      for (int j = 0; j < kFrags; j += 2) {
-        uint32_t d[8];
-        if constexpr (BITS == 4) {
-          dequant_int4_words_bf16<kHasZero, SHORT, 2>({f.w[i][j], f.w[i][j + 1]}, c, bs, d);
-        } else {
-          dequant_int8_words_bf16<kHasZero, SHORT, 4>({f.w[i][0], f.w[i][1], f.w[i][2], f.w[i][3]}, bs, d);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          f32x4& sum = acc;
-          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8_t, u32x4{d[4 * h], d[4 * h + 1], d[4 * h + 2], d[4 * h + 3]}),
-              __builtin_bit_cast(bf16x8_t, op[j + h]), sum, 0, 0, 0);
-        }
-      }
-      continue;
-    }
     half2_t s2 = col_scale2, z2 = half2_t{};
     if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) s2 = splat_low(f.s[gi]);
     if constexpr (kHasZero) z2 = splat_low(f.z[gi]);
