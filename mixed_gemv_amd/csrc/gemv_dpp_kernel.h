@@ -36,7 +36,7 @@ struct UnitFragment {
 // GROUPS_PER_RUN 1 or 2 ("regular"): the group size divides the k step (or there is a single
 // group, the per-column mode), so a lane's scale / zero offset advances by a constant per
 // unit.  GROUPS_PER_RUN 4 ("generic", any group size that is a multiple of 32): one lookup
-// per block with an integer division.
+// per block (group_of).
 template <int BITS, int GROUPS_PER_RUN>
 struct WaveCursor {
   int w_voffset;                   // byte offset of this lane's chunk of block 0 inside the wave's weight range
