@@ -623,6 +623,19 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     // The bfloat16 kernels are bound by their arithmetic, and two-unit waves are their worst
     // length by far (13824x5120: 18.9 us at 5 waves of 2 units against 14.0 at 2 waves of 5).
     if (knobs.wide_waves && !mc && split_k > 1 && ceil_div(ksteps, split_k) == 2) split_k = (split_k + 1) / 2;
+    // A single bf16 row on 700 and more tiles, up to 16 k steps.  A wave per k step leaves the SIMDs with unequal numbers
+    // of them and turns workgroups over for one unit each: int4, 3 or 4 waves instead take, geometric means (worst), with 5
+    // k steps 0.80 of the time (1.04), 6 0.87 (1.0), 7 0.91-0.95 (1.05), 8 level (but with four groups per
+    // lane run 0.85); int8 is level.  Two waves per tile, where the wave budget stops at that, are too few for one or two groups per run: four take
+    // 0.93 with 7-8 k steps (int8 0.95), 0.99 with 9-10, 0.95-0.98 with 11-16; with four groups 0.94-1.09.  So is one wave
+    // with 4 k steps (0.92, int8 0.85).
+    if (knobs.wide_waves && !mc && m_batch == 1 && tiles * 8 >= cus * 22 && ksteps <= 16) {
+      if (bits == 4 && ksteps >= 5 && split_k == ksteps) {
+        if (ksteps < 8 || knobs.generic_groups) split_k = ksteps <= 6 ? 3 : 4;
+      } else if (!knobs.generic_groups && (split_k == 2 ? ksteps >= 7 : split_k == 1 && ksteps == 4)) {
+        split_k = 4;
+      }
+    }
   }
   int tiles_per_wg = pair_tiles ? 2 : 1;
   int workgroup_cap = 0;
