@@ -90,15 +90,18 @@ MGEMV_API int mgemv_version(void);
  * Packs n_unpacked signed 4-bit values held one per int8 into n_unpacked/2 bytes (an odd
  * n_unpacked is MGEMV_ERR_SIZE):
  * element 2i in bits 0..3 of byte i, element 2i+1 in bits 4..7.  Values are truncated to
- * their low 4 bits, as in the reference. */
+ * their low 4 bits, as in the reference.
+ * packed may be unpacked itself, or begin in front of it: such a call runs on one thread, in ascending order. */
 MGEMV_API int mgemv_pack_int4(uint8_t *packed, const int8_t *unpacked, size_t n_unpacked);
 
-/* Replaces SubBytePacker<int4b_t,int8_t>::unpack (utils/preprocess.h:41-53): sign-extending inverse. */
+/* Replaces SubBytePacker<int4b_t,int8_t>::unpack (utils/preprocess.h:41-53): sign-extending inverse.
+ * packed may be the upper half of unpacked (one thread, ascending order). */
 MGEMV_API int mgemv_unpack_int4(int8_t *unpacked, const uint8_t *packed, size_t n_packed);
 
 /* Replaces ZeroPointPreprocessor<half_t,int8_t>::neg_zero_point_multiplies_scale
  * (utils/preprocess.h:94-101): out[i] = fp16(-zeros[i]) * scales[i], one fp16 multiply.
- * The result is the additive term the GEMV takes as `zero_add` (mixed_gemv_test.cu:237-239, 275). */
+ * The result is the additive term the GEMV takes as `zero_add` (mixed_gemv_test.cu:237-239, 275).
+ * out may be scales itself, or begin in front of it, and zeros may be out's upper half (one thread, ascending order). */
 MGEMV_API int mgemv_fold_zero_points(uint16_t *out, const uint16_t *scales, const int8_t *zeros, size_t n);
 
 /* Bytes that mgemv_preprocess_weights writes for this shape (>= the input size: rows are
@@ -123,7 +126,7 @@ MGEMV_API int mgemv_preprocess_weights(uint8_t *dst, const uint8_t *src, const s
 
 /* Inverse of mgemv_preprocess_weights for MGEMV_COLUMN_MAJOR input: recovers the n_out x k
  * row-major quantised weights from a preprocessed buffer.  No counterpart in the reference;
- * it exists so that layouts can be audited and round-trip tested. */
+ * it exists so that layouts can be audited and round-trip tested.  dst may not alias src_preprocessed. */
 MGEMV_API int mgemv_unpreprocess_weights(uint8_t *dst, const uint8_t *src_preprocessed, const size_t *shape,
                                          int rank, int quant_type);
 

@@ -45,10 +45,16 @@ inline void float_to_half_bits(const f32x8& f, u16x8& h) {
 // Elements a thread should have at least (a few microseconds' work: what starting the others costs).
 constexpr size_t kGrain = (size_t)1 << 15;
 
-// fn(first, last) over pieces of `grain` elements of [0, n), side by side where there is enough to do.
+bool share_memory(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+  return a0 < b0 + b_bytes && b0 < a0 + a_bytes;
+}
+
+// fn(first, last) over pieces of `grain` elements of [0, n), side by side where there is enough to do.  in_order: one
+// ascending piece, for a result that lies over its operands -- a thread would write what another has yet to read.
 template <typename Fn>
-void in_pieces(size_t n, size_t grain, Fn fn) {
-  const size_t pieces = (n + grain - 1) / grain;
+void in_pieces(size_t n, size_t grain, bool in_order, Fn fn) {
+  const size_t pieces = in_order ? 1 : (n + grain - 1) / grain;
   if (pieces <= 1) {
     fn((size_t)0, n);
     return;
@@ -208,7 +214,8 @@ int mgemv_pack_int4(uint8_t* packed, const int8_t* unpacked, size_t n_unpacked) 
   // 32 elements at a time: a 16-bit pair holds element 2i in its low byte and 2i + 1 in its high one
   typedef uint16_t pairs16 __attribute__((vector_size(32), aligned(1), may_alias));
   typedef uint8_t bytes16 __attribute__((vector_size(16), aligned(1), may_alias));
-  in_pieces(n_unpacked / 2, kGrain, [=](size_t first, size_t last) {
+  const bool in_order = share_memory(packed, n_unpacked / 2, unpacked, n_unpacked);
+  in_pieces(n_unpacked / 2, kGrain, in_order, [=](size_t first, size_t last) {
     size_t i = first;
     for (; i + 16 <= last; i += 16) {
       const pairs16 v = *reinterpret_cast<const pairs16*>(unpacked + 2 * i);
@@ -224,7 +231,8 @@ int mgemv_unpack_int4(int8_t* unpacked, const uint8_t* packed, size_t n_packed) 
   if (n_packed == 0) return MGEMV_OK;
   if (packed == nullptr || unpacked == nullptr) return MGEMV_ERR_NULL_POINTER;
   typedef int8_t bytes16 __attribute__((vector_size(16), aligned(1), may_alias));
-  in_pieces(n_packed, kGrain, [=](size_t first, size_t last) {
+  const bool in_order = share_memory(unpacked, 2 * n_packed, packed, n_packed);
+  in_pieces(n_packed, kGrain, in_order, [=](size_t first, size_t last) {
     size_t i = first;
     for (; i + 16 <= last; i += 16) {
       const bytes16 v = *reinterpret_cast<const bytes16*>(packed + i);
@@ -246,7 +254,8 @@ int mgemv_fold_zero_points(uint16_t* out, const uint16_t* scales, const int8_t* 
   if (out == nullptr || scales == nullptr || zeros == nullptr) return MGEMV_ERR_NULL_POINTER;
   // -z is an integer of magnitude <= 128: exact in binary16.  The binary32 product of two
   // halves is exact, so one rounding to binary16 is the correctly rounded fp16 multiply.
-  in_pieces(n, kGrain / 4, [=](size_t first, size_t last) {
+  const bool in_order = share_memory(out, 2 * n, scales, 2 * n) || share_memory(out, 2 * n, zeros, n);
+  in_pieces(n, kGrain / 4, in_order, [=](size_t first, size_t last) {
     for (size_t i = first; i < last; i += 8) {
       const size_t here = last - i < 8 ? last - i : 8;
       u16x8 s = {}, r;
@@ -266,7 +275,8 @@ int mgemv_fold_zero_points(uint16_t* out, const uint16_t* scales, const int8_t* 
 int mgemv_fold_zero_points_bf16(uint16_t* out, const uint16_t* scales, const int8_t* zeros, size_t n) {
   if (n == 0) return MGEMV_OK;
   if (out == nullptr || scales == nullptr || zeros == nullptr) return MGEMV_ERR_NULL_POINTER;
-  in_pieces(n, kGrain / 4, [=](size_t first, size_t last) {
+  const bool in_order = share_memory(out, 2 * n, scales, 2 * n) || share_memory(out, 2 * n, zeros, n);
+  in_pieces(n, kGrain / 4, in_order, [=](size_t first, size_t last) {
     for (size_t i = first; i < last; ++i) {
       // -z has at most 8 significant bits: exact in bfloat16.  The binary32 product of two
       // bfloat16 values is exact, so one rounding (nearest even) is the correctly rounded multiply.
