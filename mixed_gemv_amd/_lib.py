@@ -101,8 +101,8 @@ def lib():
 
 
 def py_calls():
-    """The extension module that unpacks torch tensors and calls the library (csrc/py_calls.cpp); raises if it is
-    missing.  The library is loaded in front of it, so that the two share one copy."""
+    """The extension module that unpacks torch tensors and calls the library (csrc/py_calls.cpp), for a process that has
+    PyTorch; raises if it is missing.  The library is loaded in front of it, so that the two share one copy."""
     import importlib.machinery
     import importlib.util
     lib()

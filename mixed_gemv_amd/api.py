@@ -2,7 +2,7 @@
 
 Host utilities take and return numpy arrays.  Device entry points take anything exposing a
 device address: a torch tensor on the GPU, or a plain integer address.  PyTorch is used only
-as the owner of device memory and streams.
+as the owner of device memory and streams; without it, addresses and integer streams still work.
 """
 import ctypes
 import enum
@@ -79,13 +79,46 @@ def _stream_ptr(stream):
     return ctypes.c_void_p(_stream_address(stream))
 
 
-_calls = None  # the device entry points as CPython calls (csrc/py_calls.cpp), loaded with the first of them
+_calls = None  # the device entry points, by position: py_calls.so, or _CtypesCalls where there is no PyTorch
+
+
+class _CtypesCalls:
+    """The functions of csrc/py_calls.cpp for a process without PyTorch, whose operands are integer addresses.  (The
+    extension links against PyTorch's libraries.  It takes 4 us a call; this takes 9.)"""
+
+    @staticmethod
+    def _entry(name, element, probe):
+        return getattr(_lib.lib(), name + ("_bf16" if _is_bf16(element, probe) else ""))
+
+    @classmethod
+    def gemv(cls, w, x, s, z, c, y, batch, n_out, m, k, group, op, bits, stream, batch_strides, element):
+        sa, sb, ss, sc, sd = batch_strides or (0, 0, 0, 0, 0)
+        return cls._entry("mgemv_gemv_batched", element, x)(
+            *map(_dev_ptr, (w, x, s, z, c, y)), *map(int, (batch, n_out, m, k, group, op, bits, sa, sb, ss, sc, sd)),
+            _stream_ptr(stream))
+
+    @classmethod
+    def gemv_routed(cls, w, x, s, z, c, y, route, entries, batch, n_out, m, k, group, batch_strides, op, bits, stream, element):
+        sa, sb, ss, sc, sd = batch_strides
+        return cls._entry("mgemv_gemv_routed", element, x)(
+            *map(_dev_ptr, (w, x, s, z, c, y, route)),
+            *map(int, (entries, batch, n_out, m, k, group, op, bits, sa, sb, ss, sc, sd)), _stream_ptr(stream))
+
+    @classmethod
+    def dequantize(cls, w, s, z, out, n_out, k, group, op, bits, stream, element):
+        return cls._entry("mgemv_dequantize", element, s)(
+            *map(_dev_ptr, (w, s, z, out)), *map(int, (n_out, k, group, op, bits)), _stream_ptr(stream))
 
 
 def _native_calls():
     global _calls
     if _calls is None:
-        _calls = _lib.py_calls()
+        try:
+            import torch  # noqa: F401
+        except ImportError:
+            _calls = _CtypesCalls
+        else:
+            _calls = _lib.py_calls()
     return _calls
 
 

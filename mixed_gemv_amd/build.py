@@ -97,9 +97,16 @@ def write_default_plans(path):
 
 def build_py_calls(verbose=True):
     """csrc/py_calls.cpp -> lib/py_calls.so.  PyTorch's libraries are named without a path: the process that loads the
-    module has them already."""
+    module has them already.  Without PyTorch there is nothing to build it against, nor anyone to load it (api.py goes
+    through ctypes there): returns None, and leaves none behind from an earlier build."""
     import sysconfig
-    import torch
+    try:
+        import torch
+    except ImportError:
+        if os.path.exists(PY_CALLS_PATH):
+            os.remove(PY_CALLS_PATH)
+        print("py_calls: not built, PyTorch is not installed", flush=True)
+        return None
     torch_dir = os.path.dirname(torch.__file__)
     torch_include = os.path.join(torch_dir, "include")
     rocm_include = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc()))), "include")
