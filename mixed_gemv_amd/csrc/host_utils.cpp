@@ -109,8 +109,8 @@ void transpose_quantised(uint8_t* dst, const uint8_t* src, size_t k, size_t n_ou
   }
 }
 
-// Four words at a time; the compiler makes SSE2 of it (or whatever the target has).
-typedef uint32_t word4 __attribute__((vector_size(16), aligned(4), may_alias));
+// Four words at a time, of buffers at any address; the compiler makes SSE2 of it (or whatever the target has).
+typedef uint32_t word4 __attribute__((vector_size(16), aligned(1), may_alias));
 template <typename W>
 inline W encode_int4(W natural) {
   const W b = natural ^ 0x88888888u;
