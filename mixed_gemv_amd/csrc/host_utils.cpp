@@ -111,23 +111,10 @@ void transpose_quantised(uint8_t* dst, const uint8_t* src, size_t k, size_t n_ou
 
 // Four words at a time, of buffers at any address; the compiler makes SSE2 of it (or whatever the target has).
 typedef uint32_t word4 __attribute__((vector_size(16), aligned(1), may_alias));
-template <typename W>
-inline W encode_int4(W natural) {
-  const W b = natural ^ 0x88888888u;
-  const W f5 = b & 0x00f00000u;
-  return ((b & 0x0000000fu) << 7) | ((b & 0x000000f0u) << 19) | ((b & 0x00000f00u) >> 5) | ((b & 0x0000f000u) << 7) |
-         ((b & 0x000f0000u) >> 1) | (f5 << 11) | (f5 >> 21) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
-}
-template <typename W>
-inline W decode_int4(W w) {
-  const W f5 = ((w >> 11) | (w << 21)) & 0x00f00000u;
-  return (((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) | ((w >> 7) & 0x0000f000u) |
-          ((w << 1) & 0x000f0000u) | f5 | ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u)) ^ 0x88888888u;
-}
 template <int BITS, bool DECODE>
 inline word4 recode_chunk(word4 w) {
-  if (BITS == 8) return w ^ 0x80808080u;
-  return DECODE ? decode_int4(w) : encode_int4(w);
+  if (BITS == 8) return mgemv::recode_int8(w);
+  return DECODE ? mgemv::decode_int4(w) : mgemv::encode_int4(w);
 }
 
 // One 16-row tile between rows (row_bytes apart, `rows` of them) and its units.  A lane's run -- 64 bytes of one row, whose

@@ -24,8 +24,8 @@
 // instructions, so the small-batch path consumes the identical buffer.
 //
 // A chunk is four 32-bit words in ascending k.  int4: a word holds 8 consecutive elements,
-// each stored biased (value + 8) as a 4-bit field whose least significant bit sits at bit
-// int4_field_shift(e) of the word (the field of element 5 wraps round from bit 31 to bits 0-2):
+// each stored biased (value + 8) as a 4-bit field at these bits of the word (the field of element 5
+// wraps round from bit 31 to bits 0-2):
 //     e      0   1   2   3   4   5   6   7
 //     bits  7-10 23-26 3-6 19-22 15-18 31,0-2 11-14 27-30
 // The k-adjacent pair (2h, 2h+1) always lands at the SAME position of the two 16-bit halves,
@@ -65,7 +65,6 @@ struct Geometry {
   static constexpr int kChunkK = kChunkBytes * 8 / BITS;        // 32 | 16
   static constexpr int kRunK = kBlocksPerUnit * kChunkK;        // 128 | 64
   static constexpr int kStepK = kKSlices * kRunK;               // 512 | 256
-  static constexpr int kWordK = 32 / BITS;                      // 8 | 4
 };
 
 MGEMV_HD int chunk_k(int bits) { return kChunkBytes * 8 / bits; }
@@ -79,38 +78,24 @@ MGEMV_HD size_t preprocessed_bytes(size_t n_out, size_t k, int bits) {
   return t * s * (size_t)kUnitBytes;
 }
 
-// Byte offset of the chunk holding (row n, reduction index k0), k0 a multiple of kChunkK.
-MGEMV_HD size_t chunk_offset(size_t n, size_t k0, size_t ksteps, int bits) {
-  const size_t ck = (size_t)chunk_k(bits), rk = (size_t)run_k(bits), sk = (size_t)step_k(bits);
-  size_t t = n / kTileRows, r = n % kTileRows;
-  size_t s = k0 / sk, kk = k0 % sk;
-  size_t slice = kk / rk, blk = (kk % rk) / ck;
-  size_t lane = slice * kTileRows + r;
-  return (t * ksteps + s) * (size_t)kUnitBytes + blk * (size_t)kBlockBytes + lane * (size_t)kChunkBytes;
-}
-
-// int4 word: natural order (element e in bits 4e..4e+3, two's complement) <-> stored order.
-MGEMV_HD uint32_t rotl32(uint32_t v, int s) { return s ? (v << s) | (v >> (32 - s)) : v; }
-MGEMV_HD uint32_t rotr32(uint32_t v, int s) { return s ? (v >> s) | (v << (32 - s)) : v; }
-MGEMV_HD int int4_field_shift(int e) {
-  return e == 0 ? 7 : e == 1 ? 23 : e == 2 ? 3 : e == 3 ? 19 : e == 4 ? 15 : e == 5 ? 31 : e == 6 ? 11 : 27;
-}
-// Straight-line forms of "field e moves from bit 4e to bit int4_field_shift(e)" (the host
-// preprocessor spends its time here).
-MGEMV_HD uint32_t encode_int4_word(uint32_t natural) {
-  const uint32_t b = natural ^ 0x88888888u;  // +8 on each two's-complement nibble
+// 32-bit words (W: one, or a vector of them) in natural order -- int4: element e in bits 4e..4e+3, two's complement --
+// to stored order and back.
+template <typename W>
+MGEMV_HD W encode_int4(W natural) {
+  const W b = natural ^ 0x88888888u;  // +8 on each two's-complement nibble
+  const W f5 = b & 0x00f00000u;
   return ((b & 0x0000000fu) << 7) | ((b & 0x000000f0u) << 19) | ((b & 0x00000f00u) >> 5) | ((b & 0x0000f000u) << 7) |
-         ((b & 0x000f0000u) >> 1) | rotl32(b & 0x00f00000u, 11) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
+         ((b & 0x000f0000u) >> 1) | (f5 << 11) | (f5 >> 21) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
 }
-MGEMV_HD uint32_t decode_int4_word(uint32_t stored) {
-  const uint32_t w = stored;
-  const uint32_t b = ((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) |
-                     ((w >> 7) & 0x0000f000u) | ((w << 1) & 0x000f0000u) | (rotr32(w, 11) & 0x00f00000u) |
-                     ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u);
-  return b ^ 0x88888888u;
+template <typename W>
+MGEMV_HD W decode_int4(W w) {
+  const W f5 = ((w >> 11) | (w << 21)) & 0x00f00000u;
+  return (((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) | ((w >> 7) & 0x0000f000u) |
+          ((w << 1) & 0x000f0000u) | f5 | ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u)) ^ 0x88888888u;
 }
-MGEMV_HD uint32_t encode_int8_word(uint32_t natural) { return natural ^ 0x80808080u; }
-MGEMV_HD uint32_t decode_int8_word(uint32_t stored) { return stored ^ 0x80808080u; }
+// (its own inverse)
+template <typename W>
+MGEMV_HD W recode_int8(W w) { return w ^ 0x80808080u; }
 
 }  // namespace mgemv
 
