@@ -405,15 +405,14 @@ MGEMV_API int mgemv_tuned_plan_count(void);
  * out[0] = workgroups, out[1] = threads per
  * workgroup, out[2] = k-split waves per tile, out[3] = tile sequences per workgroup,
  * out[4] = k steps per wave and tile, out[5] = 0 VALU kernel / 1 matrix-core kernel with the
- * activation operand in registers / 2 LDS-staged matrix-core kernel (bf16: also the k-stationary kernel, whose operand
- * is in LDS there) / 3 k-stationary matrix-core kernel,
+ * activation operand in registers / 2 LDS-staged matrix-core kernel / 3 k-stationary matrix-core kernel,
  * out[6] = tiles per wave (matrix-core path), out[7] = most tiles a wave walks one after the
  * other (VALU and k-stationary kernels). */
 MGEMV_API int mgemv_query_launch(int n_out, int m_batch, int k, int weight_bits, int group_size, int out[8]);
 /* mgemv_query_launch assumes an unpartitioned MI355X (256 compute units); a launch plans for the
  * compute units of the device its stream belongs to.
- * The same for the _bf16 entry points (their kernels are compiled for at most 8 waves per workgroup, and of
- * the matrix-core kernels only the LDS-staged one exists for bf16). */
+ * The same for the _bf16 entry points (their kernels are compiled for at most 8 waves per workgroup, the k-stationary one
+ * for 16, and the register-operand kernel does not exist for bf16). */
 MGEMV_API int mgemv_query_launch_bf16(int n_out, int m_batch, int k, int weight_bits, int group_size, int out[8]);
 /* The same for either element type (MGEMV_ELEMENT_*) and a device of num_compute_units compute
  * units (a partition of an MI355X has 32 per XCD), plus what the plan asks of the hardware:

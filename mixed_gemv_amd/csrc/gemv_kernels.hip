@@ -1445,8 +1445,7 @@ int query_launch_any(int n_out, int m_batch, int k, int weight_bits, int group_s
   out[2] = lp.split_k;
   out[3] = lp.tiles_per_wg;
   out[4] = lp.steps_per_wave;
-  // (the bf16 build of the k-stationary kernel keeps its operand in LDS stages: it counts as LDS-staged, with walks)
-  out[5] = !lp.matrix_core ? 0 : lp.k_stationary && act != mgemv::kActBf16 ? 3 : lp.k_stationary || lp.staged_rows != 0 ? 2 : 1;
+  out[5] = !lp.matrix_core ? 0 : lp.k_stationary ? 3 : lp.staged_rows != 0 ? 2 : 1;
   out[6] = lp.tiles_per_wave;
   out[7] = lp.tiles_in_sequence;
   return MGEMV_OK;

@@ -580,7 +580,7 @@ def test_k_stationary_clauses_found_by_the_audits_of_random_shapes():
 
 def test_bf16_launch_rules_differ_where_they_were_measured_to():
     """The bfloat16 kernels are bound by arithmetic: no tile walks, no whole-k single-wave workgroups,
-    no two-unit waves; at most 8 waves per workgroup."""
+    no two-unit waves; at most 8 waves per workgroup of the VALU and LDS-staged kernels."""
     q = lambda n, m, k: mg.query_launch(n, m, k, 4, 128, element="bf16")
     c5 = q(28672, 1, 8192)
     assert (c5["workgroups"], c5["split_k"], c5["tiles_in_sequence"]) == (1792, 4, 1), c5
@@ -588,11 +588,25 @@ def test_bf16_launch_rules_differ_where_they_were_measured_to():
     mlp = q(13824, 1, 5120)
     assert mlp["split_k"] > 1 and mlp["steps_per_wave"] != 2, mlp
     assert mg.query_launch(13824, 1, 5120, 4, 128)["split_k"] == 1                 # fp16: whole-k waves
-    assert q(28672, 2, 8192)["matrix_core"] == 0 and q(28672, 3, 8192)["matrix_core"] == 2   # 2 rows stay on the VALU kernel
+    # walks of 7 tiles fill the SIMDs as the LDS-staged workgroups do: k-stationary from 3 rows (31.3 us / 35.1 at 4 rows)
+    assert q(28672, 2, 8192)["matrix_core"] == 0 and q(28672, 3, 8192)["matrix_core"] == 3   # 2 rows stay on the VALU kernel
     assert q(8192, 1, 8192)["workgroups"] == 256                                   # one tile per sequence: kept
     for n, m, k in [(4096, 1, 4096), (1024, 1, 8192), (22016, 1, 4096), (5120, 2, 5120), (4096, 16, 4096)]:
         assert q(n, m, k)["threads"] <= 512, (n, m, k)
-        assert q(n, m, k)["matrix_core"] in (0, 2)                                 # no register-operand kernel for bf16
+        assert q(n, m, k)["matrix_core"] in (0, 2, 3)                              # no register-operand kernel for bf16
+
+
+def test_the_query_tells_the_bf16_matrix_core_kernels_apart():
+    q = lambda *p: mg.query_launch(*p, element="bf16")["matrix_core"]  # noqa: E731
+    shapes = [(4096, 16, 4096, 4, 128), (28672, 4, 8192, 4, 128), (5004, 3, 5280, 4, 96), (11008, 4, 4096, 8, 0)]
+    assert [q(*s) for s in shapes] == [3] * 4
+    assert q(28672, 8, 7168, 4, 128) == 2 and q(1024, 5, 2048, 4, 128) == 2    # walks of 7 with 14 k steps; 4 k steps
+    for variant, kind in ((mg.MATRIX_CORE_LDS_STAGED, 2), (mg.MATRIX_CORE_K_STATIONARY, 3)):
+        mg.set_matrix_core_variant(variant)
+        try:
+            assert [q(*s) for s in shapes] == [kind] * 4
+        finally:
+            mg.set_matrix_core_variant(mg.MATRIX_CORE_AUTO)
 
 
 def test_int8_weights_keep_two_to_four_rows_on_the_valu_kernel():

@@ -57,7 +57,7 @@ def test_plan_covers_the_problem(case):
         plan = mg.query_launch(n_out, rows, k, bits, k if qop == PER_COLUMN else group, element="bf16")
         cover = mg.plan_coverage(n_out, rows, k, bits, k if qop == PER_COLUMN else group, element="bf16")
     assert plan["split_k"] == ksteps and plan["steps_per_wave"] == 1 and plan["tiles_per_wg"] == 1, plan
-    assert plan["matrix_core"] == 2 and plan["tiles_in_sequence"] == -(-(-(-n_out // 16)) // (cap or 256)), plan
+    assert plan["matrix_core"] == 3 and plan["tiles_in_sequence"] == -(-(-(-n_out // 16)) // (cap or 256)), plan
     assert cover["lds_bytes"] == ksteps * rows * ((1024 if bits == 4 else 512) + 16) + plan["tiles_in_sequence"] * 4 * rows * 17 * 16
     assert cover["lds_bytes"] <= 160 * 1024 and cover["tiles_miscovered"] == 0 and cover["bad_waves"] == 0, cover
 
@@ -93,7 +93,7 @@ def test_batched_launch_matches_single_launches(gpu):
     bias = torch.randn((count, n_out), device=gpu, generator=gen).to(torch.bfloat16)
     y = torch.zeros((count, rows, n_out), dtype=torch.bfloat16, device=gpu)
     single = torch.zeros_like(y)
-    assert mg.query_launch(n_out, rows, k, 4, 128, element="bf16")["split_k"] == 8
+    assert mg.query_launch(n_out, rows, k, 4, 128, element="bf16")["matrix_core"] == 3
     mg.device_gemv(w, x, s, z, bias, y, count, n_out, rows, k, 128, SCALE_AND_ZEROS, 4,
                    batch_strides=(w_bytes, rows * k, k // 128 * n_out, n_out, rows * n_out))
     for b in range(count):
