@@ -598,7 +598,7 @@ def test_bf16_launch_rules_differ_where_they_were_measured_to():
 
 def test_the_query_tells_the_bf16_matrix_core_kernels_apart():
     q = lambda *p: mg.query_launch(*p, element="bf16")["matrix_core"]  # noqa: E731
-    shapes = [(4096, 16, 4096, 4, 128), (28672, 4, 8192, 4, 128), (5004, 3, 5280, 4, 96), (11008, 4, 4096, 8, 0)]
+    shapes = [(4096, 16, 4096, 4, 128), (28672, 4, 8192, 4, 128), (5004, 3, 5280, 4, 96), (11008, 8, 4096, 8, 0)]
     assert [q(*s) for s in shapes] == [3] * 4
     assert q(28672, 8, 7168, 4, 128) == 2 and q(1024, 5, 2048, 4, 128) == 2    # walks of 7 with 14 k steps; 4 k steps
     for variant, kind in ((mg.MATRIX_CORE_LDS_STAGED, 2), (mg.MATRIX_CORE_K_STATIONARY, 3)):
