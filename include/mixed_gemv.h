@@ -338,7 +338,7 @@ MGEMV_API int mgemv_set_dequant_form(int form);
  * Kernel choice follows the fp16 rules (mgemv_set_matrix_core_threshold), except that the register-operand kernel does
  * not exist for bf16 and that the k-stationary kernel, whose bf16 build keeps its activation rows in LDS, has a rule of its
  * own: from 3 rows and 5 k steps up to walks of 3 tiles per compute unit, and on longer ones that fill the SIMDs as well
- * as the LDS-staged kernel; two rows with 5-8 k steps (int8: only groups that do not divide the k step, from 9). */
+ * as the LDS-staged kernel; two rows from 5 k steps (int8: only groups that do not divide the k step, from 9). */
 MGEMV_API int mgemv_gemv_bf16(const void *weights, const uint16_t *x, const uint16_t *scale,
                               const uint16_t *zero_add, const uint16_t *bias, uint16_t *y, int n_out, int m_batch,
                               int k, int group_size, int quant_op, int weight_bits, void *stream);

@@ -429,15 +429,19 @@ inline bool use_k_stationary(int m_batch, int tiles, int ksteps, int bits, int c
 //     walks by the units of the busiest SIMD, here against there (a workgroup of n k steps puts ceil(n/4) waves on a
 //     SIMD): walks of 4 and 6 up to 1.15 times as many 0.90 (1.06), then 1.02 (1.13); walks from 7 up to 1.05 times
 //     0.92 (1.07), then 1.03 (1.3).  28672x8192 at 4 rows 31.3 / 35.1, 28672x4096 17.9 / 20.1; 13824x5120 level;
-//   2 rows, 5-8 k steps, 0.85 (1.1): 28672x4096 17.7 / 18.9.  (9-16 k steps are ahead by a tenth too, 28672x8192
-//     31.3 / 34.2; the plan tests hold two rows to workgroups of 8 waves and to the VALU kernel there.)  int8 at 2 rows: one scale lookup per
-//     lane run level, four 0.90 from 9 k steps;
+//   2 rows, against the VALU kernel's waves: 5-8 k steps 0.85 (1.1), 28672x4096 17.7 / 18.9; 9-16 k steps, 3500 launches,
+//     0.87 (1.07), 28672x8192 31.3 / 34.2 -- but 1.0 (1.13) on walks of 4 with 9, 10 or 13 k steps, where the waves of a
+//     workgroup leave a SIMD or two idle a sixth of the time and more, and four groups per lane run do not make up for it
+//     (15312x4608 13.5 / 12.0).  int8 at 2 rows: one scale lookup per lane run level, four 0.90 from 9 k steps;
 //   9-16 rows, where they fit: walks of 1-3 tiles 0.84 (0.96), longer ones up to 2.0;
 //   one row: 0.97 with a spread of 0.8-1.3, so it stays on the VALU kernel.
 inline bool use_k_stationary_bf16(int m_batch, int tiles, int ksteps, int bits, int cus, bool generic_groups) {
   if (m_batch < 2 || ksteps < 5 || tiles * 2 < cus) return false;
   const int walk = ceil_div(tiles, cus);
-  if (m_batch == 2) return bits == 4 ? ksteps <= 8 : generic_groups && ksteps >= 9;
+  if (m_batch == 2) {
+    if (bits == 8) return generic_groups && ksteps >= 9;
+    return ksteps <= 8 || walk != 4 || generic_groups || 4 * ceil_div(ksteps, 4) * 6 < ksteps * 7;
+  }
   if (walk <= 3) return true;
   if (m_batch > 8) return false;
   if (walk == 5) return true;

@@ -589,9 +589,15 @@ def test_bf16_launch_rules_differ_where_they_were_measured_to():
     assert mlp["split_k"] > 1 and mlp["steps_per_wave"] != 2, mlp
     assert mg.query_launch(13824, 1, 5120, 4, 128)["split_k"] == 1                 # fp16: whole-k waves
     # walks of 7 tiles fill the SIMDs as the LDS-staged workgroups do: k-stationary from 3 rows (31.3 us / 35.1 at 4 rows)
-    assert q(28672, 2, 8192)["matrix_core"] == 0 and q(28672, 3, 8192)["matrix_core"] == 3   # 2 rows stay on the VALU kernel
+    assert q(28672, 3, 8192)["matrix_core"] == 3
+    # ... and 2 rows with 9-16 k steps (28672x8192 31.3 us / 34.2 on the VALU kernel), but for walks of 4 whose k steps leave
+    # SIMDs idle (15312x4608 13.5 / 12.0)
+    assert [q(n, 2, k)["matrix_core"] for n, k in ((28672, 8192), (5120, 5120), (15312, 6144), (20480, 4608))] == [3] * 4
+    assert [q(15312, 2, 512 * ks)["matrix_core"] for ks in range(8, 17)] == [3, 0, 0, 3, 3, 0, 3, 3, 3]
+    assert mg.query_launch(15312, 2, 4608, 4, 96, element="bf16")["matrix_core"] == 3      # four groups per lane run: level at worst
+    assert q(2032, 2, 8192)["matrix_core"] == 0 and q(4096, 2, 8704)["matrix_core"] == 0   # 127 tiles; 17 k steps
     assert q(8192, 1, 8192)["workgroups"] == 256                                   # one tile per sequence: kept
-    for n, m, k in [(4096, 1, 4096), (1024, 1, 8192), (22016, 1, 4096), (5120, 2, 5120), (4096, 16, 4096)]:
+    for n, m, k in [(4096, 1, 4096), (1024, 1, 8192), (22016, 1, 4096), (4096, 16, 4096)]:
         assert q(n, m, k)["threads"] <= 512, (n, m, k)
         assert q(n, m, k)["matrix_core"] in (0, 2, 3)                              # no register-operand kernel for bf16
 

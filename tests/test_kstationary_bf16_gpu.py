@@ -17,6 +17,9 @@ CASES = [
     # tag, n_out, k, bits, quant_op, group, rows, bias, forced workgroups (0 = the built-in rule), k steps
     ("fewest_k_steps", 2048, 2304, 4, SCALE_AND_ZEROS, 128, 3, True, 0, 5),
     ("two_rows", 4100, 4096, 4, SCALE_AND_ZEROS, 64, 2, True, 0, 8),
+    ("two_rows_16_k_steps", 2052, 8192, 4, SCALE_AND_ZEROS, 128, 2, True, 0, 16),
+    ("two_rows_walk_of_4", 15312, 6104, 4, PER_COLUMN, 0, 2, False, 0, 12),
+    ("two_rows_9_k_steps_generic_groups", 15316, 4512, 4, SCALE_AND_ZEROS, 96, 2, True, 0, 9),
     ("eight_rows_lds_nearly_full", 12288, 8192, 4, SCALE_AND_ZEROS, 128, 8, False, 0, 16),
     ("nine_rows_two_rounds", 8192, 2560, 4, SCALE_ONLY, 128, 9, True, 0, 5),
     ("sixteen_rows", 4096, 4096, 4, SCALE_AND_ZEROS, 128, 16, False, 0, 8),
