@@ -189,7 +189,7 @@ __device__ __forceinline__ void settle_dot_chain(float& acc) { asm volatile("s_n
 //
 // Two forms each, as for fp16:
 //   short    int4: the products of the fp16 short form, exact in fp16, widened to fp32 by the matrix unit and rounded
-//            (dequant_int4_word_bf16_short); int8: fma(u, s, -128 s), exact for 2^-100 <= s < 2^119;
+//            (dequant_int4_words_bf16); int8: fma(u, s, -128 s), exact for 2^-100 <= s < 2^119;
 //   general  (8u - 64) * (s/8) resp. (u - 128) * s: exact for every finite s, with the sign of
 //            a zero product as the reference's multiply gives it.
 // ---------------------------------------------------------------------------------------------
@@ -212,12 +212,20 @@ __device__ __forceinline__ float byte_to_f32(uint32_t v) {
 
 // Which scales the short form takes, by bf16 bit pattern.
 // int8: 2^-100 .. 2^119 -- positive, every product with an integer a normal number, -128 s finite.
-// int4: the products q s have 11 significant bits and must not fall off either end of fp16: 2^-17 <= s < 2^-5, scaled by
-// any 2^shift that is the same for the whole wave (the widening step takes it back).
+// int4: the products q s have 11 significant bits and must not fall off either end of fp16: 2^-17 <= s < 2^-5, or 2^shift
+// times that, any shift that is the same for the four lanes of a widening step (which takes it back).
 constexpr uint32_t kShortBf16Int8First = 0x0d80, kShortBf16Int8Past = 0x7b00;
-constexpr uint32_t kShortBf16Int4First = (127 - 17) << 7, kShortBf16Int4Past = (127 - 5) << 7;
+constexpr uint32_t kShortBf16Int4FirstExponent = 127 - 17, kShortBf16Int4Binades = 12;
+constexpr uint32_t kShortBf16Int4First = kShortBf16Int4FirstExponent << 7;
+constexpr uint32_t kShortBf16Int4Past = (kShortBf16Int4FirstExponent + kShortBf16Int4Binades) << 7;
 constexpr int kShortBf16MinShift = -14, kShortBf16MaxShift = 15;  // 2^shift is a normal fp16 value
-constexpr int kNoShortForm = 0x7fffffff;
+
+// A lane's int4 scale for the short bf16 form: s 2^-shift, and 2^shift twice, as fp16.
+struct Int4ScaleBf16 {
+  float s;
+  uint32_t power;
+};
+constexpr uint32_t kNoShift = 0x3c003c00u;
 
 // One lane's row of the 4x4 identity, as a mask on four packed 16-bit values: the operand of the widening steps below.
 struct Identity4 {
@@ -266,21 +274,20 @@ struct Bf16Scale {
   float add;              // int8, short: -128 s
   f32x4 z;                // additive zero, four times: the accumulator operand of add_zero_bf16
   ShortFormScale f16;     // int4, short: of s * 2^-shift
-  u32x2 widen, identity;  // 2^shift (fp16) and 1 (bf16) times the lane's row of the identity
+  u32x2 widen, identity;  // int4, short: 2^shift (fp16) and 1 (bf16) times the lane's row of the identity
 };
 
-// shift: int4 short form only.
+// short4: int4 short form only (which does not read s_bits).
 template <int BITS, bool SHORT>
-__device__ __forceinline__ Bf16Scale make_bf16_scale(uint32_t s_bits, uint32_t z_bits, const Identity4& id, int shift) {
+__device__ __forceinline__ Bf16Scale make_bf16_scale(uint32_t s_bits, uint32_t z_bits, const Identity4& id, const Int4ScaleBf16& short4) {
   const float s = bf16_low_to_f32(s_bits), z = bf16_low_to_f32(z_bits);
   Bf16Scale f{};
   if constexpr (BITS == 4 && SHORT) {
-    auto scaled = [&](uint32_t power_bits) { return splat((half_t)(s * __builtin_bit_cast(float, power_bits - ((uint32_t)shift << 23)))); };  // exact
-    f.f16.s17 = scaled(0x48000000u);  // 2^17
-    f.f16.s21 = scaled(0x4a000000u);
-    f.f16.m8s = scaled(0xc1000000u);  // -8
-    const uint32_t unit = (uint32_t)(15 + shift) << 10;
-    f.widen = u32x2{id.lo & (unit | unit << 16), id.hi & (unit | unit << 16)};
+    auto scaled = [&](float power) { return splat((half_t)(short4.s * power)); };  // exact
+    f.f16.s17 = scaled(0x1p17f);
+    f.f16.s21 = scaled(0x1p21f);
+    f.f16.m8s = scaled(-8.0f);
+    f.widen = u32x2{id.lo & short4.power, id.hi & short4.power};
   } else {
     f.mul = BITS == 4 ? s * 0.125f : s;
     f.add = s * -128.0f;

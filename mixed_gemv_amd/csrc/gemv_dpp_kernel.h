@@ -227,11 +227,11 @@ __device__ __forceinline__ void compute_words_bf16(float (&acc)[MB], uint32_t w0
 
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool SHORT, int I, int ACT>
 __device__ __forceinline__ void compute_block(float (&acc)[MB], const UnitFragment<BITS, MB, GROUPS_PER_RUN>& f,
-                                              const ConvertRegs& c, int shift) {
+                                              const ConvertRegs& c, const Int4ScaleBf16 (&short4)[GROUPS_PER_RUN]) {
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   constexpr int gi = I * GROUPS_PER_RUN / kBlocksPerUnit;
   if constexpr (ACT == kActBf16) {
-    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(f.s[gi], kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
+    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(f.s[gi], kHasZero ? f.z[gi] : 0u, make_identity4(), short4[gi]);
     compute_words_bf16<BITS, kHasZero, SHORT, MB, I, 0>(acc, f.w[I][0], f.w[I][1], f.x, c, bs);
     compute_words_bf16<BITS, kHasZero, SHORT, MB, I, 2>(acc, f.w[I][2], f.w[I][3], f.x, c, bs);
   } else {
@@ -249,12 +249,12 @@ __device__ __forceinline__ void compute_block(float (&acc)[MB], const UnitFragme
 
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool SHORT, int ACT>
 __device__ __forceinline__ void compute_unit_form(float (&acc)[MB], const UnitFragment<BITS, MB, GROUPS_PER_RUN>& f,
-                                                  const ConvertRegs& regs, int shift) {
+                                                  const ConvertRegs& regs, const Int4ScaleBf16 (&short4)[GROUPS_PER_RUN]) {
   const ConvertRegs c = (ACT == kActF16 && BITS == 4 && !SHORT) ? general_form_regs(regs) : regs;
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 0, ACT>(acc, f, c, shift);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 1, ACT>(acc, f, c, shift);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 2, ACT>(acc, f, c, shift);
-  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 3, ACT>(acc, f, c, shift);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 0, ACT>(acc, f, c, short4);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 1, ACT>(acc, f, c, short4);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 2, ACT>(acc, f, c, short4);
+  compute_block<BITS, QOP, MB, GROUPS_PER_RUN, SHORT, 3, ACT>(acc, f, c, short4);
   // The two forms meet again after this call, and the compiler may place a register copy of
   // the accumulators at that join: make them safe to read by any instruction first.
 #pragma unroll
@@ -281,14 +281,14 @@ __device__ __forceinline__ void compute_unit(float (&acc)[MB], const UnitFragmen
     }
     return;
   }
+  Int4ScaleBf16 short4[GROUPS_PER_RUN] = {};
   if constexpr (BITS == 4 || ACT == kActBf16) {
-    const int shift = short_allowed ? wave_short_form<BITS, ACT>(f.s) : kNoShortForm;
-    if (shift != kNoShortForm) {
-      compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, true, ACT>(acc, f, c, shift);
+    if (short_allowed && wave_takes_short_form<BITS, ACT>(f.s, short4)) {
+      compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, true, ACT>(acc, f, c, short4);
       return;
     }
   }
-  compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, false, ACT>(acc, f, c, 0);
+  compute_unit_form<BITS, QOP, MB, GROUPS_PER_RUN, false, ACT>(acc, f, c, short4);
 }
 
 // Epilogue: fp32 add of the bias, one rounding to fp16

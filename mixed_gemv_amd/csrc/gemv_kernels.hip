@@ -57,7 +57,8 @@ __device__ __forceinline__ u32x4 dequantize_eight(const uint32_t (&w)[8 * BITS /
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   u32x4 out;
   if constexpr (ACT == kActBf16) {
-    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? z_bits : 0u, make_identity4(), 0);
+    const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? z_bits : 0u, make_identity4(),
+                                                      Int4ScaleBf16{bf16_low_to_f32(s_bits), kNoShift});
     uint32_t d[4];
     if constexpr (BITS == 4) dequant_int4_words_bf16<kHasZero, SHORT, 1>(w, c, bs, d);
     else dequant_int8_words_bf16<kHasZero, SHORT, 2>(w, bs, d);

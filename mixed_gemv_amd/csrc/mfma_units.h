@@ -86,7 +86,7 @@ __device__ __forceinline__ void load_block_operands(const Activations& xa, int i
 template <int BITS, int QOP, int GROUPS_PER_RUN, bool SHORT, int ACT, typename Activations>
 __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWeights<BITS, GROUPS_PER_RUN>& f,
                                                        const Activations& xa, const ConvertRegs& c,
-                                                       half2_t col_scale2, int shift) {
+                                                       half2_t col_scale2, const Int4ScaleBf16 (&short4)[GROUPS_PER_RUN]) {
   constexpr bool kHasZero = QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
   constexpr int kFrags = BITS == 4 ? 4 : 2;
   // The operands of block i+1 are requested before block i is dequantised, and the request is
@@ -110,7 +110,7 @@ __device__ __forceinline__ void compute_unit_mfma_form(f32x4& acc, const MfmaWei
       __builtin_amdgcn_sched_barrier(0);
       const int gi = i * GROUPS_PER_RUN / kBlocksPerUnit;
       const uint32_t s_bits = QOP != MGEMV_PER_COLUMN_SCALE_ONLY ? f.s[gi] : as_u32(col_scale2);
-      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u, make_identity4(), shift);
+      const Bf16Scale bs = make_bf16_scale<BITS, SHORT>(s_bits, kHasZero ? f.z[gi] : 0u, make_identity4(), short4[QOP != MGEMV_PER_COLUMN_SCALE_ONLY ? gi : 0]);
       uint32_t d[8];
       if constexpr (BITS == 4) {
         dequant_int4_words_bf16<kHasZero, SHORT, 2>({f.w[i][j], f.w[i][j + 1]}, c, bs, d);
@@ -178,22 +178,25 @@ template <int BITS, int QOP, int GROUPS_PER_RUN, int ACT = kActF16, typename Act
 __device__ __forceinline__ void compute_unit_mfma(f32x4& acc, const MfmaWeights<BITS, GROUPS_PER_RUN>& f,
                                                   const Activations& xa, const ConvertRegs& c,
                                                   half2_t col_scale2, bool short_allowed) {
+  Int4ScaleBf16 short4[GROUPS_PER_RUN] = {};
   if constexpr (BITS == 4 || ACT == kActBf16) {
-    int shift = short_allowed ? 0 : kNoShortForm;
+    bool takes = false;
     if (short_allowed) {
       if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) {
-        shift = wave_short_form<BITS, ACT>(f.s);
+        takes = wave_takes_short_form<BITS, ACT>(f.s, short4);
       } else {
         const uint32_t bits[1] = {as_u32(col_scale2)};
-        shift = wave_short_form<BITS, ACT>(bits);
+        Int4ScaleBf16 one[1] = {};
+        takes = wave_takes_short_form<BITS, ACT>(bits, one);
+        short4[0] = one[0];
       }
     }
-    if (shift != kNoShortForm) {
-      compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, true, ACT>(acc, f, xa, c, col_scale2, shift);
+    if (takes) {
+      compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, true, ACT>(acc, f, xa, c, col_scale2, short4);
       return;
     }
   }
-  compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2, 0);
+  compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2, short4);
 }
 
 // Weights, scales and zeros of unit `unit` of the wave's k range through descriptors: everything
