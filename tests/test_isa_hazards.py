@@ -97,3 +97,21 @@ def test_a_check_that_sees_nothing_fails(tmp_path, monkeypatch):
     (tmp_path / "empty-hip-amdgcn-amd-amdhsa-gfx950.s").write_text("kernel_a:\n\ts_endpgm\n")
     with pytest.raises(RuntimeError, match="did not see the kernels"):
         lib_build.lint_device_code(verbose=False)
+
+
+def test_the_k_stationary_loops_begin_at_a_64_byte_line():
+    """Their heads' place decides 2 % of the time of the fp16 build, and any change in front of them moves them."""
+    import re
+    path = os.path.join(lib_build.OBJ_DIR, "launch_mfma_kstat-hip-amdgcn-amd-amdhsa-gfx950.s")
+    if not os.path.exists(path):
+        pytest.skip("no device assembly: built elsewhere")
+    # (one or two groups per lane run; with four, loop-invariant address arithmetic may come between)
+    kernels = re.findall(r"^(_ZN5mgemv22gemv_mfma_kstat_kernelILi[48]ELi[123]ELi[12]E\S+):\s*;.*?\n(.*?)^\.Lfunc_end", open(path).read(), re.S | re.M)
+    assert len(kernels) >= 20
+    for name, body in kernels:
+        # the directive, then at most a few scalar instructions, then the label the walk comes back to
+        ahead, _, behind = body.partition(".p2align 6")
+        assert behind, name
+        head = re.search(r"^(\.LBB\S+):", behind, re.M)
+        lead = re.findall(r"^\t([a-z]\w+)", behind[:head.start()], re.M)
+        assert len(lead) <= 2 and re.search(r"s_c?branch\S* +" + re.escape(head[1]) + r"\b", behind[head.end():]), (name, lead)
