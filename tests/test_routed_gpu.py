@@ -27,6 +27,9 @@ CASES = [
      mg.MATRIX_CORE_REGISTER_OPERAND, 1),
     ("k_stationary_four_rows", 80, 2048, 4, SCALE_AND_ZEROS, 128, 4, True, "f16", mg.MATRIX_CORE_K_STATIONARY, 3),
     ("k_stationary_int8", 64, 2048, 8, SCALE_ONLY, 128, 5, False, "f16", mg.MATRIX_CORE_K_STATIONARY, 3),
+    ("k_stationary_bf16_generic_groups", 84, 2112, 4, SCALE_AND_ZEROS, 96, 5, True, "bf16", mg.MATRIX_CORE_K_STATIONARY, 3),
+    ("k_stationary_bf16_int8_sixteen_rows", 80, 1280, 8, PER_COLUMN, 0, 16, True, "bf16", mg.MATRIX_CORE_K_STATIONARY, 3),
+    ("k_stationary_bf16_by_the_rule", 2052, 2560, 4, SCALE_ONLY, 128, 3, False, "bf16", None, 3),
 ]
 
 ENTRIES = 5
@@ -120,7 +123,7 @@ def test_routed_launch_equals_one_launch_per_problem(gpu, forced_variant, case):
             assert error_report(got[b].view(np.float16), ref)[1] <= REL_TOL, (tag, b)
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[7]], ids=[CASES[i][0] for i in (0, 4, 7)])
+@pytest.mark.parametrize("case", [CASES[i] for i in (0, 4, 7, 9)], ids=[CASES[i][0] for i in (0, 4, 7, 9)])
 def test_one_token_and_its_chosen_experts(gpu, forced_variant, case):
     """stride_x = 0: every problem of the launch reads the same activations (a decode step's top-k)."""
     forced_variant(case[9])
@@ -131,7 +134,7 @@ def test_one_token_and_its_chosen_experts(gpu, forced_variant, case):
         assert np.array_equal(got[b], stack.single(entry, 0)), (case[0], b)
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[6], CASES[7]], ids=[CASES[i][0] for i in (0, 4, 6, 7)])
+@pytest.mark.parametrize("case", [CASES[i] for i in (0, 4, 6, 7, 9, 10)], ids=[CASES[i][0] for i in (0, 4, 6, 7, 9, 10)])
 def test_an_index_outside_the_stack_leaves_its_outputs_alone(gpu, forced_variant, case):
     forced_variant(case[9])
     stack = Stack(case, gpu, 4)
