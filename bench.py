@@ -748,6 +748,27 @@ def measure(wl, steps, warmup, use_graph):
 DEFAULT_EXTRA = "c1,c2,c3a,c3b,c4:m1,c4:m2,c4:m4,c4:m8,c4:m16,c5,c5:m4,c5:m16,vocab,nsx8,nsx16,routed,ns:bf16,c5:bf16"
 
 
+def short_line(out):
+    """What is printed: everything but the further workloads and ceilings, and of those their figures (the whole is 26 KB,
+    more than a reader of a run's last lines gets to see)."""
+    line = dict(out)
+    if "other_workloads" in out:  # (their kernel times and shares of the peak are roofline.by_workload)
+        line["other_workloads"] = {name: {"us_per_call": e["us_per_call"]} for name, e in out["other_workloads"].items()}
+    if "ceilings" in out:
+        line["ceilings"] = {}
+        for name, c in out["ceilings"].items():
+            if c is None:  # a workload without measurement builds
+                continue
+            short = line["ceilings"][name] = {kind: c[kind]["us_per_launch"] for kind in ("empty_grid", "loads_only", "compute_only")
+                                              if kind in c}
+            reads = c.get("stream_read", [])
+            short["stream_read"] = reads["us_per_launch"] if isinstance(reads, dict) else c.get("stream_read_best_us")
+            if "timeline_us" in c:
+                short["first_wave_start_to_last_store"] = c["timeline_us"]["first_wave_start_to_last_store"]
+        line["ceilings"]["unit"] = "us per launch"
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -776,6 +797,9 @@ def main():
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only copy 512 MiB device to device four times and exit: the known-size kernel against which "
                          "the FETCH_SIZE / WRITE_SIZE counters of `rocprofv3 --pmc` are scaled")
+    ap.add_argument("--details", metavar="FILE",
+                    help="also write the whole of the measurements there as JSON: plans, parity and repetitions of every "
+                         "workload, all ceilings with their notes and timelines (the printed line has their figures alone)")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py: this build measures one GPU only (a GEMV over one weight matrix held by one MI355X); "
@@ -960,7 +984,10 @@ def main():
     out["launch_plans"] = {"built_in_table_entries": mg.default_plan_count(), "caller_table_entries": mg.tuned_plan_count(),
                            "note": "rules of plan_launch plus the library's compiled-in table (mixed_gemv_amd/default_plans.json); "
                                    "nothing is tuned or installed by this run"}
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(short_line(out)))
 
 
 if __name__ == "__main__":
