@@ -2,6 +2,7 @@
 // and the dispatchers that pick their instantiations.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "kernel_common.h"
 #include "mfma_units.h"
@@ -311,50 +312,51 @@ gemv_mfma_lds_kernel(const uint8_t* weights, const half_t* x, const half_t* scal
       __builtin_amdgcn_wave_barrier();
     }
   };
-  int u = 0;
-  do {
-    // even step: weights in wa, stage 0
-    park_x_rows<BITS, ROUNDS>(xr, my_stages, lane, ty, p.tiles_per_wg);
+  // One k step: the rows on their way go to the stage, the next step's rows and weights are requested (not behind the last),
+  // the step is computed.
+  auto step = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& now, MfmaWeights<BITS, GROUPS_PER_RUN>& next, int stage, int u, auto last) {
+    constexpr bool kLast = decltype(last)::value;
+    park_x_rows<BITS, ROUNDS>(xr, my_stages + stage * stage_bytes, lane, ty, p.tiles_per_wg);
     stage_ready();
     if constexpr (PROBE == kProbeComputeOnly) {
-      wb = wa;
-      keep_registers(wb, xr);
-    } else {
+      next = now;
+      keep_registers(next, xr);
+    } else if constexpr (!kLast) {
       fetch_x_rows<BITS, ROUNDS>(xr, p, x_rsrc, ks_begin + u + 1, lane, ty, p.tiles_per_wg);
-      load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN>(wb, p, w_rsrc, tables, u + 1, ks_begin + u + 1, lane, row);
+      load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN>(next, p, w_rsrc, tables, u + 1, ks_begin + u + 1, lane, row);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (u < units) {
-      const LdsActivations<BITS> xa{my_stages + operand_offset};
+      const LdsActivations<BITS> xa{my_stages + stage * stage_bytes + operand_offset};
       if constexpr (PROBE == kProbeLoadsOnly)
-        consume_unit(acc, wa, xa);
+        consume_unit(acc, now, xa);
       else
-        compute_unit_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(acc, wa, xa, c, col_scale, short_ok);
+        compute_unit_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(acc, now, xa, c, col_scale, short_ok);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (u + 1 < steps) {
-      // odd step: weights in wb, stage 1
-      park_x_rows<BITS, ROUNDS>(xr, my_stages + stage_bytes, lane, ty, p.tiles_per_wg);
-      stage_ready();
-      if constexpr (PROBE == kProbeComputeOnly) {
-        wa = wb;
-        keep_registers(wa, xr);
-      } else {
-        fetch_x_rows<BITS, ROUNDS>(xr, p, x_rsrc, ks_begin + u + 2, lane, ty, p.tiles_per_wg);
-        load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN>(wa, p, w_rsrc, tables, u + 2, ks_begin + u + 2, lane, row);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (u + 1 < units) {
-        const LdsActivations<BITS> xa{my_stages + stage_bytes + operand_offset};
-        if constexpr (PROBE == kProbeLoadsOnly)
-          consume_unit(acc, wb, xa);
-        else
-          compute_unit_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(acc, wb, xa, c, col_scale, short_ok);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+  };
+  // Whole pairs of steps, and a single one behind them if need be.  With the second step of a pair conditional inside the
+  // loop, a path leads from the first step's requests straight back to the loop's head; the compiler does not know it is
+  // never taken, finds weights outstanding in the registers it computes addresses in, and waits for them there -- for every
+  // step's own weights, in front of the staging or of the next step's requests.  72 launches of random shapes take 0.955 of
+  // the time without those waits (0.83-1.01): 2032x2048 groups of 256 at 8 rows 3.92 us -> 3.42, 9072x5760 int8 at 6 rows
+  // 15.8 -> 13.8, 4096x11008 at 4 rows 8.57 -> 7.95; 8192x8192, walked by shared stages, level.
+  // int4 in bf16 with 16 rows to a wave keeps the conditional: the longer code costs it 2.5-6 % (4096x14336 at 12 rows
+  // 14.0 us / 14.8).
+  int u = 0;
+  if constexpr (BITS == 4 && ACT == kActBf16 && ROUNDS == 16) {
+    do {
+      step(wa, wb, 0, u, std::false_type{});
+      if (u + 1 < steps) step(wb, wa, 1, u + 1, std::false_type{});
+      u += 2;
+    } while (u < steps);
+  } else {
+    for (; u + 1 < steps; u += 2) {
+      step(wa, wb, 0, u, std::false_type{});
+      step(wb, wa, 1, u + 1, std::false_type{});
     }
-    u += 2;
-  } while (u < steps);
+    if (u < steps) step(wa, wb, 0, u, std::true_type{});
+  }
 
   // Lane l holds D[rows 4*(l/16) .. +3 of the tile][batch row l % 16].
   f32x4 sum = acc;
