@@ -1,6 +1,7 @@
 // The k-stationary matrix-core GEMV kernel for gfx950 (MI355X), wave64, and its dispatcher.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "kernel_common.h"
 #include "mfma_units.h"
@@ -35,7 +36,6 @@ namespace mgemv {
 // tiles of the longest walk x 4 x m_batch x 17 x 16 bytes (the partial sums) -- one behind the other where
 // both fit, else sharing the space, with a barrier between the two uses.
 // ---------------------------------------------------------------------------------------------
-constexpr int kParkSlots = kKStationaryParkSlots;  // entries of one block of partial sums: one per possible wave and one to spare
 
 template <int BITS, int QOP, int GROUPS_PER_RUN>
 __device__ __forceinline__ void load_unit_kstat(MfmaWeights<BITS, GROUPS_PER_RUN>& f, __amdgpu_buffer_rsrc_t w_rsrc,
@@ -207,13 +207,18 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   const bool short_allowed = (tail.flags & kExactIntegerFormOnly) == 0;
   const ConvertRegs c = make_convert_regs();
 
-  // Partial sums in LDS: for every (tile of the walk, row group, batch row) a block of kParkSlots entries of
-  // four floats, entry w written by wave w (the odd block length spreads the lanes over the banks).  The lane
-  // that later sums a block finds its entries side by side, at offsets known to the compiler.
+  // Partial sums in LDS: for every (tile of the walk, row group, batch row) a block of 4, 8 or 16 entries of four floats, as
+  // few as there is one for each wave, and one to spare; entry w is written by wave w (the odd block length spreads the lanes
+  // over the banks, and the launch has room for blocks of 17).  The lane that later sums a block finds its entries side by
+  // side, at offsets known to the compiler.  Blocks of 16 for every launch, those of missing waves zero, took fp16 launches of
+  // up to 4 k steps 1.1-1.15 times as long and of 5-8 1.02-1.04 (36400x2048 at 4 rows 10.7 us / 9.35, 11008x4096 7.37 / 7.24;
+  // a fourth size, 12, gains nothing and the choice costs the others 0.5 %).
+  const int pieces = waves <= 4 ? 4 : waves <= 8 ? 8 : 16;
+  const int slots = pieces + 1;
   f32x4* const park = reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(partials) +
                                                (park_behind_stage ? waves * (stage_rows * XS::kRowStride) : 0));
-  const int park_tile_stride = kKSlices * m_batch * kParkSlots;  // entries from a tile to the next
-  f32x4* const my_park = park + (slice * m_batch + m) * kParkSlots + kw;
+  const int park_tile_stride = kKSlices * m_batch * slots;  // entries from a tile to the next
+  f32x4* const my_park = park + (slice * m_batch + m) * slots + kw;
   auto compute_and_park = [&](const MfmaWeights<BITS, GROUPS_PER_RUN>& f, int i) {
     f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     half2_t col_scale = half2_t{};
@@ -276,7 +281,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   // need the other waves' sums -- addresses, the bias, zeros in the entries of waves that do not exist --
   // is done in front of it.
   const bool sums = m < m_batch && kw < my_tiles;
-  f32x4* block = park + (kw * kKSlices + slice) * (m_batch * kParkSlots) + m * kParkSlots;
+  f32x4* block = park + ((kw * kKSlices + slice) * m_batch + m) * slots;
   int n0 = (tile0 + kw) * kTileRows + 4 * slice;
   float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   auto fetch_bias = [&]() {
@@ -293,9 +298,9 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   };
   if (sums) {
     fetch_bias();
-    if (waves < kMaxWavesPerWorkgroup)
+    if (waves < pieces)
       for (int t = kw; t < my_tiles; t += waves)
-        for (int w = waves; w < kMaxWavesPerWorkgroup; ++w)
+        for (int w = waves; w < pieces; ++w)
           block[(t - kw) * park_tile_stride + w] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
   uint16_t* dst = reinterpret_cast<uint16_t*>(tail.y) + (size_t)m * (size_t)p.n_out + n0;
@@ -305,12 +310,20 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   __syncthreads();
   if (sums) {
     for (int t = kw; t < my_tiles; t += waves) {
-      f32x4 piece[kMaxWavesPerWorkgroup];
+      f32x4 sum;
+      auto sum_block = [&](auto count) {
+        f32x4 piece[decltype(count)::value];
 #pragma unroll
-      for (int w = 0; w < kMaxWavesPerWorkgroup; ++w) piece[w] = block[w];
-      f32x4 sum = piece[0];
+        for (int w = 0; w < count; ++w) piece[w] = block[w];
+        sum = piece[0];
 #pragma unroll
-      for (int w = 1; w < kMaxWavesPerWorkgroup; ++w) sum += piece[w];  // ascending k
+        for (int w = 1; w < count; ++w) sum += piece[w];  // ascending k
+      };
+      switch (pieces) {
+        case 4: sum_block(std::integral_constant<int, 4>{}); break;
+        case 8: sum_block(std::integral_constant<int, 8>{}); break;
+        default: sum_block(std::integral_constant<int, 16>{});
+      }
       // n_out is a multiple of 4 and so is n0: the four outputs of a lane are all inside or all outside, and
       // they are neighbours in y -- one 8-byte store where y allows it
       if (n0 < p.n_out) {

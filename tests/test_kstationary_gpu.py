@@ -87,6 +87,28 @@ def test_results_do_not_depend_on_how_the_tiles_are_walked(gpu):
         assert np.array_equal(got.view(np.uint16), base.view(np.uint16)), cap
 
 
+@pytest.mark.parametrize("element", ["f16", "bf16"])
+@pytest.mark.parametrize("ksteps", [3, 4, 5, 7, 8, 9, 15, 16])
+def test_blocks_of_partial_sums_of_every_size(gpu, ksteps, element):
+    """Blocks of 4, 8 and 16 partial sums, full and with a wave missing, on walks longer than the workgroup has waves: each
+    row is a one-hot of its own wave's k step, so that a wrong, missing or stale partial sum shows in every output."""
+    k, n_out, rows = 512 * ksteps, 16 * 4 * (ksteps + 1) + 8, 5
+    prob = Problem("ks_blocks", n_out, k, 4, SCALE_ONLY, 128, m_batch=rows, bias=False, element=element)
+    dev = DeviceProblem(prob, gpu)
+    x = np.zeros((rows, k), dtype=np.float32)
+    at = [(w * 512 + 37 * (w + 1)) % k for w in (0, 1 % ksteps, ksteps // 2, ksteps - 2, ksteps - 1)]
+    for r, i in enumerate(at):
+        x[r, i] = 1.0
+    import torch
+    dtype = torch.bfloat16 if element == "bf16" else torch.half
+    dev.x.copy_(torch.from_numpy(x).to(dtype).view(dev.x.dtype))
+    want = dev.dequant().view(np.uint16)[:, at].T
+    with k_stationary(4):
+        assert mg.query_launch(n_out, rows, k, 4, 128, element=element)["split_k"] == ksteps
+        got = dev.run().copy().view(np.uint16)
+    assert np.array_equal(got, want)
+
+
 def test_outputs_that_are_not_8_byte_aligned_take_the_narrow_stores(gpu):
     import torch
     prob = Problem("ks_align", 528, 2048, 4, SCALE_AND_ZEROS, 128, m_batch=3, bias=True)
