@@ -20,7 +20,8 @@ constexpr int kNumXcd = 8;
 constexpr int kNumCus = 256;
 constexpr int kKStationaryParkSlots = kMaxWavesPerWorkgroup + 1;  // k-stationary matrix-core kernel: entries of 16 bytes per block of partial sums
 constexpr int kMaxKStationaryLds = 128 * 1024;  // most LDS the k-stationary matrix-core kernel parks partial sums in
-constexpr int kMaxKStationaryBf16Lds = 160 * 1024;  // ... with bf16 operands: most LDS its activation rows and partial sums take together
+constexpr int kKStationaryZeroBytes = 256;  // ... with bf16 operands: zeros, a k run of the operand of a batch row that does not exist
+constexpr int kMaxKStationaryBf16Lds = 160 * 1024 - kKStationaryZeroBytes;  // ... most LDS its activation rows and partial sums take together
 constexpr int kMaxValuBatch = 4;  // activation rows handled per launch by the VALU kernel
 constexpr int kExactIntegerFormOnly = 1;  // GemvTail::flags: never take the short int4 dequantiser
 constexpr int kSingleStage = 2;           // GemvTail::flags: no load in flight while a unit is computed (VALU kernel)

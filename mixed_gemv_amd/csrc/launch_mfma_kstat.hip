@@ -25,7 +25,7 @@ namespace mgemv {
 // bf16: the dequantiser needs the registers, so the operand stays in the wave's stage instead and is read from LDS, two
 // matrix instructions ahead (16 LDS reads of 16 bytes beside 400 other instructions a unit; 98-128 registers, 4 waves per
 // SIMD, no spills -- with a block's operands ahead the four-group build spilled 30 and took 1.4 times as long).  What
-// bounds it is its instruction issue (53-68 % of all cycles issue a vector instruction), then the start (16 MiB of first
+// bounds it is its instruction issue (53-68 % of all cycles issue a vector instruction, at 1.9-2.1 GHz), then the start (16 MiB of first
 // units) and the last unit's arithmetic.  28672x8192, 4 rows: 31.3 us, 3.8 TB/s; the LDS-staged kernel, whose 140-164
 // registers leave 3 waves per SIMD and whose barriers line them up, 35.1.
 // It replaces nothing in the reference, whose kernel is fixed to one activation row
@@ -34,7 +34,7 @@ namespace mgemv {
 // Dynamic LDS: waves x 8 activation rows (the stage each wave turns its operand round in, at the start; bf16: waves x
 // m_batch rows, which stay) and
 // tiles of the longest walk x 4 x m_batch x 17 x 16 bytes (the partial sums) -- one behind the other where
-// both fit, else sharing the space, with a barrier between the two uses.
+// both fit, else sharing the space, with a barrier between the two uses.  Static, bf16: kKStationaryZeroBytes of zeros.
 // ---------------------------------------------------------------------------------------------
 
 template <int BITS, int QOP, int GROUPS_PER_RUN>
@@ -159,7 +159,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   uint8_t* const stage = reinterpret_cast<uint8_t*>(partials) + kw * (stage_rows * XS::kRowStride);
   typename KStatOperand<BITS, kLdsOperand>::type xa;
   if constexpr (kLdsOperand) {
-    // The stage stays: lanes of rows that do not exist read row 0 (those columns are never stored).
+    // The stage stays.
     for (int first = 0; first < m_batch; first += 8) {
       const int rows_here = m_batch - first < 8 ? m_batch - first : 8;
       XRows<BITS, 8> rows;
@@ -168,9 +168,15 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       __builtin_amdgcn_sched_barrier(0);
       park_x_rows<BITS, 8>(rows, stage, lane, first, 1, rows_here);
     }
+    // Lanes of rows that do not exist read zeros: their columns of a matrix product are never stored, but the matrix unit
+    // multiplies them all the same, and a large launch runs at the clock the power limit leaves (28672x8192 at 4 rows 1.92
+    // GHz, its loads alone 2.32).  With row 0 in the idle columns that launch took 30.3 us, with zeros 29.4; 128256x4096 at
+    // 2 rows 66.3 / 63.6, 28672x8064 g96 at 4 rows 33.2 / 32.3; up to 13 us level.
+    __shared__ u32x4 zeros[kKStationaryZeroBytes / 16];
+    if (lane < kKStationaryZeroBytes / 16) zeros[lane] = u32x4{0u, 0u, 0u, 0u};  // every wave for itself: no barrier
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the LDS executes a wave's accesses in order
     __builtin_amdgcn_wave_barrier();
-    xa.lane_base = stage + (m < m_batch ? m : 0) * XS::kRowStride + slice * (G::kRunK * 2);
+    xa.lane_base = m < m_batch ? stage + m * XS::kRowStride + slice * (G::kRunK * 2) : reinterpret_cast<const uint8_t*>(zeros);
   } else {
     // ... and are read back in operand shape -- lane (slice, m) takes the sixteen 16-byte pieces of row m that its
     // matrix instructions pair with its weights.
