@@ -360,7 +360,8 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // for every further unit; kProbeLoadsOnly keeps every load and replaces the arithmetic of a unit
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
 // records timestamps and the time spent waiting for loads, per wave.
-template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone>
+// TWO_UNITS: no wave has more than two units, on one tile.
+template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, bool TWO_UNITS = false>
 __global__ void __launch_bounds__(kWave * (MB >= 3 || ACT == kActBf16 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup))
 __attribute__((amdgpu_waves_per_eu(ACT == kActF16 && MB == 1 && GROUPS_PER_RUN == 1 ? 6 : 1)))
 gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out, int k,
@@ -472,8 +473,17 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     // end (4096x4096: 4.44 / 4.74 / 5.04 us at 2 / 3 / 4 rows against 4.55 / 4.83 / 5.19 through
     // the loop).  A three-unit path lost 5 % to the loop (4096x6144, 2 rows), and in the
     // single-row kernels, which are held to 80 registers, any extra path made the loop beside it
-    // 4-7 % slower, so those keep the loop for every length.
-    if (total == 1) {
+    // 4-7 % slower, so there the two-unit path is a build of its own, without a loop: a launch is over before the
+    // second request's latency could be hidden (through the loop / without: 4096x4096 g64 4.19 us / 3.91, scale only 3.88 /
+    // 3.74, 4096x2048 int8 3.75 / 3.60, 2500x3168 g96 4.50 / 3.93; 4096x4096 g128 with zeros 4.03 / 4.00).
+    if constexpr (TWO_UNITS) {
+      advance<MULTI>(cur, walk);
+      load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);  // past the range of a wave with one unit: nothing
+      __builtin_amdgcn_sched_barrier(0);
+      compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
+      __builtin_amdgcn_sched_barrier(0);
+      if (total > 1) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+    } else if (total == 1) {
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
       if constexpr (MULTI) finish_tile<MB>(acc, slot);
     } else if (MB >= 2 && !MULTI && total == 2) {
@@ -589,15 +599,20 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
 }
 
 // Picks the instantiation for the run-time arguments.
-template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT>
+template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, bool TWO_UNITS = false>
 hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
-  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
+  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, TWO_UNITS>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
                 g.zero_add, g.n_out, g.k, pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups,
                 g.tail.num_groups, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int MB, int GPR, int ACT>
 hipError_t launch_gemv_kernel(const GemvLaunch& g) {
+  // (bf16, bound by its arithmetic, gains nothing: 4096x4096 4.83 us / 4.83)
+  if constexpr (MB == 1 && ACT == kActF16) {
+    if (g.plan.tiles_in_sequence == 1 && g.plan.steps_per_wave == 2 && g.plan.stages == 2)
+      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, true>(g);
+  }
   return g.plan.tiles_in_sequence > 1 ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, true, ACT>(g)
                                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT>(g);
 }

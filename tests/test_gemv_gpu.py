@@ -727,3 +727,28 @@ def test_full_size_outputs_within_the_float64_bound(gpu, cfg):
         assert bad == 0 and host_check_bad == 0, (m, bad, worst)
         assert worst <= 1.25 * host_check_worst, (m, worst, host_check_worst)
     prob.m_batch, prob.x = full_rows, full_x
+
+
+@pytest.mark.parametrize("bits,qop,group,ksteps", [(4, SCALE_AND_ZEROS, 128, 8), (4, SCALE_ONLY, 64, 7), (4, SCALE_AND_ZEROS, 96, 6),
+                                                   (4, PER_COLUMN, 0, 5), (8, SCALE_AND_ZEROS, 128, 8), (8, PER_COLUMN, 0, 7),
+                                                   (8, SCALE_ONLY, 96, 6)])
+def test_single_rows_of_two_units_a_wave(gpu, bits, qop, group, ksteps):
+    """Waves of two units, the last one with one where the k steps do not divide, take a build without a loop: the bits of the
+    loop's (which the single-stage setting selects), on full and ragged tiles and a reduction that ends inside a k step."""
+    step = 512 if bits == 4 else 256
+    unit = 8 if qop == PER_COLUMN else group
+    for n_out in (2048 + 16, 3000):
+        k = ((ksteps - 1) * step + step // 2) // unit * unit
+        prob = Problem("two_units", n_out, k, bits, qop, group, m_batch=1, bias=True)
+        dev = DeviceProblem(prob, gpu)
+        plan = mg.query_launch(n_out, 1, k, bits, prob.group_size)
+        assert plan["steps_per_wave"] == 2 and plan["matrix_core"] == 0 and plan["tiles_in_sequence"] == 1, plan
+        got = dev.run().copy()
+        try:
+            mg.set_prefetch_stages(1)
+            loop = dev.run().copy()
+        finally:
+            mg.set_prefetch_stages(0)
+        assert np.array_equal(got.view(np.uint16), loop.view(np.uint16))
+        _, rel, _ = error_report(got, prob.oracle_gemv(threads=8))
+        assert rel <= REL_TOL, rel
