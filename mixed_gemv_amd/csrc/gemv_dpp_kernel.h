@@ -360,8 +360,11 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // for every further unit; kProbeLoadsOnly keeps every load and replaces the arithmetic of a unit
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
 // records timestamps and the time spent waiting for loads, per wave.
-// TWO_UNITS: no wave has more than two units, on one tile.
-template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, bool TWO_UNITS = false>
+// FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead).
+constexpr int kUnitLoop = 0;  // any number of them
+constexpr int kTwoUnits = 1;  // one or two, on one tile
+constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
+template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop>
 __global__ void __launch_bounds__(kWave * (MB >= 3 || ACT == kActBf16 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup))
 __attribute__((amdgpu_waves_per_eu(ACT == kActF16 && MB == 1 && GROUPS_PER_RUN == 1 ? 6 : 1)))
 gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out, int k,
@@ -476,7 +479,29 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     // 4-7 % slower, so there the two-unit path is a build of its own, without a loop: a launch is over before the
     // second request's latency could be hidden (through the loop / without: 4096x4096 g64 4.19 us / 3.91, scale only 3.88 /
     // 3.74, 4096x2048 int8 3.75 / 3.60, 2500x3168 g96 4.50 / 3.93; 4096x4096 g128 with zeros 4.03 / 4.00).
-    if constexpr (TWO_UNITS) {
+    // In a launch of at most one wave per SIMD nothing else runs while a wave's second unit is on its way, so there the first
+    // two are requested together.  (Where waves share a SIMD that loses: 4528x28032 g96, 1152 waves, 22.9 us / 23.2, 4260x7296
+    // 7.31 / 7.44.)  In a graph, the loop
+    // / this: 1688x17376 g96 9.87 us / 9.32, 2896x10496 int8 7.95 / 7.49, 8192x8192 8.16 / 7.92, 4096x11008 6.67 / 6.54; at 3
+    // rows 2596x3200 int8 5.04 / 4.81; bf16 1324x26752 13.2 / 12.6; 0.97 of the time on 78 launches of random shapes.
+    if constexpr (FORM == kTwoAhead) {
+      auto request = [&](UnitFragment<BITS, MB, GROUPS_PER_RUN>& f) {
+        advance<MULTI>(cur, walk);
+        load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(f, p, w_rsrc, x_rsrc, tables, cur);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      request(fb);
+      int u = 0;
+      do {
+        compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
+        __builtin_amdgcn_sched_barrier(0);
+        request(fa);
+        if (u + 1 < total) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+        __builtin_amdgcn_sched_barrier(0);
+        request(fb);
+        u += 2;
+      } while (u < total);
+    } else if constexpr (FORM == kTwoUnits) {
       advance<MULTI>(cur, walk);
       load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);  // past the range of a wave with one unit: nothing
       __builtin_amdgcn_sched_barrier(0);
@@ -599,19 +624,21 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
 }
 
 // Picks the instantiation for the run-time arguments.
-template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, bool TWO_UNITS = false>
+template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, int FORM = kUnitLoop>
 hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
-  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, TWO_UNITS>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
+  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, FORM>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
                 g.zero_add, g.n_out, g.k, pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups,
                 g.tail.num_groups, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int MB, int GPR, int ACT>
 hipError_t launch_gemv_kernel(const GemvLaunch& g) {
-  // (bf16, bound by its arithmetic, gains nothing: 4096x4096 4.83 us / 4.83)
-  if constexpr (MB == 1 && ACT == kActF16) {
-    if (g.plan.tiles_in_sequence == 1 && g.plan.steps_per_wave == 2 && g.plan.stages == 2)
-      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, true>(g);
+  if (g.plan.tiles_in_sequence == 1 && g.plan.stages == 2) {
+    // (bf16, bound by its arithmetic, gains nothing from kTwoUnits: 4096x4096 4.83 us / 4.83)
+    if constexpr (MB == 1 && ACT == kActF16) {
+      if (g.plan.steps_per_wave == 2) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits>(g);
+    }
+    if (g.plan.wave_per_simd && g.plan.steps_per_wave > 2) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead>(g);
   }
   return g.plan.tiles_in_sequence > 1 ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, true, ACT>(g)
                                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT>(g);

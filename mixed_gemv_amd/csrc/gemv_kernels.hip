@@ -708,6 +708,7 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
             (long long)seq_tiles() * tiles_per_wg * split_k * rows * kWave * 4 > 64 * 1024))
       lp.workgroups = lp.workgroups * 2 < ceil_div(groups, tiles_per_wg) ? lp.workgroups * 2 : ceil_div(groups, tiles_per_wg);
     lp.tiles_in_sequence = seq_tiles();
+    lp.wave_per_simd = (long long)lp.workgroups * split_k * tiles_per_wg <= 4ll * cus;
   }
   lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
   lp.threads = kWave * split_k * tiles_per_wg;

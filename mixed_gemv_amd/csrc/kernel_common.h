@@ -272,6 +272,7 @@ struct LaunchPlan {
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
   int staged_rows;        // LDS-staged matrix-core kernel: 8 or 16 activation rows per stage; 0 = other kernels
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
+  bool wave_per_simd;     // VALU path: one problem's waves are at most one for each SIMD
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
   bool k_stationary;      // the matrix-core kernel whose waves keep one k step each while the workgroup walks tiles_in_sequence tiles
 };

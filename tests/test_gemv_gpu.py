@@ -752,3 +752,30 @@ def test_single_rows_of_two_units_a_wave(gpu, bits, qop, group, ksteps):
         assert np.array_equal(got.view(np.uint16), loop.view(np.uint16))
         _, rel, _ = error_report(got, prob.oracle_gemv(threads=8))
         assert rel <= REL_TOL, rel
+
+
+@pytest.mark.parametrize("element", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,qop,group,ksteps,rows", [(4, SCALE_AND_ZEROS, 128, 9, 1), (4, SCALE_ONLY, 96, 13, 1), (4, PER_COLUMN, 0, 17, 2),
+                                                        (8, SCALE_AND_ZEROS, 64, 18, 1), (8, SCALE_ONLY, 128, 21, 3),
+                                                        (8, SCALE_AND_ZEROS, 96, 19, 4)])
+def test_first_two_units_requested_together(gpu, bits, qop, group, ksteps, rows, element):
+    """Launches of at most one wave per SIMD whose waves have three or more units, odd and even numbers of them and a shorter
+    last wave: the bits of the loop that holds one unit less (which the single-stage setting selects)."""
+    step = 512 if bits == 4 else 256
+    unit = 8 if qop == PER_COLUMN else group
+    k = ((ksteps - 1) * step + step // 2) // unit * unit
+    for n_out in (2064, 4092):
+        prob = Problem("two_ahead", n_out, k, bits, qop, group, m_batch=rows, bias=True, element=element)
+        dev = DeviceProblem(prob, gpu)
+        try:
+            mg.set_matrix_core_threshold(17)
+            plan = mg.query_launch(n_out, rows, k, bits, prob.group_size, element=element)
+            assert plan["steps_per_wave"] > 2 and plan["tiles_in_sequence"] == 1 and plan["matrix_core"] == 0, plan
+            assert plan["workgroups"] * plan["split_k"] * plan["tiles_per_wg"] <= 1024, plan
+            got = dev.run().copy()
+            mg.set_prefetch_stages(1)
+            loop = dev.run().copy()
+        finally:
+            mg.set_prefetch_stages(0)
+            mg.set_matrix_core_threshold(0)
+        assert np.array_equal(got.view(np.uint16), loop.view(np.uint16))
