@@ -186,15 +186,21 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     for (int i = 0; i < kBlocksPerUnit; ++i)
 #pragma unroll
       for (int j = 0; j < (BITS == 4 ? 4 : 2); ++j) xa.x[i][j] = u32x4{0u, 0u, 0u, 0u};
-    for (int first = 0; first < m_batch; first += 8) {
-      const int rows_here = m_batch - first < 8 ? m_batch - first : 8;
-      XRows<BITS, 8> rows;
-      fetch_x_rows<BITS, 8>(rows, p, x_rsrc, kw, lane, first, 1, rows_here);
-      // The first unit of weights is requested behind the first rows of x (an L2 hit, back long before it):
-      // the operand is turned round while the weights are still on their way.
-      if (first == 0) request_first_unit();
-      __builtin_amdgcn_sched_barrier(0);
-      park_x_rows<BITS, 8>(rows, stage, lane, 0, 1, rows_here);
+    // Rows 8-15 are requested with the others: they are in registers that the operand takes later.  (In front of their own
+    // turn, a load latency more, 4096x4096 at 16 rows took 5.85 us / 5.25, 11008x4096 8.3 / 7.8, 8192x8192 g64 12.7 / 12.1.
+    // int8, whose rows are half as long, gains nothing, and four groups per run would spill them.)
+    constexpr bool kAllRowsAhead = BITS == 4 && GROUPS_PER_RUN != 4;
+    const int rows_ahead = m_batch < 8 ? m_batch : 8;
+    XRows<BITS, 8> rows, more;
+    auto fetch_more = [&]() { fetch_x_rows<BITS, 8>(more, p, x_rsrc, kw, lane, 8, 1, m_batch - 8); };
+    fetch_x_rows<BITS, 8>(rows, p, x_rsrc, kw, lane, 0, 1, rows_ahead);
+    if (kAllRowsAhead && m_batch > 8) fetch_more();
+    // The first unit of weights is requested behind the rows of x (an L2 hit, back long before it):
+    // the operand is turned round while the weights are still on their way.
+    request_first_unit();
+    __builtin_amdgcn_sched_barrier(0);
+    auto turn_round = [&](const XRows<BITS, 8>& r, int first, int rows_here) {
+      park_x_rows<BITS, 8>(r, stage, lane, 0, 1, rows_here);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the LDS executes a wave's accesses in order
       __builtin_amdgcn_wave_barrier();
       if (m >= first && m < first + rows_here) {
@@ -206,7 +212,10 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-    }
+    };
+    turn_round(rows, 0, rows_ahead);
+    if (!kAllRowsAhead && m_batch > 8) fetch_more();
+    if (m_batch > 8) turn_round(more, 8, m_batch - 8);
   }
   const bool park_behind_stage = kLdsOperand || (tail.flags & kParkBehindStage) != 0;
   if (!park_behind_stage) __syncthreads();  // the stages make room for the partial sums
