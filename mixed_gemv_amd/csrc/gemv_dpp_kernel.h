@@ -309,6 +309,21 @@ __device__ __forceinline__ void store_outputs(const GemvTail& tail, bool has_bia
   }
 }
 
+// The same with the bias in a register.
+template <int ACT>
+__device__ __forceinline__ void store_outputs(const GemvTail& tail, uint32_t bias_bits, int n_out, int m, int tile, int lane, float sum) {
+  const int n = tile * kTileRows + lane;
+  if (lane < kTileRows && n < n_out) {
+    if constexpr (ACT == kActBf16) {
+      sum = epilogue_value(tail, sum, true, bf16_low_to_f32(bias_bits));
+      reinterpret_cast<uint16_t*>(tail.y)[(size_t)m * (size_t)n_out + n] = (uint16_t)pack_bf16(sum, 0.0f);
+    } else {
+      sum = epilogue_value(tail, sum, true, (float)splat_low(bias_bits)[0]);
+      tail.y[(size_t)m * (size_t)n_out + n] = (half_t)sum;
+    }
+  }
+}
+
 // A wave has computed the last unit of a tile: park the tile's 64 per-lane partial sums in the
 // wave's LDS slot for that tile and start afresh.  (Nothing but LDS is touched inside the unit
 // loop: a global store or bias load there would make the compiler drain the prefetched loads.)
@@ -364,7 +379,9 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 constexpr int kUnitLoop = 0;  // any number of them
 constexpr int kTwoUnits = 1;  // one or two, on one tile
 constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
-template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop>
+// EARLY_BIAS: the launch has a bias; it is requested behind the first two units (kTwoUnits, kTwoAhead).
+template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop,
+          bool EARLY_BIAS = false>
 __global__ void __launch_bounds__(kWave * (MB >= 3 || ACT == kActBf16 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup))
 __attribute__((amdgpu_waves_per_eu(ACT == kActF16 && MB == 1 && GROUPS_PER_RUN == 1 ? 6 : 1)))
 gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out, int k,
@@ -428,6 +445,18 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
 
   GemvTail late;
   if (my_tiles <= 0) late = read_tail_here();
+  // EARLY_BIAS: the bias of the tile's rows, in lanes 0-15.  Behind the barrier it is a load from memory that nothing hides.  A
+  // build of its own: a branch would leave the number of loads in flight unknown, and the waits for the units would wait for
+  // the bias as well (4096x4096 4.03 us); an empty descriptor costs launches without a bias up to 1 %.  4096x4096 with a bias
+  // 3.62 us / 3.48, int8 per column 4.86 / 4.74, 4096x11008 6.67 / 6.48.
+  uint32_t tile_bias = 0;
+  auto request_bias = [&]() {
+    if constexpr (EARLY_BIAS) {
+      const __amdgpu_buffer_rsrc_t bias_rsrc = make_rsrc(late.bias + owner * late.stride_bias, (uint32_t)p.n_out * 2u);
+      tile_bias = load_b16_low(bias_rsrc, (tile_begin * kTileRows + lane) * 2);  // rows past n_out: zero, never stored
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   if (my_tiles > 0) {
     const int total = MULTI ? my_tiles * units : units;
     const int tile_stride = p.ksteps * kUnitBytes;
@@ -491,6 +520,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
         __builtin_amdgcn_sched_barrier(0);
       };
       request(fb);
+      request_bias();
       int u = 0;
       do {
         compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
@@ -505,6 +535,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
       advance<MULTI>(cur, walk);
       load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);  // past the range of a wave with one unit: nothing
       __builtin_amdgcn_sched_barrier(0);
+      request_bias();
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
       __builtin_amdgcn_sched_barrier(0);
       if (total > 1) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
@@ -603,7 +634,11 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
       sum = (((sum + a0) + a1) + a2) + a3;
     }
     for (; w < split_k; ++w) sum += part[w * MB * kWave];
-    store_outputs<ACT>(late, has_bias, p.n_out, m, tile_begin + j, lane_c, reduce_k_slices(sum));
+    const float total_sum = reduce_k_slices(sum);
+    if constexpr (EARLY_BIAS)
+      store_outputs<ACT>(late, tile_bias, p.n_out, m, tile_begin + j, lane_c, total_sum);
+    else
+      store_outputs<ACT>(late, has_bias, p.n_out, m, tile_begin + j, lane_c, total_sum);
   }
   if constexpr (PROBE == kProbeTimeline) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // the outputs are on their way
@@ -624,9 +659,9 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
 }
 
 // Picks the instantiation for the run-time arguments.
-template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, int FORM = kUnitLoop>
+template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, int FORM = kUnitLoop, bool EARLY_BIAS = false>
 hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
-  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, FORM>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
+  return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, FORM, EARLY_BIAS>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
                 g.zero_add, g.n_out, g.k, pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups,
                 g.tail.num_groups, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
 }
@@ -636,9 +671,16 @@ hipError_t launch_gemv_kernel(const GemvLaunch& g) {
   if (g.plan.tiles_in_sequence == 1 && g.plan.stages == 2) {
     // (bf16, bound by its arithmetic, gains nothing from kTwoUnits: 4096x4096 4.83 us / 4.83)
     if constexpr (MB == 1 && ACT == kActF16) {
-      if (g.plan.steps_per_wave == 2) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits>(g);
+      if (g.plan.steps_per_wave == 2)
+        return g.tail.bias != nullptr ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits, true>(g)
+                                      : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits>(g);
     }
-    if (g.plan.wave_per_simd && g.plan.steps_per_wave > 2) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead>(g);
+    if (g.plan.wave_per_simd && g.plan.steps_per_wave > 2) {
+      if constexpr (MB == 1) {
+        if (g.tail.bias != nullptr) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead, true>(g);
+      }
+      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead>(g);
+    }
   }
   return g.plan.tiles_in_sequence > 1 ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, true, ACT>(g)
                                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT>(g);

@@ -752,6 +752,9 @@ def test_single_rows_of_two_units_a_wave(gpu, bits, qop, group, ksteps):
         assert np.array_equal(got.view(np.uint16), loop.view(np.uint16))
         _, rel, _ = error_report(got, prob.oracle_gemv(threads=8))
         assert rel <= REL_TOL, rel
+        plain = DeviceProblem(Problem("two_units", n_out, k, bits, qop, group, m_batch=1, bias=False), gpu)  # builds without the early bias
+        _, rel, _ = error_report(plain.run(), plain.p.oracle_gemv(threads=8))
+        assert rel <= REL_TOL, rel
 
 
 @pytest.mark.parametrize("element", ["f16", "bf16"])
