@@ -375,11 +375,12 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // for every further unit; kProbeLoadsOnly keeps every load and replaces the arithmetic of a unit
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
 // records timestamps and the time spent waiting for loads, per wave.
-// FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead).
+// FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead, kOneUnit).
 constexpr int kUnitLoop = 0;  // any number of them
 constexpr int kTwoUnits = 1;  // one or two, on one tile
 constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
-// EARLY_BIAS: the launch has a bias; it is requested behind the first two units (kTwoUnits, kTwoAhead).
+constexpr int kOneUnit = 3;   // one, on one tile
+// EARLY_BIAS: the launch has a bias; it is requested behind the first one or two units (not kUnitLoop).
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop,
           bool EARLY_BIAS = false>
 __global__ void __launch_bounds__(kWave * (MB >= 3 || ACT == kActBf16 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup))
@@ -513,7 +514,15 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     // 7.31 / 7.44.)  In a graph, the loop
     // / this: 1688x17376 g96 9.87 us / 9.32, 2896x10496 int8 7.95 / 7.49, 8192x8192 8.16 / 7.92, 4096x11008 6.67 / 6.54; at 3
     // rows 2596x3200 int8 5.04 / 4.81; bf16 1324x26752 13.2 / 12.6; 0.97 of the time on 78 launches of random shapes.
-    if constexpr (FORM == kTwoAhead) {
+    // A wave of one unit needs no loop, and without one the kernel takes 36-50 registers instead of 64-142 (the loop's copies of
+    // a unit): 8 waves per SIMD instead of 3-6, so more of a launch is in flight at once.  The general build / this, one row:
+    // 22016x4096 scale only 10.1 us / 9.2, 18944x3584 9.3 / 8.4, 11008x4096 g64 7.4 / 6.5, 11008x3072 g96 6.7 / 6.0, 36864x2560
+    // 11.7 / 11.0, 22016x4096 10.8 / 10.7; with a bias 11008x4096 6.1 / 5.9; bf16 13824x2048 6.1 / 6.0; 2-4 rows level.
+    if constexpr (FORM == kOneUnit) {
+      request_bias();
+      __builtin_amdgcn_sched_barrier(0);
+      compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
+    } else if constexpr (FORM == kTwoAhead) {
       auto request = [&](UnitFragment<BITS, MB, GROUPS_PER_RUN>& f) {
         advance<MULTI>(cur, walk);
         load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(f, p, w_rsrc, x_rsrc, tables, cur);
@@ -669,6 +678,12 @@ hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
 template <int BITS, int QOP, int MB, int GPR, int ACT>
 hipError_t launch_gemv_kernel(const GemvLaunch& g) {
   if (g.plan.tiles_in_sequence == 1 && g.plan.stages == 2) {
+    if (g.plan.steps_per_wave == 1) {
+      if constexpr (MB == 1) {
+        if (g.tail.bias != nullptr) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kOneUnit, true>(g);
+      }
+      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kOneUnit>(g);
+    }
     // (bf16, bound by its arithmetic, gains nothing from kTwoUnits: 4096x4096 4.83 us / 4.83)
     if constexpr (MB == 1 && ACT == kActF16) {
       if (g.plan.steps_per_wave == 2)
