@@ -14,6 +14,8 @@
 #ifndef MIXED_GEMV_AMD_GEMV_DPP_KERNEL_H_
 #define MIXED_GEMV_AMD_GEMV_DPP_KERNEL_H_
 
+#include <type_traits>
+
 #include "kernel_common.h"
 
 namespace mgemv {
@@ -366,8 +368,7 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 
 // blockDim = (64 * split_k, tiles_per_wg).  Dynamic LDS: ceil(tiles / sequences) * tiles_per_wg *
 // split_k * MB * 64 floats.
-// One activation row, one group per run: ask for 6 resident waves per SIMD (at most 80 VGPRs).
-// The allocation unit is 8 registers, so 81 would already cost a whole wave of occupancy.
+// (One row and one group per run: at most 80 VGPRs, 6 waves per SIMD; the product's builds take 36-58, the time-stamped one more.)
 // ACT: kActF16 or kActBf16 -- the type of activations, scales, zeros, bias and outputs (the
 // pointers are typed as 16-bit storage either way).
 // PROBE (measurement builds of this same kernel, see mixed_gemv.h "Measurement probes"):
@@ -482,9 +483,6 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
 
     // Two fragments in flight: the loads of unit u+1 are issued before unit u is computed, so
     // a wave that is waiting for its turn on the VALU still has memory requests outstanding.
-    // (The first fragment is loaded ahead of the loop and reaches it through register copies,
-    // which wait for its data before the second unit is requested.  A loop that loads both
-    // fragments inside, without that wait, measured the same to 2 % on every shape.)
     UnitFragment<BITS, MB, GROUPS_PER_RUN> fa, fb;
     load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fa, p, w_rsrc, x_rsrc, tables, cur);
     __builtin_amdgcn_sched_barrier(0);
@@ -501,23 +499,19 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     if constexpr (PROBE == kProbeComputeOnly) fb = fa;  // (waits for the first unit; every later "load" re-uses it)
     const bool short_ok = (late.flags & kExactIntegerFormOnly) == 0;
     const ConvertRegs c = make_convert_regs();
-    // With two or more activation rows, a wave of exactly two units runs straight-line code: the
-    // second unit is requested without waiting for the first and nothing is prefetched past the
-    // end (4096x4096: 4.44 / 4.74 / 5.04 us at 2 / 3 / 4 rows against 4.55 / 4.83 / 5.19 through
-    // the loop).  A three-unit path lost 5 % to the loop (4096x6144, 2 rows), and in the
-    // single-row kernels, which are held to 80 registers, any extra path made the loop beside it
-    // 4-7 % slower, so there the two-unit path is a build of its own, without a loop: a launch is over before the
-    // second request's latency could be hidden (through the loop / without: 4096x4096 g64 4.19 us / 3.91, scale only 3.88 /
-    // 3.74, 4096x2048 int8 3.75 / 3.60, 2500x3168 g96 4.50 / 3.93; 4096x4096 g128 with zeros 4.03 / 4.00).
-    // In a launch of at most one wave per SIMD nothing else runs while a wave's second unit is on its way, so there the first
-    // two are requested together.  (Where waves share a SIMD that loses: 4528x28032 g96, 1152 waves, 22.9 us / 23.2, 4260x7296
-    // 7.31 / 7.44.)  In a graph, the loop
-    // / this: 1688x17376 g96 9.87 us / 9.32, 2896x10496 int8 7.95 / 7.49, 8192x8192 8.16 / 7.92, 4096x11008 6.67 / 6.54; at 3
-    // rows 2596x3200 int8 5.04 / 4.81; bf16 1324x26752 13.2 / 12.6; 0.97 of the time on 78 launches of random shapes.
-    // A wave of one unit needs no loop, and without one the kernel takes 36-50 registers instead of 64-142 (the loop's copies of
-    // a unit): 8 waves per SIMD instead of 3-6, so more of a launch is in flight at once.  The general build / this, one row:
-    // 22016x4096 scale only 10.1 us / 9.2, 18944x3584 9.3 / 8.4, 11008x4096 g64 7.4 / 6.5, 11008x3072 g96 6.7 / 6.0, 36864x2560
-    // 11.7 / 11.0, 22016x4096 10.8 / 10.7; with a bias 11008x4096 6.1 / 5.9; bf16 13824x2048 6.1 / 6.0; 2-4 rows level.
+    // Builds for the lengths a wave has.  A path of its own for waves of one or two units beside the loop made the compiler copy
+    // units between two sets of registers (80-142 of them, where the loop alone takes 57-116), and each copy waits for its data.
+    // kOneUnit: 36-50 registers, 8 waves per SIMD, so more of a launch is in flight at once.  Beside the loop / alone, one row:
+    //   22016x4096 scale only 10.1 us / 9.2, 18944x3584 9.3 / 8.4, 11008x4096 g64 7.4 / 6.5, 11008x3072 g96 6.7 / 6.0, 36864x2560
+    //   11.7 / 11.0, 22016x4096 10.8 / 10.7; with a bias 11008x4096 6.1 / 5.9; bf16 13824x2048 6.1 / 6.0; 2-4 rows level.
+    // kTwoUnits: both are requested at once; such a launch is over before the second request's latency could be hidden.
+    // Through the loop / without: 4096x4096 g64 4.19 us / 3.91, scale only 3.88 / 3.74, 4096x2048 int8 3.75 / 3.60, 2500x3168
+    //   g96 4.50 / 3.93; 4096x4096 g128 with zeros 4.03 / 4.00, in bf16 level.
+    // kTwoAhead: in a launch of at most one wave per SIMD nothing else runs while a wave's second unit is on its way, so there
+    // the first two are requested together.  (Where waves share a SIMD that loses: 4528x28032 g96, 1152 waves, 22.9 us / 23.2,
+    // 4260x7296 7.31 / 7.44.)  The loop / this: 1688x17376 g96 9.87 us / 9.32, 2896x10496 int8 7.95 / 7.49, 8192x8192 8.16 /
+    //   7.92, 4096x11008 6.67 / 6.54; at 3 rows 2596x3200 int8 5.04 / 4.81; bf16 1324x26752 13.2 / 12.6; 0.97 of the time on 78
+    //   launches of random shapes.
     if constexpr (FORM == kOneUnit) {
       request_bias();
       __builtin_amdgcn_sched_barrier(0);
@@ -548,17 +542,6 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
       __builtin_amdgcn_sched_barrier(0);
       if (total > 1) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
-    } else if (total == 1) {
-      compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
-      if constexpr (MULTI) finish_tile<MB>(acc, slot);
-    } else if (MB >= 2 && !MULTI && total == 2) {
-      advance<MULTI>(cur, walk);
-      if constexpr (PROBE == kProbeComputeOnly) reuse_unit<BITS, MB, GROUPS_PER_RUN>(fb);
-      else load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);
-      __builtin_amdgcn_sched_barrier(0);
-      compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
-      __builtin_amdgcn_sched_barrier(0);
-      compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
     } else {
       // The prefetches are unconditional: past the wave's last unit every weight offset is out
       // of the descriptor's range, the loads return zero without touching memory, and the
@@ -569,6 +552,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
       // issued, which gives that behaviour -- loads and arithmetic strictly one after the other -- to the
       // same code; results do not change.
       const bool single_stage = (late.flags & kSingleStage) != 0;
+      asm volatile(".p2align 6");
       int u = 0;
       do {
         advance<MULTI>(cur, walk);
@@ -677,25 +661,19 @@ hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
 
 template <int BITS, int QOP, int MB, int GPR, int ACT>
 hipError_t launch_gemv_kernel(const GemvLaunch& g) {
+  // Waves on one tile: the build for their length, with the bias requested early for a single row.
   if (g.plan.tiles_in_sequence == 1 && g.plan.stages == 2) {
-    if (g.plan.steps_per_wave == 1) {
-      if constexpr (MB == 1) {
-        if (g.tail.bias != nullptr) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kOneUnit, true>(g);
-      }
-      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kOneUnit>(g);
-    }
-    // (bf16, bound by its arithmetic, gains nothing from kTwoUnits: 4096x4096 4.83 us / 4.83)
-    if constexpr (MB == 1 && ACT == kActF16) {
-      if (g.plan.steps_per_wave == 2)
-        return g.tail.bias != nullptr ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits, true>(g)
-                                      : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoUnits>(g);
-    }
-    if (g.plan.wave_per_simd && g.plan.steps_per_wave > 2) {
-      if constexpr (MB == 1) {
-        if (g.tail.bias != nullptr) return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead, true>(g);
-      }
-      return launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kTwoAhead>(g);
-    }
+    const int steps = g.plan.steps_per_wave;
+    const int form = steps == 1 ? kOneUnit : steps == 2 ? kTwoUnits : g.plan.wave_per_simd ? kTwoAhead : kUnitLoop;
+    const bool early_bias = MB == 1 && g.tail.bias != nullptr;
+    auto go = [&](auto f) {
+      constexpr int kForm = decltype(f)::value;
+      return early_bias ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm, MB == 1>(g)
+                        : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm>(g);
+    };
+    if (form == kOneUnit) return go(std::integral_constant<int, kOneUnit>{});
+    if (form == kTwoUnits) return go(std::integral_constant<int, kTwoUnits>{});
+    if (form == kTwoAhead) return go(std::integral_constant<int, kTwoAhead>{});
   }
   return g.plan.tiles_in_sequence > 1 ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, true, ACT>(g)
                                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT>(g);
