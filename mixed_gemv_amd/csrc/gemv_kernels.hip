@@ -231,9 +231,95 @@ PlanKnobs knobs_of_plan(const mgemv_tuned_plan& plan) {
   return kn;
 }
 
+inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Tile sequences of a four-wave workgroup (4, 2 or 1, the waves left over splitting k) with which one workgroup per compute
+// unit takes the tiles in walks of up to longest_walk that are even to 3 %; 0: none.
+inline int even_fit(int tiles, int ksteps, int longest_walk, int cus) {
+  for (int tw = 4; tw >= 1; tw /= 2) {
+    const int sequences = cus * tw, walk = ceil_div(tiles, sequences);
+    if (walk > longest_walk) continue;
+    // The k steps must divide evenly over the 4 / tw waves of a sequence as well, or a SIMD of every compute
+    // unit idles (6 k steps on 4 waves are 2 + 2 + 2 + 0): against one workgroup per tile with a wave per k step,
+    // 12288x3072 7.09 us / 5.68, 20480x3072 10.10 / 8.79, 28672x3072 12.95 / 11.05, 12288x2560 7.13 / 5.24,
+    // 12288x3584 7.18 / 6.24, 12288x5120 9.39 / 8.58; with four k steps or fewer that launch is ahead on every
+    // even fit (12288x2048 5.10 / 4.52; 20480x2048 6.78 / 5.93; 28672x2048 8.32 / 7.64; 16384x2048 5.42 / 5.23).
+    if (ksteps % (4 / tw) != 0) continue;
+    // ... and with up to 8 k steps a single tile sequence of four k-split waves (two units a wave, then the next
+    // tile) is behind a workgroup of one-unit waves per tile: 12288x4096 6.6 us / 7.3; 20480x4096 9.8 / 10.4; 20048x3840
+    // 10.0 / 11.0; 28672x4096 level (two or four sequences side by side stay: 16384x4096 8.0 / 9.0; 24576x3072 9.5 / 10.1)
+    if (ksteps <= 8 && tw == 1) continue;
+    if ((long long)walk * sequences * 100 <= (long long)tiles * 103) return tw;
+  }
+  return 0;
+}
+
+// 1 or 2: the group size divides the k step ("regular" scale addressing, one or two groups per
+// lane run); 4: any other legal group size ("generic", one lookup per block).
+int groups_per_run(int group_size, int bits) {
+  const int run = run_k(bits);
+  if (step_k(bits) % group_size != 0) return 4;
+  return group_size % run == 0 ? 1 : 2;
+}
+
+// The group size does not divide the k step: one scale / zero lookup per block of a unit.
+inline bool looks_up_per_block(int k, int group_size, int bits) {
+  return group_size > 0 && group_size != k && groups_per_run(group_size, bits) == 4;
+}
+
+// Waves per tile, each workgroup one tile, of a single row on more tiles than compute units; 0: as the rules of plan_launch
+// have it.  Those rules are older than the builds of the VALU kernel without a loop (waves of one or two units), of which more
+// are in flight at once and which request all they need up front: most launches that used to want longer waves -- walks of
+// several tiles, whole-k waves, two tiles per workgroup -- now want two units a wave.  Part of the built-in measured
+// plans, so for the device these were measured on only.
+// fp16, int4, us of the rules / here:
+//   9-16 k steps, more than 512 tiles: two units.  49152x8192 g96 48.9 / 40.9, 48672x7680 37.6 / 33.4, 16384x8192 14.0 / 13.4,
+//     20272x6144 14.5 / 13.0, 12288x5600 8.65 / 7.68, 28384x7680 20.0 / 18.5; 17456x6656 per column 11.65 / 11.9.  With the rules
+//     stay 9 and 10 k steps on 769-1024 tiles (they gain 2-6 %), 9-12 on even fits of 1025-2048 (24576x6144 level, 28672x6144 17.8 /
+//     17.4) and, on up to 640 tiles, 16 k steps (four waves of four units each) and lookups per block (8400x5280 g96 8.67 / 8.97).
+//   9-16 k steps, up to 512 tiles: one unit.  6704x5472 g96 8.05 / 6.92, 4960x4608 5.50 / 4.93, 5120x4608 5.65 / 4.99, 8192x6144
+//     6.74 / 6.65; with the rules stay 10 k steps of a regular group size (8192x5120 level) and, where they are ahead by 2-4 %,
+//     14 and more on evenly filled 512 tiles.
+//   5-8 k steps: one unit up to 5.5 tiles per compute unit (7 and 8 k steps), 8 (5) or 12 (6), then two: 71904x3584 22.5 /
+//     20.7, 99104x4096 39.4 / 37.0, 96464x2464 27.8 / 23.5, 88000x3072 27.5 / 26.7; 22016x4096 10.09, 10.18 with two.  Even fits
+//     on up to 8 tiles per compute unit stay with the rules (24576x4096 11.6 us, 11.8 with two units).
+//   17-32 k steps, up to 768 tiles: two units (8336x9216 11.8 / 10.6, 12288x9216 14.1 / 12.0, 10128x14848 17.8 / 16.8); more
+//     tiles or k steps: four waves (13488x9728 15.0 / 13.4, 28672x10240 30.1 / 28.0, 24576x15360 37.5 / 34.9; 15200x11264 16.9 /
+//     17.3) but where whole-k waves fill the SIMDs (16384x9216 15.2, four waves 15.9).
+// fp16, int8, more than 4 tiles per compute unit: one unit a wave at 10-12 k steps (85264x2560 g96 35.1 / 32.5, 40960x2816
+//   19.8 / 18.6, 20480x3072 11.5 / 11.1); more than 8: at 5-9 and 13 as well (82624x1280 g96 20.5 / 17.7, 49152x1280 11.5 / 10.8);
+//   with 14 it loses (20480x3584 12.9 / 13.8).
+// bf16 with a lookup per block, up to 2 tiles per compute unit and 16 k steps: up to eight waves (5168x2560 int8 g96 7.38 / 6.18,
+//   5248x8160 g96 10.95 / 9.15, 5360x3328 int8 9.31 / 7.65); other group sizes gain and lose.
+inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16, bool generic_groups) {
+  if (tiles <= cus || ksteps < 5) return 0;
+  if (bf16) {
+    const bool two_per_cu = tiles * 8 >= cus * 9 && tiles <= 2 * cus && ksteps >= 9 && ksteps <= 16;
+    return two_per_cu && generic_groups ? kMaxWavesPerWideWorkgroup : 0;
+  }
+  const int two_units = ceil_div(ksteps, 2);
+  if (bits == 8) {
+    if (ksteps <= 8 && tiles <= 8 * cus) return 0;
+    if (ksteps >= 10 && ksteps <= 12) return tiles > 4 * cus ? ksteps : 0;
+    return ksteps <= 13 && tiles > 8 * cus ? ksteps : 0;
+  }
+  if (ksteps <= 8) {
+    if (tiles <= 8 * cus && even_fit(tiles, ksteps, 7, cus) != 0) return 0;
+    return tiles * 2 > cus * (ksteps == 5 ? 16 : ksteps == 6 ? 24 : 11) ? two_units : 0;
+  }
+  if (ksteps <= 16) {
+    if (tiles <= 2 * cus) return (ksteps == 10 && !generic_groups) || (ksteps >= 14 && tiles * 103 >= cus * 200) ? 0 : ksteps;
+    if ((ksteps == 16 || generic_groups) && tiles * 2 <= 5 * cus) return 0;
+    if (ksteps <= 10 && tiles > 3 * cus && tiles <= 4 * cus) return 0;
+    return ksteps <= 12 && tiles > 4 * cus && tiles <= 8 * cus && even_fit(tiles, ksteps, 7, cus) != 0 ? 0 : two_units;
+  }
+  if (tiles <= 2 * cus || (tiles <= 4 * cus && tiles * 107 >= cus * 400)) return 0;
+  return tiles <= 3 * cus && ksteps <= 32 ? two_units : 4;
+}
+
 // Process-wide overrides win over the tables (they are what a tuner sweeps); then the caller's
-// entry for exactly this group size, then its entry for any group size, then the built-in table,
-// then the built-in rules.
+// entry for exactly this group size, then its entry for any group size, then the built-in table and
+// the measured ranges of single rows, then the built-in rules.
 PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus) {
   PlanKnobs kn;
   kn.split_k = g_override_split_k.load();
@@ -258,6 +344,12 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
       if (p->n_out == n_out && p->k == k && p->weight_bits == bits && p->m_batch == m_batch && p->element == element &&
           (p->group_size == group_size || p->group_size == 0))
         return knobs_of_plan(*p);
+    const int split = m_batch != 1 ? 0 : single_row_split(num_tiles(n_out), num_ksteps(k, bits), bits, num_cus, act == kActBf16,
+                                                          looks_up_per_block(k, group_size, bits));
+    if (split != 0) {
+      kn.split_k = split;
+      kn.tiles_per_wg = 1;
+    }
   }
   return kn;
 }
@@ -289,7 +381,6 @@ inline bool use_matrix_cores(int m_batch, int tiles, int ksteps, int forced, boo
          (m_batch >= 2 && !bf16 && tiles >= 6 * cus && (ksteps >= 8 || units > 64ll * cus));  // bf16, 28672x8192, 2 rows: 40.6 us against 37.8
 }
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // Tiles per workgroup of the LDS-staged matrix-core kernel (= waves that share one activation stage): as few as
 // bring the launch down to one workgroup per compute unit or fewer, at most 8 and at most a quarter of the staged
@@ -656,26 +747,11 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     // 51.5 us against 47.3; 151936x2048, 19 tiles: 31.9 against 29.8), so those are left out.
     // (The bfloat16 kernels want every SIMD busy more than they want equal walks: 28672x8192 takes
     // 35.5 us with one tile and four waves per workgroup against 38.4 with walks of 7 tiles.)
-    const int longest_walk = knobs.wide_waves ? 1 : 7;
-    for (int tw = 4; tw >= 1; tw /= 2) {
-      const int sequences = cus * tw;
-      if (ceil_div(tiles, sequences) > longest_walk) continue;
-      // The k steps must divide evenly over the 4 / tw waves of a sequence as well, or a SIMD of every compute
-      // unit idles (6 k steps on 4 waves are 2 + 2 + 2 + 0): against one workgroup per tile with a wave per k step,
-      // 12288x3072 7.09 us / 5.68, 20480x3072 10.10 / 8.79, 28672x3072 12.95 / 11.05, 12288x2560 7.13 / 5.24,
-      // 12288x3584 7.18 / 6.24, 12288x5120 9.39 / 8.58; with four k steps or fewer that launch is ahead on every
-      // even fit (12288x2048 5.10 / 4.52; 20480x2048 6.78 / 5.93; 28672x2048 8.32 / 7.64; 16384x2048 5.42 / 5.23).
-      if (ksteps % (4 / tw) != 0) continue;
-      // ... and with up to 8 k steps a single tile sequence of four k-split waves (two units a wave, then the next
-      // tile) is behind a workgroup of one-unit waves per tile: 12288x4096 6.6 us / 7.3; 20480x4096 9.8 / 10.4; 20048x3840
-      // 10.0 / 11.0; 28672x4096 level (two or four sequences side by side stay: 16384x4096 8.0 / 9.0; 24576x3072 9.5 / 10.1)
-      if (ksteps <= 8 && tw == 1) continue;
-      if ((long long)ceil_div(tiles, sequences) * sequences * 100 <= (long long)tiles * 103) {
-        tiles_per_wg = tw;
-        split_k = 4 / tw;
-        workgroup_cap = cus;
-        break;
-      }
+    const int tw = even_fit(tiles, ksteps, knobs.wide_waves ? 1 : 7, cus);
+    if (tw != 0) {
+      tiles_per_wg = tw;
+      split_k = 4 / tw;
+      workgroup_cap = cus;
     }
   }
   if (ov_sk > 0) split_k = ov_sk;
@@ -741,14 +817,6 @@ int check_problem(const void* weights, const void* scale, const void* zero_add, 
   if (reinterpret_cast<uintptr_t>(weights) % 16) return MGEMV_ERR_ALIGNMENT;
   if (reinterpret_cast<uintptr_t>(scale) % 2 || reinterpret_cast<uintptr_t>(zero_add) % 2) return MGEMV_ERR_ALIGNMENT;
   return MGEMV_OK;
-}
-
-// 1 or 2: the group size divides the k step ("regular" scale addressing, one or two groups per
-// lane run); 4: any other legal group size ("generic", one lookup per block).
-int groups_per_run(int group_size, int bits) {
-  const int run = run_k(bits);
-  if (step_k(bits) % group_size != 0) return 4;
-  return group_size % run == 0 ? 1 : 2;
 }
 
 // What a plan asks of the hardware: dynamic LDS of its (largest) launch, the workgroup size limit the
@@ -836,7 +904,7 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
   PlanKnobs knobs = knobs_for(n_out, k, bits, group_size, m_batch, act, num_cus);
   knobs.num_cus = num_cus;
   // (a group as long as k is the per-column mode, whose kernels look one scale up per row)
-  knobs.generic_groups = group_size > 0 && group_size != k && groups_per_run(group_size, bits) == 4;
+  knobs.generic_groups = looks_up_per_block(k, group_size, bits);
   if (act == kActBf16) {
     // bf16: of the matrix-core kernels the LDS-staged and the k-stationary one (both need two tiles here); the VALU
     // kernel's dequantiser wants the registers of 8-wave workgroups
