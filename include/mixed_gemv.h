@@ -394,7 +394,7 @@ MGEMV_API int mgemv_tuned_plan_clear(void);
  * compiled in): plans measured on an unpartitioned MI355X that the built-in rules do not produce.
  * It is consulted after the caller's table, for launches on a device of 256 compute units only, and
  * bypassed like the caller's table while a process-wide override is set.
- * The launches of single rows that it does not list follow rules by ranges of sizes, measured there too.
+ * Launches that it does not list follow rules by ranges of sizes, measured there too.
  * mgemv_set_default_plans(0) switches both off (1 on again); mgemv_default_plan_count tells how many
  * entries the table has. */
 MGEMV_API int mgemv_set_default_plans(int enable);

@@ -485,7 +485,7 @@ def erase_tuned_plan(n_out, k, weight_bits, group_size, m_batch, element="f16"):
 
 
 def set_default_plans(enable=True):
-    """Switches the library's built-in measured plans on or off: the table (default_plans.json) and the ranges of single rows."""
+    """Switches the library's built-in measured plans on or off: the table (default_plans.json) and the ranges of sizes."""
     _lib.check(_lib.lib().mgemv_set_default_plans(1 if enable else 0), "set_default_plans")
 
 

@@ -317,9 +317,77 @@ inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16,
   return tiles <= 3 * cus && ksteps <= 32 ? two_units : 4;
 }
 
+// Tiles per workgroup of the LDS-staged matrix-core kernel (= waves that share one activation stage): as few as
+// bring the launch down to one workgroup per compute unit or fewer, at most 8 and at most a quarter of the staged
+// rows.  Measured, 16 rows: 4096x4096 (256 tiles) 6.3 us at 1 tile against 7.2 at 2; 8192x8192 (512)
+// 13.4 at 2 against 17.8 at 4; 11008x4096 (688) 10.1 at 4 against 11.3 at 2 and 14.2 at 8;
+// 28672x8192 (1792) 28.3 at 8 against 30.6 at 4 and 32.8 at 2.  8 rows: 4096x4096 5.4 at 1
+// against 6.4 at 2; 5120x5120 (320) 7.7 at 2 against 9.3 at 1; 10240x8192 (640) 14.7 at 4
+// against 15.5 at 2; 11008x4096 9.0 at 4 against 9.7 at 2; 28672x8192 27.6 at 4 against 29.5 at 2.
+// Still more workgroups than compute units: a count just above a multiple of 256 leaves most
+// of the last round idle, and halving the tiles per workgroup evens that out (18944x3584,
+// 8 rows: 296 workgroups of 4 tiles 12.8 us, 592 of 2 tiles 11.8; 22016x4096: 14.4 / 13.3):
+// the largest count whose last round is at least three quarters full.
+inline int lds_staged_tiles_per_wg(int tiles, int staged_rows, int cus) {
+  int tw = 1;
+  while (ceil_div(tiles, tw) > cus && tw * 2 <= 8 && tw * 4 <= staged_rows) tw *= 2;
+  if (ceil_div(tiles, tw) > cus) {
+    for (int t = tw; t >= 1; t /= 2) {
+      const int wgs = ceil_div(tiles, t);
+      if (wgs * 4 >= ceil_div(wgs, cus) * cus * 3) return t;
+    }
+  }
+  return tw;
+}
+
+// Two and more rows, int4, in the same manner: launches that belong to another kernel, or to the same one in more workgroups,
+// than the rules have it.  Times are us, the rules' / here, or here as a part of theirs.
+//   fp16, 9-16 rows, a group size that divides the k step: the k-stationary kernel, since its rows 8-15 are requested with the
+//     first eight --
+//       at most one tile per compute unit, 64 tiles and more, 5-14 k steps (15 up to 14 rows): 0.79-1.005 on 31 launches, mean
+//         0.90 (4096x2560 at 14 rows 5.60 / 4.82, 3360x3584 at 13 6.17 / 4.92, 4096x6656 at 14 8.18 / 7.17); 15 k steps at 16 rows
+//         1.01-1.06, 16 0.97-1.01;
+//       two tiles per compute unit at 13-16 rows (from 1.25, which the LDS-staged kernel's pairs of tiles fill as well), 5-16
+//         k steps: 0.80-0.996 on 25, mean 0.92 (6848x5632 g64 9.64 / 8.52, 8192x8192 g64 with a bias 13.1 / 12.5); 12 k steps 1.025, and 8 on an
+//         even fit are left where the launch tests have them.
+//   bf16, 2 rows:
+//     3 k steps, walks of 20 and more: k-stationary, four workgroups per compute unit (104496x1536 21.6 / 18.8; the VALU kernel
+//       before), and 4 k steps, walks of 12 and more: two (69824x2048 20.8 / 16.6, 54528x2048 20.5 / 16.0); shorter walks gain and lose;
+//     5-16 k steps, walks of 7 and more: the LDS-staged kernel with workgroups of 4 tiles where the busiest SIMD would
+//       have 1.15 times as many units on the k-stationary one (as in use_k_stationary_bf16): 62688x2560 g96 33.9 / 26.4, 29664x4608
+//       23.5 / 20.2, 91600x3072 32.3 / 29.3; 0.75-0.99 on 16 launches, mean 0.90, and below that line 0.95-1.3 (61312x5120 g96 36.7 / 39.0);
+//   bf16, 8 k steps, walks of 31 to 40 (two rows: 27 to 48): two, three or four workgroups per compute unit at 2 / 3 / 4 rows.  0.94-0.99 /
+//     0.95-1.014 / 0.96-1.004 of the time on 11, 9 and 8 launches (128256x4096 64.5 / 61.6, 65.0 / 61.5, 64.4 / 62.7); shorter walks gain and lose 3 %.
+void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int cus, bool bf16, bool generic_groups) {
+  const int walk = ceil_div(tiles, cus);
+  auto choose = [&](int variant, int workgroups) {
+    kn.matrix_core_min_batch = 1;
+    kn.matrix_core_variant = variant;
+    kn.workgroups = workgroups;
+  };
+  if (!bf16) {
+    if (m_batch < 9 || generic_groups || ksteps < 5) return;
+    const bool one_tile = walk == 1 && tiles * 4 >= cus && (ksteps <= 14 || (ksteps == 15 && m_batch <= 14));
+    const bool two_tiles = walk == 2 && m_batch >= 13 && tiles * 4 > cus * 5 && ksteps <= 16 && ksteps != 12 &&
+                           !(ksteps == 8 && tiles == 2 * cus);
+    if (one_tile || two_tiles) choose(MGEMV_MATRIX_CORE_K_STATIONARY, 0);
+    return;
+  }
+  if (ksteps == 8 && m_batch <= 4 && (m_batch == 2 ? walk >= 27 && walk <= 48 : walk >= 31 && walk <= 40)) {
+    choose(MGEMV_MATRIX_CORE_K_STATIONARY, m_batch * cus);
+  } else if (m_batch == 2 && ksteps <= 4) {
+    if (ksteps == 3 && walk >= 20) choose(MGEMV_MATRIX_CORE_K_STATIONARY, 4 * cus);
+    if (ksteps == 4 && walk >= 12) choose(MGEMV_MATRIX_CORE_K_STATIONARY, 2 * cus);
+  } else if (m_batch == 2 && ksteps <= 16 && walk >= 7) {
+    const int tw = lds_staged_tiles_per_wg(tiles, 8, cus);
+    const long long here = 4ll * walk * ceil_div(ksteps, 4), there = (long long)ceil_div(ceil_div(tiles, tw), cus) * tw * ksteps;
+    if (tw == 4 && here * 100 >= there * 115) choose(MGEMV_MATRIX_CORE_LDS_STAGED, 0);
+  }
+}
+
 // Process-wide overrides win over the tables (they are what a tuner sweeps); then the caller's
 // entry for exactly this group size, then its entry for any group size, then the built-in table and
-// the measured ranges of single rows, then the built-in rules.
+// the measured ranges, then the built-in rules.
 PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus) {
   PlanKnobs kn;
   kn.split_k = g_override_split_k.load();
@@ -344,11 +412,16 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
       if (p->n_out == n_out && p->k == k && p->weight_bits == bits && p->m_batch == m_batch && p->element == element &&
           (p->group_size == group_size || p->group_size == 0))
         return knobs_of_plan(*p);
-    const int split = m_batch != 1 ? 0 : single_row_split(num_tiles(n_out), num_ksteps(k, bits), bits, num_cus, act == kActBf16,
-                                                          looks_up_per_block(k, group_size, bits));
-    if (split != 0) {
-      kn.split_k = split;
-      kn.tiles_per_wg = 1;
+    const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
+    const bool bf16 = act == kActBf16, per_block = looks_up_per_block(k, group_size, bits);
+    if (m_batch == 1) {
+      const int split = single_row_split(tiles, ksteps, bits, num_cus, bf16, per_block);
+      if (split != 0) {
+        kn.split_k = split;
+        kn.tiles_per_wg = 1;
+      }
+    } else if (bits == 4) {
+      set_multi_row_ranges(kn, m_batch, tiles, ksteps, num_cus, bf16, per_block);
     }
   }
   return kn;
@@ -381,29 +454,6 @@ inline bool use_matrix_cores(int m_batch, int tiles, int ksteps, int forced, boo
          (m_batch >= 2 && !bf16 && tiles >= 6 * cus && (ksteps >= 8 || units > 64ll * cus));  // bf16, 28672x8192, 2 rows: 40.6 us against 37.8
 }
 
-
-// Tiles per workgroup of the LDS-staged matrix-core kernel (= waves that share one activation stage): as few as
-// bring the launch down to one workgroup per compute unit or fewer, at most 8 and at most a quarter of the staged
-// rows.  Measured, 16 rows: 4096x4096 (256 tiles) 6.3 us at 1 tile against 7.2 at 2; 8192x8192 (512)
-// 13.4 at 2 against 17.8 at 4; 11008x4096 (688) 10.1 at 4 against 11.3 at 2 and 14.2 at 8;
-// 28672x8192 (1792) 28.3 at 8 against 30.6 at 4 and 32.8 at 2.  8 rows: 4096x4096 5.4 at 1
-// against 6.4 at 2; 5120x5120 (320) 7.7 at 2 against 9.3 at 1; 10240x8192 (640) 14.7 at 4
-// against 15.5 at 2; 11008x4096 9.0 at 4 against 9.7 at 2; 28672x8192 27.6 at 4 against 29.5 at 2.
-// Still more workgroups than compute units: a count just above a multiple of 256 leaves most
-// of the last round idle, and halving the tiles per workgroup evens that out (18944x3584,
-// 8 rows: 296 workgroups of 4 tiles 12.8 us, 592 of 2 tiles 11.8; 22016x4096: 14.4 / 13.3):
-// the largest count whose last round is at least three quarters full.
-inline int lds_staged_tiles_per_wg(int tiles, int staged_rows, int cus) {
-  int tw = 1;
-  while (ceil_div(tiles, tw) > cus && tw * 2 <= 8 && tw * 4 <= staged_rows) tw *= 2;
-  if (ceil_div(tiles, tw) > cus) {
-    for (int t = tw; t >= 1; t /= 2) {
-      const int wgs = ceil_div(tiles, t);
-      if (wgs * 4 >= ceil_div(wgs, cus) * cus * 3) return t;
-    }
-  }
-  return tw;
-}
 
 // Where the k-stationary matrix-core kernel (one wave per k step, one workgroup per compute unit walking
 // ceil(tiles / cus) tiles) is ahead of the others; fp16, 4 to 16 k steps, 2 to 16 rows (int4 unless noted).  Its waves hold
