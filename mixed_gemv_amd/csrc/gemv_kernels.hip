@@ -340,6 +340,13 @@ inline int lds_staged_tiles_per_wg(int tiles, int staged_rows, int cus) {
   return tw;
 }
 
+// Two fp16 rows, int8, more than 8 tiles per compute unit and 5-14 k steps: up to eight waves of one or two units instead of
+// whole-k waves or walks (us of the rules / here: 63808x1280 g256 16.4 / 14.5, 80768x2816 g96 45.1 / 38.6, 69392x2560 g256 29.9 /
+// 28.9; 0.85-1.002 of the time on 24 launches, mean 0.95).  Fewer tiles and longer reductions gain and lose.
+inline int two_int8_rows_split(int tiles, int ksteps, int cus) {
+  return tiles > 8 * cus && ksteps >= 5 && ksteps <= 14 ? (ksteps < 8 ? ksteps : 8) : 0;
+}
+
 // Two and more rows, int4, in the same manner: launches that belong to another kernel, or to the same one in more workgroups,
 // than the rules have it.  Times are us, the rules' / here, or here as a part of theirs.
 //   fp16, 9-16 rows, a group size that divides the k step: the k-stationary kernel, since its rows 8-15 are requested with the
@@ -414,8 +421,9 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
         return knobs_of_plan(*p);
     const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
     const bool bf16 = act == kActBf16, per_block = looks_up_per_block(k, group_size, bits);
-    if (m_batch == 1) {
-      const int split = single_row_split(tiles, ksteps, bits, num_cus, bf16, per_block);
+    if (m_batch == 1 || (m_batch == 2 && bits == 8 && !bf16)) {
+      const int split = m_batch == 1 ? single_row_split(tiles, ksteps, bits, num_cus, bf16, per_block)
+                                     : two_int8_rows_split(tiles, ksteps, num_cus);
       if (split != 0) {
         kn.split_k = split;
         kn.tiles_per_wg = 1;

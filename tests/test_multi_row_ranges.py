@@ -50,6 +50,32 @@ def test_bf16_two_to_four_rows(tiles, rows, ksteps, want):
         assert got != rules and got["matrix_core"] == want[0] and got["workgroups"] == (want[1] or got["workgroups"]), got
 
 
+@pytest.mark.parametrize("tiles, ksteps, want", [(2049, 5, 5), (2500, 8, 8), (3500, 14, 7), (2048, 8, None), (3500, 15, None),
+                                                 (3500, 4, None)])
+def test_two_fp16_rows_int8(tiles, ksteps, want):
+    args = (16 * tiles, 2, 256 * ksteps, 8, 128)
+    got = mg.query_launch(*args, num_compute_units=256)
+    cov = mg.plan_coverage(*args, num_compute_units=256)
+    assert cov["tiles_miscovered"] == 0 and cov["bad_waves"] == 0
+    mg.set_default_plans(False)
+    try:
+        rules = mg.query_launch(*args, num_compute_units=256)
+    finally:
+        mg.set_default_plans(True)
+    if want is None:
+        assert got == rules
+    else:
+        assert (got["matrix_core"], got["split_k"], got["tiles_per_wg"], got["tiles_in_sequence"]) == (VALU, want, 1, 1), got
+
+
+@pytest.mark.gpu
+def test_two_fp16_rows_int8_results(gpu):
+    prob = Problem("ranges", 32788, 2568, 8, PER_COLUMN, 0, m_batch=2, bias=True, x_dist="normal")   # 2050 tiles, 11 k steps: 2 x 5 + 1
+    assert mg.query_launch(32788, 2, 2568, 8, 2568, num_compute_units=256)["split_k"] == 6
+    _, rel, _ = error_report(DeviceProblem(prob, gpu).run(), prob.oracle_gemv(threads=16))
+    assert rel <= 2e-3, rel
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n_out, rows, k, qop, group, bias, element, kind", [
     (1028, 9, 2576, PER_COLUMN, 0, True, "f16", KSTAT),                 # 65 tiles, the last of four rows; the last k step of 16 elements
