@@ -262,9 +262,9 @@ int groups_per_run(int group_size, int bits) {
   return group_size % run == 0 ? 1 : 2;
 }
 
-// The group size does not divide the k step: one scale / zero lookup per block of a unit.
-inline bool looks_up_per_block(int k, int group_size, int bits) {
-  return group_size > 0 && group_size != k && groups_per_run(group_size, bits) == 4;
+// Scale / zero lookups per lane run of a launch: groups_per_run, one for a group as long as k (per-column mode) or none given.
+inline int lookups_per_run(int k, int group_size, int bits) {
+  return group_size > 0 && group_size != k ? groups_per_run(group_size, bits) : 1;
 }
 
 // Waves per tile, each workgroup one tile, of a single row on more tiles than compute units; 0: as the rules of plan_launch
@@ -276,7 +276,8 @@ inline bool looks_up_per_block(int k, int group_size, int bits) {
 //   9-16 k steps, more than 512 tiles: two units.  49152x8192 g96 48.9 / 40.9, 48672x7680 37.6 / 33.4, 16384x8192 14.0 / 13.4,
 //     20272x6144 14.5 / 13.0, 12288x5600 8.65 / 7.68, 28384x7680 20.0 / 18.5; 17456x6656 per column 11.65 / 11.9.  With the rules
 //     stay 9 and 10 k steps on 769-1024 tiles (they gain 2-6 %), 9-12 on even fits of 1025-2048 (24576x6144 level, 28672x6144 17.8 /
-//     17.4) and, on up to 640 tiles, 16 k steps (four waves of four units each) and lookups per block (8400x5280 g96 8.67 / 8.97).
+//     17.4) and, on up to 640 tiles, 16 k steps (four waves of four units each) and lookups per block (8400x5280 g96 8.67 / 8.97),
+//     and two lookups per run where a wave per tile fills the SIMDs (16384x6144 g64 scale only 9.85 / 10.3, 16384x8192 g64 14.1 / 14.5).
 //   9-16 k steps, up to 512 tiles: one unit.  6704x5472 g96 8.05 / 6.92, 4960x4608 5.50 / 4.93, 5120x4608 5.65 / 4.99, 8192x6144
 //     6.74 / 6.65; with the rules stay 10 k steps of a regular group size (8192x5120 level) and, where they are ahead by 2-4 %,
 //     14 and more on evenly filled 512 tiles.
@@ -284,15 +285,16 @@ inline bool looks_up_per_block(int k, int group_size, int bits) {
 //     20.7, 99104x4096 39.4 / 37.0, 96464x2464 27.8 / 23.5, 88000x3072 27.5 / 26.7; 22016x4096 10.09, 10.18 with two.  Even fits
 //     on up to 8 tiles per compute unit stay with the rules (24576x4096 11.6 us, 11.8 with two units).
 //   17-32 k steps, up to 768 tiles: two units (8336x9216 11.8 / 10.6, 12288x9216 14.1 / 12.0, 10128x14848 17.8 / 16.8); more
-//     tiles or k steps: four waves (13488x9728 15.0 / 13.4, 28672x10240 30.1 / 28.0, 24576x15360 37.5 / 34.9; 15200x11264 16.9 /
-//     17.3) but where whole-k waves fill the SIMDs (16384x9216 15.2, four waves 15.9).
+//     than 1024: four waves (28672x10240 30.1 / 28.0, 24576x15360 37.5 / 34.9; in between 0.89-1.045, left with the rules).
 // fp16, int8, more than 4 tiles per compute unit: one unit a wave at 10-12 k steps (85264x2560 g96 35.1 / 32.5, 40960x2816
 //   19.8 / 18.6, 20480x3072 11.5 / 11.1); more than 8: at 5-9 and 13 as well (82624x1280 g96 20.5 / 17.7, 49152x1280 11.5 / 10.8);
 //   with 14 it loses (20480x3584 12.9 / 13.8).
 // bf16 with a lookup per block, up to 2 tiles per compute unit and 16 k steps: up to eight waves (5168x2560 int8 g96 7.38 / 6.18,
 //   5248x8160 g96 10.95 / 9.15, 5360x3328 int8 9.31 / 7.65); other group sizes gain and lose.
-inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16, bool generic_groups) {
+inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16, int lookups) {
   if (tiles <= cus || ksteps < 5) return 0;
+  const bool generic_groups = lookups == 4;
+  const bool fills_simds = tiles <= 4 * cus && tiles * 103 >= cus * 400;  // with a wave per tile
   if (bf16) {
     const bool two_per_cu = tiles * 8 >= cus * 9 && tiles <= 2 * cus && ksteps >= 9 && ksteps <= 16;
     return two_per_cu && generic_groups ? kMaxWavesPerWideWorkgroup : 0;
@@ -310,10 +312,10 @@ inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16,
   if (ksteps <= 16) {
     if (tiles <= 2 * cus) return (ksteps == 10 && !generic_groups) || (ksteps >= 14 && tiles * 103 >= cus * 200) ? 0 : ksteps;
     if ((ksteps == 16 || generic_groups) && tiles * 2 <= 5 * cus) return 0;
-    if (ksteps <= 10 && tiles > 3 * cus && tiles <= 4 * cus) return 0;
+    if ((ksteps <= 10 && tiles > 3 * cus && tiles <= 4 * cus) || (fills_simds && lookups == 2)) return 0;
     return ksteps <= 12 && tiles > 4 * cus && tiles <= 8 * cus && even_fit(tiles, ksteps, 7, cus) != 0 ? 0 : two_units;
   }
-  if (tiles <= 2 * cus || (tiles <= 4 * cus && tiles * 107 >= cus * 400)) return 0;
+  if (tiles <= 2 * cus || (tiles > 3 * cus && tiles <= 4 * cus)) return 0;
   return tiles <= 3 * cus && ksteps <= 32 ? two_units : 4;
 }
 
@@ -420,16 +422,17 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
           (p->group_size == group_size || p->group_size == 0))
         return knobs_of_plan(*p);
     const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
-    const bool bf16 = act == kActBf16, per_block = looks_up_per_block(k, group_size, bits);
+    const bool bf16 = act == kActBf16;
+    const int lookups = lookups_per_run(k, group_size, bits);
     if (m_batch == 1 || (m_batch == 2 && bits == 8 && !bf16)) {
-      const int split = m_batch == 1 ? single_row_split(tiles, ksteps, bits, num_cus, bf16, per_block)
+      const int split = m_batch == 1 ? single_row_split(tiles, ksteps, bits, num_cus, bf16, lookups)
                                      : two_int8_rows_split(tiles, ksteps, num_cus);
       if (split != 0) {
         kn.split_k = split;
         kn.tiles_per_wg = 1;
       }
     } else if (bits == 4) {
-      set_multi_row_ranges(kn, m_batch, tiles, ksteps, num_cus, bf16, per_block);
+      set_multi_row_ranges(kn, m_batch, tiles, ksteps, num_cus, bf16, lookups == 4);
     }
   }
   return kn;
@@ -962,7 +965,7 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
   PlanKnobs knobs = knobs_for(n_out, k, bits, group_size, m_batch, act, num_cus);
   knobs.num_cus = num_cus;
   // (a group as long as k is the per-column mode, whose kernels look one scale up per row)
-  knobs.generic_groups = looks_up_per_block(k, group_size, bits);
+  knobs.generic_groups = lookups_per_run(k, group_size, bits) == 4;
   if (act == kActBf16) {
     // bf16: of the matrix-core kernels the LDS-staged and the k-stationary one (both need two tiles here); the VALU
     // kernel's dequantiser wants the registers of 8-wave workgroups

@@ -34,8 +34,8 @@ def waves(tiles, ksteps, bits=4, group=128, element="f16"):
     (3072, 16, 8), (9000, 12, 6),
     # 5-8 k steps: two units where there are many tiles, but for even fits
     (2049, 5, 3), (3073, 6, 3), (2050, 6, None), (1409, 8, 4), (1408, 8, None), (1536, 8, None), (2000, 7, None), (8000, 7, 4),
-    # longer reductions: two units up to 768 tiles and 32 k steps, else four waves unless whole-k waves fill the SIMDs
-    (513, 17, 9), (768, 32, 16), (768, 33, 4), (769, 20, 4), (1000, 20, None), (512, 20, None), (2000, 30, 4)])
+    # longer reductions: two units up to 768 tiles and 32 k steps, four waves above 1024
+    (513, 17, 9), (768, 32, 16), (768, 33, 4), (769, 20, None), (1024, 20, None), (1100, 33, None), (512, 20, None), (2000, 30, 4)])
 def test_fp16_int4(tiles, ksteps, want):
     assert waves(tiles, ksteps) == want
 
@@ -50,6 +50,11 @@ def test_groups_that_do_not_divide_the_k_step():
     assert waves(400, 10, group=96) == 10                                            # fp16: ten of them too
     assert [waves(400, ks, group=96, element="bf16") for ks in (8, 9, 16, 17)] == [None, 5, 8, None]
     assert waves(400, 12, element="bf16") is None and waves(513, 12, group=96, element="bf16") is None
+
+
+def test_two_lookups_per_run_where_a_wave_per_tile_fills_the_simds():
+    assert [waves(tiles, 12, group=64) for tiles in (993, 994, 995, 1024)] == [6, 6, None, None]
+    assert waves(1024, 12) == 6
 
 
 def test_other_devices_and_overrides_keep_the_rules():
