@@ -18,6 +18,14 @@ extern "C" {
  * shape cannot read faster than X" is a kernel anybody can run, not a remark.
  * ---------------------------------------------------------------------------------------- */
 
+/* Which build of the VALU kernel a launch of batch_count problems takes on a device of num_compute_units compute
+ * units: MGEMV_UNIT_FORM_LOOP (any number of units per wave; also reported for matrix-core launches),
+ * _TWO (waves of one or two units), _TWO_AHEAD (longer waves that have a SIMD to themselves, the first two units
+ * requested together) or _ONE (waves of one unit).  The results do not depend on it. */
+enum { MGEMV_UNIT_FORM_LOOP = 0, MGEMV_UNIT_FORM_TWO = 1, MGEMV_UNIT_FORM_TWO_AHEAD = 2, MGEMV_UNIT_FORM_ONE = 3 };
+MGEMV_API int mgemv_probe_unit_form(int n_out, int m_batch, int k, int weight_bits, int group_size, int element,
+                                    int batch_count, int num_compute_units, int *form);
+
 /* One empty kernel launch (one wave, no instruction but the end of the program). */
 MGEMV_API int mgemv_probe_empty_launch(void *stream);
 /* The same with a grid of `workgroups` workgroups of `waves_per_workgroup` waves (1-16), e.g. the

@@ -48,6 +48,7 @@ SIGNATURES = {
     "mgemv_set_prefetch_stages": (_c.c_int, [_c.c_int]),
     "mgemv_plan_coverage": (_c.c_int, [_c.c_int] * 7 + [_c.POINTER(_c.c_int64 * 8)]),
     "mgemv_gemv_arguments": (_c.c_int, [_vp, _vp]),
+    "mgemv_probe_unit_form": (_c.c_int, [_c.c_int] * 8 + [_c.POINTER(_c.c_int)]),
     "mgemv_probe_empty_launch": (_c.c_int, [_vp]),
     "mgemv_probe_empty_grid": (_c.c_int, [_c.c_int, _c.c_int, _vp]),
     "mgemv_probe_stream_read": (_c.c_int, [_vp, _c.c_size_t, _c.c_int, _c.c_int, _c.c_int, _vp, _vp]),

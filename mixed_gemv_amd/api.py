@@ -429,6 +429,21 @@ PROBE_COMPUTE_ONLY = 3
 PROBE_TIMELINE_WAITS = 4
 
 
+UNIT_FORM_LOOP = 0
+UNIT_FORM_TWO = 1
+UNIT_FORM_TWO_AHEAD = 2
+UNIT_FORM_ONE = 3
+
+
+def probe_unit_form(n_out, m_batch, k, weight_bits=4, group_size=0, element="f16", batch_count=1, num_compute_units=256):
+    """Which build of the VALU kernel a launch of batch_count problems takes: UNIT_FORM_* (mgemv_probe_unit_form)."""
+    out = ctypes.c_int()
+    _lib.check(_lib.lib().mgemv_probe_unit_form(int(n_out), int(m_batch), int(k), int(weight_bits), int(group_size),
+                                                1 if _is_bf16(element, None) else 0, int(batch_count), int(num_compute_units),
+                                                ctypes.byref(out)), "probe_unit_form")
+    return out.value
+
+
 def probe_empty_launch(stream=None):
     """One empty kernel launch (mgemv_probe_empty_launch)."""
     _lib.check(_lib.lib().mgemv_probe_empty_launch(_stream_ptr(stream)), "probe_empty_launch")

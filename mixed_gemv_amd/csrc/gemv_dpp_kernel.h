@@ -377,10 +377,6 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
 // records timestamps and the time spent waiting for loads, per wave.
 // FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead, kOneUnit).
-constexpr int kUnitLoop = 0;  // any number of them
-constexpr int kTwoUnits = 1;  // one or two, on one tile
-constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
-constexpr int kOneUnit = 3;   // one, on one tile
 // EARLY_BIAS: the launch has a bias; it is requested behind the first one or two units (not kUnitLoop).
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop,
           bool EARLY_BIAS = false>
@@ -662,18 +658,17 @@ hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
 template <int BITS, int QOP, int MB, int GPR, int ACT>
 hipError_t launch_gemv_kernel(const GemvLaunch& g) {
   // Waves on one tile: the build for their length, with the bias requested early for a single row.
-  if (g.plan.tiles_in_sequence == 1 && g.plan.stages == 2) {
-    const int steps = g.plan.steps_per_wave;
-    const int form = steps == 1 ? kOneUnit : steps == 2 ? kTwoUnits : g.plan.wave_per_simd ? kTwoAhead : kUnitLoop;
-    const bool early_bias = MB == 1 && g.tail.bias != nullptr;
-    auto go = [&](auto f) {
-      constexpr int kForm = decltype(f)::value;
-      return early_bias ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm, MB == 1>(g)
-                        : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm>(g);
-    };
-    if (form == kOneUnit) return go(std::integral_constant<int, kOneUnit>{});
-    if (form == kTwoUnits) return go(std::integral_constant<int, kTwoUnits>{});
-    if (form == kTwoAhead) return go(std::integral_constant<int, kTwoAhead>{});
+  const bool early_bias = MB == 1 && g.tail.bias != nullptr;
+  auto go = [&](auto f) {
+    constexpr int kForm = decltype(f)::value;
+    return early_bias ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm, MB == 1>(g)
+                      : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm>(g);
+  };
+  switch (g.form) {
+    case kOneUnit: return go(std::integral_constant<int, kOneUnit>{});
+    case kTwoUnits: return go(std::integral_constant<int, kTwoUnits>{});
+    case kTwoAhead: return go(std::integral_constant<int, kTwoAhead>{});
+    default: break;
   }
   return g.plan.tiles_in_sequence > 1 ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, true, ACT>(g)
                                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT>(g);

@@ -845,7 +845,6 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
             (long long)seq_tiles() * tiles_per_wg * split_k * rows * kWave * 4 > 64 * 1024))
       lp.workgroups = lp.workgroups * 2 < ceil_div(groups, tiles_per_wg) ? lp.workgroups * 2 : ceil_div(groups, tiles_per_wg);
     lp.tiles_in_sequence = seq_tiles();
-    lp.wave_per_simd = (long long)lp.workgroups * split_k * tiles_per_wg <= 4ll * cus;
   }
   lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
   lp.threads = kWave * split_k * tiles_per_wg;
@@ -1008,6 +1007,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.group_size = group_size;
   g.plan = plan_launch(n_out, k, weight_bits, m_batch,
                        knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus));
+  g.form = unit_form(g.plan, batch_count, info.num_cus);
   g.tail.bias = reinterpret_cast<const half_t*>(bias);
   g.tail.split_k = g.plan.split_k;
   g.tail.num_groups = k / group_size;
@@ -1560,6 +1560,21 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
   out[5] = busy_waves;
   out[6] = idle_waves;
   out[7] = max_units;             // most units any wave computes
+  return MGEMV_OK;
+}
+
+int mgemv_probe_unit_form(int n_out, int m_batch, int k, int weight_bits, int group_size, int element, int batch_count,
+                          int num_compute_units, int* form) {
+  using namespace mgemv;
+  if (form == nullptr) return MGEMV_ERR_NULL_POINTER;
+  if (element != MGEMV_ELEMENT_F16 && element != MGEMV_ELEMENT_BF16) return MGEMV_ERR_QUANT_TYPE;
+  if (num_compute_units < 1 || num_compute_units > 4096) return MGEMV_ERR_SIZE;
+  if (batch_count < 1 || batch_count > 65535) return MGEMV_ERR_BATCH;
+  if (const int st = check_tuned_key(n_out, k, weight_bits, group_size, m_batch)) return st;
+  const int act = element == MGEMV_ELEMENT_BF16 ? kActBf16 : kActF16;
+  const LaunchPlan lp = plan_launch(n_out, k, weight_bits, m_batch,
+                                    knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, num_compute_units));
+  *form = unit_form(lp, batch_count, num_compute_units);
   return MGEMV_OK;
 }
 

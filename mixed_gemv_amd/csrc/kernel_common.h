@@ -272,10 +272,26 @@ struct LaunchPlan {
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
   int staged_rows;        // LDS-staged matrix-core kernel: 8 or 16 activation rows per stage; 0 = other kernels
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
-  bool wave_per_simd;     // VALU path: one problem's waves are at most one for each SIMD
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
   bool k_stationary;      // the matrix-core kernel whose waves keep one k step each while the workgroup walks tiles_in_sequence tiles
 };
+
+// How a wave of the VALU kernel goes through its units (one build of the kernel each).
+constexpr int kUnitLoop = 0;  // any number of them
+constexpr int kTwoUnits = 1;  // one or two, on one tile
+constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
+constexpr int kOneUnit = 3;   // one, on one tile
+
+// The build a launch takes.  All four compute the same bits, so the number of problems in a batched or routed launch may
+// count here, which it does not in the plan.  kTwoAhead is for launches of at most one wave per SIMD, all problems taken
+// together: nine problems of 4516x2112 int8 g96 18.7 us / 17.7 in the loop, ten of 3504x5568 g96 25.0 / 24.2, eleven of
+// 1740x5120 int8 17.4 / 16.8; 0.946-1.026 of the time on 109 launches of random shapes, mean 0.99.  The figures of single problems
+// stand at the kernel's builds.
+inline int unit_form(const LaunchPlan& plan, int batch_count, int cus) {
+  if (plan.matrix_core || plan.tiles_in_sequence != 1 || plan.stages != 2) return kUnitLoop;
+  if (plan.steps_per_wave <= 2) return plan.steps_per_wave == 1 ? kOneUnit : kTwoUnits;
+  return (long long)plan.workgroups * plan.split_k * plan.tiles_per_wg * batch_count <= 4ll * cus ? kTwoAhead : kUnitLoop;
+}
 
 // Launches through hipLaunchKernel so that the status returned is this launch's own, not a
 // stale sticky error left behind by some other runtime call of the process.
@@ -293,6 +309,7 @@ struct GemvLaunch {
   const half_t* zero_add;
   int n_out, k, group_size;
   LaunchPlan plan;
+  int form;  // VALU kernel: unit_form
   GemvTail tail;
   dim3 grid, block;
   size_t lds;
