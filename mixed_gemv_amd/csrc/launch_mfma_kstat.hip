@@ -188,19 +188,20 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       for (int j = 0; j < (BITS == 4 ? 4 : 2); ++j) xa.x[i][j] = u32x4{0u, 0u, 0u, 0u};
     // Rows 8-15 are requested with the others: they are in registers that the operand takes later.  (In front of their own
     // turn, a load latency more, 4096x4096 at 16 rows took 5.85 us / 5.25, 11008x4096 8.3 / 7.8, 8192x8192 g64 12.7 / 12.1.
-    // int8, whose rows are half as long, gains nothing, and four groups per run would spill them.)
+    // int8, whose rows are half as long, gains nothing.)  Four groups per run leave no registers for them: eight rows at a time,
+    // in their own turn, spill 48 registers of the build with zeros, four at a time 16 (4096x4032 g96 at 16 rows 9.4 us / 7.35,
+    // 8192x8064 22.1 / 17.5, 28672x8064 42.6 / 38.5; at 12 rows 0.95 of the time, up to 9 rows 1.02).
     constexpr bool kAllRowsAhead = BITS == 4 && GROUPS_PER_RUN != 4;
+    constexpr int kLateRows = BITS == 4 ? 4 : 8;  // rows 8-15 requested at once where they are not ahead
     const int rows_ahead = m_batch < 8 ? m_batch : 8;
     XRows<BITS, 8> rows, more;
-    auto fetch_more = [&]() { fetch_x_rows<BITS, 8>(more, p, x_rsrc, kw, lane, 8, 1, m_batch - 8); };
     fetch_x_rows<BITS, 8>(rows, p, x_rsrc, kw, lane, 0, 1, rows_ahead);
-    if (kAllRowsAhead && m_batch > 8) fetch_more();
+    if (kAllRowsAhead && m_batch > 8) fetch_x_rows<BITS, 8>(more, p, x_rsrc, kw, lane, 8, 1, m_batch - 8);
     // The first unit of weights is requested behind the rows of x (an L2 hit, back long before it):
     // the operand is turned round while the weights are still on their way.
     request_first_unit();
     __builtin_amdgcn_sched_barrier(0);
-    auto turn_round = [&](const XRows<BITS, 8>& r, int first, int rows_here) {
-      park_x_rows<BITS, 8>(r, stage, lane, 0, 1, rows_here);
+    auto read_back = [&](int first, int rows_here) {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the LDS executes a wave's accesses in order
       __builtin_amdgcn_wave_barrier();
       if (m >= first && m < first + rows_here) {
@@ -213,9 +214,22 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     };
-    turn_round(rows, 0, rows_ahead);
-    if (!kAllRowsAhead && m_batch > 8) fetch_more();
-    if (m_batch > 8) turn_round(more, 8, m_batch - 8);
+    park_x_rows<BITS, 8>(rows, stage, lane, 0, 1, rows_ahead);
+    read_back(0, rows_ahead);
+    if (m_batch > 8) {
+      if constexpr (kAllRowsAhead) {
+        park_x_rows<BITS, 8>(more, stage, lane, 0, 1, m_batch - 8);
+      } else {
+        for (int first = 8; first < 16; first += kLateRows) {
+          if (kLateRows < 8 && first >= m_batch) break;
+          const int rows_here = m_batch - first < kLateRows ? m_batch - first : kLateRows;
+          XRows<BITS, kLateRows> late_rows;
+          fetch_x_rows<BITS, kLateRows>(late_rows, p, x_rsrc, kw, lane, first, 1, rows_here);
+          park_x_rows<BITS, kLateRows>(late_rows, stage, lane, first - 8, 1, rows_here);
+        }
+      }
+      read_back(8, m_batch - 8);
+    }
   }
   const bool park_behind_stage = kLdsOperand || (tail.flags & kParkBehindStage) != 0;
   if (!park_behind_stage) __syncthreads();  // the stages make room for the partial sums
