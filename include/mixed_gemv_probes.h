@@ -41,7 +41,8 @@ MGEMV_API int mgemv_probe_stream_read(const void *src, size_t bytes, int workgro
                                       int units_in_flight, uint32_t *sink, void *stream);
 
 /* Measurement builds of the single-row int4 scale-and-zero fp16 GEMV kernel (one group per lane
- * run: group sizes that are multiples of 128), launched with the geometry mgemv_gemv would use:
+ * run: group sizes that are multiples of 128), launched with the geometry mgemv_gemv would use, in the
+ * build that it would use for waves of that length (mgemv_probe_unit_form):
  *   MGEMV_PROBE_LOADS_ONLY  every load of the kernel, the arithmetic of a unit replaced by an
  *                           exclusive-or over its registers; y receives meaningless values;
  *   MGEMV_PROBE_TIMELINE    the kernel as it is, plus MGEMV_PROBE_TIMELINE_WORDS 64-bit words per

@@ -371,7 +371,7 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // (One row and one group per run: at most 80 VGPRs, 6 waves per SIMD; the product's builds take 36-58, the time-stamped one more.)
 // ACT: kActF16 or kActBf16 -- the type of activations, scales, zeros, bias and outputs (the
 // pointers are typed as 16-bit storage either way).
-// PROBE (measurement builds of this same kernel, see mixed_gemv.h "Measurement probes"):
+// PROBE (measurement builds, one for each way through the units, see mixed_gemv_probes.h):
 // kProbeNone the product; kProbeComputeOnly loads a wave's first unit only and repeats its arithmetic
 // for every further unit; kProbeLoadsOnly keeps every load and replaces the arithmetic of a unit
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
@@ -488,10 +488,24 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     if constexpr (PROBE == kProbeTimeline) {
       __builtin_amdgcn_sched_barrier(0);
       stamp[1] = __builtin_amdgcn_s_memrealtime();      // the first unit is requested
-      asm volatile("s_waitcnt vmcnt(3)" ::: "memory");   // ... and all but its last three blocks are in
-      stamp[2] = __builtin_amdgcn_s_memrealtime();
       __builtin_amdgcn_sched_barrier(0);
     }
+    // Timeline probe, in front of unit u's arithmetic, with `behind` loads of the next unit issued behind its own.
+    constexpr int kLoadsOfUnit = MB + GROUPS_PER_RUN * 2 + kBlocksPerUnit;
+    auto timeline_unit = [&](auto behind, int u, int total) {
+      if constexpr (PROBE == kProbeTimeline) {
+        constexpr int kBehindFirstBlock = kBlocksPerUnit - 1 + decltype(behind)::value;
+        if (u == 0) {
+          asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kBehindFirstBlock) : "memory");  // all but the first unit's last three blocks are in
+          stamp[2] = __builtin_amdgcn_s_memrealtime();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (late.flags & kTimelineWaits) timeline_wait<kBehindFirstBlock>(waits, u, total);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    using NoLoadsBehind = std::integral_constant<int, 0>;
+    using NextUnitBehind = std::integral_constant<int, kLoadsOfUnit>;
     if constexpr (PROBE == kProbeComputeOnly) fb = fa;  // (waits for the first unit; every later "load" re-uses it)
     const bool short_ok = (late.flags & kExactIntegerFormOnly) == 0;
     const ConvertRegs c = make_convert_regs();
@@ -511,33 +525,44 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     if constexpr (FORM == kOneUnit) {
       request_bias();
       __builtin_amdgcn_sched_barrier(0);
+      timeline_unit(NoLoadsBehind{}, 0, total);
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
     } else if constexpr (FORM == kTwoAhead) {
       auto request = [&](UnitFragment<BITS, MB, GROUPS_PER_RUN>& f) {
         advance<MULTI>(cur, walk);
-        load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(f, p, w_rsrc, x_rsrc, tables, cur);
+        if constexpr (PROBE == kProbeComputeOnly) reuse_unit<BITS, MB, GROUPS_PER_RUN>(f);
+        else load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(f, p, w_rsrc, x_rsrc, tables, cur);
         __builtin_amdgcn_sched_barrier(0);
       };
       request(fb);
       request_bias();
       int u = 0;
       do {
+        timeline_unit(NextUnitBehind{}, u, total);
         compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
         __builtin_amdgcn_sched_barrier(0);
         request(fa);
-        if (u + 1 < total) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+        if (u + 1 < total) {
+          timeline_unit(NextUnitBehind{}, u + 1, total);
+          compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+        }
         __builtin_amdgcn_sched_barrier(0);
         request(fb);
         u += 2;
       } while (u < total);
     } else if constexpr (FORM == kTwoUnits) {
       advance<MULTI>(cur, walk);
-      load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);  // past the range of a wave with one unit: nothing
+      if constexpr (PROBE == kProbeComputeOnly) reuse_unit<BITS, MB, GROUPS_PER_RUN>(fb);
+      else load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);  // past the range of a wave with one unit: nothing
       __builtin_amdgcn_sched_barrier(0);
       request_bias();
+      timeline_unit(NextUnitBehind{}, 0, total);
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
       __builtin_amdgcn_sched_barrier(0);
-      if (total > 1) compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+      if (total > 1) {
+        timeline_unit(NoLoadsBehind{}, 1, total);
+        compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
+      }
     } else {
       // The prefetches are unconditional: past the wave's last unit every weight offset is out
       // of the descriptor's range, the loads return zero without touching memory, and the
@@ -556,10 +581,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
         else load_unit<BITS, QOP, MB, GROUPS_PER_RUN>(fb, p, w_rsrc, x_rsrc, tables, cur);
         if (single_stage) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the arithmetic it overlaps
-        if constexpr (PROBE == kProbeTimeline) {
-          if (late.flags & kTimelineWaits) timeline_wait<kBlocksPerUnit - 1 + MB + GROUPS_PER_RUN * 2 + kBlocksPerUnit>(waits, u, total);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        timeline_unit(NextUnitBehind{}, u, total);
         compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
         if constexpr (MULTI) {
           if (--pending == 0) {
@@ -574,10 +596,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
         if (single_stage) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         if (u + 1 < total) {
-          if constexpr (PROBE == kProbeTimeline) {
-            if (late.flags & kTimelineWaits) timeline_wait<kBlocksPerUnit - 1 + MB + GROUPS_PER_RUN * 2 + kBlocksPerUnit>(waits, u + 1, total);
-            __builtin_amdgcn_sched_barrier(0);
-          }
+          timeline_unit(NextUnitBehind{}, u + 1, total);
           compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fb, c, short_ok);
           if constexpr (MULTI) {
             if (--pending == 0) {

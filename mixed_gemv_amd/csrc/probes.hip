@@ -56,9 +56,14 @@ hipError_t launch_gemv_probe_kind(const GemvLaunch& g) {
                   pack_steps(num_ksteps(g.k, 4), g.plan.steps_per_wave), g.plan.workgroups, g.tail.num_groups,
                   pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
   };
-  return g.plan.tiles_in_sequence > 1
-             ? args(gemv_dpp_kernel<4, MGEMV_FINEGRAINED_SCALE_AND_ZEROS, 1, 1, true, kActF16, PROBE>)
-             : args(gemv_dpp_kernel<4, MGEMV_FINEGRAINED_SCALE_AND_ZEROS, 1, 1, false, kActF16, PROBE>);
+  constexpr int kQuant = MGEMV_FINEGRAINED_SCALE_AND_ZEROS;
+  if (g.plan.tiles_in_sequence > 1) return args(gemv_dpp_kernel<4, kQuant, 1, 1, true, kActF16, PROBE>);
+  switch (g.form) {  // the build the product launches
+    case kOneUnit: return args(gemv_dpp_kernel<4, kQuant, 1, 1, false, kActF16, PROBE, kOneUnit>);
+    case kTwoUnits: return args(gemv_dpp_kernel<4, kQuant, 1, 1, false, kActF16, PROBE, kTwoUnits>);
+    case kTwoAhead: return args(gemv_dpp_kernel<4, kQuant, 1, 1, false, kActF16, PROBE, kTwoAhead>);
+    default: return args(gemv_dpp_kernel<4, kQuant, 1, 1, false, kActF16, PROBE>);
+  }
 }
 
 hipError_t launch_gemv_probe(const GemvLaunch& g, int probe) {
