@@ -573,7 +573,7 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
       // issued, which gives that behaviour -- loads and arithmetic strictly one after the other -- to the
       // same code; results do not change.
       const bool single_stage = (late.flags & kSingleStage) != 0;
-      asm volatile(".p2align 6");
+      asm volatile(".p2align 6");  // the loop begins at most a few moves behind a 64-byte line, whatever is in front of it
       int u = 0;
       do {
         advance<MULTI>(cur, walk);
