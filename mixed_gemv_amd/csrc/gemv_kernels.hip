@@ -786,16 +786,21 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     // A single bf16 row on 700 and more tiles, up to 16 k steps.  A wave per k step leaves the SIMDs with unequal numbers
     // of them and turns workgroups over for one unit each: int4, 3 or 4 waves instead take, geometric means (worst), with 5
     // k steps 0.80 of the time (1.04), 6 0.87 (1.0), 7 0.91-0.95 (1.05), 8 level (but with four groups per
-    // lane run 0.85); int8 is level.  Two waves per tile, where the wave budget stops at that, are too few for one or two groups per run: four take
-    // 0.93 with 7-8 k steps (int8 0.95), 0.99 with 9-10, 0.95-0.98 with 11-16; with four groups 0.94-1.09.  So is one wave
-    // with 4 k steps (0.92, int8 0.85).
+    // lane run 0.85); int8 is level.  So is one wave with 4 k steps (0.92, int8 0.85).
     if (knobs.wide_waves && !mc && m_batch == 1 && tiles * 8 >= cus * 22 && ksteps <= 16) {
       if (bits == 4 && ksteps >= 5 && split_k == ksteps) {
         if (ksteps < 8 || knobs.generic_groups) split_k = ksteps <= 6 ? 3 : 4;
-      } else if (!knobs.generic_groups && (split_k == 2 ? ksteps >= 7 : split_k == 1 && ksteps == 4)) {
+      } else if (!knobs.generic_groups && split_k == 1 && ksteps == 4) {
         split_k = 4;
       }
     }
+    // Where the wave budget stops at two bf16 waves per tile, four (three with 5 and 6 k steps).  Two do not give a SIMD enough to
+    // choose from, and 2300-2560 tiles of them are on the machine all at once with nothing left to even out its end:
+    // two / four waves 37976x4352 int8 34.3 us / 30.9, 38400x5376 g96 37.4 / 32.7, 38232x8576 g64 at two rows 58.7 / 51.1; over 3300
+    // launches of 1300-8000 tiles 0.80-1.04, mean 0.936.  int8 with
+    // 9 and 10 k steps is level (0.99-1.02) and keeps two, but for single rows with one or two groups per run, which take 0.99.
+    const bool level = bits == 8 && (ksteps == 9 || ksteps == 10) && (m_batch > 1 || knobs.generic_groups);
+    if (knobs.wide_waves && !mc && split_k == 2 && ksteps >= 5 && !level) split_k = 4;
   }
   int tiles_per_wg = pair_tiles ? 2 : 1;
   int workgroup_cap = 0;
