@@ -417,9 +417,10 @@ MGEMV_API int mgemv_query_launch(int n_out, int m_batch, int k, int weight_bits,
 MGEMV_API int mgemv_query_launch_bf16(int n_out, int m_batch, int k, int weight_bits, int group_size, int out[8]);
 /* The same for either element type (MGEMV_ELEMENT_*) and a device of num_compute_units compute
  * units (a partition of an MI355X has 32 per XCD), plus what the plan asks of the hardware:
- * out[8] = bytes of dynamic LDS per workgroup, out[9] = the workgroup size limit the chosen
- * kernel is compiled for, out[10] = prefetch stages (1 or 2), out[11] = launches that serve all
- * activation rows (the VALU kernel takes four rows per launch). */
+ * out[8] = bytes of dynamic LDS per workgroup (the bf16 k-stationary kernel has 256 static ones
+ * besides), out[9] = the workgroup size limit the chosen kernel is compiled for, out[10] = prefetch
+ * stages (1 or 2), out[11] = launches that serve all activation rows (the VALU kernel takes four
+ * rows per launch). */
 MGEMV_API int mgemv_query_launch_for(int n_out, int m_batch, int k, int weight_bits, int group_size, int element,
                                      int num_compute_units, int out[12]);
 
