@@ -363,8 +363,10 @@ inline int two_int8_rows_split(int tiles, int ksteps, int cus) {
 //     3 k steps, walks of 20 and more: k-stationary, four workgroups per compute unit (104496x1536 21.6 / 18.8; the VALU kernel
 //       before), and 4 k steps, walks of 12 and more: two (69824x2048 20.8 / 16.6, 54528x2048 20.5 / 16.0); shorter walks gain and lose;
 //     5-16 k steps, walks of 7 and more: the LDS-staged kernel with workgroups of 4 tiles where the busiest SIMD would
-//       have 1.15 times as many units on the k-stationary one (as in use_k_stationary_bf16): 62688x2560 g96 33.9 / 26.4, 29664x4608
-//       23.5 / 20.2, 91600x3072 32.3 / 29.3; 0.75-0.99 on 16 launches, mean 0.90, and below that line 0.95-1.3 (61312x5120 g96 36.7 / 39.0);
+//       have 1.15 times as many units on the k-stationary one (as in use_k_stationary_bf16): 58536x2560 g64 32.9 / 24.5, 29560x4608
+//       24.8 / 21.8; 0.64-1.02 on 420 launches, mean 0.84.  A lookup per block moves that line, since the LDS-staged kernel does
+//       more of them: 1.25 on walks of 7 and 8, 1.16 on longer ones (1.15 on all of them took 24992x3072 g96 scale only from 13.6 to 14.8,
+//       25152x4608 18.4 / 19.6, 57600x6624 47.2 / 52.3; the launches between the lines took 1.05 times as long);
 //   bf16, 8 k steps, walks of 31 to 40 (two rows: 27 to 48): two, three or four workgroups per compute unit at 2 / 3 / 4 rows.  0.94-0.99 /
 //     0.95-1.014 / 0.96-1.004 of the time on 11, 9 and 8 launches (128256x4096 64.5 / 61.6, 65.0 / 61.5, 64.4 / 62.7); shorter walks gain and lose 3 %.
 void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int cus, bool bf16, bool generic_groups) {
@@ -390,7 +392,8 @@ void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int
   } else if (m_batch == 2 && ksteps <= 16 && walk >= 7) {
     const int tw = lds_staged_tiles_per_wg(tiles, 8, cus);
     const long long here = 4ll * walk * ceil_div(ksteps, 4), there = (long long)ceil_div(ceil_div(tiles, tw), cus) * tw * ksteps;
-    if (tw == 4 && here * 100 >= there * 115) choose(MGEMV_MATRIX_CORE_LDS_STAGED, 0);
+    const int ahead_from = !generic_groups ? 115 : walk <= 8 ? 125 : 116;
+    if (tw == 4 && here * 100 >= there * ahead_from) choose(MGEMV_MATRIX_CORE_LDS_STAGED, 0);
   }
 }
 
