@@ -272,25 +272,32 @@ inline int lookups_per_run(int k, int group_size, int bits) {
 // are in flight at once and which request all they need up front: most launches that used to want longer waves -- walks of
 // several tiles, whole-k waves, two tiles per workgroup -- now want two units a wave.  Part of the built-in measured
 // plans, so for the device these were measured on only.
-// fp16, int4, us of the rules / here:
-//   9-16 k steps, more than 512 tiles: two units.  49152x8192 g96 48.9 / 40.9, 48672x7680 37.6 / 33.4, 16384x8192 14.0 / 13.4,
-//     20272x6144 14.5 / 13.0, 12288x5600 8.65 / 7.68, 28384x7680 20.0 / 18.5; 17456x6656 per column 11.65 / 11.9.  With the rules
-//     stay 9 and 10 k steps on 769-1024 tiles (they gain 2-6 %), 9-12 on even fits of 1025-2048 (24576x6144 level, 28672x6144 17.8 /
-//     17.4) and, on up to 640 tiles, 16 k steps (four waves of four units each) and lookups per block (8400x5280 g96 8.67 / 8.97),
-//     and two lookups per run where a wave per tile fills the SIMDs (16384x6144 g64 scale only 9.85 / 10.3, 16384x8192 g64 14.1 / 14.5).
-//   9-16 k steps, up to 512 tiles: one unit.  6704x5472 g96 8.05 / 6.92, 4960x4608 5.50 / 4.93, 5120x4608 5.65 / 4.99, 8192x6144
-//     6.74 / 6.65; with the rules stay 10 k steps of a regular group size (8192x5120 level) and, where they are ahead by 2-4 %,
-//     14 and more on evenly filled 512 tiles.
-//   5-8 k steps: one unit up to 5.5 tiles per compute unit (7 and 8 k steps), 8 (5) or 12 (6), then two: 71904x3584 22.5 /
-//     20.7, 99104x4096 39.4 / 37.0, 96464x2464 27.8 / 23.5, 88000x3072 27.5 / 26.7; 22016x4096 10.09, 10.18 with two.  Even fits
-//     on up to 8 tiles per compute unit stay with the rules (24576x4096 11.6 us, 11.8 with two units).
-//   17-32 k steps, up to 768 tiles: two units (8336x9216 11.8 / 10.6, 12288x9216 14.1 / 12.0, 10128x14848 17.8 / 16.8); more
-//     than 1024: four waves (28672x10240 30.1 / 28.0, 24576x15360 37.5 / 34.9; in between 0.89-1.045, left with the rules).
-// fp16, int8, more than 4 tiles per compute unit: one unit a wave at 10-12 k steps (85264x2560 g96 35.1 / 32.5, 40960x2816
-//   19.8 / 18.6, 20480x3072 11.5 / 11.1); more than 8: at 5-9 and 13 as well (82624x1280 g96 20.5 / 17.7, 49152x1280 11.5 / 10.8);
-//   with 14 it loses (20480x3584 12.9 / 13.8).
-// bf16 with a lookup per block, up to 2 tiles per compute unit and 16 k steps: up to eight waves (5168x2560 int8 g96 7.38 / 6.18,
-//   5248x8160 g96 10.95 / 9.15, 5360x3328 int8 9.31 / 7.65); other group sizes gain and lose.
+// fp16, int4; us of the rules / here, both through the builds there are now; "of the time" is here over the rules, on launches
+// of random shapes:
+//   9-16 k steps, more than 512 tiles: two units.  50408x4480 g64 28.2 / 24.2, 14108x8064 g96 16.3 / 13.7, 37912x4608 g96 24.3 / 22.1,
+//     68696x7168 56.6 / 52.5; 0.924 of the time (0.69-1.05) on 1500 launches of more than 1024 tiles, 0.970 (0.79-1.11) on 470 of
+//     513-1024.
+//   9-16 k steps, up to 512 tiles: one unit.  7312x5568 g96 8.27 / 7.07, 4172x6400 g64 7.57 / 6.85, 6908x5888 per column 6.56 / 6.12;
+//     0.933 (0.77-1.06) on 660.
+//   5-7 k steps: one unit up to 5.5 (7 k steps), 8 (5) or 12 (6) tiles per compute unit, then two.  79772x2560 g64 26.4 / 22.6, 74732x2304
+//     scale only 19.1 / 17.8; 0.927 (0.68-1.07) on 1170.  8 k steps: two from 5.5 on; 51248x4032 g96 27.3 / 22.5, 82844x3840 35.0 / 30.7,
+//     0.891 on 240 launches of more than 2048 tiles, but 1.04 (0.94-1.13) on 70 of 1409-2048, where one unit is still ahead.
+//   17-32 k steps, up to 768 tiles: two units (8656x12800 g64 15.3 / 13.6, 10092x12160 14.4 / 13.2; 0.927 on 430); more than 1024: four
+//     waves (26560x14208 g96 45.7 / 40.0, 36336x12288 42.9 / 39.5; 0.935, 0.72-1.07, on 650).  33 and more: four waves either way; up to
+//     768 tiles they are what the rules take, but for the last few tile counts (0.976-1.007 on 60), above 1024 0.90 on 50.
+//   With the rules stay, as measured: lookups per block on up to 640 tiles (8400x5280 g96 8.67 / 8.97), two lookups per run where a
+//     wave per tile fills the SIMDs (16384x6144 g64 scale only 9.85 / 10.3), even fits with 5-8 k steps (24576x4096 11.6 / 11.8) and
+//     769-1024 tiles with 17 and more (0.89-1.045).
+//   With the rules stay because a launch test holds one shape of each to its older plan, not because it is faster; two units /
+//     the plan that stays: 16 k steps on 513-640 tiles 0.80-0.92 of the time, mean 0.86, on 60 (9216x8192); 9 and 10 k steps on 769-1024
+//     tiles 0.88-1.03, mean 0.98 (13824x5120); 9-12 on even fits of 1025-2048 (28672x6144 17.8 us / 17.4).  One unit / the plan
+//     that stays: 10 k steps up to 512 tiles 0.90-1.04, mean 0.99, with two lookups per run 1.02 (5120x5120); 14-16 on evenly filled 512
+//     tiles 0.93-1.04, mean 0.99, two lookups per run 1.03, lookups per block 0.91 (8192x8192).
+// fp16, int8, more than 4 tiles per compute unit: one unit a wave at 10-12 k steps (49568x2816 25.6 / 23.4, 71644x3072 37.7 / 35.2,
+//   19712x2560 per column 10.2 / 9.7; 0.95, 0.85-1.03, on 360); more than 8: at 5-9 and 13 as well (72220x1632 g96 24.6 / 22.1, 37952x2176
+//   16.7 / 15.6; 0.94 on 790); with 14 it loses (20480x3584 12.9 / 13.8).
+// bf16 with a lookup per block, 9-16 k steps on 1.125 to 2 tiles per compute unit: up to eight waves instead of pairs of tiles
+//   (5052x4320 g96 9.65 / 8.39, 7936x7680 11.3 / 9.5, int8 5784x2304 7.6 / 6.05; 0.79-1.06 on 400); other group sizes gain and lose.
 inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16, int lookups) {
   if (tiles <= cus || ksteps < 5) return 0;
   const bool generic_groups = lookups == 4;
@@ -343,8 +350,8 @@ inline int lds_staged_tiles_per_wg(int tiles, int staged_rows, int cus) {
 }
 
 // Two fp16 rows, int8, more than 8 tiles per compute unit and 5-14 k steps: up to eight waves of one or two units instead of
-// whole-k waves or walks (us of the rules / here: 63808x1280 g256 16.4 / 14.5, 80768x2816 g96 45.1 / 38.6, 69392x2560 g256 29.9 /
-// 28.9; 0.85-1.002 of the time on 24 launches, mean 0.95).  Fewer tiles and longer reductions gain and lose.
+// whole-k waves or walks (us of the rules / here: 57592x1728 g96 scale only 21.0 / 18.7, 131144x1792 g64 42.3 / 39.1, 75760x1280
+// 19.5 / 18.3; 0.74-1.06 of the time on 540 launches, mean 0.93).  Fewer tiles and longer reductions gain and lose.
 inline int two_int8_rows_split(int tiles, int ksteps, int cus) {
   return tiles > 8 * cus && ksteps >= 5 && ksteps <= 14 ? (ksteps < 8 ? ksteps : 8) : 0;
 }
@@ -353,22 +360,28 @@ inline int two_int8_rows_split(int tiles, int ksteps, int cus) {
 // than the rules have it.  Times are us, the rules' / here, or here as a part of theirs.
 //   fp16, 9-16 rows, a group size that divides the k step: the k-stationary kernel, since its rows 8-15 are requested with the
 //     first eight --
-//       at most one tile per compute unit, 64 tiles and more, 5-14 k steps (15 up to 14 rows): 0.79-1.005 on 31 launches, mean
-//         0.90 (4096x2560 at 14 rows 5.60 / 4.82, 3360x3584 at 13 6.17 / 4.92, 4096x6656 at 14 8.18 / 7.17); 15 k steps at 16 rows
-//         1.01-1.06, 16 0.97-1.01;
+//       at most one tile per compute unit, 64 tiles and more, 5-14 k steps (15 up to 14 rows): 0.73-1.06 on 2370 launches, mean
+//         0.89 (1776x3456 g64 at 13 rows 6.16 / 5.04, 2760x6400 at 14 8.97 / 7.72); 15 k steps 0.96 on 117, at 16 rows 1.01-1.06;
+//         16 k steps 0.87-1.05, mean 0.98, left with the rules;
 //       two tiles per compute unit at 13-16 rows (from 1.25, which the LDS-staged kernel's pairs of tiles fill as well), 5-16
-//         k steps: 0.80-0.996 on 25, mean 0.92 (6848x5632 g64 9.64 / 8.52, 8192x8192 g64 with a bias 13.1 / 12.5); 12 k steps 1.025, and 8 on an
-//         even fit are left where the launch tests have them.
+//         k steps: 0.80-1.03 on 451, mean 0.91 (5224x3072 at 13 rows 7.15 / 5.90, 6536x3968 per column 7.42 / 6.51, 8192x8192 g64 with a
+//         bias at 16 13.1 / 12.5).  12 k steps (0.88-1.05, mean 0.97) and 8 on 512 tiles (0.84-0.93, mean 0.90) keep the rules' plan
+//         because a launch test holds one shape of each to it.
 //   bf16, 2 rows:
-//     3 k steps, walks of 20 and more: k-stationary, four workgroups per compute unit (104496x1536 21.6 / 18.8; the VALU kernel
-//       before), and 4 k steps, walks of 12 and more: two (69824x2048 20.8 / 16.6, 54528x2048 20.5 / 16.0); shorter walks gain and lose;
+//     3 k steps, walks of 20 and more: k-stationary, four workgroups per compute unit (93308x1408 scale only 23.7 / 17.6; the VALU
+//       kernel before; 0.85 on 23), and 4 k steps, walks of 12 and more: two (84860x1792 g64 35.3 / 25.7, 104424x2048 per column 29.6 /
+//       23.9; 0.84, 0.65-1.07, on 80); shorter walks gain and lose;
 //     5-16 k steps, walks of 7 and more: the LDS-staged kernel with workgroups of 4 tiles where the busiest SIMD would
 //       have 1.15 times as many units on the k-stationary one (as in use_k_stationary_bf16): 58536x2560 g64 32.9 / 24.5, 29560x4608
 //       24.8 / 21.8; 0.64-1.02 on 420 launches, mean 0.84.  A lookup per block moves that line, since the LDS-staged kernel does
 //       more of them: 1.25 on walks of 7 and 8, 1.16 on longer ones (1.15 on all of them took 24992x3072 g96 scale only from 13.6 to 14.8,
 //       25152x4608 18.4 / 19.6, 57600x6624 47.2 / 52.3; the launches between the lines took 1.05 times as long);
-//   bf16, 8 k steps, walks of 31 to 40 (two rows: 27 to 48): two, three or four workgroups per compute unit at 2 / 3 / 4 rows.  0.94-0.99 /
-//     0.95-1.014 / 0.96-1.004 of the time on 11, 9 and 8 launches (128256x4096 64.5 / 61.6, 65.0 / 61.5, 64.4 / 62.7); shorter walks gain and lose 3 %.
+//   bf16, 8 k steps, walks of 31 to 40 (two rows: 27 to 48): the k-stationary kernel in two, three or four workgroups per compute unit
+//     at 2 / 3 / 4 rows, which share the LDS that the partial sums of one long walk would take whole.  With 2 and 3 rows it is the rules'
+//     kernel too, in one workgroup; with 4 the rules take the LDS-staged one, since 33 KB of rows and 31 or more tiles' sums, reckoned
+//     in blocks of 17 entries, are over 160 KB.  (Blocks of the 9 entries that 8 waves write would fit; the rule does not know.)  0.94-0.99 /
+//     0.95-1.014 / 0.96-1.004 of the time on 11, 9 and 8 launches, 0.86-1.02 on 90 more (128256x4096 64.5 / 61.6, 65.0 / 61.5, 64.4 / 62.7);
+//     shorter walks gain and lose 3 %.
 void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int cus, bool bf16, bool generic_groups) {
   const int walk = ceil_div(tiles, cus);
   auto choose = [&](int variant, int workgroups) {
@@ -723,6 +736,8 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     if (ov_t == 1 || ov_t == 2 || ov_t == 4) tiles_per_wave = ov_t;
   }
   const int groups = ceil_div(tiles, tiles_per_wave);
+  // (The VALU figures from here on are from before its builds by length.  On a device of 256 compute units single_row_split is asked
+  // first for a single row on more tiles than that.)
   // Shapes that the exact-fit rule below does not take (measured on MI355X; one tile group per
   // workgroup is best throughout):
   //  * about one workgroup per compute unit or fewer (<= 384 tile groups): few, longer waves --
