@@ -174,6 +174,7 @@ std::atomic<int> g_matrix_core_variant{MGEMV_MATRIX_CORE_AUTO};
 // What steers plan_launch besides the shape: zeros mean "built-in rule".
 struct PlanKnobs {
   int split_k = 0, tiles_per_wg = 0, tiles_per_wave = 0, workgroups = 0;
+  int parts = 0;            // part-tile matrix-core kernel: workgroups per tile
   int matrix_core_min_batch = 0;
   int matrix_core_variant = MGEMV_MATRIX_CORE_AUTO;
   bool wide_waves = false;  // the kernel is one of those compiled for at most 8 waves per workgroup
@@ -410,6 +411,41 @@ void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int
   }
 }
 
+// Two and more rows: workgroups per tile on the part-tile matrix-core kernel (launch_mfma_parts.hip); 0: not on that kernel.
+// Part of the built-in measured plans, as the ranges above.  Over 2500 launches of random shapes whose plan it changes
+// (2 tiles and more, up to 32768 k) 0.76 of the time of what was there (0.32-1.035, 3 of them above 1.02).  Geometric means:
+//   at most a quarter as many tiles as compute units, 2-4 rows: four parts -- fp16 0.73 at 2 rows, 0.68 at 3 and 4, bf16 0.61 and
+//     0.59, int8 0.75-0.84 and 0.64-0.75 (964x12416 3 rows 8.7 us / 5.7; 616x13368 per column bf16 2 rows 12.3 / 5.2);
+//   at most half as many: two parts -- 2-4 rows fp16 0.84 and 0.74, bf16 0.75 and 0.66, 5-8 rows 0.82 and 0.76, int8 0.75-0.86
+//     (2048x11008 4 rows 8.4 / 6.1; 1924x28288 bf16 8 rows 20.9 / 15.1); four parts there, two workgroups per compute unit, 1.0-1.2;
+//   at most as many: one part, four waves with a stage of their own, where the reduction is long, or as rows and bits say: 0.91-0.96
+//     from 17 k steps (4096x14336 bf16 8 rows 12.8 / 11.9), 9-16 rows on few tiles 0.80-0.90, int8 0.83-0.91.  Two parts 1.1-1.5;
+//   more, int4 from 17 k steps: bf16 at 2-4 rows up to 1.5 tiles per compute unit two parts 0.85, one part where the LDS-staged kernel's
+//     pairs of tiles fill the machine badly, 2 to 3 tiles per compute unit 0.87 (bf16 4 to 5 as well, 0.92).  Elsewhere 0.95-1.4.
+// Fewer than 5 k steps gain less, and launch tests hold such shapes to their older plans, as they hold: 3 and 4 rows of int8 on more than
+// a quarter as many tiles up to 17 k steps (0.85-0.91 here), bf16 on exactly half as many up to 8 (0.80-0.88) and two bf16 rows on
+// 112-127 (16 k steps) and 128 tiles.  9-16 fp16 rows of up to 8 k steps on few tiles (0.94) keep the rules' plan for the same reason.
+inline int part_tiles(int m_batch, int tiles, int ksteps, int bits, bool bf16, int cus) {
+  if (m_batch < 2 || tiles < 2 || ksteps < (m_batch == 2 && bits == 8 ? 8 : 5)) return 0;
+  if (tiles * 4 <= cus && m_batch <= 4) return 4;
+  if (tiles * 2 <= cus && m_batch <= 8) {
+    if (bits == 8 && m_batch <= 4 && ksteps <= 17) return 0;
+    if (bf16 && m_batch == 2 && tiles * (ksteps > 16 ? 2 : 16) >= cus * (ksteps > 16 ? 1 : 7)) return 0;
+    if (bf16 && tiles * 2 == cus && ksteps <= 8) return 0;
+    return 2;
+  }
+  if (tiles <= cus) {
+    if (m_batch == 2 || (bits == 8 && m_batch <= 4)) return 0;
+    if (ksteps > 16) return 1;
+    if (bits == 8) return !bf16 || tiles * 2 < cus ? 1 : 0;
+    return m_batch >= 9 && (bf16 ? tiles * 2 < cus : tiles * 4 < cus && ksteps > 8) ? 1 : 0;
+  }
+  if (bits == 8 || ksteps <= 16) return 0;
+  if (bf16 && m_batch <= 4 && tiles * 2 <= 3 * cus) return 2;
+  if (m_batch >= 3 && m_batch <= (bf16 ? 8 : 4) && tiles > 2 * cus && tiles <= 3 * cus) return 1;
+  return bf16 && m_batch >= 3 && m_batch <= 8 && tiles > 4 * cus && tiles <= 5 * cus ? 1 : 0;
+}
+
 // Process-wide overrides win over the tables (they are what a tuner sweeps); then the caller's
 // entry for exactly this group size, then its entry for any group size, then the built-in table and
 // the measured ranges, then the built-in rules.
@@ -447,7 +483,12 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
         kn.split_k = split;
         kn.tiles_per_wg = 1;
       }
-    } else if (bits == 4) {
+    }
+    if (const int parts = kn.split_k != 0 ? 0 : part_tiles(m_batch, tiles, ksteps, bits, bf16, num_cus)) {
+      kn.matrix_core_min_batch = 1;
+      kn.matrix_core_variant = MGEMV_MATRIX_CORE_LDS_STAGED;
+      kn.parts = parts;
+    } else if (m_batch > 1 && bits == 4) {
       set_multi_row_ranges(kn, m_batch, tiles, ksteps, num_cus, bf16, lookups == 4);
     }
   }
@@ -696,6 +737,25 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
       const bool four = lp.staged_rows == 16 ? ceil_div(tiles, 2) * 4 > cus * 11 : wgs4 * 4 >= ceil_div(wgs4, cus) * cus * 3;
       lp.tiles_per_wg = four ? 4 : 2;
     }
+    // Parts of tiles (measured ranges only): the waves of a workgroup share the units of `parts` k steps.
+    if (knobs.parts > 0 && knobs.parts * m_batch <= kTileRows) {
+      lp.tiles_per_wg = lp.tiles_per_wave = lp.tiles_in_sequence = 1;
+      lp.parts = knobs.parts;
+      lp.staged_rows = lp.parts < 4 && lp.parts * m_batch <= 8 ? 8 : 16;
+      lp.workgroups = tiles * lp.parts;
+      // Up to 8 units a wave each (0.90-0.96 of the time of half as many waves of two); more of them four waves, one per SIMD:
+      // what such a launch waits for is a compute unit's path to memory, not latency, and 8 take 1.0-1.08 times as long
+      // (bf16 on up to 64 tiles 0.97-1.0).
+      const int units = ceil_div(ksteps, lp.parts);
+      const int waves = ov_sk > 0 ? (ov_sk < kMaxWavesPerMfmaWorkgroup ? ov_sk : kMaxWavesPerMfmaWorkgroup) : units <= kMaxWavesPerMfmaWorkgroup ? units : 4;
+      const int units_per_wave = ceil_div(units, waves < units ? waves : units);
+      lp.steps_per_wave = units_per_wave * lp.parts;
+      lp.split_k = ceil_div(units, units_per_wave);
+      lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
+      lp.threads = kWave * lp.split_k;
+      lp.stages = 2;
+      return lp;
+    }
     // the kernel exists for 2, 4, 8 or 16 staged rows per wave of a k range
     if (ov_tw > 0 && ov_tw <= 8 && lp.staged_rows % ov_tw == 0 && lp.staged_rows / ov_tw >= 2) lp.tiles_per_wg = ov_tw;
     lp.workgroups = ceil_div(tiles, lp.tiles_per_wg);
@@ -923,8 +983,9 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
     r.max_threads = kWave * kMaxWavesPerMfmaWorkgroup;
     if (lp.staged_rows != 0) {
       const int row_stride = step_k(bits) * 2 + 16;
-      r.lds_bytes = (size_t)lp.split_k * 2 * lp.staged_rows * row_stride +
-                    (lp.split_k > 1 ? (size_t)lp.tiles_per_wg * lp.split_k * kWave * 4 * sizeof(float) : 0);
+      // (a wave of the part-tile kernel has one stage, its own)
+      r.lds_bytes = (size_t)lp.split_k * (lp.parts != 0 ? 1 : 2) * lp.staged_rows * row_stride +
+                    (lp.split_k > 1 || lp.parts > 1 ? (size_t)lp.tiles_per_wg * lp.split_k * kWave * 4 * sizeof(float) : 0);
     } else {
       r.lds_bytes = lp.split_k == 1 ? 0 : (size_t)lp.tiles_per_wg * lp.split_k * lp.tiles_per_wave * kWave * 4 * sizeof(float);
     }
@@ -1077,6 +1138,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
         return MGEMV_ERR_QUANT_OP;
       return launch_mfma_lds_probe(g, gpr, rounds, probe) == hipSuccess ? MGEMV_OK : MGEMV_ERR_LAUNCH;
     }
+    if (g.plan.parts != 0) return launch_mfma_parts(g, weight_bits, quant_op, gpr, act) == hipSuccess ? MGEMV_OK : MGEMV_ERR_LAUNCH;
     if (g.plan.staged_rows != 0) {
       return launch_mfma_lds(g, weight_bits, quant_op, gpr, g.plan.staged_rows / g.plan.tiles_per_wg, act) == hipSuccess
                  ? MGEMV_OK
@@ -1531,7 +1593,8 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
   const int seq_base = tiles / sequences, seq_rem = tiles % sequences;  // as gemv_any passes them
   const bool multi = (!lp.matrix_core || lp.k_stationary) && lp.tiles_in_sequence > 1;
   const int rows = m_batch < kMaxValuBatch ? m_batch : kMaxValuBatch;
-  std::vector<int> covered((size_t)tiles, 0);
+  const int parts = lp.parts > 0 ? lp.parts : 1;
+  std::vector<int> covered((size_t)tiles * parts, 0);  // k steps of each tile, or part of one
   std::vector<char> block_seen((size_t)lp.workgroups, 0);
   int64_t idle_waves = 0, busy_waves = 0, max_span = 0, max_lds = 0, bad_ranges = 0, max_units = 0;
   for (int block = 0; block < grid; ++block) {
@@ -1540,7 +1603,9 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
     if (block_seen[(size_t)wg]++) ++bad_ranges;   // two blocks with one logical id
     for (int ty = 0; ty < lp.tiles_per_wg; ++ty) {
       for (int kw = 0; kw < lp.split_k; ++kw) {
-        const WaveWork w = lp.matrix_core && !lp.k_stationary
+        const PartWork part = part_wave_work(parts, wg, kw, lp.steps_per_wave, ksteps);
+        const WaveWork w = lp.parts != 0 ? WaveWork{part.tile, part.tile < tiles ? 1 : 0, part.ks_begin, part.units}
+                           : lp.matrix_core && !lp.k_stationary
                                ? (lp.staged_rows != 0
                                       ? staged_wave_work(wg, ty, kw, lp.tiles_per_wg, tiles, lp.steps_per_wave, ksteps)
                                       : mfma_wave_work(lp.tiles_per_wave, wg, ty, kw, lp.tiles_per_wg, tiles,
@@ -1548,6 +1613,7 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
                                : valu_wave_work(multi, wg, ty, kw, lp.tiles_per_wg, seq_base, seq_rem, tiles,
                                                 lp.steps_per_wave, ksteps);
         if (w.units <= 0) ++bad_ranges;  // every kernel relies on each wave along k having units
+        if (lp.steps_per_wave % parts != 0 || parts * m_batch > kTileRows) ++bad_ranges;  // whole units, a column for every row and k step
         if (w.tiles <= 0 || w.units <= 0) {
           ++idle_waves;
           continue;
@@ -1557,7 +1623,7 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
           ++bad_ranges;
           continue;
         }
-        for (int t = 0; t < w.tiles; ++t) covered[(size_t)(w.tile_begin + t)] += w.units;
+        for (int t = 0; t < w.tiles; ++t) covered[(size_t)(w.tile_begin + t) * parts + (lp.parts != 0 ? part.part : 0)] += w.units;
         // the bytes one weight descriptor spans: tiles are ksteps units apart
         const int64_t span = (int64_t)(w.tiles - 1) * ksteps * kUnitBytes + (int64_t)w.units * kUnitBytes;
         max_span = span > max_span ? span : max_span;
@@ -1574,7 +1640,7 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
     }
   }
   int64_t wrong = 0;
-  for (int t = 0; t < tiles; ++t) wrong += covered[(size_t)t] != ksteps;
+  for (const int steps : covered) wrong += steps != ksteps;
   out[0] = wrong;                 // tiles whose k steps are not covered exactly once
   out[1] = bad_ranges;            // waves with a range outside the problem or without units, duplicate workgroup ids
   out[2] = max_span;              // most bytes behind one weight descriptor

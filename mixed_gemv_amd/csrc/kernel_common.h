@@ -137,6 +137,16 @@ __host__ __device__ __forceinline__ WaveWork staged_wave_work(int wg, int ty, in
   return w;
 }
 
+// Part-tile matrix-core kernel: a workgroup takes 16 / parts rows of one tile, a wave a range of whole units of `parts` k steps.
+struct PartWork {
+  int tile, part, ks_begin, units;  // units: k steps, the last unit of the reduction may be short
+};
+__host__ __device__ __forceinline__ PartWork part_wave_work(int parts, int wg, int kw, int steps_per_wave, int ksteps) {
+  WaveWork w;
+  wave_k_range(w, kw, steps_per_wave, ksteps);
+  return PartWork{wg / parts, wg % parts, w.ks_begin, w.units};
+}
+
 __device__ __forceinline__ int logical_workgroup(const Problem& p) {
   return logical_workgroup_of((int)blockIdx.x, p.wgs_per_xcd);
 }
@@ -270,7 +280,8 @@ struct LaunchPlan {
   int split_k, tiles_per_wg, steps_per_wave, workgroups, wgs_per_xcd, threads;
   int tiles_per_wave;  // 1 on the VALU path; 1, 2 or 4 on the matrix-core path
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
-  int staged_rows;        // LDS-staged matrix-core kernel: 8 or 16 activation rows per stage; 0 = other kernels
+  int staged_rows;        // LDS-staged and part-tile matrix-core kernels: 8 or 16 activation rows per stage; 0 = other kernels
+  int parts;              // part-tile matrix-core kernel: workgroups per tile (1, 2 or 4); 0 = other kernels
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
   bool k_stationary;      // the matrix-core kernel whose waves keep one k step each while the workgroup walks tiles_in_sequence tiles
@@ -323,6 +334,7 @@ hipError_t launch_gemv_f16(const GemvLaunch& g, int bits, int qop, int mb, int g
 hipError_t launch_gemv_bf16(const GemvLaunch& g, int bits, int qop, int mb, int gpr);
 hipError_t launch_mfma(const GemvLaunch& g, int bits, int qop, int gpr);
 hipError_t launch_mfma_lds(const GemvLaunch& g, int bits, int qop, int gpr, int rounds, int act);
+hipError_t launch_mfma_parts(const GemvLaunch& g, int bits, int qop, int gpr, int act);
 hipError_t launch_mfma_kstat(const GemvLaunch& g, int bits, int qop, int gpr, int act);
 // ... and of the k-stationary matrix-core kernel (kProbeLoadsOnly / kProbeComputeOnly), where they exist.
 bool mfma_kstat_probe_exists(int bits, int qop, int gpr, int act);

@@ -199,19 +199,16 @@ __device__ __forceinline__ void compute_unit_mfma(f32x4& acc, const MfmaWeights<
   compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2, short4);
 }
 
-// Weights, scales and zeros of unit `unit` of the wave's k range through descriptors: everything
-// unit-dependent sits in the bounds-checked VGPR offset, so a prefetch past the range reads zeros.
+// Weights, scales and zeros of a unit through descriptors: everything unit-dependent sits in the bounds-checked VGPR
+// offset, so a prefetch past the range reads zeros.  k_run: first reduction index of the lane's run; row: its weight row.
 template <int BITS, int QOP, int GROUPS_PER_RUN>
-__device__ __forceinline__ void load_weights_lds_mfma(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p,
-                                                      __amdgpu_buffer_rsrc_t w_rsrc, const ScaleTables& tables, int unit,
-                                                      int kstep, int lane, int row) {
+__device__ __forceinline__ void load_weights_at(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p, __amdgpu_buffer_rsrc_t w_rsrc,
+                                                const ScaleTables& tables, int voffset, int k_run, int row) {
   using G = Geometry<BITS>;
-  const int voffset = unit * kUnitBytes + lane * kChunkBytes;
 #pragma unroll
   for (int i = 0; i < kBlocksPerUnit; ++i)
     f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, voffset + i * kBlockBytes, 0, kCacheStream);
   if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) {
-    const int k_run = kstep * G::kStepK + (lane / kTileRows) * G::kRunK;
 #pragma unroll
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
       const int grp = group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
@@ -220,6 +217,15 @@ __device__ __forceinline__ void load_weights_lds_mfma(MfmaWeights<BITS, GROUPS_P
       if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) f.z[gi] = load_b16_low(tables.zero, off);
     }
   }
+}
+// ... of unit `unit` of the wave's k range, a whole tile's rows.
+template <int BITS, int QOP, int GROUPS_PER_RUN>
+__device__ __forceinline__ void load_weights_lds_mfma(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p,
+                                                      __amdgpu_buffer_rsrc_t w_rsrc, const ScaleTables& tables, int unit,
+                                                      int kstep, int lane, int row) {
+  using G = Geometry<BITS>;
+  load_weights_at<BITS, QOP, GROUPS_PER_RUN>(f, p, w_rsrc, tables, unit * kUnitBytes + lane * kChunkBytes,
+                                             kstep * G::kStepK + (lane / kTileRows) * G::kRunK, row);
 }
 
 // Activation rows on their way through LDS: a wave fetches whole rows of a k step (64 lanes x 16 or 8 bytes,
