@@ -175,6 +175,7 @@ std::atomic<int> g_matrix_core_variant{MGEMV_MATRIX_CORE_AUTO};
 struct PlanKnobs {
   int split_k = 0, tiles_per_wg = 0, tiles_per_wave = 0, workgroups = 0;
   int parts = 0;            // part-tile matrix-core kernel: workgroups per tile
+  bool split_left_over = false;  // k-stationary kernel: tiles that do not divide over the workgroups go to two or four of them
   int matrix_core_min_batch = 0;
   int matrix_core_variant = MGEMV_MATRIX_CORE_AUTO;
   bool wide_waves = false;  // the kernel is one of those compiled for at most 8 waves per workgroup
@@ -476,6 +477,7 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
     const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
     const bool bf16 = act == kActBf16;
     const int lookups = lookups_per_run(k, group_size, bits);
+    kn.split_left_over = true;
     if (m_batch == 1 || (m_batch == 2 && bits == 8 && !bf16)) {
       const int split = m_batch == 1 ? single_row_split(tiles, ksteps, bits, num_cus, bf16, lookups)
                                      : two_int8_rows_split(tiles, ksteps, num_cus);
@@ -664,8 +666,42 @@ inline bool use_k_stationary_bf16(int m_batch, int tiles, int ksteps, int bits, 
 }
 
 // LDS stages of the k-stationary kernel's waves: 8 rows each to turn the operand round in (fp16), or the rows that stay (bf16).
-inline size_t kstat_stage_bytes(int waves, int bits, int m_batch, bool bf16) {
-  return (size_t)waves * (bf16 ? m_batch : 8) * (step_k(bits) * 2 + 16);
+// (With left-over tiles in parts the rows stay in fp16 as well.)
+inline size_t kstat_stage_bytes(int waves, int bits, int m_batch, bool bf16, int parts = 0) {
+  return (size_t)waves * (bf16 || parts != 0 ? m_batch : 8) * (step_k(bits) * 2 + 16);
+}
+
+// Workgroups per left-over tile of a k-stationary launch; 0: walks of whole tiles, some one longer than the others.  313 tiles
+// on 256 compute units are walks of two for 57 of them, and the launch takes as long as two tiles everywhere; with four parts to
+// a left-over tile each compute unit has a quarter more than its first.  What a launch has to gain is units of its busiest SIMD (a
+// wave per k step, dealt out to four SIMDs in turn); what it pays is one barrier at its start and a unit in code nobody has
+// fetched yet, 0.4-0.5 us, so one unit saved is not enough but with 8 bf16 k steps, and fp16, whose units are shorter, pays less
+// often.  Part of the built-in measured plans.  Of the time of whole tiles, same kernel, 1300 launches of random shapes:
+//   bf16 walks of 1 / 2 / 3: four parts 0.93 / 0.92 / 0.95 (9 k steps 0.87; 5004x5280 g96 at 3 rows 9.7 us / 8.8, 9104x5632 at 3 rows
+//     12.5 / 11.5), two parts 0.97 / 0.93 / 0.96 (14-16 k steps on other walks than 2: 0.99-1.01, left out);
+//   fp16: four parts 0.93-0.96 (4608x8192 at 4 rows 9.4 / 8.6; 11-14 k steps 0.98-1.02, left out), two parts on walks of 2 and 3
+//     0.94 / 0.97 (9104x8192 at 4 rows 13.1 / 11.2), on walks of 1 1.0.
+// Longer walks and one unit saved: 0.98-1.1.  int8, whose rows are half as long, 1.03-1.15; four lookups per run in fp16 have
+// no registers for it.
+inline int left_over_parts(int m_batch, int tiles, int ksteps, int bits, int cus, bool bf16, bool generic_groups) {
+  const int walk = tiles / cus, left_over = tiles % cus;
+  if (bits != 4 || walk < 1 || walk > 3 || left_over == 0 || ksteps < 5 || (!bf16 && generic_groups)) return 0;
+  const int parts = m_batch <= 4 && left_over * 4 <= cus ? 4 : m_batch <= 8 && left_over * 2 <= cus ? 2 : 0;
+  if (parts == 0) return 0;
+  // units of the busiest SIMD: now, and with a part's units dealt out as kstat_tail_unit has it
+  int most = 0;
+  for (int simd = 0; simd < 4; ++simd) {
+    int units = 0;
+    for (int kw = simd; kw < ksteps; kw += 4) units += walk + (kstat_tail_unit(kw, ksteps) * parts < ksteps ? 1 : 0);
+    most = units > most ? units : most;
+  }
+  const int saved = (walk + 1) * ceil_div(ksteps, 4) - most;
+  if (bf16) {
+    if (ksteps == 8) return parts;
+    return saved >= 2 && (walk < 3 || ksteps != 12) && (parts == 4 || ksteps <= 13 || walk == 2) ? parts : 0;
+  }
+  if (saved < 2) return 0;
+  return parts == 4 ? (ksteps <= 10 || ksteps >= 15 ? parts : 0) : walk >= 2 ? parts : 0;
 }
 
 LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs& knobs) {
@@ -707,6 +743,12 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     lp.tiles_in_sequence = walk();
     lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
     lp.threads = kWave * lp.split_k;
+    if (knobs.split_left_over && lp.workgroups == cus) {
+      const int parts = left_over_parts(m_batch, tiles, ksteps, bits, cus, knobs.wide_waves, knobs.generic_groups);
+      if (parts != 0 && (long long)kstat_stage_bytes(ksteps, bits, m_batch, true, parts) + walk() * park_bytes <=
+                            kMaxKStationaryBf16Lds - kKStationaryStagedBytes)
+        lp.parts = parts;
+    }
     return lp;
   }
   // The LDS-staged kernel serves every matrix-core launch of two or more tiles.  (While its loop
@@ -974,9 +1016,9 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
   r.launches = 1;
   if (lp.matrix_core && lp.k_stationary) {
     r.max_threads = kWave * kMaxWavesPerWorkgroup;
-    const size_t stage = kstat_stage_bytes(lp.split_k, bits, m_batch, act == kActBf16), park = (size_t)lp.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16;
+    const size_t stage = kstat_stage_bytes(lp.split_k, bits, m_batch, act == kActBf16, lp.parts), park = (size_t)lp.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16;
     // both when they fit (then no barrier stands between a wave's operand and its walk), else the larger of the two
-    r.lds_bytes = act == kActBf16 || stage + park <= (size_t)kMaxKStationaryLds ? stage + park : stage > park ? stage : park;
+    r.lds_bytes = act == kActBf16 || lp.parts != 0 || stage + park <= (size_t)kMaxKStationaryLds ? stage + park : stage > park ? stage : park;
     return r;
   }
   if (lp.matrix_core) {
@@ -1102,7 +1144,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   {
     const int sequences = g.plan.workgroups * g.plan.tiles_per_wg;
     g.tail.seq_base = num_tiles(n_out) / sequences;
-    g.tail.seq_rem = num_tiles(n_out) % sequences;
+    g.tail.seq_rem = g.plan.k_stationary && g.plan.parts != 0 ? 0 : num_tiles(n_out) % sequences;  // the rest in parts
   }
   g.tail.stride_weights = stride_weights;
   g.tail.stride_x = stride_x;
@@ -1122,7 +1164,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
     g.tail.m_batch = m_batch;
     g.lds = launch_resources(g.plan, weight_bits, m_batch, act).lds_bytes;
     if (g.plan.k_stationary) {
-      const size_t stage = kstat_stage_bytes(g.plan.split_k, weight_bits, m_batch, act == kActBf16);
+      const size_t stage = kstat_stage_bytes(g.plan.split_k, weight_bits, m_batch, act == kActBf16, g.plan.parts);
       if (g.lds > stage && g.lds - stage >= (size_t)g.plan.tiles_in_sequence * kKSlices * m_batch * kKStationaryParkSlots * 16)
         g.tail.flags |= kParkBehindStage;
       if (probe != kProbeNone) {
@@ -1590,7 +1632,8 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
   const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, weight_bits);
   const int grid = lp.wgs_per_xcd * kNumXcd;
   const int sequences = lp.workgroups * lp.tiles_per_wg;
-  const int seq_base = tiles / sequences, seq_rem = tiles % sequences;  // as gemv_any passes them
+  const bool left_over_parts = lp.k_stationary && lp.parts != 0;
+  const int seq_base = tiles / sequences, seq_rem = left_over_parts ? 0 : tiles % sequences;  // as gemv_any passes them
   const bool multi = (!lp.matrix_core || lp.k_stationary) && lp.tiles_in_sequence > 1;
   const int rows = m_batch < kMaxValuBatch ? m_batch : kMaxValuBatch;
   const int parts = lp.parts > 0 ? lp.parts : 1;
@@ -1604,7 +1647,7 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
     for (int ty = 0; ty < lp.tiles_per_wg; ++ty) {
       for (int kw = 0; kw < lp.split_k; ++kw) {
         const PartWork part = part_wave_work(parts, wg, kw, lp.steps_per_wave, ksteps);
-        const WaveWork w = lp.parts != 0 ? WaveWork{part.tile, part.tile < tiles ? 1 : 0, part.ks_begin, part.units}
+        const WaveWork w = lp.parts != 0 && !lp.k_stationary ? WaveWork{part.tile, part.tile < tiles ? 1 : 0, part.ks_begin, part.units}
                            : lp.matrix_core && !lp.k_stationary
                                ? (lp.staged_rows != 0
                                       ? staged_wave_work(wg, ty, kw, lp.tiles_per_wg, tiles, lp.steps_per_wave, ksteps)
@@ -1613,7 +1656,13 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
                                : valu_wave_work(multi, wg, ty, kw, lp.tiles_per_wg, seq_base, seq_rem, tiles,
                                                 lp.steps_per_wave, ksteps);
         if (w.units <= 0) ++bad_ranges;  // every kernel relies on each wave along k having units
-        if (lp.steps_per_wave % parts != 0 || parts * m_batch > kTileRows) ++bad_ranges;  // whole units, a column for every row and k step
+        // whole units, a column for every row and k step
+        if (parts * m_batch > kTileRows || (!lp.k_stationary && lp.steps_per_wave % parts != 0)) ++bad_ranges;
+        if (left_over_parts) {  // the wave's unit of its workgroup's part of a left-over tile
+          const int tile = seq_base * lp.workgroups + wg / parts, unit = kstat_tail_unit(kw, lp.split_k);
+          if (tile < tiles && unit * parts < ksteps)
+            covered[(size_t)tile * parts + wg % parts] += ksteps - unit * parts < parts ? ksteps - unit * parts : parts;
+        }
         if (w.tiles <= 0 || w.units <= 0) {
           ++idle_waves;
           continue;
@@ -1623,7 +1672,9 @@ int mgemv_plan_coverage(int n_out, int m_batch, int k, int weight_bits, int grou
           ++bad_ranges;
           continue;
         }
-        for (int t = 0; t < w.tiles; ++t) covered[(size_t)(w.tile_begin + t) * parts + (lp.parts != 0 ? part.part : 0)] += w.units;
+        for (int t = 0; t < w.tiles; ++t)
+          for (int q = 0; q < parts; ++q)
+            if (lp.k_stationary || q == part.part || lp.parts == 0) covered[(size_t)(w.tile_begin + t) * parts + q] += w.units;
         // the bytes one weight descriptor spans: tiles are ksteps units apart
         const int64_t span = (int64_t)(w.tiles - 1) * ksteps * kUnitBytes + (int64_t)w.units * kUnitBytes;
         max_span = span > max_span ? span : max_span;

@@ -22,6 +22,7 @@ constexpr int kKStationaryParkSlots = kMaxWavesPerWorkgroup + 1;  // k-stationar
 constexpr int kMaxKStationaryLds = 128 * 1024;  // most LDS the k-stationary matrix-core kernel parks partial sums in
 constexpr int kKStationaryZeroBytes = 256;  // ... with bf16 operands: zeros, a k run of the operand of a batch row that does not exist
 constexpr int kMaxKStationaryBf16Lds = 160 * 1024 - kKStationaryZeroBytes;  // ... most LDS its activation rows and partial sums take together
+constexpr int kKStationaryStagedBytes = kMaxWavesPerWorkgroup * 4;  // ... with left-over tiles in parts: a word for each wave
 constexpr int kMaxValuBatch = 4;  // activation rows handled per launch by the VALU kernel
 constexpr int kExactIntegerFormOnly = 1;  // GemvTail::flags: never take the short int4 dequantiser
 constexpr int kSingleStage = 2;           // GemvTail::flags: no load in flight while a unit is computed (VALU kernel)
@@ -145,6 +146,13 @@ __host__ __device__ __forceinline__ PartWork part_wave_work(int parts, int wg, i
   WaveWork w;
   wave_k_range(w, kw, steps_per_wave, ksteps);
   return PartWork{wg / parts, wg % parts, w.ks_begin, w.units};
+}
+
+// K-stationary kernel with left-over tiles split into parts: which unit of `parts` k steps of its workgroup's part a wave takes (one
+// past the last: none).  The waves are dealt out to the four SIMDs in turn; the first units go to those that have a wave less.
+__host__ __device__ __forceinline__ int kstat_tail_unit(int kw, int waves) {
+  const int unit = kw - waves % 4;
+  return unit < 0 ? unit + waves : unit;
 }
 
 __device__ __forceinline__ int logical_workgroup(const Problem& p) {
@@ -282,6 +290,7 @@ struct LaunchPlan {
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
   int staged_rows;        // LDS-staged and part-tile matrix-core kernels: 8 or 16 activation rows per stage; 0 = other kernels
   int parts;              // part-tile matrix-core kernel: workgroups per tile (1, 2 or 4); 0 = other kernels
+                          // k-stationary kernel: workgroups per tile left over (2 or 4); 0 = walks of whole tiles
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
   bool k_stationary;      // the matrix-core kernel whose waves keep one k step each while the workgroup walks tiles_in_sequence tiles

@@ -35,6 +35,7 @@ namespace mgemv {
 // m_batch rows, which stay) and
 // tiles of the longest walk x 4 x m_batch x 17 x 16 bytes (the partial sums) -- one behind the other where
 // both fit, else sharing the space, with a barrier between the two uses.  Static, bf16: kKStationaryZeroBytes of zeros.
+// TAIL: m_batch rows that stay in either type, the zeros, and kKStationaryStagedBytes of words.
 // ---------------------------------------------------------------------------------------------
 
 template <int BITS, int QOP, int GROUPS_PER_RUN>
@@ -60,7 +61,11 @@ struct KStatOperand<BITS, true> { typedef LdsActivations<BITS> type; };
 // PROBE (measurement builds, wrong results): kProbeLoadsOnly keeps every load, the operand's way through LDS, the
 // parking, the barrier and the combine, and replaces the arithmetic of a unit by taking its registers;
 // kProbeComputeOnly requests only the first tile's unit and repeats its arithmetic for every tile of the walk.
-template <int BITS, int QOP, int GROUPS_PER_RUN, int ACT, int PROBE = kProbeNone>
+// TAIL: the tiles that do not divide over the workgroups are split into parts, two or four workgroups to a tile: behind its walk a
+// workgroup takes 16 / parts rows of one of them, and a wave a unit of `parts` k steps of those, mapped to the matrix operands as in
+// the part-tile kernel.  A column of a product holds one k step's sums in the order of every other unit's, so the bits are the same.
+// (Which launches, and what it is worth: left_over_parts.)
+template <int BITS, int QOP, int GROUPS_PER_RUN, int ACT, int PROBE = kProbeNone, bool TAIL = false>
 __global__ void __launch_bounds__(kWave * kMaxWavesPerWorkgroup)
 gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out,
                        int k, uint32_t packed_steps, int workgroups, int num_groups, uint32_t packed_group,
@@ -125,6 +130,16 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   const int tile0 = work.tile_begin;
   const int my_tiles = work.tiles;  // >= 1 by the host's geometry
   const int m = lane % kTileRows;
+  // This workgroup's part of a left-over tile, and this wave's unit of it: `parts` k steps of 16 / parts rows (the mapping of
+  // the part-tile kernel).  Everything else about the part is worked out where it is needed.
+  const int parts = TAIL ? tiles_per_wg_of(packed_group) : 1;
+  const int tail_tile = TAIL ? tail.seq_base * p.workgroups + wg / parts : 0;
+  const bool has_tail = TAIL && tail_tile * kTileRows < p.n_out;
+  const int tail_unit = TAIL ? kstat_tail_unit(kw, waves) : 0;
+  const int tail_units = TAIL ? (waves + parts - 1) / parts : 0;
+  const bool computes_tail = has_tail && tail_unit < tail_units;
+  const int part_rows = kTileRows / parts;
+  const int tail_row0 = tail_tile * kTileRows + wg % parts * part_rows;
 
   const int tile_stride = p.ksteps * kUnitBytes;  // bytes from a unit to the same k step of the next tile
   const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(
@@ -151,13 +166,56 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     offsets_of_tile(0, off);
     load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(wa, w_rsrc, tables, lane * kChunkBytes, off);
   };
+  // A unit of the part meets the rows of several waves.  Each wave says when its own are in its stage, and the first time a part's
+  // unit looks they have long been there; the words are cleared in front of a barrier that waits for nothing but the waves'
+  // starts.  (A barrier behind the rows costs 0.8 us a launch, one behind the walk 0.5, the rows fetched once more, straight to the
+  // LDS, 0.5-1.)
+  __shared__ uint32_t staged[TAIL ? kMaxWavesPerWorkgroup : 1];
+  auto clear_staged = [&]() {
+    if constexpr (TAIL) {
+      if (lane == 0) staged[kw] = 0;
+      __syncthreads();
+    }
+  };
+  auto say_staged = [&]() {
+    if constexpr (TAIL) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      if (lane == 0) __hip_atomic_store(&staged[kw], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  };
+  // Unit i of the walk; the one behind it is this wave's unit of the workgroup's part.
+  auto request_unit = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& to, int i) {
+    int off[GROUPS_PER_RUN];
+    if (TAIL && computes_tail && i == my_tiles) {
+      const int kstep = tail_unit * parts;
+      const int steps = waves - kstep < parts ? waves - kstep : parts;
+      const __amdgpu_buffer_rsrc_t part_rsrc = make_rsrc(
+          p.weights + ((size_t)tail_tile * (size_t)p.ksteps + (size_t)kstep) * (size_t)kUnitBytes, (uint32_t)steps * (uint32_t)kUnitBytes);
+      const int l = lane_after_loop(), k_part = l % kTileRows / part_rows, row_in_part = l % part_rows;
+      const int row_raw = tail_row0 + row_in_part;
+      const int row = row_raw < p.n_out ? row_raw : p.n_out - 1;
+      const int k_run = (kstep + k_part) * G::kStepK + l / kTileRows * G::kRunK;
+#pragma unroll
+      for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
+        const int grp = QOP == MGEMV_PER_COLUMN_SCALE_ONLY ? 0 : group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
+        off[gi] = (grp * p.n_out + row) * 2;
+      }
+      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(
+          to, part_rsrc, tables, k_part * kUnitBytes + (l / kTileRows * kTileRows + wg % parts * part_rows + row_in_part) * kChunkBytes, off);
+    } else {
+      offsets_of_tile(i, off);
+      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(to, w_rsrc, tables, i * tile_stride + lane * kChunkBytes, off);
+    }
+  };
   // The activation operand: rows of this wave's k step come in whole (one fully coalesced load per row) and pass
   // through a stage that belongs to this wave alone.
   // (Read straight from x in operand shape, every load instruction touches 64 cache lines for 16 bytes each.)
   using XS = XStage<BITS>;
-  const int stage_rows = kLdsOperand ? m_batch : 8;
+  const int stage_rows = kLdsOperand || TAIL ? m_batch : 8;
   uint8_t* const stage = reinterpret_cast<uint8_t*>(partials) + kw * (stage_rows * XS::kRowStride);
+  __shared__ u32x4 zeros[kLdsOperand || TAIL ? kKStationaryZeroBytes / 16 : 1];
   typename KStatOperand<BITS, kLdsOperand>::type xa;
+  clear_staged();
   if constexpr (kLdsOperand) {
     // The stage stays.
     for (int first = 0; first < m_batch; first += 8) {
@@ -168,11 +226,11 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       __builtin_amdgcn_sched_barrier(0);
       park_x_rows<BITS, 8>(rows, stage, lane, first, 1, rows_here);
     }
+    say_staged();
     // Lanes of rows that do not exist read zeros: their columns of a matrix product are never stored, but the matrix unit
     // multiplies them all the same, and a large launch runs at the clock the power limit leaves (28672x8192 at 4 rows 1.92
     // GHz, its loads alone 2.32).  With row 0 in the idle columns that launch took 30.3 us, with zeros 29.4; 128256x4096 at
     // 2 rows 66.3 / 63.6, 28672x8064 g96 at 4 rows 33.2 / 32.3; up to 13 us level.
-    __shared__ u32x4 zeros[kKStationaryZeroBytes / 16];
     if (lane < kKStationaryZeroBytes / 16) zeros[lane] = u32x4{0u, 0u, 0u, 0u};  // every wave for itself: no barrier
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the LDS executes a wave's accesses in order
     __builtin_amdgcn_wave_barrier();
@@ -215,6 +273,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       __builtin_amdgcn_wave_barrier();
     };
     park_x_rows<BITS, 8>(rows, stage, lane, 0, 1, rows_ahead);
+    say_staged();
     read_back(0, rows_ahead);
     if (m_batch > 8) {
       if constexpr (kAllRowsAhead) {
@@ -231,7 +290,10 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       read_back(8, m_batch - 8);
     }
   }
-  const bool park_behind_stage = kLdsOperand || (tail.flags & kParkBehindStage) != 0;
+  if constexpr (TAIL) {
+    if (!kLdsOperand && lane < kKStationaryZeroBytes / 16) zeros[lane] = u32x4{0u, 0u, 0u, 0u};
+  }
+  const bool park_behind_stage = kLdsOperand || TAIL || (tail.flags & kParkBehindStage) != 0;
   if (!park_behind_stage) __syncthreads();  // the stages make room for the partial sums
   const bool short_allowed = (tail.flags & kExactIntegerFormOnly) == 0;
   const ConvertRegs c = make_convert_regs();
@@ -247,8 +309,46 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   f32x4* const park = reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(partials) +
                                                (park_behind_stage ? waves * (stage_rows * XS::kRowStride) : 0));
   const int park_tile_stride = kKSlices * m_batch * slots;  // entries from a tile to the next
-  f32x4* const my_park = park + (slice * m_batch + m) * slots + kw;
-  auto compute_and_park = [&](const MfmaWeights<BITS, GROUPS_PER_RUN>& f, int i) {
+  f32x4* my_park = park + (slice * m_batch + m) * slots + kw;
+  bool parks = m < m_batch;
+  // The unit of a left-over part: its operand, its scales past the reduction and its entries take the place of the walk's.
+  // (Through the loop itself, as one more unit of the walk, bf16 and longer walks lose 1-2 % and short fp16 ones gain as much.)
+  auto turn_to_part = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& f) {
+    const int l = lane_after_loop(), slice = l / kTileRows, k_part = l % kTileRows / part_rows, row_in_part = l % part_rows;
+    const int kstep = tail_unit * parts + k_part;
+    const uint8_t* const base =
+        row_in_part < m_batch && kstep < waves
+            ? reinterpret_cast<const uint8_t*>(partials) + (kstep * stage_rows + row_in_part) * XS::kRowStride + slice * (G::kRunK * 2)
+            : reinterpret_cast<const uint8_t*>(zeros);
+    const int of = tail_unit * parts + l % parts;
+    // (every wave of the workgroup says so in front of its walk, whatever the others do)
+    while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(&staged[of < waves ? of : kw], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u) != 0)
+      __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    if constexpr (kLdsOperand) {
+      xa.lane_base = base;
+    } else {
+      const LdsActivations<BITS> from{base};
+#pragma unroll
+      for (int i = 0; i < kBlocksPerUnit; ++i)
+#pragma unroll
+        for (int j = 0; j < (BITS == 4 ? 4 : 2); ++j) xa.x[i][j] = mfma_operand<BITS>(from, i, j);
+    }
+    // Past the reduction the activations are zero, but an infinite scale or zero times zero is not: finite ones of the short form's range.
+    constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
+    const int k_run = kstep * G::kStepK + slice * G::kRunK;
+#pragma unroll
+    for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
+      const bool past = k_run + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
+      f.s[gi] = past ? kAnyScale : f.s[gi];
+      f.z[gi] = past ? 0u : f.z[gi];
+    }
+    // The product's rows 4 * slice .. + 3 are the part's at one of the unit's k steps; a column is a batch row at one of them.
+    const int quads = part_rows / 4;
+    parks = slice / quads == k_part && row_in_part < m_batch;
+    my_park = park + ((slice % quads) * m_batch + row_in_part) * slots + kstep;
+  };
+  auto compute_and_park = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& f, int i) {
     f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     half2_t col_scale = half2_t{};
     bool short_ok = short_allowed;
@@ -265,7 +365,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     } else {
       compute_unit_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(acc, f, xa, c, col_scale, short_ok);
     }
-    if (m < m_batch) my_park[i * park_tile_stride] = acc;
+    if (TAIL ? parks : m < m_batch) my_park[i * park_tile_stride] = acc;
   };
   // arithmetic-only build: the next unit is the first one again; the compiler must assume its registers changed
   auto repeat_first_unit = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& to, const MfmaWeights<BITS, GROUPS_PER_RUN>& from) {
@@ -284,9 +384,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     if constexpr (PROBE == kProbeComputeOnly) {
       repeat_first_unit(wb, wa);
     } else {
-      int off[GROUPS_PER_RUN];
-      offsets_of_tile(i + 1, off);
-      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(wb, w_rsrc, tables, (i + 1) * tile_stride + lane * kChunkBytes, off);
+      request_unit(wb, i + 1);
     }
     __builtin_amdgcn_sched_barrier(0);
     compute_and_park(wa, i);
@@ -294,24 +392,37 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     if constexpr (PROBE == kProbeComputeOnly) {
       repeat_first_unit(wa, wb);
     } else {
-      int off[GROUPS_PER_RUN];
-      offsets_of_tile(i + 2, off);
-      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(wa, w_rsrc, tables, (i + 2) * tile_stride + lane * kChunkBytes, off);
+      request_unit(wa, i + 2);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (i + 1 < my_tiles) compute_and_park(wb, i + 1);
     __builtin_amdgcn_sched_barrier(0);
     i += 2;
   } while (i < my_tiles);
+  if constexpr (TAIL) {
+    if (computes_tail) {
+      if (my_tiles & 1) wa = wb;  // requested last
+      turn_to_part(wa);
+      compute_and_park(wa, my_tiles);
+    }
+  }
 
   // The combine.  Wave r sums tiles r, r + waves, ... of the walk; lane (slice, m) the four rows
   // 4 * slice .. + 3 of batch row m.  A wave that reaches the barrier waits for the slowest one, and behind
   // the barrier it is alone on its SIMD, where every instruction costs its full latency: whatever does not
   // need the other waves' sums -- addresses, the bias, zeros in the entries of waves that do not exist --
   // is done in front of it.
-  const bool sums = m < m_batch && kw < my_tiles;
+  const int summed_tiles = my_tiles + (has_tail ? 1 : 0);
+  const bool sums = m < m_batch && kw < summed_tiles;
   f32x4* block = park + ((kw * kKSlices + slice) * m_batch + m) * slots;
   int n0 = (tile0 + kw) * kTileRows + 4 * slice;
+  uint16_t* dst = reinterpret_cast<uint16_t*>(tail.y) + (size_t)m * (size_t)p.n_out + n0;
+  // the part: lanes of the first slices, one for every four of its rows
+  auto move_to_part = [&]() {
+    n0 = slice * 4 < part_rows ? tail_row0 + 4 * slice : p.n_out;
+    dst = reinterpret_cast<uint16_t*>(tail.y) + (size_t)m * (size_t)p.n_out + n0;
+  };
+  if (TAIL && has_tail && kw == my_tiles) move_to_part();
   float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   auto fetch_bias = [&]() {
     if (has_bias) {
@@ -327,18 +438,17 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   };
   if (sums) {
     fetch_bias();
-    if (waves < pieces)
-      for (int t = kw; t < my_tiles; t += waves)
-        for (int w = waves; w < pieces; ++w)
+    if (TAIL || waves < pieces)
+      for (int t = kw; t < summed_tiles; t += waves)
+        for (int w = TAIL && t == my_tiles ? tail_units * parts : waves; w < pieces; ++w)
           block[(t - kw) * park_tile_stride + w] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  uint16_t* dst = reinterpret_cast<uint16_t*>(tail.y) + (size_t)m * (size_t)p.n_out + n0;
   const size_t dst_step = (size_t)waves * kTileRows;  // outputs from a tile this wave sums to the next
   const bool wide_store = ((reinterpret_cast<uintptr_t>(tail.y) | (uintptr_t)((size_t)p.n_out * 2)) & 7u) == 0;
 
   __syncthreads();
   if (sums) {
-    for (int t = kw; t < my_tiles; t += waves) {
+    for (int t = kw; t < summed_tiles; t += waves) {
       f32x4 sum;
       auto sum_block = [&](auto count) {
         f32x4 piece[decltype(count)::value];
@@ -377,14 +487,17 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
       block += waves * park_tile_stride;
       n0 += waves * kTileRows;
       dst += dst_step;
-      if (t + waves < my_tiles) fetch_bias();
+      if (TAIL && has_tail && t + waves == my_tiles) move_to_part();
+      if (t + waves < summed_tiles) fetch_bias();
     }
   }
 }
 
-template <int BITS, int QOP, int GPR, int ACT, int PROBE = kProbeNone>
+template <int BITS, int QOP, int GPR, int ACT, int PROBE = kProbeNone, bool TAIL = false>
 hipError_t launch_mfma_kstat_kernel(const GemvLaunch& g) {
-  const auto kernel = gemv_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE>;
+  if constexpr (PROBE == kProbeNone && !TAIL && BITS == 4 && (ACT == kActBf16 || GPR != 4))  // (left_over_parts asks for no others)
+    if (g.plan.parts != 0) return launch_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE, true>(g);
+  const auto kernel = gemv_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE, TAIL>;
   if (g.lds > 48 * 1024) {
     // More than 48 KiB of dynamic LDS has to be granted per kernel and device; remember the
     // largest grant so that only the first such launch pays for the call.
@@ -404,7 +517,8 @@ hipError_t launch_mfma_kstat_kernel(const GemvLaunch& g) {
     }
   }
   return launch(kernel, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale, g.zero_add, g.n_out, g.k,
-                pack_steps(num_ksteps(g.k, BITS), 1), g.plan.workgroups, g.tail.num_groups, pack_group(g.group_size, 1, g.tail.route != nullptr),
+                pack_steps(num_ksteps(g.k, BITS), 1), g.plan.workgroups, g.tail.num_groups,
+                pack_group(g.group_size, TAIL ? g.plan.parts : 1, g.tail.route != nullptr),
                 g.tail);
 }
 
