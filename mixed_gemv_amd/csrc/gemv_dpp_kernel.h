@@ -412,22 +412,9 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
   // unbatched launch whose waves stay on one tile reads the tail, so those loads do not wait
   // for any scalar load at all: `tail` itself is only touched by batched launches and tile
   // walks, everything else reads the copy `late`, fetched once the first unit is requested.
-  // Batched launch (gemv/kernel/mixed_gemv.h:140-149, 222-223): problems past the first fetch
-  // their strides first.  A routed launch (a bit of a preloaded word says so) looks up whose
-  // weights, scales, zeros and bias each problem takes; x and y stay with the problem.
   const long long batch = blockIdx.z;
-  long long owner = batch;
-  if ((blockIdx.z | (packed_group & kRoutedLaunch)) != 0) {  // one test on the way of an unbatched launch
-    if ((packed_group & kRoutedLaunch) != 0) {
-      const int entry = tail.route[batch];
-      if ((unsigned)entry >= (unsigned)tail.route_extent) return;  // whole workgroup, before any barrier
-      owner = entry;
-    }
-    p.weights += owner * tail.stride_weights;
-    p.x += batch * tail.stride_x;
-    p.scale += owner * tail.stride_scale;
-    p.zero_add += owner * tail.stride_scale;  // only dereferenced in scale+zero mode
-  }
+  long long owner;
+  if (!place_problem(p, tail, packed_group, owner)) return;  // whole workgroup, before any barrier
 
   const int wg = logical_workgroup(p);
   if (wg >= p.workgroups) return;  // whole workgroup leaves before any barrier
@@ -671,7 +658,7 @@ template <int BITS, int QOP, int MB, int GPR, bool MULTI, int ACT, int FORM = kU
 hipError_t launch_gemv_kernel_m(const GemvLaunch& g) {
   return launch(gemv_dpp_kernel<BITS, QOP, MB, GPR, MULTI, ACT, kProbeNone, FORM, EARLY_BIAS>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
                 g.zero_add, g.n_out, g.k, pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups,
-                g.tail.num_groups, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
+                g.tail.num_groups, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.stack != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int MB, int GPR, int ACT>

@@ -1151,8 +1151,11 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.tail.stride_scale = stride_scale;
   g.tail.stride_bias = stride_bias;
   g.tail.stride_y = stride_y;
-  g.tail.route = route;
-  g.tail.route_extent = route_extent;
+  if (route != nullptr) {  // the two change places (place_problem)
+    g.tail.stack = g.weights;
+    g.weights = reinterpret_cast<const uint8_t*>(route);
+    g.tail.route_extent = route_extent;
+  }
   g.grid = dim3((unsigned)(g.plan.wgs_per_xcd * kNumXcd), 1, (unsigned)batch_count);
   g.block = dim3((unsigned)(kWave * g.plan.split_k), (unsigned)g.plan.tiles_per_wg, 1);
   g.stream = static_cast<hipStream_t>(stream);

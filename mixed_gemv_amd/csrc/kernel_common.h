@@ -41,12 +41,14 @@ struct GemvTail {
   int m_batch;         // activation rows (matrix-core kernel)
   int num_groups;      // k / group_size (1 in per-column mode): extent of the scale / zero tables
   int flags;           // kExactIntegerFormOnly | kSingleStage
-  float alpha, beta;   // epilogue: y = alpha * acc + beta * bias (gemv/device/gemv_adaptor.h:123, epilogue{alpha, beta})
-  int seq_base;        // VALU kernel: tiles / sequences ...
-  int seq_rem;         // ... and tiles % sequences (the first seq_rem sequences get one tile more)
-  long long stride_weights, stride_x, stride_scale, stride_bias, stride_y;  // per batch problem
-  const int* route;    // routed launch: problem b takes weights, scales, zeros and bias of entry route[b] of the stack
+  // Routed launch: problem b takes weights, scales, zeros and bias of entry route[b] of the stack; route itself is the launch's
+  // `weights` argument (place_problem).  From here to stride_scale: one 64-byte line of the arguments.
+  const uint8_t* stack;  // the weights of entry 0; null: not routed
   int route_extent;    // entries in the stack: a problem routed outside [0, route_extent) is left alone
+  int seq_base;        // VALU kernel: tiles / sequences ...
+  long long stride_weights, stride_x, stride_scale, stride_bias, stride_y;  // per batch problem
+  float alpha, beta;   // epilogue: y = alpha * acc + beta * bias (gemv/device/gemv_adaptor.h:123, epilogue{alpha, beta})
+  int seq_rem;         // ... and tiles % sequences (the first seq_rem sequences get one tile more)
   unsigned long long* trace;  // timeline probe: kTimelineWordsPerWave words per wave, else unused
 };
 
@@ -67,7 +69,7 @@ struct Problem {
 };
 
 constexpr uint32_t pack_steps(int ksteps, int steps_per_wave) { return (uint32_t)ksteps | ((uint32_t)steps_per_wave << 16); }
-// group size in bits 0-23, tiles per workgroup in bits 24-30, bit 31: the launch is routed (GemvTail::route)
+// group size in bits 0-23, tiles per workgroup in bits 24-30, bit 31: the launch is routed (GemvTail::stack)
 constexpr uint32_t kRoutedLaunch = 0x80000000u;
 constexpr uint32_t pack_group(int group_size, int tiles_per_wg, bool routed) {
   return (uint32_t)group_size | ((uint32_t)tiles_per_wg << 24) | (routed ? kRoutedLaunch : 0u);
@@ -157,6 +159,35 @@ __host__ __device__ __forceinline__ int kstat_tail_unit(int kw, int waves) {
 
 __device__ __forceinline__ int logical_workgroup(const Problem& p) {
   return logical_workgroup_of((int)blockIdx.x, p.wgs_per_xcd);
+}
+
+// Where the operands of problem blockIdx.z begin (gemv/kernel/mixed_gemv.h:140-149, 222-223): moves the pointers of p, gives the
+// entry whose weights, scales, zeros and bias it takes (x and y stay with the problem), or false: routed outside the stack.
+// The way to the first weight of a routed launch was three scalar loads one behind the other, each a miss of the cold cache: the
+// route's address, the entry, the strides.  The route's address is a preloaded argument now (the weights' is not, which needs
+// the entry first), and the rest is requested with the entry.  8 of 64 matrices of 1408x2048 4.63 us / 4.34; 0.93-0.99 of the time on 40
+// routed launches of random shapes.
+__device__ __forceinline__ bool place_problem(Problem& p, const GemvTail& tail, uint32_t packed_group, long long& owner) {
+  const long long batch = blockIdx.z;
+  owner = batch;
+  if ((blockIdx.z | (packed_group & kRoutedLaunch)) == 0) return true;  // one test on the way of an unbatched launch
+  long long stride_weights = tail.stride_weights, stride_x = tail.stride_x, stride_scale = tail.stride_scale;
+  bool there = true;
+  if ((packed_group & kRoutedLaunch) != 0) {
+    typedef const __attribute__((address_space(4))) int* Route;
+    int entry = ((Route)p.weights)[batch], extent = tail.route_extent;
+    const uint8_t* stack = tail.stack;
+    // (in front of the first use of any of them, or the compiler requests the strides behind the test of the entry)
+    asm volatile("" : "+s"(entry), "+s"(extent), "+s"(stack), "+s"(stride_weights), "+s"(stride_x), "+s"(stride_scale));
+    there = (unsigned)entry < (unsigned)extent;
+    owner = entry;
+    p.weights = stack;
+  }
+  p.weights += owner * stride_weights;
+  p.x += batch * stride_x;
+  p.scale += owner * stride_scale;
+  p.zero_add += owner * stride_scale;  // only dereferenced in scale+zero mode
+  return there;
 }
 
 // Group index of reduction position k_index (host/mixed_gemv.h:88), clamped to the last

@@ -51,16 +51,8 @@ gemv_mfma_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, c
                "s"(tail.m_batch), "s"(tail.num_groups), "s"(tail.flags), "s"(tail.stride_weights), "s"(tail.stride_x), "s"(tail.stride_scale),
                "s"(tail.stride_bias), "s"(tail.stride_y));
   const long long batch = blockIdx.z;
-  long long owner = batch;  // routed launch: whose weights, scales, zeros and bias the problem takes
-  if (packed_group & kRoutedLaunch) {
-    const int entry = tail.route[batch];
-    if ((unsigned)entry >= (unsigned)tail.route_extent) return;  // whole workgroup, before any barrier
-    owner = entry;
-  }
-  p.weights += owner * tail.stride_weights;
-  p.x += batch * tail.stride_x;
-  p.scale += owner * tail.stride_scale;
-  p.zero_add += owner * tail.stride_scale;
+  long long owner;
+  if (!place_problem(p, tail, packed_group, owner)) return;  // whole workgroup, before any barrier
   const bool has_bias = tail.bias != nullptr;
   tail.bias += owner * tail.stride_bias;
   tail.y += batch * tail.stride_y;
@@ -236,18 +228,8 @@ gemv_mfma_lds_kernel(const uint8_t* weights, const half_t* x, const half_t* scal
   p.group_size = (int)(packed_group & 0xffffffu);
   p.tiles_per_wg = tiles_per_wg_of(packed_group);
   const long long batch = blockIdx.z;
-  long long owner = batch;  // routed launch: whose weights, scales, zeros and bias the problem takes
-  if ((blockIdx.z | (packed_group & kRoutedLaunch)) != 0) {
-    if ((packed_group & kRoutedLaunch) != 0) {
-      const int entry = tail.route[batch];
-      if ((unsigned)entry >= (unsigned)tail.route_extent) return;  // whole workgroup, before any barrier
-      owner = entry;
-    }
-    p.weights += owner * tail.stride_weights;
-    p.x += batch * tail.stride_x;
-    p.scale += owner * tail.stride_scale;
-    p.zero_add += owner * tail.stride_scale;
-  }
+  long long owner;
+  if (!place_problem(p, tail, packed_group, owner)) return;  // whole workgroup, before any barrier
   const bool has_bias = tail.bias != nullptr;
   tail.bias += owner * tail.stride_bias;
   tail.y += batch * tail.stride_y;
@@ -394,7 +376,7 @@ template <int BITS, int QOP, int GPR, int T>
 hipError_t launch_mfma_kernel_t(const GemvLaunch& g) {
   return launch(gemv_mfma_kernel<BITS, QOP, GPR, T>, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale,
                 g.zero_add, g.n_out, g.k, pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups,
-                g.plan.wgs_per_xcd, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
+                g.plan.wgs_per_xcd, pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.stack != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int GPR>
@@ -458,7 +440,7 @@ hipError_t launch_mfma_lds_kernel_r(const GemvLaunch& g) {
   }
   return launch(kernel, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale, g.zero_add, g.n_out, g.k,
                 pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups, g.tail.num_groups,
-                pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.route != nullptr), g.tail);
+                pack_group(g.group_size, g.plan.tiles_per_wg, g.tail.stack != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int GPR, int ACT>
