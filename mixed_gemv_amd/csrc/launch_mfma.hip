@@ -280,7 +280,7 @@ gemv_mfma_lds_kernel(const uint8_t* weights, const half_t* x, const half_t* scal
   XRows<BITS, ROUNDS> xr;
   MfmaWeights<BITS, GROUPS_PER_RUN> wa, wb;
   fetch_x_rows<BITS, ROUNDS>(xr, p, x_rsrc, ks_begin, lane, ty, p.tiles_per_wg);
-  load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN>(wa, p, w_rsrc, tables, 0, ks_begin, lane, row);
+  load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(wa, p, w_rsrc, tables, 0, ks_begin, lane, row);
   // A stage is shared by the tiles_per_wg waves that cover the same k range of neighbouring tiles
   // (SHARED).  With one tile per workgroup every wave has its stages to itself: the LDS executes
   // a wave's accesses in order, so nothing but the compiler has to be kept from reordering them,
@@ -305,7 +305,7 @@ gemv_mfma_lds_kernel(const uint8_t* weights, const half_t* x, const half_t* scal
       keep_registers(next, xr);
     } else if constexpr (!kLast) {
       fetch_x_rows<BITS, ROUNDS>(xr, p, x_rsrc, ks_begin + u + 1, lane, ty, p.tiles_per_wg);
-      load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN>(next, p, w_rsrc, tables, u + 1, ks_begin + u + 1, lane, row);
+      load_weights_lds_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(next, p, w_rsrc, tables, u + 1, ks_begin + u + 1, lane, row);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (u < units) {

@@ -38,20 +38,6 @@ namespace mgemv {
 // TAIL: m_batch rows that stay in either type, the zeros, and kKStationaryStagedBytes of words.
 // ---------------------------------------------------------------------------------------------
 
-template <int BITS, int QOP, int GROUPS_PER_RUN>
-__device__ __forceinline__ void load_unit_kstat(MfmaWeights<BITS, GROUPS_PER_RUN>& f, __amdgpu_buffer_rsrc_t w_rsrc,
-                                                const ScaleTables& tables, int weight_offset,
-                                                const int (&table_offset)[GROUPS_PER_RUN]) {
-#pragma unroll
-  for (int i = 0; i < kBlocksPerUnit; ++i)
-    f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, weight_offset + i * kBlockBytes, 0, kCacheStream);
-#pragma unroll
-  for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-    f.s[gi] = load_b16_low(tables.scale, table_offset[gi]);  // per-column mode: the row's scale, group 0
-    if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) f.z[gi] = load_b16_low(tables.zero, table_offset[gi]);
-  }
-}
-
 // Where a wave keeps its activation operand: in registers, or in its stage.
 template <int BITS, bool LDS_OPERAND>
 struct KStatOperand { typedef MfmaActivations<BITS> type; };
@@ -154,7 +140,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   auto request_first_unit = [&]() {
     int off[GROUPS_PER_RUN];
     offsets_of_tile(0, off);
-    load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(wa, w_rsrc, tables, lane * kChunkBytes, off);
+    load_unit_mfma<BITS, GROUPS_PER_RUN, true, QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS, ACT>(wa, w_rsrc, tables, lane * kChunkBytes, [&](int gi) { return off[gi]; });
   };
   // A unit of the part meets the rows of several waves.  Each wave says when its own are in its stage, and the first time a part's
   // unit looks they have long been there; the words are cleared in front of a barrier that waits for nothing but the waves'
@@ -190,11 +176,11 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
         const int grp = QOP == MGEMV_PER_COLUMN_SCALE_ONLY ? 0 : group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
         off[gi] = (grp * p.n_out + row) * 2;
       }
-      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(
-          to, part_rsrc, tables, k_part * kUnitBytes + (l / kTileRows * kTileRows + wg % parts * part_rows + row_in_part) * kChunkBytes, off);
+      load_unit_mfma<BITS, GROUPS_PER_RUN, true, QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS, ACT>(
+          to, part_rsrc, tables, k_part * kUnitBytes + (l / kTileRows * kTileRows + wg % parts * part_rows + row_in_part) * kChunkBytes, [&](int gi) { return off[gi]; });
     } else {
       offsets_of_tile(i, off);
-      load_unit_kstat<BITS, QOP, GROUPS_PER_RUN>(to, w_rsrc, tables, i * tile_stride + lane * kChunkBytes, off);
+      load_unit_mfma<BITS, GROUPS_PER_RUN, true, QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS, ACT>(to, w_rsrc, tables, i * tile_stride + lane * kChunkBytes, [&](int gi) { return off[gi]; });
     }
   };
   // The activation operand: rows of this wave's k step come in whole (one fully coalesced load per row) and pass

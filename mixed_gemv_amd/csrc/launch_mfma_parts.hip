@@ -145,7 +145,7 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   }
   auto request = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& w, int u) {
     fetch_part_rows<BITS, ROWS, PARTS>(xr, x_rows, p.k, x_rsrc, ks_begin + u * PARTS, lane);
-    load_weights_at<BITS, QOP, GROUPS_PER_RUN>(w, p, w_rsrc, tables, u * (PARTS * kUnitBytes) + w_lane,
+    load_weights_at<BITS, QOP, GROUPS_PER_RUN, ACT>(w, p, w_rsrc, tables, u * (PARTS * kUnitBytes) + w_lane,
                                                (ks_begin + u * PARTS + k_part) * G::kStepK + slice * G::kRunK, row);
   };
   request(wa, 0);

@@ -199,33 +199,55 @@ __device__ __forceinline__ void compute_unit_mfma(f32x4& acc, const MfmaWeights<
   compute_unit_mfma_form<BITS, QOP, GROUPS_PER_RUN, false, ACT>(acc, f, xa, c, col_scale2, short4);
 }
 
-// Weights, scales and zeros of a unit through descriptors: everything unit-dependent sits in the bounds-checked VGPR
-// offset, so a prefetch past the range reads zeros.  k_run: first reduction index of the lane's run; row: its weight row.
-template <int BITS, int QOP, int GROUPS_PER_RUN>
-__device__ __forceinline__ void load_weights_at(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p, __amdgpu_buffer_rsrc_t w_rsrc,
-                                                const ScaleTables& tables, int voffset, int k_run, int row) {
-  using G = Geometry<BITS>;
+// Weights, scales and zeros of a unit through descriptors; scale_offset(gi): bytes into the tables, group gi of the lane's run (the
+// per-column mode of the k-stationary kernel takes the row's scale for group 0's).
+// Loads come back in order.  fp16: the scales are requested first, so that a wave starts on a unit's first block while the others
+// are on their way; behind the weights they made it wait for the whole unit.  In front / behind, geometric means over 118 launches of
+// random shapes: int4 on more tiles than compute units 0.98 of the time up to 16 k steps and 0.99 beyond, on fewer 0.988,
+// int8 0.99-1.0; 8192x8192 g64 at 16 rows 13.85 us behind, 13.5 in front (cold).  bf16, which waits for the vector unit: 0.985-1.003,
+// and with four lookups per run 1.03 (5004x5280 g96 at 3 rows 8.0 / 8.25), so there the weights stay in front.
+template <int BITS, int GROUPS_PER_RUN, bool HAS_SCALE, bool HAS_ZERO, int ACT, typename ScaleOffset>
+__device__ __forceinline__ void load_unit_mfma(MfmaWeights<BITS, GROUPS_PER_RUN>& f, __amdgpu_buffer_rsrc_t w_rsrc, const ScaleTables& tables,
+                                               int voffset, const ScaleOffset& scale_offset) {
+  auto load_scales = [&]() {
+    if constexpr (HAS_SCALE) {
+#pragma unroll
+      for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
+        const int off = scale_offset(gi);
+        f.s[gi] = load_b16_low(tables.scale, off);
+        if constexpr (HAS_ZERO) f.z[gi] = load_b16_low(tables.zero, off);
+      }
+    }
+  };
+  if constexpr (ACT == kActF16) {
+    load_scales();
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int i = 0; i < kBlocksPerUnit; ++i)
     f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, voffset + i * kBlockBytes, 0, kCacheStream);
-  if constexpr (QOP != MGEMV_PER_COLUMN_SCALE_ONLY) {
-#pragma unroll
-    for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-      const int grp = group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN));
-      const int off = (grp * p.n_out + row) * 2;
-      f.s[gi] = load_b16_low(tables.scale, off);
-      if constexpr (QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS) f.z[gi] = load_b16_low(tables.zero, off);
-    }
-  }
+  if constexpr (ACT != kActF16) load_scales();
+}
+
+// ... everything unit-dependent in the bounds-checked VGPR offset, so a prefetch past the range reads zeros.  k_run: first reduction
+// index of the lane's run; row: its weight row.
+template <int BITS, int QOP, int GROUPS_PER_RUN, int ACT>
+__device__ __forceinline__ void load_weights_at(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p, __amdgpu_buffer_rsrc_t w_rsrc,
+                                                const ScaleTables& tables, int voffset, int k_run, int row) {
+  using G = Geometry<BITS>;
+  load_unit_mfma<BITS, GROUPS_PER_RUN, QOP != MGEMV_PER_COLUMN_SCALE_ONLY, QOP == MGEMV_FINEGRAINED_SCALE_AND_ZEROS, ACT>(
+      f, w_rsrc, tables, voffset, [&](int gi) {
+        return (group_of<GROUPS_PER_RUN>(p, k_run + gi * (G::kRunK / GROUPS_PER_RUN)) * p.n_out + row) * 2;
+      });
 }
 // ... of unit `unit` of the wave's k range, a whole tile's rows.
-template <int BITS, int QOP, int GROUPS_PER_RUN>
+template <int BITS, int QOP, int GROUPS_PER_RUN, int ACT>
 __device__ __forceinline__ void load_weights_lds_mfma(MfmaWeights<BITS, GROUPS_PER_RUN>& f, const Problem& p,
                                                       __amdgpu_buffer_rsrc_t w_rsrc, const ScaleTables& tables, int unit,
                                                       int kstep, int lane, int row) {
   using G = Geometry<BITS>;
-  load_weights_at<BITS, QOP, GROUPS_PER_RUN>(f, p, w_rsrc, tables, unit * kUnitBytes + lane * kChunkBytes,
-                                             kstep * G::kStepK + (lane / kTileRows) * G::kRunK, row);
+  load_weights_at<BITS, QOP, GROUPS_PER_RUN, ACT>(f, p, w_rsrc, tables, unit * kUnitBytes + lane * kChunkBytes,
+                                                  kstep * G::kStepK + (lane / kTileRows) * G::kRunK, row);
 }
 
 // Activation rows on their way through LDS: a wave fetches whole rows of a k step (64 lanes x 16 or 8 bytes,
