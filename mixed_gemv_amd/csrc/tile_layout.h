@@ -79,23 +79,23 @@ MGEMV_HD size_t preprocessed_bytes(size_t n_out, size_t k, int bits) {
 }
 
 // 32-bit words (W: one, or a vector of them) in natural order -- int4: element e in bits 4e..4e+3, two's complement --
-// to stored order and back.
+// to stored order and back.  (In place: a wide vector as an argument or a result has no agreed place without the instructions for it.)
 template <typename W>
-MGEMV_HD W encode_int4(W natural) {
-  const W b = natural ^ 0x88888888u;  // +8 on each two's-complement nibble
+MGEMV_HD void encode_int4(W& w) {
+  const W b = w ^ 0x88888888u;  // +8 on each two's-complement nibble
   const W f5 = b & 0x00f00000u;
-  return ((b & 0x0000000fu) << 7) | ((b & 0x000000f0u) << 19) | ((b & 0x00000f00u) >> 5) | ((b & 0x0000f000u) << 7) |
-         ((b & 0x000f0000u) >> 1) | (f5 << 11) | (f5 >> 21) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
+  w = ((b & 0x0000000fu) << 7) | ((b & 0x000000f0u) << 19) | ((b & 0x00000f00u) >> 5) | ((b & 0x0000f000u) << 7) |
+      ((b & 0x000f0000u) >> 1) | (f5 << 11) | (f5 >> 21) | ((b & 0x0f000000u) >> 13) | ((b & 0xf0000000u) >> 1);
 }
 template <typename W>
-MGEMV_HD W decode_int4(W w) {
+MGEMV_HD void decode_int4(W& w) {
   const W f5 = ((w >> 11) | (w << 21)) & 0x00f00000u;
-  return (((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) | ((w >> 7) & 0x0000f000u) |
-          ((w << 1) & 0x000f0000u) | f5 | ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u)) ^ 0x88888888u;
+  w = (((w >> 7) & 0x0000000fu) | ((w >> 19) & 0x000000f0u) | ((w << 5) & 0x00000f00u) | ((w >> 7) & 0x0000f000u) |
+       ((w << 1) & 0x000f0000u) | f5 | ((w << 13) & 0x0f000000u) | ((w << 1) & 0xf0000000u)) ^ 0x88888888u;
 }
 // (its own inverse)
 template <typename W>
-MGEMV_HD W recode_int8(W w) { return w ^ 0x80808080u; }
+MGEMV_HD void recode_int8(W& w) { w = w ^ 0x80808080u; }
 
 }  // namespace mgemv
 
