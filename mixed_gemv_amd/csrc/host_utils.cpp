@@ -22,9 +22,9 @@ namespace {
 #define MGEMV_VARIANTS 0
 #endif
 #define MGEMV_INLINE inline __attribute__((always_inline))
-typedef uint32_t word4 __attribute__((vector_size(16), aligned(1), may_alias));  // of buffers at any address
-typedef uint32_t word8 __attribute__((vector_size(32), aligned(1), may_alias));
-typedef uint32_t word16 __attribute__((vector_size(64), aligned(1), may_alias));
+typedef uint32_t word4 __attribute__((vector_size(16)));
+typedef uint32_t word8 __attribute__((vector_size(32)));
+typedef uint32_t word16 __attribute__((vector_size(64)));
 
 template <typename Loop, typename... Args>
 void run_plain(Args... args) { Loop::template run<word4>(args...); }
