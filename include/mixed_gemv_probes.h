@@ -18,7 +18,8 @@ extern "C" {
  * shape cannot read faster than X" is a kernel anybody can run, not a remark.
  * ---------------------------------------------------------------------------------------- */
 
-/* Which build of the VALU kernel a launch of batch_count problems takes on a device of num_compute_units compute
+/* Which build of the VALU kernel for whole tiles (of which the measurement builds below are; a single row on few tiles takes the
+ * kernel for parts of tiles instead, which has one build) a launch of batch_count problems takes on a device of num_compute_units compute
  * units: MGEMV_UNIT_FORM_LOOP (any number of units per wave; also reported for matrix-core launches),
  * _TWO (waves of one or two units), _TWO_AHEAD (longer waves that have a SIMD to themselves, the first two units
  * requested together) or _ONE (waves of one unit).  The results do not depend on it. */
@@ -41,14 +42,16 @@ MGEMV_API int mgemv_probe_stream_read(const void *src, size_t bytes, int workgro
                                       int units_in_flight, uint32_t *sink, void *stream);
 
 /* Measurement builds of the single-row int4 scale-and-zero fp16 GEMV kernel (one group per lane
- * run: group sizes that are multiples of 128), launched with the geometry mgemv_gemv would use, in the
+ * run: group sizes that are multiples of 128), launched with the geometry mgemv_gemv would use (whole tiles), in the
  * build that it would use for waves of that length (mgemv_probe_unit_form):
  *   MGEMV_PROBE_LOADS_ONLY  every load of the kernel, the arithmetic of a unit replaced by an
  *                           exclusive-or over its registers; y receives meaningless values;
  *   MGEMV_PROBE_TIMELINE    the kernel as it is, plus MGEMV_PROBE_TIMELINE_WORDS 64-bit words per
  *                           wave, written to trace[wave * MGEMV_PROBE_TIMELINE_WORDS + i] (wave =
  *                           workgroup * waves per workgroup + wave in workgroup; workgroups and
- *                           threads as mgemv_query_launch_for reports for the device).  Words 0-4
+ *                           threads as mgemv_query_launch_for reports for the device; where the
+ *                           product takes parts of tiles, as it reports with mgemv_set_default_plans(0),
+ *                           which are no more waves).  Words 0-4
  *                           are readings of the 100 MHz constant clock (s_memrealtime): 0 the wave
  *                           starts, 1 its first unit is requested, 2 that unit's first block has
  *                           arrived, 3 its last unit is computed, 4 its outputs are stored;
@@ -57,7 +60,8 @@ MGEMV_API int mgemv_probe_stream_read(const void *src, size_t bytes, int workgro
  *                           start and after its stores, so that (13 - 12) / (4 - 0) * 100 MHz is the
  *                           clock the compute unit ran at.
  *                           trace_capacity_waves: waves the buffer has room for; a launch with
- *                           more returns MGEMV_ERR_SIZE and writes nothing.  y is the GEMV's result;
+ *                           more returns MGEMV_ERR_SIZE and writes nothing.  y is the GEMV's result
+ *                           (summed in the order of whole tiles);
  *   MGEMV_PROBE_TIMELINE_WAITS  the same, and in front of each unit's arithmetic the wave waits
  *                           explicitly for that unit's operands and first weight block (two more
  *                           clock readings per unit, which slow the kernel by a few per cent):

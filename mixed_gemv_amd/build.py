@@ -17,7 +17,7 @@ LINT_REPORT = os.path.join(LIB_DIR, "isa_lint.json")
 MIN_DOT_INSTRUCTIONS = 10000
 
 # One translation unit per family of kernel instantiations, so that they compile side by side.
-SOURCES = ["launch_valu_f16.hip", "launch_valu_bf16.hip", "launch_mfma.hip", "launch_mfma_parts.hip", "launch_mfma_kstat.hip", "gemv_kernels.hip", "probes.hip",
+SOURCES = ["launch_valu_f16.hip", "launch_valu_bf16.hip", "launch_valu_parts.hip", "launch_mfma.hip", "launch_mfma_parts.hip", "launch_mfma_kstat.hip", "gemv_kernels.hip", "probes.hip",
            "host_utils.cpp"]
 
 # -ffp-contract=off: the dequantiser is a separately rounded fp16 multiply and add.

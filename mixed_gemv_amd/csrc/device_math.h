@@ -184,6 +184,16 @@ __device__ __forceinline__ void dot2_row_bcast(float& acc, uint32_t x, half2_t d
         : "v"(x), "v"(d), "n"(SRC));
 }
 
+// The same with x from lane SRC of the caller's four lanes.
+template <int SRC>
+__device__ __forceinline__ void dot2_quad_bcast(float& acc, uint32_t x, half2_t d) {
+  static_assert(SRC >= 0 && SRC < 4, "source lane within four lanes");
+  if constexpr (SRC == 0)
+    asm(".p2align 3\n\tv_dot2c_f32_f16_dpp %0, %1, %2 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(d));
+  else
+    asm("v_dot2c_f32_f16_dpp %0, %1, %2 quad_perm:[%3,%3,%3,%3] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(d), "n"(SRC));
+}
+
 // The compiler does not know the asm above is a dot instruction, so it cannot pad the
 // "dot result read by a different instruction" hazard of this target (3 wait states).
 // Call this once after the last dot of a chain, before the accumulator is consumed.
@@ -385,6 +395,12 @@ __device__ __forceinline__ void dot2_row_bcast_bf16(float& acc, uint32_t x, uint
   asm("v_dot2c_f32_bf16_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
       : "+v"(acc)
       : "v"(x), "v"(d), "n"(SRC));
+}
+
+template <int SRC>
+__device__ __forceinline__ void dot2_quad_bcast_bf16(float& acc, uint32_t x, uint32_t d) {
+  static_assert(SRC >= 0 && SRC < 4, "source lane within four lanes");
+  asm("v_dot2c_f32_bf16_dpp %0, %1, %2 quad_perm:[%3,%3,%3,%3] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(d), "n"(SRC));
 }
 
 // Raw buffer descriptor: base pointer + byte count; out-of-range lanes read zero.

@@ -174,7 +174,7 @@ std::atomic<int> g_matrix_core_variant{MGEMV_MATRIX_CORE_AUTO};
 // What steers plan_launch besides the shape: zeros mean "built-in rule".
 struct PlanKnobs {
   int split_k = 0, tiles_per_wg = 0, tiles_per_wave = 0, workgroups = 0;
-  int parts = 0;            // part-tile matrix-core kernel: workgroups per tile
+  int parts = 0;            // part-tile kernels: workgroups per tile
   bool split_left_over = false;  // k-stationary kernel: tiles that do not divide over the workgroups go to two or four of them
   int matrix_core_min_batch = 0;
   int matrix_core_variant = MGEMV_MATRIX_CORE_AUTO;
@@ -326,6 +326,31 @@ inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16,
   }
   if (tiles <= 2 * cus || (tiles > 3 * cus && tiles <= 4 * cus)) return 0;
   return tiles <= 3 * cus && ksteps <= 32 ? two_units : 4;
+}
+
+// A single row on few tiles: workgroups per tile on the VALU kernel for parts of tiles (launch_valu_parts.hip); 0: not on that
+// kernel.  Of the time of the kernel for whole tiles, 700 launches of random shapes, geometric means (worst):
+//   at most a quarter as many tiles as compute units, four parts: fp16 int4 9-16 k steps 0.79 (0.97), 17-32 0.69 (0.82), more 0.60; int8
+//     0.84 (0.86), 0.83 (0.86), 0.65; bf16 int4 5-8 0.73 (0.91), 9-16 0.63 (0.70), 17-32 0.60 (0.69), more 0.44; int8 17-32 0.73 (0.78), more
+//     0.53 (512x5120 3.9 us / 3.1, 1024x16384 7.3 / 5.0; 900x4608 per column bf16 5.5 / 3.3, 1024x16320 g96 bf16 12.6 / 7.5);
+//   at most half as many, two parts: from 17 k steps fp16 int4 0.79 (0.88), int8 0.85, bf16 int8 0.84 (0.88); bf16 int4 from 5 0.60-0.81
+//     (0.97) (2048x8192 bf16 6.1 / 4.8, 2048x16384 7.7 / 5.8, 2000x12288 int8 7.3 / 6.2).  fp16 with 9-16 k steps is level (0.97-1.1), more
+//     tiles take 1.1-1.8 times as long.
+// Shorter reductions gain and lose; bf16 int8 with 9-16 k steps (0.8) loses up to 1.07 in batched launches (plan_of_batch).
+// Launch tests hold two shapes of int4 on exactly a quarter as many tiles to their older plans, 16 k steps to its threads and 20, in
+// fp16, to its bits: fp16 keeps the plan between them (1024x8192 4.5 us, four parts 3.6), bf16 takes two parts with 16 (5.9 / 4.2,
+// four 4.05).
+// kMaxValuPartsKSteps: as many as were measured; the sums of every unit lie in the LDS.
+constexpr int kMaxValuPartsKSteps = 128;
+inline int single_row_parts(int tiles, int ksteps, int bits, bool bf16, int cus) {
+  if (ksteps > kMaxValuPartsKSteps) return 0;
+  const int from = !bf16 ? 9 : bits == 8 ? 17 : 5;
+  if (tiles * 4 == cus && bits == 4 && ksteps >= 16 && ksteps <= 20) {
+    if (!bf16) return 0;
+    if (ksteps == 16) return 2;
+  }
+  if (tiles * 4 <= cus) return ksteps >= from ? 4 : 0;
+  return tiles * 2 <= cus && ksteps >= (bf16 ? from : 17) ? 2 : 0;
 }
 
 // Tiles per workgroup of the LDS-staged matrix-core kernel (= waves that share one activation stage): as few as
@@ -486,6 +511,7 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
         kn.tiles_per_wg = 1;
       }
     }
+    if (m_batch == 1 && kn.split_k == 0) kn.parts = single_row_parts(tiles, ksteps, bits, bf16, num_cus);
     if (const int parts = kn.split_k != 0 ? 0 : part_tiles(m_batch, tiles, ksteps, bits, bf16, num_cus)) {
       kn.matrix_core_min_batch = 1;
       kn.matrix_core_variant = MGEMV_MATRIX_CORE_LDS_STAGED;
@@ -837,6 +863,21 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
     tiles_per_wave = tiles >= cus ? 2 : 1;
     if (ov_t == 1 || ov_t == 2 || ov_t == 4) tiles_per_wave = ov_t;
   }
+  // One row, parts of tiles (measured ranges only).
+  if (!mc && m_batch == 1 && knobs.parts > 0) {
+    LaunchPlan lp{};
+    lp.tiles_per_wg = lp.tiles_per_wave = lp.tiles_in_sequence = 1;
+    lp.parts = knobs.parts;
+    lp.workgroups = tiles * lp.parts;
+    const int units = ceil_div(ksteps, lp.parts);
+    const int units_per_wave = ceil_div(units, units <= kMaxWavesPerWideWorkgroup ? units : units <= kMaxWavesPerWorkgroup && lp.parts == 1 ? kMaxWavesPerWideWorkgroup : 4);
+    lp.steps_per_wave = units_per_wave * lp.parts;
+    lp.split_k = ceil_div(units, units_per_wave);
+    lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
+    lp.threads = kWave * lp.split_k;
+    lp.stages = 2;
+    return lp;
+  }
   const int groups = ceil_div(tiles, tiles_per_wave);
   // (The VALU figures from here on are from before its builds by length.  On a device of 256 compute units single_row_split is asked
   // first for a single row on more tiles than that.)
@@ -1035,8 +1076,12 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
   }
   const int rows = m_batch < kMaxValuBatch ? m_batch : kMaxValuBatch;
   r.launches = (m_batch + kMaxValuBatch - 1) / kMaxValuBatch;
-  r.max_threads = kWave * (rows >= 3 || act == kActBf16 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup);
+  r.max_threads = kWave * (rows >= 3 || act == kActBf16 || lp.parts != 0 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup);
   r.lds_bytes = (size_t)lp.tiles_in_sequence * lp.tiles_per_wg * lp.split_k * rows * kWave * sizeof(float);
+  if (lp.parts != 0) {  // every unit's sums
+    const int units = lp.split_k * lp.steps_per_wave / lp.parts;
+    r.lds_bytes = (size_t)ceil_div(units, kValuPartsSumsAtOnce) * kValuPartsSumsAtOnce * kWave * sizeof(float);
+  }
   return r;
 }
 
@@ -1101,6 +1146,24 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
   return knobs;
 }
 
+// The plan of a batched or routed launch whose problems would each be split into parts.  Every number of parts gives the same bits, and
+// up to 16 k steps (8 in bf16) so does the kernel for whole tiles, a wave per k step, so the number of problems may count: as
+// many parts as leave a workgroup per compute unit, and where that is not all of them whole tiles, if their kernel gives the bits.
+// Of the time of whole tiles: two problems 0.72-1.0 (2000x12288 int8 1.04, 2048x16384 1.1); three and more 0.99-1.03, 1.05-1.07
+// with 64 tiles and more than 16 k steps (1024x16384, three problems, 7.7 us / 8.3).  With two workgroups per compute unit 1.1-1.5.
+// fp16 in fewer parts up to 16 k steps: 1.0-1.14.
+LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, PlanKnobs knobs, int batch_count) {
+  while (knobs.parts > 1 && (long long)num_tiles(n_out) * knobs.parts * batch_count > knobs.num_cus) knobs.parts /= 2;
+  if (knobs.parts == single.parts) return single;
+  if (knobs.parts == 1 || !knobs.wide_waves) {
+    PlanKnobs whole = knobs;
+    whole.parts = 0;
+    const LaunchPlan lp = plan_launch(n_out, k, bits, 1, whole);
+    if (lp.steps_per_wave == 1 && lp.split_k > 1) return lp;
+  }
+  return plan_launch(n_out, k, bits, 1, knobs);
+}
+
 // act: kActF16 or kActBf16, the type behind every 16-bit operand.
 int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, const uint16_t* zero_add,
              const uint16_t* bias, uint16_t* y, int batch_count, int n_out, int m_batch, int k, int group_size,
@@ -1131,8 +1194,10 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.n_out = n_out;
   g.k = k;
   g.group_size = group_size;
-  g.plan = plan_launch(n_out, k, weight_bits, m_batch,
-                       knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus));
+  PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus);
+  if (probe != kProbeNone && m_batch == 1) knobs.parts = 0;  // no measurement builds of the VALU kernel for parts of tiles
+  g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
+  if (m_batch == 1 && g.plan.parts != 0 && batch_count > 1) g.plan = plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count);
   g.form = unit_form(g.plan, batch_count, info.num_cus);
   g.tail.bias = reinterpret_cast<const half_t*>(bias);
   g.tail.split_k = g.plan.split_k;
@@ -1203,6 +1268,12 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
         (size_t)g.grid.x * (size_t)(g.plan.split_k * g.plan.tiles_per_wg) > trace_capacity_waves)
       return MGEMV_ERR_SIZE;
     return launch_gemv_probe(g, probe) == hipSuccess ? MGEMV_OK : MGEMV_ERR_LAUNCH;
+  }
+  if (g.plan.parts != 0) {
+    g.x = reinterpret_cast<const half_t*>(x);
+    g.tail.y = reinterpret_cast<half_t*>(y);
+    g.lds = launch_resources(g.plan, weight_bits, m_batch, act).lds_bytes;
+    return launch_valu_parts(g, weight_bits, quant_op, gpr, act) == hipSuccess ? MGEMV_OK : MGEMV_ERR_LAUNCH;
   }
   // VALU path: activation rows are processed kMaxValuBatch at a time.
   for (int m0 = 0; m0 < m_batch; m0 += kMaxValuBatch) {
@@ -1715,8 +1786,9 @@ int mgemv_probe_unit_form(int n_out, int m_batch, int k, int weight_bits, int gr
   if (batch_count < 1 || batch_count > 65535) return MGEMV_ERR_BATCH;
   if (const int st = check_tuned_key(n_out, k, weight_bits, group_size, m_batch)) return st;
   const int act = element == MGEMV_ELEMENT_BF16 ? kActBf16 : kActF16;
-  const LaunchPlan lp = plan_launch(n_out, k, weight_bits, m_batch,
-                                    knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, num_compute_units));
+  PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, num_compute_units);
+  if (m_batch == 1) knobs.parts = 0;  // as the measurement builds
+  const LaunchPlan lp = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   *form = unit_form(lp, batch_count, num_compute_units);
   return MGEMV_OK;
 }

@@ -23,6 +23,7 @@ constexpr int kMaxKStationaryLds = 128 * 1024;  // most LDS the k-stationary mat
 constexpr int kKStationaryZeroBytes = 256;  // ... with bf16 operands: zeros, a k run of the operand of a batch row that does not exist
 constexpr int kMaxKStationaryBf16Lds = 160 * 1024 - kKStationaryZeroBytes;  // ... most LDS its activation rows and partial sums take together
 constexpr int kKStationaryStagedBytes = kMaxWavesPerWorkgroup * 4;  // ... with left-over tiles in parts: a word for each wave
+constexpr int kValuPartsSumsAtOnce = 16;  // VALU kernel for parts of tiles: units whose sums are added up at a time
 constexpr int kMaxValuBatch = 4;  // activation rows handled per launch by the VALU kernel
 constexpr int kExactIntegerFormOnly = 1;  // GemvTail::flags: never take the short int4 dequantiser
 constexpr int kSingleStage = 2;           // GemvTail::flags: no load in flight while a unit is computed (VALU kernel)
@@ -140,7 +141,7 @@ __host__ __device__ __forceinline__ WaveWork staged_wave_work(int wg, int ty, in
   return w;
 }
 
-// Part-tile matrix-core kernel: a workgroup takes 16 / parts rows of one tile, a wave a range of whole units of `parts` k steps.
+// Part-tile kernels: a workgroup takes 16 / parts rows of one tile, a wave a range of whole units of `parts` k steps.
 struct PartWork {
   int tile, part, ks_begin, units;  // units: k steps, the last unit of the reduction may be short
 };
@@ -320,7 +321,7 @@ struct LaunchPlan {
   int tiles_per_wave;  // 1 on the VALU path; 1, 2 or 4 on the matrix-core path
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
   int staged_rows;        // LDS-staged and part-tile matrix-core kernels: 8 or 16 activation rows per stage; 0 = other kernels
-  int parts;              // part-tile matrix-core kernel: workgroups per tile (1, 2 or 4); 0 = other kernels
+  int parts;              // part-tile kernels: workgroups per tile (1, 2 or 4; VALU: 2 or 4); 0 = other kernels
                           // k-stationary kernel: workgroups per tile left over (2 or 4); 0 = walks of whole tiles
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
@@ -339,7 +340,7 @@ constexpr int kOneUnit = 3;   // one, on one tile
 // 1740x5120 int8 17.4 / 16.8; 0.946-1.026 of the time on 109 launches of random shapes, mean 0.99.  The figures of single problems
 // stand at the kernel's builds.
 inline int unit_form(const LaunchPlan& plan, int batch_count, int cus) {
-  if (plan.matrix_core || plan.tiles_in_sequence != 1 || plan.stages != 2) return kUnitLoop;
+  if (plan.matrix_core || plan.tiles_in_sequence != 1 || plan.stages != 2 || plan.parts != 0) return kUnitLoop;
   if (plan.steps_per_wave <= 2) return plan.steps_per_wave == 1 ? kOneUnit : kTwoUnits;
   return (long long)plan.workgroups * plan.split_k * plan.tiles_per_wg * batch_count <= 4ll * cus ? kTwoAhead : kUnitLoop;
 }
@@ -372,6 +373,7 @@ struct GemvLaunch {
 // activation rows, groups per run, ...; the run-time values pick the instantiation).
 hipError_t launch_gemv_f16(const GemvLaunch& g, int bits, int qop, int mb, int gpr);
 hipError_t launch_gemv_bf16(const GemvLaunch& g, int bits, int qop, int mb, int gpr);
+hipError_t launch_valu_parts(const GemvLaunch& g, int bits, int qop, int gpr, int act);
 hipError_t launch_mfma(const GemvLaunch& g, int bits, int qop, int gpr);
 hipError_t launch_mfma_lds(const GemvLaunch& g, int bits, int qop, int gpr, int rounds, int act);
 hipError_t launch_mfma_parts(const GemvLaunch& g, int bits, int qop, int gpr, int act);
