@@ -300,13 +300,18 @@ inline int lookups_per_run(int k, int group_size, int bits) {
 //   16.7 / 15.6; 0.94 on 790); with 14 it loses (20480x3584 12.9 / 13.8).
 // bf16 with a lookup per block, 9-16 k steps on 1.125 to 2 tiles per compute unit: up to eight waves instead of pairs of tiles
 //   (5052x4320 g96 9.65 / 8.39, 7936x7680 11.3 / 9.5, int8 5784x2304 7.6 / 6.05; 0.79-1.06 on 400); other group sizes gain and lose.
+// A lookup per block, half a tile to one tile per compute unit, 9-16 k steps, both types: eight waves of one or two units instead of four of
+//   three and four: both are requested at once, and nine k steps on four waves are 3 + 3 + 3 and a SIMD idle.  int4 0.92 of the time
+//   (0.74-1.04) on 185 (4096x8064 g96 6.37 / 6.16, in bf16 8.25 / 7.79), int8 0.86 (0.75-0.94) on 63 (3072x3072 g96 4.65 / 4.37); two to
+//   six problems 0.89-1.0.  Longer reductions take 0.85-0.96 alone and 1.05-1.2 in batched launches, with one or two lookups 0.9-1.2.
 // bf16, 1.5 to 2 tiles per compute unit and longer reductions: four waves per tile instead of pairs of tiles with two each, which leave a wave
 //   alone on every SIMD they have and some without one.  A lookup per block, from 18 k steps (17, as fast, is held by a launch test): 0.88 of the time (0.81-0.96) on 70 (8192x23040 g96
 //   33.2 / 30.4, int8 8192x16224 g96 33.9 / 28.8); int4 otherwise, from 25: 0.92 (0.74-1.03) on 130 (8192x27904 32.8 / 31.0, 8192x21248
 //   26.0 / 24.6; with 17-24 k steps 0.96, up to 1.03, left).  int8 otherwise 1.0-1.1, up to 1.5 tiles 1.03-1.3.
 inline int single_row_split(int tiles, int ksteps, int bits, int cus, bool bf16, int lookups) {
-  if (tiles <= cus || ksteps < 5) return 0;
   const bool generic_groups = lookups == 4;
+  if (generic_groups && tiles * 2 > cus && tiles <= cus && ksteps >= 9 && ksteps <= 16) return 8;
+  if (tiles <= cus || ksteps < 5) return 0;
   const bool fills_simds = tiles <= 4 * cus && tiles * 103 >= cus * 400;  // with a wave per tile
   if (bf16) {
     const bool two_per_cu = tiles * 8 >= cus * 9 && tiles <= 2 * cus && ksteps >= 9 && ksteps <= 16;
