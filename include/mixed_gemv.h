@@ -402,7 +402,9 @@ MGEMV_API int mgemv_default_plan_count(void);
 MGEMV_API int mgemv_tuned_plan_count(void);
 
 /* Reports the geometry mgemv_gemv would use for this problem (group_size as passed to mgemv_gemv,
- * k for per-column problems, 0 to consult only table entries for any group size):
+ * k for per-column problems, 0 to consult only table entries for any group size; a launch with scales by
+ * group and one group as long as k has the geometry of the per-column one, but it may keep a k-stationary
+ * workgroup's tiles whole where that one splits left-over tiles, with other LDS than out[8] below):
  * out[0] = workgroups, out[1] = threads per
  * workgroup, out[2] = k-split waves per tile, out[3] = tile sequences per workgroup,
  * out[4] = k steps per wave and tile, out[5] = 0 VALU kernel / 1 matrix-core kernel with the

@@ -1205,6 +1205,9 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.k = k;
   g.group_size = group_size;
   PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus);
+  const int gpr = groups_per_run(group_size, weight_bits);
+  // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
+  if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
   if (probe != kProbeNone && m_batch == 1) knobs.parts = 0;  // no measurement builds of the VALU kernel for parts of tiles
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   if (m_batch == 1 && g.plan.parts != 0 && batch_count > 1) g.plan = plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count);
@@ -1234,7 +1237,6 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.grid = dim3((unsigned)(g.plan.wgs_per_xcd * kNumXcd), 1, (unsigned)batch_count);
   g.block = dim3((unsigned)(kWave * g.plan.split_k), (unsigned)g.plan.tiles_per_wg, 1);
   g.stream = static_cast<hipStream_t>(stream);
-  const int gpr = groups_per_run(group_size, weight_bits);
 
   if (g.plan.matrix_core) {
     g.x = reinterpret_cast<const half_t*>(x);

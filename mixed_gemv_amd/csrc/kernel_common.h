@@ -378,6 +378,9 @@ hipError_t launch_mfma(const GemvLaunch& g, int bits, int qop, int gpr);
 hipError_t launch_mfma_lds(const GemvLaunch& g, int bits, int qop, int gpr, int rounds, int act);
 hipError_t launch_mfma_parts(const GemvLaunch& g, int bits, int qop, int gpr, int act);
 hipError_t launch_mfma_kstat(const GemvLaunch& g, int bits, int qop, int gpr, int act);
+// Which launches of the k-stationary kernel have a build for left-over tiles in parts; lookups: of scales per lane run, as launched.
+// (int8 gains nothing by it, and four lookups per run in fp16 have no registers for it.)
+constexpr bool kstat_has_left_over_parts(int bits, int lookups, int act) { return bits == 4 && (act == kActBf16 || lookups != 4); }
 // ... and of the k-stationary matrix-core kernel (kProbeLoadsOnly / kProbeComputeOnly), where they exist.
 bool mfma_kstat_probe_exists(int bits, int qop, int gpr, int act);
 hipError_t launch_mfma_kstat_probe(const GemvLaunch& g, int gpr, int probe);

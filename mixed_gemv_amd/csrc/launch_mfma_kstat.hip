@@ -471,8 +471,14 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
 
 template <int BITS, int QOP, int GPR, int ACT, int PROBE = kProbeNone, bool TAIL = false>
 hipError_t launch_mfma_kstat_kernel(const GemvLaunch& g) {
-  if constexpr (PROBE == kProbeNone && !TAIL && BITS == 4 && (ACT == kActBf16 || GPR != 4))  // (left_over_parts asks for no others)
-    if (g.plan.parts != 0) return launch_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE, true>(g);
+  if constexpr (!TAIL) {
+    if (g.plan.parts != 0) {  // whole tiles only would leave the rest of the matrix out, in stages of another size
+      if constexpr (PROBE == kProbeNone && kstat_has_left_over_parts(BITS, GPR, ACT))
+        return launch_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE, true>(g);
+      else
+        return hipErrorInvalidValue;
+    }
+  }
   const auto kernel = gemv_mfma_kstat_kernel<BITS, QOP, GPR, ACT, PROBE, TAIL>;
   if (g.lds > 48 * 1024) {
     // More than 48 KiB of dynamic LDS has to be granted per kernel and device; remember the

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import mixed_gemv_amd as mg
-from helpers import PER_COLUMN, SCALE_AND_ZEROS, SCALE_ONLY, DeviceProblem, Problem
+from helpers import PER_COLUMN, SCALE_AND_ZEROS, SCALE_ONLY, DeviceProblem, Problem, float64_bound_violations
 
 CASES = [
     # tiles, k steps, k short of whole steps by, quant_op, group, rows, bias, element, tiles' parts
@@ -122,3 +122,15 @@ def test_batched_and_routed_launches_have_the_bits_of_single_ones(gpu, case):
     mg.device_gemv_routed(w, x, scale, zero, b, y, route, 2, 2, n_out, rows, k, group, strides, qop, 4, element=element)
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy().view(np.uint16), np.stack([single[1]] * 2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qop", [SCALE_ONLY, SCALE_AND_ZEROS])
+@pytest.mark.parametrize("n_out, k, rows", [(5004, 4640, 4), (9596, 4640, 8)])
+def test_one_group_as_long_as_the_reduction(gpu, n_out, k, rows, qop):
+    """Plans take such a group for the per-column mode, whose left-over tiles go in parts; by group the fp16 launch looks four scales
+    up per run, for which no such build exists: every output is there all the same."""
+    assert covered_in_parts(n_out, rows, k, 4, k, "f16")
+    prob = Problem("one group", n_out, k, 4, qop, k, m_batch=rows, bias=True)
+    y = DeviceProblem(prob, gpu).run()
+    assert float64_bound_violations(prob, y)[0] == 0
