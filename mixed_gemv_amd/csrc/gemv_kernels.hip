@@ -1207,7 +1207,8 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus);
   const int gpr = groups_per_run(group_size, weight_bits);
   // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
-  if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
+  // Nor do the measurement builds have parts.
+  if (probe != kProbeNone || !kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
   if (probe != kProbeNone && m_batch == 1) knobs.parts = 0;  // no measurement builds of the VALU kernel for parts of tiles
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   if (m_batch == 1 && g.plan.parts != 0 && batch_count > 1) g.plan = plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count);

@@ -105,6 +105,22 @@ def test_matrix_core_measurement_builds_run(gpu, m_batch):
             mg.probe_gemv_rows(mg.PROBE_TIMELINE, m_batch, dev.w, dev.x, dev.scale, dev.zero, dev.y, n_out, k, 64)
 
 
+@pytest.mark.parametrize("n_out, k, m_batch", [(4608, 8192, 4), (9596, 4608, 8)])   # 32 and 88 tiles more than walks of one and two
+def test_measurement_builds_walk_left_over_tiles_whole(gpu, n_out, k, m_batch):
+    """The product takes left-over tiles of the k-stationary kernel in parts, which its measurement builds do not have: they take every
+    tile whole, in stages of their own size."""
+    import torch
+    prob = Problem("probe_left_over", n_out, k, 4, SCALE_AND_ZEROS, 128, m_batch=m_batch, x_dist="normal")
+    dev = DeviceProblem(prob, gpu)
+    assert mg.query_launch(n_out, m_batch, k, 4, 128)["matrix_core"] == 3
+    assert mg.plan_coverage(n_out, m_batch, k, 4, 128)["max_units_per_wave"] < -(-n_out // 16 // 256)     # in parts
+    for kind in (mg.PROBE_LOADS_ONLY, mg.PROBE_COMPUTE_ONLY):
+        dev.y.fill_(0x7e00)
+        mg.probe_gemv_rows(kind, m_batch, dev.w, dev.x, dev.scale, dev.zero, dev.y, n_out, k, 128)
+        torch.cuda.synchronize()
+        assert not np.any(dev.y.cpu().numpy().view(np.uint16) == 0x7e00)
+
+
 def test_stream_read_and_empty_launch_run_and_check_their_arguments(gpu):
     import torch
     buf = torch.zeros(8 << 20, dtype=torch.uint8, device=gpu)
