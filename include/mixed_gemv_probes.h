@@ -79,7 +79,8 @@ MGEMV_API int mgemv_probe_gemv(int kind, unsigned long long *trace, size_t trace
                                int group_size, void *stream);
 
 /* The same two builds -- MGEMV_PROBE_LOADS_ONLY, MGEMV_PROBE_COMPUTE_ONLY -- for a launch of m_batch
- * activation rows, where they exist: one row as above; on the matrix cores the LDS-staged kernel whose
+ * activation rows on whole tiles (where the product takes tiles in parts, as it would without those; see above), where they
+ * exist: one row as above; on the matrix cores the LDS-staged kernel whose
  * workgroups share their activation stage between two or more tiles (int4, scale and zero, fp16,
  * group sizes 64-512; e.g. 8192 x 8192 at 8-16 rows), and the k-stationary kernel (same operand types;
  * e.g. 28672 x 8192 at 2-16 rows).  On the LDS-staged kernel "loads only" keeps the staging of the

@@ -484,8 +484,8 @@ inline int part_tiles(int m_batch, int tiles, int ksteps, int bits, bool bf16, i
 
 // Process-wide overrides win over the tables (they are what a tuner sweeps); then the caller's
 // entry for exactly this group size, then its entry for any group size, then the built-in table and
-// the measured ranges, then the built-in rules.
-PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus) {
+// the measured ranges, then the built-in rules.  whole_tiles: nothing in parts (the measurement builds, which have none).
+PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus, bool whole_tiles) {
   PlanKnobs kn;
   kn.split_k = g_override_split_k.load();
   kn.tiles_per_wg = g_override_tiles_per_wg.load();
@@ -512,7 +512,7 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
     const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
     const bool bf16 = act == kActBf16;
     const int lookups = lookups_per_run(k, group_size, bits);
-    kn.split_left_over = true;
+    kn.split_left_over = !whole_tiles;
     if (m_batch == 1 || (m_batch == 2 && bits == 8 && !bf16)) {
       const int split = m_batch == 1 ? single_row_split(tiles, ksteps, bits, num_cus, bf16, lookups)
                                      : two_int8_rows_split(tiles, ksteps, num_cus);
@@ -521,8 +521,9 @@ PlanKnobs knobs_for(int n_out, int k, int bits, int group_size, int m_batch, int
         kn.tiles_per_wg = 1;
       }
     }
-    if (m_batch == 1 && kn.split_k == 0) kn.parts = single_row_parts(tiles, ksteps, bits, bf16, num_cus);
-    if (const int parts = kn.split_k != 0 ? 0 : part_tiles(m_batch, tiles, ksteps, bits, bf16, num_cus)) {
+    const bool in_parts = !whole_tiles && kn.split_k == 0;
+    if (in_parts && m_batch == 1) kn.parts = single_row_parts(tiles, ksteps, bits, bf16, num_cus);
+    if (const int parts = in_parts ? part_tiles(m_batch, tiles, ksteps, bits, bf16, num_cus) : 0) {
       kn.matrix_core_min_batch = 1;
       kn.matrix_core_variant = MGEMV_MATRIX_CORE_LDS_STAGED;
       kn.parts = parts;
@@ -1141,8 +1142,8 @@ int device_info(int device, DeviceInfo& info) {
 }
 
 // The knobs of a problem with the element type taken into account.
-PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus = kNumCus) {
-  PlanKnobs knobs = knobs_for(n_out, k, bits, group_size, m_batch, act, num_cus);
+PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_batch, int act, int num_cus = kNumCus, bool whole_tiles = false) {
+  PlanKnobs knobs = knobs_for(n_out, k, bits, group_size, m_batch, act, num_cus, whole_tiles);
   knobs.num_cus = num_cus;
   // (a group as long as k is the per-column mode, whose kernels look one scale up per row)
   knobs.generic_groups = lookups_per_run(k, group_size, bits) == 4;
@@ -1204,12 +1205,10 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   g.n_out = n_out;
   g.k = k;
   g.group_size = group_size;
-  PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus);
+  PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, info.num_cus, probe != kProbeNone);
   const int gpr = groups_per_run(group_size, weight_bits);
   // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
-  // Nor do the measurement builds have parts.
-  if (probe != kProbeNone || !kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
-  if (probe != kProbeNone && m_batch == 1) knobs.parts = 0;  // no measurement builds of the VALU kernel for parts of tiles
+  if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   if (m_batch == 1 && g.plan.parts != 0 && batch_count > 1) g.plan = plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count);
   g.form = unit_form(g.plan, batch_count, info.num_cus);
@@ -1799,9 +1798,9 @@ int mgemv_probe_unit_form(int n_out, int m_batch, int k, int weight_bits, int gr
   if (batch_count < 1 || batch_count > 65535) return MGEMV_ERR_BATCH;
   if (const int st = check_tuned_key(n_out, k, weight_bits, group_size, m_batch)) return st;
   const int act = element == MGEMV_ELEMENT_BF16 ? kActBf16 : kActF16;
-  PlanKnobs knobs = knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, num_compute_units);
-  if (m_batch == 1) knobs.parts = 0;  // as the measurement builds
-  const LaunchPlan lp = plan_launch(n_out, k, weight_bits, m_batch, knobs);
+  // a single row on whole tiles, as the measurement builds have it
+  const LaunchPlan lp = plan_launch(n_out, k, weight_bits, m_batch,
+                                    knobs_for_element(n_out, k, weight_bits, group_size, m_batch, act, num_compute_units, m_batch == 1));
   *form = unit_form(lp, batch_count, num_compute_units);
   return MGEMV_OK;
 }

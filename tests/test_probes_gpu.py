@@ -121,6 +121,21 @@ def test_measurement_builds_walk_left_over_tiles_whole(gpu, n_out, k, m_batch):
         assert not np.any(dev.y.cpu().numpy().view(np.uint16) == 0x7e00)
 
 
+@pytest.mark.parametrize("n_out, k, m_batch", [(2048, 5120, 3), (2048, 4096, 5)])
+def test_measurement_builds_where_the_product_takes_parts_of_tiles(gpu, n_out, k, m_batch):
+    """The part-tile kernel has no measurement builds: those of the kernel for whole tiles answer, here the k-stationary one."""
+    import torch
+    assert mg.query_launch(n_out, m_batch, k, 4, 128)["matrix_core"] == 2
+    assert mg.query_launch(n_out, m_batch, k, 4, 128)["tiles_per_wg"] == 1     # the part-tile kernel
+    prob = Problem("probe_parts", n_out, k, 4, SCALE_AND_ZEROS, 128, m_batch=m_batch, x_dist="normal")
+    dev = DeviceProblem(prob, gpu)
+    for kind in (mg.PROBE_LOADS_ONLY, mg.PROBE_COMPUTE_ONLY):
+        dev.y.fill_(0x7e00)
+        mg.probe_gemv_rows(kind, m_batch, dev.w, dev.x, dev.scale, dev.zero, dev.y, n_out, k, 128)
+        torch.cuda.synchronize()
+        assert not np.any(dev.y.cpu().numpy().view(np.uint16) == 0x7e00)
+
+
 def test_stream_read_and_empty_launch_run_and_check_their_arguments(gpu):
     import torch
     buf = torch.zeros(8 << 20, dtype=torch.uint8, device=gpu)
