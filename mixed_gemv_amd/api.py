@@ -482,6 +482,9 @@ KERNEL_MATRIX_CORE_LDS_STAGED = 3
 KERNEL_MATRIX_CORE_K_STATIONARY = 4
 
 
+_tuned_plans = {}  # (n_out, k, weight_bits, group_size, m_batch, bf16) -> the other arguments of set_tuned_plan
+
+
 def set_tuned_plan(n_out, k, weight_bits, group_size, m_batch, kernel=KERNEL_AUTO, split_k=0, tiles_per_wg=0,
                    tiles_per_wave=0, max_workgroups=0, stages=0, element="f16"):
     """Installs the launch plan for exactly this problem and element type; see mgemv_tuned_plan_set
@@ -490,6 +493,8 @@ def set_tuned_plan(n_out, k, weight_bits, group_size, m_batch, kernel=KERNEL_AUT
                                int(split_k), int(tiles_per_wg), int(tiles_per_wave), int(max_workgroups), int(stages),
                                1 if _is_bf16(element, None) else 0)
     _lib.check(_lib.lib().mgemv_tuned_plan_set(ctypes.byref(plan)), "set_tuned_plan")
+    _tuned_plans[(*plan[:5], plan[11])] = dict(kernel=plan[5], split_k=plan[6], tiles_per_wg=plan[7], tiles_per_wave=plan[8],
+                                               max_workgroups=plan[9], stages=plan[10])
 
 
 def erase_tuned_plan(n_out, k, weight_bits, group_size, m_batch, element="f16"):
@@ -497,6 +502,7 @@ def erase_tuned_plan(n_out, k, weight_bits, group_size, m_batch, element="f16"):
     plan = (ctypes.c_int * 12)(int(n_out), int(k), int(weight_bits), int(group_size), int(m_batch), 0, 0, 0, 0, 0, 0,
                                1 if _is_bf16(element, None) else 0)
     _lib.check(_lib.lib().mgemv_tuned_plan_erase(ctypes.byref(plan)), "erase_tuned_plan")
+    _tuned_plans.pop((*plan[:5], plan[11]), None)
 
 
 def set_default_plans(enable=True):
@@ -510,6 +516,7 @@ def default_plan_count():
 
 def clear_tuned_plans():
     _lib.check(_lib.lib().mgemv_tuned_plan_clear(), "clear_tuned_plans")
+    _tuned_plans.clear()
 
 
 def tuned_plan_count():

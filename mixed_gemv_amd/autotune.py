@@ -12,6 +12,7 @@ Timing is cold-cache: weight / scale / zero sets are rotated so that more than t
 Infinity Cache is touched between two uses of a set, the launches are replayed from a HIP
 graph, and the kernel time is taken with an event pair on the launch stream.
 """
+import contextlib
 import json
 import time
 
@@ -23,6 +24,9 @@ _KERNEL_NAMES = {api.KERNEL_AUTO: "auto", api.KERNEL_VALU: "valu",
                  api.KERNEL_MATRIX_CORE_LDS_STAGED: "matrix_core_lds_staged",
                  api.KERNEL_MATRIX_CORE_K_STATIONARY: "matrix_core_k_stationary"}
 _installed = {}  # key tuple -> entry dict, what save_table writes
+
+
+_BUILTIN = dict(builtin=True)  # what a launch takes without an override or an entry of its own; set_tuned_plan cannot say it
 
 
 def candidate_plans(n_out, k, weight_bits, m_batch):
@@ -133,15 +137,37 @@ def erase(key):
     _installed.pop(key, None)
 
 
+@contextlib.contextmanager
+def _without_entry(key):
+    """The library's table without the entry of this key; one that was there comes back afterwards."""
+    knobs = api._tuned_plans.get((*key[:5], 1 if key[5] == "bf16" else 0))
+    api.erase_tuned_plan(*key[:5], element=key[5])
+    try:
+        yield
+    finally:
+        if knobs is not None:
+            api.set_tuned_plan(*key[:5], **knobs, element=key[5])
+
+
+def _plan(key, num_compute_units):
+    """What a launch of this key does now: the reported geometry, and that with what else tells two plans apart (left-over
+    tiles whole or in parts)."""
+    args = (key[0], key[4], key[1], key[2], key[3])
+    geometry = api.query_launch(*args, element=key[5], num_compute_units=num_compute_units)
+    coverage = api.plan_coverage(*args, element=key[5], num_compute_units=num_compute_units)
+    return geometry, (*sorted(geometry.items()), coverage["max_units_per_wave"])
+
+
 def tune(n_out, k, weight_bits=4, quant_op=api.WeightOnlyQuantOp.FINEGRAINED_SCALE_AND_ZEROS, group_size=128,
          m_batch=1, bias=False, device="cuda:0", launches=400, rounds=2, min_gain=0.02, seed=1,
          cold_bytes=_CACHE_BYTES, log=None, element="f16"):
     """Measures the candidate plans for this problem and installs the fastest, unless it beats the
     built-in plan by less than `min_gain` (then the key ends up without an entry: one left by an
-    earlier run is removed, since the built-in plan has just been measured to be as good).  Every
-    candidate, the built-in plan included, is measured with a process-wide override set, which
-    makes the library ignore the table, so an entry that already exists never stands in for the
-    built-in plan.  Returns a
+    earlier run is removed, since the built-in plan has just been measured to be as good).  The
+    built-in plan is what a launch takes without an override and without an entry of this key, which
+    is out of the table meanwhile: the library's measured plans and ranges, parts of tiles among them,
+    which no entry can ask for (or the caller's entry for any group size).  The candidates are measured
+    with a process-wide override set, which makes the library ignore the table.  Returns a
     dict with the chosen entry (or None), the built-in time and every measurement.  `cold_bytes`
     is how much operand data is rotated between two uses of the same buffers (default: more than
     the Infinity Cache).  `element` ("f16" / "bf16") picks the entry points that are timed; an entry
@@ -157,24 +183,23 @@ def tune(n_out, k, weight_bits=4, quant_op=api.WeightOnlyQuantOp.FINEGRAINED_SCA
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     prob = _Problem(n_out, k, weight_bits, api.WeightOnlyQuantOp(quant_op), key[3], m_batch, bias, device, seed,
                     cold_bytes, element)
-    seen, results = {}, []
+    seen, results = set(), []
     try:
-        with torch.cuda.device(device):
-            _apply(dict(kernel=api.KERNEL_AUTO))
+        with torch.cuda.device(device), _without_entry(key):
+            _apply(_BUILTIN)
             spin = time.perf_counter()
             while time.perf_counter() - spin < 0.5:  # an idle device needs a while to reach its clocks
                 prob.time_us(launches)
-            for cand in candidate_plans(n_out, k, weight_bits, m_batch):
+            for cand in [_BUILTIN, *candidate_plans(n_out, k, weight_bits, m_batch)]:
                 _apply(cand)
-                geometry = tuple(sorted(api.query_launch(n_out, m_batch, k, weight_bits, key[3], element=element,
-                                                         num_compute_units=cus).items()))
-                if geometry in seen:
+                geometry, plan = _plan(key, cus)
+                if plan in seen:
                     continue
-                seen[geometry] = cand
+                seen.add(plan)
                 us = min(prob.time_us(launches) for _ in range(rounds))
-                results.append((us, cand, dict(geometry)))
+                results.append((us, cand, geometry))
                 if log:
-                    log(f"{us:8.2f} us  {_describe(cand)}  -> {dict(geometry)}")
+                    log(f"{us:8.2f} us  {_describe(cand)}  -> {geometry}")
             builtin_us = results[0][0]
             best_us, best, best_geometry = min(results, key=lambda r: r[0])
             if best is not results[0][1]:
@@ -185,8 +210,7 @@ def tune(n_out, k, weight_bits=4, quant_op=api.WeightOnlyQuantOp.FINEGRAINED_SCA
                     _apply(best)
                     best_us = min(best_us, prob.time_us(launches))
     finally:
-        _apply(dict(kernel=api.KERNEL_AUTO))
-        api.set_prefetch_stages(0)
+        _apply(_BUILTIN)
     entry = None
     if best is not results[0][1] and best_us < builtin_us * (1.0 - min_gain):
         entry = dict(n_out=key[0], k=key[1], weight_bits=key[2], group_size=key[3], m_batch=key[4],
@@ -203,9 +227,9 @@ def tune(n_out, k, weight_bits=4, quant_op=api.WeightOnlyQuantOp.FINEGRAINED_SCA
 
 
 def reconfirm(entry, device="cuda:0", launches=400, rounds=5, seed=1, cold_bytes=_CACHE_BYTES, quant_op=None, bias=False):
-    """Measures an existing table entry against the built-in plan once more, in alternation, on the
-    device at hand, and appends the gain in per cent (positive: the entry is ahead) to
-    entry["confirmations"].  A gain found on one machine at one time can be that machine's: boxes of
+    """Measures an existing table entry against the built-in plan once more (as in tune(); an entry that the library ships
+    against its rules), in alternation, on the device at hand, and appends the gain in per cent (positive: the entry is
+    ahead) to entry["confirmations"].  A gain found on one machine at one time can be that machine's: boxes of
     the same kind differ by several per cent among themselves (28672 x 8192: 22.4-24.4 us from lease
     to lease), so an entry should only ship after `confirmed()` -- the gain shown again on another
     lease.  Returns the gain.  Like tune(), must not run while other threads launch GEMVs."""
@@ -222,20 +246,25 @@ def reconfirm(entry, device="cuda:0", launches=400, rounds=5, seed=1, cold_bytes
     if entry.get("stages"):
         cand["stages"] = entry["stages"]
     builtin, tuned = [], []
+    key = _entry_key(entry)
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
     try:
-        with torch.cuda.device(device):
-            _apply(dict(kernel=api.KERNEL_AUTO))
+        with torch.cuda.device(device), _without_entry(key):
+            _apply(cand)
+            own = _plan(key, cus)
+            _apply(_BUILTIN)
+            base = dict(kernel=api.KERNEL_AUTO) if _plan(key, cus) == own else _BUILTIN
+            _apply(base)
             spin = time.perf_counter()
             while time.perf_counter() - spin < 0.5:
                 prob.time_us(launches)
             for _ in range(rounds):
-                _apply(dict(kernel=api.KERNEL_AUTO))
+                _apply(base)
                 builtin.append(prob.time_us(launches))
                 _apply(cand)
                 tuned.append(prob.time_us(launches))
     finally:
-        _apply(dict(kernel=api.KERNEL_AUTO))
-        api.set_prefetch_stages(0)
+        _apply(_BUILTIN)
     gain = round(100.0 * (statistics.median(builtin) / statistics.median(tuned) - 1.0), 2)
     entry.setdefault("confirmations", []).append(gain)
     return gain
@@ -250,7 +279,8 @@ def confirmed(entry, min_gain=0.02, leases=2):
 
 def _apply(cand):
     kernel = cand.get("kernel", api.KERNEL_AUTO)
-    api.set_prefetch_stages(cand.get("stages", 2))  # 2 is the built-in value; any override set bypasses the table
+    # 2 is the built-in value; any override set bypasses the table and the measured ranges
+    api.set_prefetch_stages(0 if cand.get("builtin") else cand.get("stages", 2))
     api.set_launch_override(cand.get("split_k", 0), cand.get("tiles_per_wg", 0), cand.get("tiles_per_wave", 0),
                             cand.get("max_workgroups", 0))
     api.set_matrix_core_threshold({api.KERNEL_AUTO: 0, api.KERNEL_VALU: 17}.get(kernel, 1))
@@ -261,6 +291,8 @@ def _apply(cand):
 
 
 def _describe(cand):
+    if cand.get("builtin"):
+        return "builtin"
     knobs = ", ".join(f"{k}={v}" for k, v in cand.items() if k != "kernel" and v)
     return f"{_KERNEL_NAMES[cand.get('kernel', 0)]}({knobs})"
 
