@@ -411,7 +411,7 @@ MGEMV_API int mgemv_tuned_plan_count(void);
  * activation operand in registers / 2 LDS-staged matrix-core kernel / 3 k-stationary matrix-core kernel,
  * out[6] = tiles per wave (matrix-core path), out[7] = most tiles a wave walks one after the
  * other (VALU and k-stationary kernels).  Where workgroups share a tile, each taking a part of its rows,
- * out[0] counts all of them.  A batched or routed launch of one row may take fewer parts; its results are the same. */
+ * out[0] counts all of them.  A batched or routed launch may take fewer parts; its results are the same. */
 MGEMV_API int mgemv_query_launch(int n_out, int m_batch, int k, int weight_bits, int group_size, int out[8]);
 /* mgemv_query_launch assumes an unpartitioned MI355X (256 compute units); a launch plans for the
  * compute units of the device its stream belongs to.

@@ -460,7 +460,7 @@ void set_multi_row_ranges(PlanKnobs& kn, int m_batch, int tiles, int ksteps, int
 //     pairs of tiles fill the machine badly, 2 to 3 tiles per compute unit 0.87 (bf16 4 to 5 as well, 0.92).  Elsewhere 0.95-1.4.
 // Fewer than 5 k steps gain less, and launch tests hold such shapes to their older plans, as they hold: 3 and 4 rows of int8 on more than
 // a quarter as many tiles up to 17 k steps (0.85-0.91 here), bf16 on exactly half as many up to 8 (0.80-0.88) and two bf16 rows on
-// 112-127 (16 k steps) and 128 tiles.  9-16 fp16 rows of up to 8 k steps on few tiles (0.94) keep the rules' plan for the same reason.
+// 112-127 (16 k steps) and 128 tiles.  (Several problems: plan_of_batch_rows.)  9-16 fp16 rows of up to 8 k steps on few tiles (0.94) keep the rules' plan for the same reason.
 inline int part_tiles(int m_batch, int tiles, int ksteps, int bits, bool bf16, int cus) {
   if (m_batch < 2 || tiles < 2 || ksteps < (m_batch == 2 && bits == 8 ? 8 : 5)) return 0;
   if (tiles * 4 <= cus && m_batch <= 4) return 4;
@@ -1079,7 +1079,8 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
       const int row_stride = step_k(bits) * 2 + 16;
       // (a wave of the part-tile kernel has one stage, its own)
       r.lds_bytes = (size_t)lp.split_k * (lp.parts != 0 ? 1 : 2) * lp.staged_rows * row_stride +
-                    (lp.split_k > 1 || lp.parts > 1 ? (size_t)lp.tiles_per_wg * lp.split_k * kWave * 4 * sizeof(float) : 0);
+                    (lp.split_k > 1 || lp.parts > 1 || lp.chains != 0
+                         ? (size_t)lp.tiles_per_wg * lp.split_k * (lp.chains != 0 ? lp.chains_per_wave : 1) * kWave * 4 * sizeof(float) : 0);
     } else {
       r.lds_bytes = lp.split_k == 1 ? 0 : (size_t)lp.tiles_per_wg * lp.split_k * lp.tiles_per_wave * kWave * 4 * sizeof(float);
     }
@@ -1157,6 +1158,14 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
   return knobs;
 }
 
+// As many parts, at most the single launch's, as leave a workgroup per compute unit when all problems are taken together.  A problem's
+// workgroups are dealt out to the XCDs in equal numbers (the last XCD gets what is left), so each XCD is looked at: six problems of
+// 42 workgroups are 36 for the 32 compute units of seven XCDs, and none for the eighth (328x7168 at 8 rows 8.0 us; 21 each 6.0).
+int parts_of_batch(int parts, int tiles, int cus, int batch_count) {
+  while (parts > 1 && (long long)ceil_div(tiles * parts, kNumXcd) * kNumXcd * batch_count > cus) parts /= 2;
+  return parts;
+}
+
 // The plan of a batched or routed launch whose problems would each be split into parts.  Every number of parts gives the same bits, and
 // up to 16 k steps (8 in bf16) so does the kernel for whole tiles, a wave per k step, so the number of problems may count: as
 // many parts as leave a workgroup per compute unit, and where that is not all of them whole tiles, if their kernel gives the bits.
@@ -1164,7 +1173,7 @@ PlanKnobs knobs_for_element(int n_out, int k, int bits, int group_size, int m_ba
 // with 64 tiles and more than 16 k steps (1024x16384, three problems, 7.7 us / 8.3).  With two workgroups per compute unit 1.1-1.5.
 // fp16 in fewer parts up to 16 k steps: 1.0-1.14.
 LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, PlanKnobs knobs, int batch_count) {
-  while (knobs.parts > 1 && (long long)num_tiles(n_out) * knobs.parts * batch_count > knobs.num_cus) knobs.parts /= 2;
+  knobs.parts = parts_of_batch(knobs.parts, num_tiles(n_out), knobs.num_cus, batch_count);
   if (knobs.parts == single.parts) return single;
   if (knobs.parts == 1 || !knobs.wide_waves) {
     PlanKnobs whole = knobs;
@@ -1173,6 +1182,28 @@ LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, P
     if (lp.steps_per_wave == 1 && lp.split_k > 1) return lp;
   }
   return plan_launch(n_out, k, bits, 1, knobs);
+}
+
+// The same for two and more rows on the part-tile matrix-core kernel, in the order of the single launch's sums (CHAINS).  Whole
+// chains to eight waves where all problems leave a compute unit to each workgroup, else to four: eight there 1.0-1.2 of the
+// time, two 1.1-1.5 (and level from 2 workgroups per compute unit on).
+// Two to eight problems of at most half as many tiles as compute units, 1445 launches of random shapes, of the time of the
+// kernels that were there before parts: 0.89 (39 of them above 1.1, worst 1.26; 2 rows 0.93, 3 and 4 0.84, 5-8 0.93), where the
+// single launch's parts took up to 2.2 (eight problems of 1024x9344 at 3 rows in bf16 14.1 us before, 30.8 in four parts each, 12.3
+// here; of 2048x4352 at 8 rows 11.8, 24.5, 12.0).  Two rows of short reductions gain least: the VALU kernel had them.
+LaunchPlan plan_of_batch_rows(const LaunchPlan& single, int m_batch, int tiles, int cus, int batch_count) {
+  LaunchPlan lp = single;
+  lp.parts = parts_of_batch(single.parts, tiles, cus, batch_count);
+  if (lp.parts == single.parts) return single;
+  lp.chains = single.parts / lp.parts;
+  lp.workgroups = tiles * lp.parts;
+  const int chains = single.split_k * lp.chains, waves = (long long)lp.workgroups * batch_count <= cus ? kMaxWavesPerMfmaWorkgroup : 4;
+  lp.chains_per_wave = ceil_div(chains, waves);
+  lp.split_k = ceil_div(chains, lp.chains_per_wave);
+  lp.staged_rows = lp.parts * m_batch <= 4 && lp.parts == 1 ? 4 : 8;
+  lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
+  lp.threads = kWave * lp.split_k;
+  return lp;
 }
 
 // act: kActF16 or kActBf16, the type behind every 16-bit operand.
@@ -1210,7 +1241,9 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
   if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
-  if (m_batch == 1 && g.plan.parts != 0 && batch_count > 1) g.plan = plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count);
+  if (batch_count > 1 && g.plan.parts != 0 && !g.plan.k_stationary)
+    g.plan = m_batch == 1 ? plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count)
+                          : plan_of_batch_rows(g.plan, m_batch, num_tiles(n_out), info.num_cus, batch_count);
   g.form = unit_form(g.plan, batch_count, info.num_cus);
   g.tail.bias = reinterpret_cast<const half_t*>(bias);
   g.tail.split_k = g.plan.split_k;

@@ -323,6 +323,8 @@ struct LaunchPlan {
   int staged_rows;        // LDS-staged and part-tile matrix-core kernels: 8 or 16 activation rows per stage; 0 = other kernels
   int parts;              // part-tile kernels: workgroups per tile (1, 2 or 4; VALU: 2 or 4); 0 = other kernels
                           // k-stationary kernel: workgroups per tile left over (2 or 4); 0 = walks of whole tiles
+  int chains, chains_per_wave;  // part-tile matrix-core kernel, batched launches in fewer parts than a single one (else 0): the single
+                          // launch's parts are parts * chains, split_k waves take chains_per_wave chains of units each
   int stages;             // VALU path: 2 = the next unit is in flight while one is computed, 1 = it is not
   bool matrix_core;       // one of the matrix-core kernels (else the VALU kernel)
   bool k_stationary;      // the matrix-core kernel whose waves keep one k step each while the workgroup walks tiles_in_sequence tiles

@@ -31,12 +31,12 @@ namespace mgemv {
 // weights per unit, which the L2 hands a compute unit at 85 GB/s, behind weights at 40-60: per unit 0.29 us at 16 rows, 0.20 of it x
 // (0.10 without x and arithmetic), 0.23 at 4 rows, where the arithmetic (0.2) takes over.  Eight waves are therefore no faster
 // than four beyond one unit each, and two parts no faster than one once every compute unit has a workgroup.
-// ROWS: activation rows staged per unit and wave, 8 or 16, at least PARTS * m_batch (row b at k step s + p is number
+// ROWS: activation rows staged per unit and wave, 4 (CHAINS > 1), 8 or 16, at least PARTS * m_batch (row b at k step s + p is number
 // b * PARTS + p).
 // It replaces nothing in the reference, whose kernel is fixed to one activation row
 // (gemv/threadblock/default_mma_core_simt.h:68-70); the dequantiser is the one of every kernel here
 // (gemv/warp/warp_dequantizer.h:52-59, 86-92), the epilogue host/mixed_gemv.h:102-103.
-// blockDim = 64 * split_k.  Dynamic LDS: split_k stages of ROWS x kRowStride bytes, then split_k * 256 floats.
+// blockDim = 64 * split_k.  Dynamic LDS: split_k stages of ROWS x kRowStride bytes, then split_k * chains_per_wave * 256 floats.
 // ---------------------------------------------------------------------------------------------
 // Byte offsets of the activation rows, in scalar registers; rows that do not exist lie past the descriptor.
 constexpr uint32_t kPastActivations = 0x80000000u;  // m_batch * k * 2 bytes are fewer
@@ -68,7 +68,12 @@ __device__ __forceinline__ void fetch_part_rows(XRows<BITS, ROWS>& r, const RowO
   }
 }
 
-template <int BITS, int QOP, int GROUPS_PER_RUN, int ROWS, int PARTS, int ACT>
+// CHAINS > 1 (batched and routed launches in fewer parts than a single one: plan_of_batch_rows): the bits of the single launch, whose
+// parts are PARTS * CHAINS.  A wave of that one adds its products up along `parts` chains at once, chain c the k steps of its range that are
+// c modulo the parts; here a unit holds PARTS of them, CHAINS units come to the same k steps, and a wave takes chains_per_wave
+// whole chains of units one after the other, whichever range they are of, and parks each one's sums as the single launch's
+// wave does.
+template <int BITS, int QOP, int GROUPS_PER_RUN, int ROWS, int PARTS, int ACT, int CHAINS = 1>
 __global__ void __launch_bounds__(kWave * kMaxWavesPerMfmaWorkgroup)
 gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out,
                        int k, uint32_t packed_steps, int workgroups, int num_groups, uint32_t packed_group, GemvTail tail) {
@@ -89,12 +94,16 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   p.wgs_per_xcd = (workgroups + kNumXcd - 1) / kNumXcd;
   p.group_size = (int)(packed_group & 0xffffffu);
   p.tiles_per_wg = 1;
+  constexpr bool kChained = CHAINS > 1;
+  const int chains_per_wave = kChained ? tiles_per_wg_of(packed_group) : 1;  // in the place of the tiles per workgroup, which is one
   const long long batch = blockIdx.z;
   long long owner;
   if (!place_problem(p, tail, packed_group, owner)) return;  // whole workgroup, before any barrier
   const bool has_bias = tail.bias != nullptr;
-  tail.bias += owner * tail.stride_bias;
-  tail.y += batch * tail.stride_y;
+  if constexpr (!kChained) {
+    tail.bias += owner * tail.stride_bias;
+    tail.y += batch * tail.stride_y;
+  }
   const int m_batch = tail.m_batch;
 
   const int wg = logical_workgroup(p);
@@ -103,7 +112,11 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   const int lane = threadIdx.x % kWave;
   const int kw = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int split_k = tail.split_k;
-  const PartWork work = part_wave_work(PARTS, wg, kw, p.steps_per_wave, p.ksteps);
+  PartWork work = part_wave_work(PARTS, wg, kw, p.steps_per_wave, p.ksteps);
+  if constexpr (kChained) {
+    work.ks_begin = 0;
+    work.units = p.ksteps;
+  }
   const int slice = lane / kTileRows, column = lane % kTileRows;
   const int k_part = column / kPartRows, row_in_part = column % kPartRows;  // this lane's k step of the unit and its weight row
   const int row0 = work.tile * kTileRows + work.part * kPartRows;
@@ -143,23 +156,23 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     x_rows.v[j] = j < m_batch ? (uint32_t)(j * p.k) * 2u : kPastActivations;
     asm volatile("" : "+s"(x_rows.v[j]));
   }
-  auto request = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& w, int u) {
-    fetch_part_rows<BITS, ROWS, PARTS>(xr, x_rows, p.k, x_rsrc, ks_begin + u * PARTS, lane);
-    load_weights_at<BITS, QOP, GROUPS_PER_RUN, ACT>(w, p, w_rsrc, tables, u * (PARTS * kUnitBytes) + w_lane,
-                                               (ks_begin + u * PARTS + k_part) * G::kStepK + slice * G::kRunK, row);
+  // The unit whose first k step is `kstep` behind the wave's first; past the reduction it reads zeros.
+  auto request = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& w, int kstep) {
+    fetch_part_rows<BITS, ROWS, PARTS>(xr, x_rows, p.k, x_rsrc, ks_begin + kstep, lane);
+    load_weights_at<BITS, QOP, GROUPS_PER_RUN, ACT>(w, p, w_rsrc, tables, kstep * kUnitBytes + w_lane,
+                                               (ks_begin + kstep + k_part) * G::kStepK + slice * G::kRunK, row);
   };
-  request(wa, 0);
   // One unit: the rows on their way go to the stage, the next unit's rows and weights are requested (not behind the last),
   // the unit is computed.  The stage belongs to the wave, and the LDS executes a wave's accesses in order: nothing but the
   // compiler has to be kept from reordering them, and one stage is enough.
-  auto step = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& now, MfmaWeights<BITS, GROUPS_PER_RUN>& next, int u, auto last) {
+  auto step = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& now, MfmaWeights<BITS, GROUPS_PER_RUN>& next, int kstep, int next_kstep, auto last) {
     park_x_rows<BITS, ROWS>(xr, stage, lane, 0, 1);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    if constexpr (!decltype(last)::value) request(next, u + 1);
+    if constexpr (!decltype(last)::value) request(next, next_kstep);
     __builtin_amdgcn_sched_barrier(0);
     half2_t s2 = col_scale;
-    const int k_unit = (ks_begin + u * PARTS) * G::kStepK;
+    const int k_unit = (ks_begin + kstep) * G::kStepK;
     if (k_unit + PARTS * G::kStepK > p.k) {
       // The last unit of the reduction is short.  Activations past it are zero, but an infinite scale or zero times zero is
       // not: what lies past it takes finite ones, of the short form's range.
@@ -177,14 +190,66 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_sched_barrier(0);
   };
-  // whole pairs of units, and a single one behind them (as in the LDS-staged kernel)
-  int u = 0;
-  for (; u + 1 < units; u += 2) {
-    step(wa, wb, u, std::false_type{});
-    step(wb, wa, u + 1, std::false_type{});
+  f32x4* const combine = reinterpret_cast<f32x4*>(lds + split_k * kStageBytes);
+  if constexpr (kChained) {
+    // Chain e of the workgroup: k steps from range e / CHAINS on, every CHAINS * PARTS.  Chains without a unit (the end of the
+    // reduction) and, in the last wave, of no range park zeros.
+    f32x4* park = combine + kw * chains_per_wave * kWave + lane;
+    for (int j = 0; j < chains_per_wave; ++j) park[j * kWave] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int kStride = CHAINS * PARTS;
+    auto first_of = [&](int chain) { return chain / CHAINS * p.steps_per_wave + chain % CHAINS * PARTS; };
+    auto end_of = [&](int chain) {
+      const int end = (chain / CHAINS + 1) * p.steps_per_wave;
+      return end < p.ksteps ? end : p.ksteps;
+    };
+    int chain = kw * chains_per_wave, kstep = first_of(chain), end = end_of(chain);
+    const int past = chain + chains_per_wave;
+    auto find_unit = [&]() {  // from kstep on; past the wave's last: past the reduction
+      while (kstep >= end && chain < past) {
+        ++chain;
+        kstep = chain < past ? first_of(chain) : p.ksteps;
+        end = end_of(chain);
+      }
+    };
+    find_unit();
+    request(wa, kstep);
+    int count = 0;
+    for (int c = kw * chains_per_wave; c < past; ++c) {
+      const int steps = end_of(c) - first_of(c);
+      count += steps > 0 ? (steps + kStride - 1) / kStride : 0;
+    }
+    auto one = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& now, MfmaWeights<BITS, GROUPS_PER_RUN>& next, auto last) {
+      const int here = kstep, chain_here = chain;
+      kstep += kStride;
+      find_unit();
+      step(now, next, here, kstep, last);
+      if (chain != chain_here) {
+        park[(chain_here - (past - chains_per_wave)) * kWave] = acc;
+        acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    };
+    int u = 0;
+    for (; u + 1 < count; u += 2) {
+      one(wa, wb, std::false_type{});
+      one(wb, wa, std::false_type{});
+    }
+    if (u < count) one(wa, wb, std::true_type{});
+  } else {
+    // whole pairs of units, and a single one behind them (as in the LDS-staged kernel)
+    request(wa, 0);
+    int u = 0;
+    for (; u + 1 < units; u += 2) {
+      step(wa, wb, u * PARTS, (u + 1) * PARTS, std::false_type{});
+      step(wb, wa, (u + 1) * PARTS, (u + 2) * PARTS, std::false_type{});
+    }
+    if (u < units) step(wa, wb, u * PARTS, 0, std::true_type{});
   }
-  if (u < units) step(wa, wb, u, std::true_type{});
 
+  if constexpr (kChained) {  // (read again: there are no registers for it in the loop)
+    tail = read_tail_here();
+    tail.bias += owner * tail.stride_bias;
+    tail.y += batch * tail.stride_y;
+  }
   // Lane l holds rows 4 * (l / 16) .. + 3 of the product in column l % 16.  Lane (quad, b) of wave 0 adds up what belongs to
   // rows 4 * quad .. + 3 of the part and batch row b: one entry of every wave and k step of a unit, ascending.
   constexpr int kQuads = kPartRows / 4;
@@ -203,24 +268,24 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     }
   }
   f32x4 sum = acc;
-  if (PARTS > 1 || split_k > 1) {
-    f32x4* const combine = reinterpret_cast<f32x4*>(lds + split_k * kStageBytes);
-    combine[kw * kWave + lane] = acc;
+  if (kChained || PARTS > 1 || split_k > 1) {
+    if constexpr (!kChained) combine[kw * kWave + lane] = acc;
+    const int entries = split_k * chains_per_wave;
     __syncthreads();
     if (!sums) return;
-    // entry of k step pt of wave w: column pt * kPartRows + b of quad pt * kQuads + quad
+    // entry of k step pt of wave (or chain) w: column pt * kPartRows + b of quad pt * kQuads + quad
     const f32x4* part = combine + quad * kTileRows + b;
     constexpr int kEntry = kQuads * kTileRows + kPartRows;
     sum = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     int w = 0;
-    for (; w + 4 <= split_k; w += 4) {
+    for (; w + 4 <= entries; w += 4) {
       f32x4 piece[4 * PARTS];
 #pragma unroll
       for (int i = 0; i < 4 * PARTS; ++i) piece[i] = part[(w + i / PARTS) * kWave + i % PARTS * kEntry];
 #pragma unroll
       for (int i = 0; i < 4 * PARTS; ++i) sum += piece[i];
     }
-    for (; w < split_k; ++w) {
+    for (; w < entries; ++w) {
 #pragma unroll
       for (int i = 0; i < PARTS; ++i) sum += part[w * kWave + i * kEntry];
     }
@@ -239,9 +304,9 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   }
 }
 
-template <int BITS, int QOP, int GPR, int ROWS, int PARTS, int ACT>
+template <int BITS, int QOP, int GPR, int ROWS, int PARTS, int ACT, int CHAINS = 1>
 hipError_t launch_mfma_parts_kernel(const GemvLaunch& g) {
-  const auto kernel = gemv_mfma_parts_kernel<BITS, QOP, GPR, ROWS, PARTS, ACT>;
+  const auto kernel = gemv_mfma_parts_kernel<BITS, QOP, GPR, ROWS, PARTS, ACT, CHAINS>;
   if (g.lds > 48 * 1024) {
     // More than 48 KiB of dynamic LDS has to be granted per kernel and device; remember the
     // largest grant so that only the first such launch pays for the call.
@@ -262,11 +327,16 @@ hipError_t launch_mfma_parts_kernel(const GemvLaunch& g) {
   }
   return launch(kernel, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale, g.zero_add, g.n_out, g.k,
                 pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups, g.tail.num_groups,
-                pack_group(g.group_size, 1, g.tail.stack != nullptr), g.tail);
+                pack_group(g.group_size, CHAINS > 1 ? g.plan.chains_per_wave : 1, g.tail.stack != nullptr), g.tail);
 }
 
 template <int BITS, int QOP, int GPR, int ACT>
 hipError_t launch_mfma_parts_rows(const GemvLaunch& g) {
+  if (g.plan.chains != 0) {
+    if (g.plan.parts == 2) return launch_mfma_parts_kernel<BITS, QOP, GPR, 8, 2, ACT, 2>(g);
+    if (g.plan.staged_rows == 8) return launch_mfma_parts_kernel<BITS, QOP, GPR, 8, 1, ACT, 2>(g);
+    return g.plan.chains == 2 ? launch_mfma_parts_kernel<BITS, QOP, GPR, 4, 1, ACT, 2>(g) : launch_mfma_parts_kernel<BITS, QOP, GPR, 4, 1, ACT, 4>(g);
+  }
   if (g.plan.staged_rows == 8)
     return g.plan.parts == 1 ? launch_mfma_parts_kernel<BITS, QOP, GPR, 8, 1, ACT>(g) : launch_mfma_parts_kernel<BITS, QOP, GPR, 8, 2, ACT>(g);
   switch (g.plan.parts) {
