@@ -1091,7 +1091,8 @@ LaunchResources launch_resources(const LaunchPlan& lp, int bits, int m_batch, in
   r.max_threads = kWave * (rows >= 3 || act == kActBf16 || lp.parts != 0 ? kMaxWavesPerWideWorkgroup : kMaxWavesPerWorkgroup);
   r.lds_bytes = (size_t)lp.tiles_in_sequence * lp.tiles_per_wg * lp.split_k * rows * kWave * sizeof(float);
   if (lp.parts != 0) {  // every unit's sums
-    const int units = lp.split_k * lp.steps_per_wave / lp.parts;
+    int units = lp.split_k * lp.steps_per_wave / lp.parts;
+    if (lp.parts == 1 && units > kValuPartsSumsAtOnce) units = lp.split_k;  // every wave adds up its own
     r.lds_bytes = (size_t)ceil_div(units, kValuPartsSumsAtOnce) * kValuPartsSumsAtOnce * kWave * sizeof(float);
   }
   return r;
@@ -1169,9 +1170,9 @@ int parts_of_batch(int parts, int tiles, int cus, int batch_count) {
 // The plan of a batched or routed launch whose problems would each be split into parts.  Every number of parts gives the same bits, and
 // up to 16 k steps (8 in bf16) so does the kernel for whole tiles, a wave per k step, so the number of problems may count: as
 // many parts as leave a workgroup per compute unit, and where that is not all of them whole tiles, if their kernel gives the bits.
-// Of the time of whole tiles: two problems 0.72-1.0 (2000x12288 int8 1.04, 2048x16384 1.1); three and more 0.99-1.03, 1.05-1.07
-// with 64 tiles and more than 16 k steps (1024x16384, three problems, 7.7 us / 8.3).  With two workgroups per compute unit 1.1-1.5.
-// fp16 in fewer parts up to 16 k steps: 1.0-1.14.
+// Of the time of whole tiles, 1770 launches of two to eight problems: four parts 0.69, two 0.78, one 0.97 (1.13 at worst, 5
+// launches above 1.05, all with four lookups per run).  With two workgroups per compute unit 1.1-1.5.  fp16 in fewer parts up to 16 k
+// steps: 1.0-1.14.
 LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, PlanKnobs knobs, int batch_count) {
   knobs.parts = parts_of_batch(knobs.parts, num_tiles(n_out), knobs.num_cus, batch_count);
   if (knobs.parts == single.parts) return single;

@@ -19,11 +19,12 @@ namespace mgemv {
 // before, in pieces of 16 / PARTS neighbouring chunks.  512x5120, one row, groups of 128 with zeros 3.9 us / 3.1, 1024x16384 7.3 / 5.0
 // (1.8 TB/s); 900x4608 per column in bf16 5.5 / 3.3.  What bounds it: start and end of a launch, then a compute unit's path to
 // memory.
-// PARTS 1, by row broadcast, is for batched launches, which have the bits of single ones (plan_of_batch): the sums of every
-// unit are parked in the LDS and added up in an order of their own.  That costs them 1-3 %, 5-7 where three or four problems leave a workgroup
-// or less to a compute unit.
-// Not taken: eight waves beyond eight units (1.0-1.1 of the time of four); sums kept in registers over a wave's units, which ties
-// the waves of every PARTS to the same k steps (batched launches 1.04-1.3); requests behind a wave's last unit (1.05-1.2, half of
+// PARTS 1, by row broadcast, is for batched launches, which have the bits of single ones (plan_of_batch): the sums of every unit
+// are added up in an order of their own, parked in the LDS up to 16 k steps, beyond by a wave for every fourth k step (LONG).
+// 1224 such launches of two to eight problems take 0.97 of the time of the kernel for whole tiles, 1.0 with four lookups per run (0.57-1.13).
+// (Every sum parked and units in one loop: 1.02, with a lookup per block on 9-16 k steps up to 1.35: 2048x4896 g96 in bf16, six
+// problems, 9.65 us whole, 13.0 so, 9.7 here.)
+// Not taken: eight waves beyond eight units (1.0-1.1 of the time of four); requests behind a wave's last unit (1.05-1.2, half of
 // what a wave of two units issues).
 // ---------------------------------------------------------------------------------------------
 
@@ -118,7 +119,9 @@ __device__ __forceinline__ void compute_part_unit(float& acc, const PartFragment
 }
 
 // blockDim = 64 * split_k.  Dynamic LDS: 64 floats for each unit, units in whole kValuPartsSumsAtOnce.
-template <int BITS, int QOP, int GROUPS_PER_RUN, int PARTS, int ACT>
+// LONG: PARTS 1 and more k steps than kValuPartsSumsAtOnce -- four waves, each every fourth k step, which adds up their sums itself.
+// (PARTS 1 otherwise: waves of one or two units.)
+template <int BITS, int QOP, int GROUPS_PER_RUN, int PARTS, int ACT, bool LONG = false>
 __global__ void __launch_bounds__(kWave * kMaxWavesPerWideWorkgroup)
 gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, const half_t* zero_add, int n_out, int k,
                       uint32_t packed_steps, int workgroups, int num_groups, uint32_t packed_group, GemvTail tail) {
@@ -151,11 +154,13 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   const int slice = lane / kTileRows, k_part = lane % kTileRows / kPartRows, row_in_part = lane % kPartRows;
   const int row0 = work.tile * kTileRows + work.part * kPartRows;
   const int row = row0 + row_in_part < p.n_out ? row0 + row_in_part : p.n_out - 1;  // padding: never stored
-  const int units = (work.units + PARTS - 1) / PARTS;  // >= 1 by the host's geometry
-  const int ks_begin = work.ks_begin;
+  constexpr int kUnitSteps = LONG ? 4 : PARTS;  // k steps from a unit to the next
+  const int ks_begin = LONG ? kw : work.ks_begin;
+  const int wave_steps = LONG ? p.ksteps - kw : work.units;
+  const int units = (wave_steps + kUnitSteps - 1) / kUnitSteps;  // >= 1 by the host's geometry
   const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(
       p.weights + ((size_t)work.tile * (size_t)p.ksteps + (size_t)ks_begin) * (size_t)kUnitBytes,
-      (uint32_t)work.units * (uint32_t)kUnitBytes);  // k steps past the reduction read zeros, and so do their activations
+      (uint32_t)wave_steps * (uint32_t)kUnitBytes);  // k steps past the reduction read zeros, and so do their activations
   const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(p.x, (uint32_t)p.k * 2u);
   ScaleTables tables;
   const uint32_t table_bytes = (uint32_t)num_groups * (uint32_t)p.n_out * 2u;
@@ -169,7 +174,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   if constexpr (GROUPS_PER_RUN != 4) {
     const int shift = __builtin_ctz((unsigned)p.group_size);
     const bool per_column = QOP == MGEMV_PER_COLUMN_SCALE_ONLY;
-    offset_step = per_column ? 0 : PARTS * (G::kStepK >> shift) * p.n_out * 2;
+    offset_step = per_column ? 0 : kUnitSteps * (G::kStepK >> shift) * p.n_out * 2;
 #pragma unroll
     for (int gi = 0; gi < GROUPS_PER_RUN; ++gi)
       first_offset[gi] = ((per_column ? 0 : (k_lane + gi * (G::kRunK / GROUPS_PER_RUN)) >> shift) * p.n_out + row) * 2;
@@ -179,7 +184,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   // A unit past the wave's is sent past every descriptor: such loads come back at once.
   auto request = [&](PartFragment<BITS, GROUPS_PER_RUN, PARTS>& f, int u) {
     const int away = u < units ? 0 : 0x40000000;
-    const int k_run = k_lane + u * (PARTS * G::kStepK);
+    const int k_run = k_lane + u * (kUnitSteps * G::kStepK);
     const int x_voffset = (k_run + lane % (PARTS == 1 ? 16 : 4) * (G::kChunkK / 4)) * 2 + away;
 #pragma unroll
     for (int i = 0; i < f.kXPieces; ++i) {
@@ -201,7 +206,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
     }
 #pragma unroll
     for (int i = 0; i < kBlocksPerUnit; ++i)
-      f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + u * (PARTS * kUnitBytes) + i * kBlockBytes, 0, kCacheStream);
+      f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + u * (kUnitSteps * kUnitBytes) + i * kBlockBytes, 0, kCacheStream);
     __builtin_amdgcn_sched_barrier(0);
   };
   request(fa, 0);
@@ -214,26 +219,31 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   const bool short_ok = (late.flags & kExactIntegerFormOnly) == 0;
   const ConvertRegs c = make_convert_regs();
   float* const my_sums = partials + ks_begin / PARTS * kWave + lane;
+  float so_far = 0.0f;  // LONG
   auto compute = [&](PartFragment<BITS, GROUPS_PER_RUN, PARTS>& f, int u) {
-    const int k_unit = (ks_begin + u * PARTS) * G::kStepK;
+    const int k_unit = (ks_begin + u * kUnitSteps) * G::kStepK;
     if (k_unit + PARTS * G::kStepK > p.k) {
       // The last unit of the reduction is short.  Activations past it are zero, but an infinite scale or zero times zero is
       // not: what lies past it takes finite ones, of the short form's range.
       constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
 #pragma unroll
       for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-        const bool past = k_lane + u * (PARTS * G::kStepK) + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
+        const bool past = k_lane + u * (kUnitSteps * G::kStepK) + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
         f.s[gi] = past ? kAnyScale : f.s[gi];
         f.z[gi] = past ? 0u : f.z[gi];
       }
     }
     float acc = 0.0f;
     compute_part_unit<BITS, QOP, GROUPS_PER_RUN, PARTS, ACT>(acc, f, c, short_ok);
-    my_sums[u * kWave] = acc;
+    if constexpr (LONG) so_far += acc;
+    else my_sums[u * kWave] = acc;
     __builtin_amdgcn_sched_barrier(0);
   };
   int u = 0;
-  if constexpr (GROUPS_PER_RUN == 4) {
+  if constexpr (PARTS == 1 && !LONG) {
+    compute(fa, 0);
+    if (units > 1) compute(fb, 1);
+  } else if constexpr (GROUPS_PER_RUN == 4) {
     // (in the form below 149-183 registers of a bf16 build with zeros, and 1.05-1.2 of the time where workgroups share a compute unit)
     do {
       compute(fa, u);
@@ -255,6 +265,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
     if (u + 1 < units) compute(fb, u + 1);
   }
 
+  if constexpr (LONG) *my_sums = so_far;
   __syncthreads();
   if (kw != 0) return;
   // The order of the sums depends on the number of k steps alone, neither on PARTS nor on the waves, so that a launch of many
@@ -266,7 +277,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   const int l = lane_after_loop();
   constexpr int kAtOnce = kValuPartsSumsAtOnce;
   float sum = 0.0f;
-  if (ksteps <= kAtOnce) {
+  if (PARTS == 1 ? !LONG : ksteps <= kAtOnce) {
     // as the waves of one k step each of the kernel for whole tiles: k steps ascending, then the slices
     const float* part = partials + l / kTileRows * kTileRows + l % kPartRows;
     float piece[kAtOnce];
@@ -279,7 +290,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
     // every fourth k step ascending, the slices, then (0 + 2) + (1 + 3)
     constexpr int kChains = 4 / PARTS;
     float chain[kChains] = {};
-    const int total = (ksteps + PARTS - 1) / PARTS;
+    const int total = LONG ? 4 : (ksteps + PARTS - 1) / PARTS;  // entries
     const float* part = partials + l;
     for (int i = 0; i < total; i += kAtOnce) {
       float piece[kAtOnce];
@@ -306,9 +317,10 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
 
 template <int BITS, int QOP, int GPR, int ACT>
 hipError_t launch_valu_parts_kernel(const GemvLaunch& g) {
-  const auto kernel = g.plan.parts == 1   ? gemv_dpp_parts_kernel<BITS, QOP, GPR, 1, ACT>
+  const auto kernel = g.plan.parts == 4   ? gemv_dpp_parts_kernel<BITS, QOP, GPR, 4, ACT>
                       : g.plan.parts == 2 ? gemv_dpp_parts_kernel<BITS, QOP, GPR, 2, ACT>
-                                          : gemv_dpp_parts_kernel<BITS, QOP, GPR, 4, ACT>;
+                      : num_ksteps(g.k, BITS) > kValuPartsSumsAtOnce ? gemv_dpp_parts_kernel<BITS, QOP, GPR, 1, ACT, true>
+                                                                     : gemv_dpp_parts_kernel<BITS, QOP, GPR, 1, ACT>;
   return launch(kernel, g.grid, g.block, g.lds, g.stream, g.weights, g.x, g.scale, g.zero_add, g.n_out, g.k,
                 pack_steps(num_ksteps(g.k, BITS), g.plan.steps_per_wave), g.plan.workgroups, g.tail.num_groups,
                 pack_group(g.group_size, 1, g.tail.stack != nullptr), g.tail);
