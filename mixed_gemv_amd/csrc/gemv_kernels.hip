@@ -741,6 +741,16 @@ inline int left_over_parts(int m_batch, int tiles, int ksteps, int bits, int cus
   return parts == 4 ? (ksteps <= 10 || ksteps >= 15 ? parts : 0) : walk >= 2 ? parts : 0;
 }
 
+// Several problems: the next one's workgroups fill the place of the shorter walks, so parts pay only where they are a quarter of the
+// compute units or more: 0.96 of the time of whole tiles (0.82-1.06, 157 launches of two to eight problems).  Fewer took 1.03-1.09,
+// up to 1.18 (eight problems of 4232x4608 at 8 rows in bf16 39.0 us / 46.2).  Nor do they in fp16 up to 8 k steps and in bf16 with 5
+// and 8, where the busiest SIMD saves a unit or none: 1.0 (0.92-1.19).
+inline bool left_over_parts_of_batch(int m_batch, int tiles, int ksteps, int cus, bool bf16) {
+  if (bf16 ? ksteps < 6 || ksteps == 8 : ksteps <= 8) return false;
+  const int left_over = tiles % cus, parts = m_batch <= 4 && left_over * 4 <= cus ? 4 : 2;
+  return left_over * parts * 4 >= cus;
+}
+
 LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs& knobs) {
   const int tiles = num_tiles(n_out), ksteps = num_ksteps(k, bits);
   const int cus = knobs.num_cus > 0 ? knobs.num_cus : kNumCus;  // the thresholds below were measured on 256 and scale with it
@@ -1241,6 +1251,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   const int gpr = groups_per_run(group_size, weight_bits);
   // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
   if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
+  if (batch_count > 1 && !left_over_parts_of_batch(m_batch, num_tiles(n_out), num_ksteps(k, weight_bits), info.num_cus, act == kActBf16)) knobs.split_left_over = false;  // the bits are the same
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   if (batch_count > 1 && g.plan.parts != 0 && !g.plan.k_stationary)
     g.plan = m_batch == 1 ? plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count)

@@ -134,3 +134,10 @@ def test_one_group_as_long_as_the_reduction(gpu, n_out, k, rows, qop):
     prob = Problem("one group", n_out, k, 4, qop, k, m_batch=rows, bias=True)
     y = DeviceProblem(prob, gpu).run()
     assert float64_bound_violations(prob, y)[0] == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[1], (288, 8, 0, SCALE_AND_ZEROS, 128, 4, True, "f16", 0), (266, 16, 128, SCALE_ONLY, 128, 4, False, "f16", 4)], ids=str)
+def test_batched_launches_with_few_tiles_left_over_have_the_bits_of_single_ones(gpu, case):
+    """A single launch may take them in parts, a batched one takes whole tiles."""
+    test_batched_and_routed_launches_have_the_bits_of_single_ones(gpu, case)
