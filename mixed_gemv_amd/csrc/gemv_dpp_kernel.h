@@ -376,7 +376,7 @@ __device__ __forceinline__ void timeline_wait(TimelineWaits& t, int u, int total
 // for every further unit; kProbeLoadsOnly keeps every load and replaces the arithmetic of a unit
 // by an exclusive-or over its registers -- what the access pattern alone takes; kProbeTimeline
 // records timestamps and the time spent waiting for loads, per wave.
-// FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead, kOneUnit).
+// FORM: how a wave goes through its units (kUnitLoop, kTwoUnits, kTwoAhead, kOneUnit, kOneUnitFinitePast).
 // EARLY_BIAS: the launch has a bias; it is requested behind the first one or two units (not kUnitLoop).
 template <int BITS, int QOP, int MB, int GROUPS_PER_RUN, bool MULTI, int ACT, int PROBE = kProbeNone, int FORM = kUnitLoop,
           bool EARLY_BIAS = false>
@@ -509,10 +509,12 @@ gemv_dpp_kernel(const uint8_t* weights, const half_t* x, const half_t* scale, co
     // 4260x7296 7.31 / 7.44.)  The loop / this: 1688x17376 g96 9.87 us / 9.32, 2896x10496 int8 7.95 / 7.49, 8192x8192 8.16 /
     //   7.92, 4096x11008 6.67 / 6.54; at 3 rows 2596x3200 int8 5.04 / 4.81; bf16 1324x26752 13.2 / 12.6; 0.97 of the time on 78
     //   launches of random shapes.
-    if constexpr (FORM == kOneUnit) {
+    if constexpr (FORM == kOneUnit || FORM == kOneUnitFinitePast) {
       request_bias();
       __builtin_amdgcn_sched_barrier(0);
       timeline_unit(NoLoadsBehind{}, 0, total);
+      if constexpr (FORM == kOneUnitFinitePast)
+        if ((ks_begin + 1) * Geometry<BITS>::kStepK > p.k) finite_past_reduction<ACT>(fa.s, fa.z, cur.k_run, Geometry<BITS>::kRunK / GROUPS_PER_RUN, p.k);
       compute_unit<BITS, QOP, MB, GROUPS_PER_RUN, ACT, PROBE>(acc, fa, c, short_ok);
     } else if constexpr (FORM == kTwoAhead) {
       auto request = [&](UnitFragment<BITS, MB, GROUPS_PER_RUN>& f) {
@@ -670,7 +672,10 @@ hipError_t launch_gemv_kernel(const GemvLaunch& g) {
     return early_bias ? launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm, MB == 1>(g)
                       : launch_gemv_kernel_m<BITS, QOP, MB, GPR, false, ACT, kForm>(g);
   };
+  if constexpr (MB == 1 && (GPR == 4 || QOP == MGEMV_PER_COLUMN_SCALE_ONLY))
+    if (g.form == kOneUnitFinitePast) return go(std::integral_constant<int, kOneUnitFinitePast>{});
   switch (g.form) {
+    case kOneUnitFinitePast:  // (one and two groups per run read zeros past the tables)
     case kOneUnit: return go(std::integral_constant<int, kOneUnit>{});
     case kTwoUnits: return go(std::integral_constant<int, kTwoUnits>{});
     case kTwoAhead: return go(std::integral_constant<int, kTwoAhead>{});

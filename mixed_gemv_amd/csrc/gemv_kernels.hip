@@ -1253,10 +1253,12 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
   if (batch_count > 1 && !left_over_parts_of_batch(m_batch, num_tiles(n_out), num_ksteps(k, weight_bits), info.num_cus, act == kActBf16)) knobs.split_left_over = false;  // the bits are the same
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
-  if (batch_count > 1 && g.plan.parts != 0 && !g.plan.k_stationary)
+  const bool in_parts = g.plan.parts != 0 && !g.plan.k_stationary;  // a single problem
+  if (batch_count > 1 && in_parts)
     g.plan = m_batch == 1 ? plan_of_batch(g.plan, n_out, k, weight_bits, knobs, batch_count)
                           : plan_of_batch_rows(g.plan, m_batch, num_tiles(n_out), info.num_cus, batch_count);
   g.form = unit_form(g.plan, batch_count, info.num_cus);
+  if (in_parts && g.plan.parts == 0 && g.form == kOneUnit) g.form = kOneUnitFinitePast;
   g.tail.bias = reinterpret_cast<const half_t*>(bias);
   g.tail.split_k = g.plan.split_k;
   g.tail.num_groups = k / group_size;

@@ -223,6 +223,21 @@ __device__ __forceinline__ half2_t splat_low(uint32_t bits) {
   return half2_t{h, h};
 }
 
+// The last k step of a reduction may be short.  Activations past it are zero, but an infinite scale (there the last group's, or the
+// row's) or zero point times zero is not: groups of a lane's run that lie past it take finite ones, of the short form's range.  k_run:
+// first reduction index of the run; group_k: from a group to the next.
+template <int ACT>
+constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
+template <int ACT, int GROUPS>
+__device__ __forceinline__ void finite_past_reduction(uint32_t (&s)[GROUPS], uint32_t (&z)[GROUPS], int k_run, int group_k, int k) {
+#pragma unroll
+  for (int gi = 0; gi < GROUPS; ++gi) {
+    const bool past = k_run + gi * group_k >= k;
+    s[gi] = past ? kAnyScale<ACT> : s[gi];
+    z[gi] = past ? 0u : z[gi];
+  }
+}
+
 struct ScaleTables {
   __amdgpu_buffer_rsrc_t scale, zero;
 };
@@ -335,6 +350,9 @@ constexpr int kUnitLoop = 0;  // any number of them
 constexpr int kTwoUnits = 1;  // one or two, on one tile
 constexpr int kTwoAhead = 2;  // any number, on one tile; the first two are requested together
 constexpr int kOneUnit = 3;   // one, on one tile
+// The same for batched launches whose problems take parts of tiles by themselves: with finite scales past the reduction, as the kernel
+// for parts has them (finite_past_reduction).  A build of its own: kOneUnit with it takes 1.01 of the time of short launches.
+constexpr int kOneUnitFinitePast = 4;
 
 // The build a launch takes.  All four compute the same bits, so the number of problems in a batched or routed launch may
 // count here, which it does not in the plan.  kTwoAhead is for launches of at most one wave per SIMD, all problems taken

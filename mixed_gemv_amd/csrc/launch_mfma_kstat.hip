@@ -287,7 +287,7 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
   const int park_tile_stride = kKSlices * m_batch * slots;  // entries from a tile to the next
   f32x4* my_park = park + (slice * m_batch + m) * slots + kw;
   bool parks = m < m_batch;
-  // The unit of a left-over part: its operand, its scales past the reduction and its entries take the place of the walk's.
+  // The unit of a left-over part: its operand and its entries take the place of the walk's.
   // (Through the loop itself, as one more unit of the walk, bf16 and longer walks lose 1-2 % and short fp16 ones gain as much.)
   auto turn_to_part = [&](MfmaWeights<BITS, GROUPS_PER_RUN>& f) {
     const int l = lane_after_loop(), slice = l / kTileRows, k_part = l % kTileRows / part_rows, row_in_part = l % part_rows;
@@ -310,15 +310,9 @@ gemv_mfma_kstat_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
 #pragma unroll
         for (int j = 0; j < (BITS == 4 ? 4 : 2); ++j) xa.x[i][j] = mfma_operand<BITS>(from, i, j);
     }
-    // Past the reduction the activations are zero, but an infinite scale or zero times zero is not: finite ones of the short form's range.
-    constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
-    const int k_run = kstep * G::kStepK + slice * G::kRunK;
-#pragma unroll
-    for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-      const bool past = k_run + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
-      f.s[gi] = past ? kAnyScale : f.s[gi];
-      f.z[gi] = past ? 0u : f.z[gi];
-    }
+    // K steps that are not there must not make a NaN of an infinite scale.  (In the last one an infinite scale does, where it is short, as in
+    // whole tiles.)
+    finite_past_reduction<ACT>(f.s, f.z, kstep, 0, waves);
     // The product's rows 4 * slice .. + 3 are the part's at one of the unit's k steps; a column is a batch row at one of them.
     const int quads = part_rows / 4;
     parks = slice / quads == k_part && row_in_part < m_batch;

@@ -174,17 +174,9 @@ gemv_mfma_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sc
     half2_t s2 = col_scale;
     const int k_unit = (ks_begin + kstep) * G::kStepK;
     if (k_unit + PARTS * G::kStepK > p.k) {
-      // The last unit of the reduction is short.  Activations past it are zero, but an infinite scale or zero times zero is
-      // not: what lies past it takes finite ones, of the short form's range.
       const int k_run = k_unit + k_part * G::kStepK + slice * G::kRunK;
-      constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
-      s2 = k_run < p.k ? s2 : as_half2(kAnyScale | kAnyScale << 16);
-#pragma unroll
-      for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-        const bool past = k_run + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
-        now.s[gi] = past ? kAnyScale : now.s[gi];
-        now.z[gi] = past ? 0u : now.z[gi];
-      }
+      s2 = k_run < p.k ? s2 : as_half2(kAnyScale<ACT> | kAnyScale<ACT> << 16);
+      finite_past_reduction<ACT>(now.s, now.z, k_run, G::kRunK / GROUPS_PER_RUN, p.k);
     }
     compute_unit_mfma<BITS, QOP, GROUPS_PER_RUN, ACT>(acc, now, xa, c, s2, short_ok);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -223,15 +223,7 @@ gemv_dpp_parts_kernel(const uint8_t* weights, const half_t* x, const half_t* sca
   auto compute = [&](PartFragment<BITS, GROUPS_PER_RUN, PARTS>& f, int u) {
     const int k_unit = (ks_begin + u * kUnitSteps) * G::kStepK;
     if (k_unit + PARTS * G::kStepK > p.k) {
-      // The last unit of the reduction is short.  Activations past it are zero, but an infinite scale or zero times zero is
-      // not: what lies past it takes finite ones, of the short form's range.
-      constexpr uint32_t kAnyScale = ACT == kActBf16 ? 0x3c00u : 0x2000u;  // 2^-7
-#pragma unroll
-      for (int gi = 0; gi < GROUPS_PER_RUN; ++gi) {
-        const bool past = k_lane + u * (kUnitSteps * G::kStepK) + gi * (G::kRunK / GROUPS_PER_RUN) >= p.k;
-        f.s[gi] = past ? kAnyScale : f.s[gi];
-        f.z[gi] = past ? 0u : f.z[gi];
-      }
+      finite_past_reduction<ACT>(f.s, f.z, k_lane + u * (kUnitSteps * G::kStepK), G::kRunK / GROUPS_PER_RUN, p.k);
     }
     float acc = 0.0f;
     compute_part_unit<BITS, QOP, GROUPS_PER_RUN, PARTS, ACT>(acc, f, c, short_ok);

@@ -141,3 +141,25 @@ def test_one_group_as_long_as_the_reduction(gpu, n_out, k, rows, qop):
 def test_batched_launches_with_few_tiles_left_over_have_the_bits_of_single_ones(gpu, case):
     """A single launch may take them in parts, a batched one takes whole tiles."""
     test_batched_and_routed_launches_have_the_bits_of_single_ones(gpu, case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[2], CASES[8], CASES[10], (576, 6, 128, PER_COLUMN, 0, 3, True, "bf16", 4),
+                                  (257, 9, 0, PER_COLUMN, 0, 4, False, "bf16", 4), (288, 16, 256, PER_COLUMN, 0, 4, False, "f16", 4)], ids=str)
+def test_infinities_are_those_of_whole_tiles(gpu, case):
+    """Infinite scales of the last group (of the column): an output is infinite or not a number in a part where it is in a whole tile,
+    the oracle's where the last k step is whole."""
+    prob = problem(case)
+    prob.q[:] = np.abs(prob.q.astype(np.int16)).clip(1, 7)
+    from oracle import pack_int4
+    prob.w_raw = pack_int4(prob.q)
+    prob.scale[-1, ::5] = 0x7F80 if prob.element == "bf16" else np.inf
+    prob.x[:] = 0x3F80 if prob.element == "bf16" else 1.0
+    inf = 0x7F80 if prob.element == "bf16" else 0x7C00
+    special = lambda y: np.where((y.view(np.uint16) & 0x7FFF) > inf, 2, np.where((y.view(np.uint16) & 0x7FFF) == inf, 1, 0))  # noqa: E731
+    dev = DeviceProblem(prob, gpu)
+    got = dev.run().copy()
+    whole = on_whole_tiles(lambda: dev.run().copy())
+    assert (special(got)[:, ::5] > 0).all() and np.array_equal(special(whole), special(got))
+    if prob.k % 512 == 0:
+        assert np.array_equal(special(got), special(prob.oracle_gemv(threads=16).reshape(got.shape)))
