@@ -836,8 +836,7 @@ LaunchPlan plan_launch(int n_out, int k, int bits, int m_batch, const PlanKnobs&
       // what such a launch waits for is a compute unit's path to memory, not latency, and 8 take 1.0-1.08 times as long
       // (bf16 on up to 64 tiles 0.97-1.0).
       const int units = ceil_div(ksteps, lp.parts);
-      const int waves = ov_sk > 0 ? (ov_sk < kMaxWavesPerMfmaWorkgroup ? ov_sk : kMaxWavesPerMfmaWorkgroup) : units <= kMaxWavesPerMfmaWorkgroup ? units : 4;
-      const int units_per_wave = ceil_div(units, waves < units ? waves : units);
+      const int units_per_wave = ceil_div(units, units <= kMaxWavesPerMfmaWorkgroup ? units : 4);
       lp.steps_per_wave = units_per_wave * lp.parts;
       lp.split_k = ceil_div(units, units_per_wave);
       lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);

@@ -336,7 +336,7 @@ struct LaunchPlan {
   int tiles_per_wave;  // 1 on the VALU path; 1, 2 or 4 on the matrix-core path
   int tiles_in_sequence;  // VALU path: most tiles any wave walks one after the other
   int staged_rows;        // LDS-staged and part-tile matrix-core kernels: 8 or 16 activation rows per stage; 0 = other kernels
-  int parts;              // part-tile kernels: workgroups per tile (1, 2 or 4; VALU: 2 or 4); 0 = other kernels
+  int parts;              // part-tile kernels: workgroups per tile (1, 2 or 4; VALU: 1 in batched launches only); 0 = other kernels
                           // k-stationary kernel: workgroups per tile left over (2 or 4); 0 = walks of whole tiles
   int chains, chains_per_wave;  // part-tile matrix-core kernel, batched launches in fewer parts than a single one (else 0): the single
                           // launch's parts are parts * chains, split_k waves take chains_per_wave chains of units each

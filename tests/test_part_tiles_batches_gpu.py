@@ -58,3 +58,27 @@ def test_the_bits_of_single_launches(gpu, case):
         for i in range(count - 1):
             assert np.array_equal(got[i], single[(2 * i + 1) % 3, i]), (count, i)
         assert (got[count - 1:] == 0x7E00).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_out, k, rows, element", [(996, 17000, 4, "f16"), (1020, 9000, 3, "bf16"), (2000, 9000, 6, "f16")])
+def test_infinite_columns_where_a_run_lies_partly_past_the_reduction(gpu, n_out, k, rows, element):
+    """Per-column scales: those rows' outputs are infinite or not a number, the same ones however many problems, the others finite."""
+    import torch
+    assert mg.query_launch(n_out, rows, k, 4, k, element=element, num_compute_units=256)["workgroups"] > 2 * (n_out // 16) - 8
+    prob = Problem("infinite columns", n_out, k, 4, PER_COLUMN, 0, m_batch=rows, element=element)
+    prob.scale[0, ::5] = 0x7F80 if element == "bf16" else np.inf
+    inf = 0x7F80 if element == "bf16" else 0x7C00
+    special = lambda y: np.where((y & 0x7FFF) > inf, 2, np.where((y & 0x7FFF) == inf, 1, 0))  # noqa: E731
+    dev = DeviceProblem(prob, gpu)
+    single = dev.run().copy().view(np.uint16).reshape(rows, n_out)
+    assert (special(single)[:, ::5] > 0).all() and (np.delete(special(single), np.s_[::5], axis=1) == 0).all()
+    w, scale, x = (torch.stack([t] * 6) for t in (dev.w, dev.scale, dev.x))
+    strides = (w[0].numel(), rows * k, n_out, 0, rows * n_out)
+    for count in (2, 3, 6):
+        y = torch.full((6, rows, n_out), 0x7E01, dtype=torch.int16, device=gpu)
+        mg.device_gemv(w, x, scale, None, None, y, count, n_out, rows, k, k, PER_COLUMN, 4, batch_strides=strides, element=element)
+        torch.cuda.synchronize()
+        for got in y.cpu().numpy().view(np.uint16)[:count]:
+            assert np.array_equal(special(got), special(single)), count
+            assert np.array_equal(got[special(got) < 2], single[special(got) < 2]), count
