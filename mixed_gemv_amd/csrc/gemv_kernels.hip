@@ -1195,8 +1195,9 @@ LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, P
 }
 
 // The same for two and more rows on the part-tile matrix-core kernel, in the order of the single launch's sums (CHAINS).  Whole
-// chains to eight waves where all problems leave a compute unit to each workgroup, else to four: eight there 1.0-1.2 of the
-// time, two 1.1-1.5 (and level from 2 workgroups per compute unit on).
+// chains to up to eight waves where all problems leave a compute unit to each workgroup, else to four: eight there 1.0-1.2 of
+// the time, two 1.1-1.5 (and level from 2 workgroups per compute unit on).  As many of them as leave the busiest SIMD the fewest
+// chains: twelve on six waves are four, on four waves three (five problems of 800x5456 at 5 rows 8.6 us / 7.2).
 // Two to eight problems of at most half as many tiles as compute units, 1445 launches of random shapes, of the time of the
 // kernels that were there before parts: 0.89 (39 of them above 1.1, worst 1.26; 2 rows 0.93, 3 and 4 0.84, 5-8 0.93), where the
 // single launch's parts took up to 2.2 (eight problems of 1024x9344 at 3 rows in bf16 14.1 us before, 30.8 in four parts each, 12.3
@@ -1207,8 +1208,15 @@ LaunchPlan plan_of_batch_rows(const LaunchPlan& single, int m_batch, int tiles, 
   if (lp.parts == single.parts) return single;
   lp.chains = single.parts / lp.parts;
   lp.workgroups = tiles * lp.parts;
-  const int chains = single.split_k * lp.chains, waves = (long long)lp.workgroups * batch_count <= cus ? kMaxWavesPerMfmaWorkgroup : 4;
-  lp.chains_per_wave = ceil_div(chains, waves);
+  const int chains = single.split_k * lp.chains, most_waves = (long long)lp.workgroups * batch_count <= cus ? kMaxWavesPerMfmaWorkgroup : 4;
+  int least = chains;  // of the busiest SIMD
+  for (int waves = most_waves; waves >= 4; --waves) {
+    const int per_wave = ceil_div(chains, waves), simd = ceil_div(ceil_div(chains, per_wave), 4) * per_wave;
+    if (simd < least || waves == most_waves) {
+      least = simd;
+      lp.chains_per_wave = per_wave;
+    }
+  }
   lp.split_k = ceil_div(chains, lp.chains_per_wave);
   lp.staged_rows = lp.parts * m_batch <= 4 && lp.parts == 1 ? 4 : 8;
   lp.wgs_per_xcd = ceil_div(lp.workgroups, kNumXcd);
