@@ -716,8 +716,9 @@ inline size_t kstat_stage_bytes(int waves, int bits, int m_batch, bool bf16, int
 // often.  Part of the built-in measured plans.  Of the time of whole tiles, same kernel, 1300 launches of random shapes:
 //   bf16 walks of 1 / 2 / 3: four parts 0.93 / 0.92 / 0.95 (9 k steps 0.87; 5004x5280 g96 at 3 rows 9.7 us / 8.8, 9104x5632 at 3 rows
 //     12.5 / 11.5), two parts 0.97 / 0.93 / 0.96 (14-16 k steps on other walks than 2: 0.99-1.01, left out);
-//   fp16: four parts 0.93-0.96 (4608x8192 at 4 rows 9.4 / 8.6; 11-14 k steps 0.98-1.02, left out), two parts on walks of 2 and 3
-//     0.94 / 0.97 (9104x8192 at 4 rows 13.1 / 11.2), on walks of 1 1.0.
+//   fp16, from 9 k steps: four parts 0.90-0.99 (4608x8192 at 4 rows 9.4 / 8.6; 11-14 k steps 0.98-1.02, left out), two parts on walks
+//     of 2 and 3 0.94-0.97 / 0.97-0.99 (9104x8192 at 4 rows 13.1 / 11.2), on walks of 1 1.0.  5 and 6 k steps take 1.03-1.07 on 180
+//     launches (9700x2440 at 7 rows 5.7 / 6.0): a part's unit in code nobody has fetched yet is longer than the two short ones saved.
 // Longer walks and one unit saved: 0.98-1.1.  int8, whose rows are half as long, 1.03-1.15; four lookups per run in fp16 have
 // no registers for it.
 inline int left_over_parts(int m_batch, int tiles, int ksteps, int bits, int cus, bool bf16, bool generic_groups) {
@@ -737,16 +738,16 @@ inline int left_over_parts(int m_batch, int tiles, int ksteps, int bits, int cus
     if (ksteps == 8) return parts;
     return saved >= 2 && (walk < 3 || ksteps != 12) && (parts == 4 || ksteps <= 13 || walk == 2) ? parts : 0;
   }
-  if (saved < 2) return 0;
+  if (saved < 2 || ksteps < 9) return 0;
   return parts == 4 ? (ksteps <= 10 || ksteps >= 15 ? parts : 0) : walk >= 2 ? parts : 0;
 }
 
 // Several problems: the next one's workgroups fill the place of the shorter walks, so parts pay only where they are a quarter of the
 // compute units or more: 0.96 of the time of whole tiles (0.82-1.06, 157 launches of two to eight problems).  Fewer took 1.03-1.09,
-// up to 1.18 (eight problems of 4232x4608 at 8 rows in bf16 39.0 us / 46.2).  Nor do they in fp16 up to 8 k steps and in bf16 with 5
-// and 8, where the busiest SIMD saves a unit or none: 1.0 (0.92-1.19).
-inline bool left_over_parts_of_batch(int m_batch, int tiles, int ksteps, int cus, bool bf16) {
-  if (bf16 ? ksteps < 6 || ksteps == 8 : ksteps <= 8) return false;
+// up to 1.18 (eight problems of 4232x4608 at 8 rows in bf16 39.0 us / 46.2).  Nor do they with 5 and 8 k steps, where the busiest SIMD
+// saves a unit or none: 1.0 (0.92-1.19).
+inline bool left_over_parts_of_batch(int m_batch, int tiles, int ksteps, int cus) {
+  if (ksteps < 6 || ksteps == 8) return false;
   const int left_over = tiles % cus, parts = m_batch <= 4 && left_over * 4 <= cus ? 4 : 2;
   return left_over * parts * 4 >= cus;
 }
@@ -1258,7 +1259,7 @@ int gemv_any(const void* weights, const uint16_t* x, const uint16_t* scale, cons
   const int gpr = groups_per_run(group_size, weight_bits);
   // The plan takes a group as long as k for the per-column mode; with scales or zeros by group such a launch may look up four.
   if (!kstat_has_left_over_parts(weight_bits, quant_op == MGEMV_PER_COLUMN_SCALE_ONLY ? 1 : gpr, act)) knobs.split_left_over = false;
-  if (batch_count > 1 && !left_over_parts_of_batch(m_batch, num_tiles(n_out), num_ksteps(k, weight_bits), info.num_cus, act == kActBf16)) knobs.split_left_over = false;  // the bits are the same
+  if (batch_count > 1 && !left_over_parts_of_batch(m_batch, num_tiles(n_out), num_ksteps(k, weight_bits), info.num_cus)) knobs.split_left_over = false;  // the bits are the same
   g.plan = plan_launch(n_out, k, weight_bits, m_batch, knobs);
   const bool in_parts = g.plan.parts != 0 && !g.plan.k_stationary;  // a single problem
   if (batch_count > 1 && in_parts)

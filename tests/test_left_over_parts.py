@@ -64,6 +64,12 @@ def test_whole_tiles_where_parts_do_not_pay(tiles, ksteps, rows, element, bits):
     assert plan["matrix_core"] != 3 or cover["max_units_per_wave"] == -(-tiles // plan["workgroups"]), (plan, cover)
 
 
+@pytest.mark.parametrize("tiles, ksteps, rows", [(607, 5, 7), (574, 5, 4), (312, 6, 4), (518, 6, 3), (816, 6, 4)])
+def test_short_fp16_reductions_walk_whole_tiles(tiles, ksteps, rows):
+    for k in (512 * ksteps, 512 * ksteps - 128):
+        assert not covered_in_parts(16 * tiles, rows, k, 4, 128, "f16")
+
+
 def problem(case, buffer=0):
     n_out, k = shape(case)
     tiles, ksteps, short, qop, group, rows, bias, element, parts = case
