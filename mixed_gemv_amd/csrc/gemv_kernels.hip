@@ -303,7 +303,7 @@ inline int lookups_per_run(int k, int group_size, int bits) {
 // A lookup per block, half a tile to one tile per compute unit, 9-16 k steps, both types: eight waves of one or two units instead of four of
 //   three and four: both are requested at once, and nine k steps on four waves are 3 + 3 + 3 and a SIMD idle.  int4 0.92 of the time
 //   (0.74-1.04) on 185 (4096x8064 g96 6.37 / 6.16, in bf16 8.25 / 7.79), int8 0.86 (0.75-0.94) on 63 (3072x3072 g96 4.65 / 4.37); two to
-//   six problems 0.89-1.0.  Longer reductions take 0.85-0.96 alone and 1.05-1.2 in batched launches, with one or two lookups 0.9-1.2.
+//   six problems 0.87-0.98, eight 0.93, but bf16 int4 1.03, up to 1.15.  Longer reductions take 0.85-0.96 alone and 1.05-1.2 in batched launches, with one or two lookups 0.9-1.2.
 // bf16, 1.5 to 2 tiles per compute unit and longer reductions: four waves per tile instead of pairs of tiles with two each, which leave a wave
 //   alone on every SIMD they have and some without one.  A lookup per block, from 18 k steps (17, as fast, is held by a launch test): 0.88 of the time (0.81-0.96) on 70 (8192x23040 g96
 //   33.2 / 30.4, int8 8192x16224 g96 33.9 / 28.8); int4 otherwise, from 25: 0.92 (0.74-1.03) on 130 (8192x27904 32.8 / 31.0, 8192x21248
@@ -1200,7 +1200,7 @@ LaunchPlan plan_of_batch(const LaunchPlan& single, int n_out, int k, int bits, P
 // the time, two 1.1-1.5 (and level from 2 workgroups per compute unit on).  As many of them as leave the busiest SIMD the fewest
 // chains: twelve on six waves are four, on four waves three (five problems of 800x5456 at 5 rows 8.6 us / 7.2).
 // Two to eight problems of at most half as many tiles as compute units, 1445 launches of random shapes, of the time of the
-// kernels that were there before parts: 0.89 (39 of them above 1.1, worst 1.26; 2 rows 0.93, 3 and 4 0.84, 5-8 0.93), where the
+// kernels that were there before parts: 0.89 (41 of them above 1.1, worst 1.26; 2 rows 0.93, 3 and 4 0.84, 5-8 0.93), where the
 // single launch's parts took up to 2.2 (eight problems of 1024x9344 at 3 rows in bf16 14.1 us before, 30.8 in four parts each, 12.3
 // here; of 2048x4352 at 8 rows 11.8, 24.5, 12.0).  Two rows of short reductions gain least: the VALU kernel had them.
 LaunchPlan plan_of_batch_rows(const LaunchPlan& single, int m_batch, int tiles, int cus, int batch_count) {

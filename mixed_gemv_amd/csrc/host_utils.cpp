@@ -13,6 +13,7 @@ namespace {
 // The loops below are written on vectors and compiled three times: for any x86-64 (SSE2), for AVX2 and for AVX-512; the
 // processor says which one runs.  Called from Python on 16 threads of an EPYC, SSE2 / AVX-512: a 4096x4096 int4 matrix laid out
 // 54 us / 24, packed 27 / 17, 131072 zero points folded 15.5 / 11 (most of it the call and the threads); the three together 113 / 63.
+// (New inputs with every result kept, as loading a model has it: 515-645 us / 475-535, most of it page faults of the results.)
 // A loop is a class whose run<W> takes the variant's vector of 32-bit words and is inlined into a function of that variant.
 #if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
 #define MGEMV_FOR(isa) __attribute__((target(isa)))
